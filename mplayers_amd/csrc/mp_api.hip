@@ -1105,33 +1105,31 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
   p.L = s->n_disp;
   p.ctx2d = s->ctx2d ? 1 : 0;
   p.rho = rho;
-  p.a_out = dunary;
   p.h = dmsg;
   p.edge = edge_weights;
   p.ctx = context;
   p.dedge = dedge_weights;
   p.dctx = dcontext;
   p.same_label = (flags & MPL_F_DCONTEXT_SAME_LABEL) ? 1 : 0;
-  bool first = true;
+  const float* a_cur = dcost_final;  // CostAggregateKernelBack: every g_k starts as dcost
   for (int it = n_iter - 1; it >= 0; --it) {
     for (int d = s->n_dir - 1; d >= 0; --d) {  // TRWP_backward.cu:337-424
       fill_dirs(s, d, 1, p.dirs, p.block_prefix, &p.n_dirs);
       p.pack = decide_pack(s, p, opts);
-      p.a_in = first ? dcost_final : dunary;  // CostAggregateKernelBack: every g_k starts as dcost
-      p.first_touch = (it == n_iter - 1) && (d & 1);
-      p.inv_from_a = (d & 1) ? 0 : 1;  // the launch before an even direction swept d + 1 = d ^ 1
-      // in the last iteration walked (it == 0) the even sweeps leave h planes nobody reads again
-      p.skip_hd_store = ((d & 1) || it == 0) ? 1 : 0;
-      p.skip_hi_store = (!(d & 1) && it == 0) ? 1 : 0;
+      p.a_in = a_cur;
+      float* const plane_e = dmsg + (int64_t)(d & ~1) * N;
+      p.a_out = (it == 0 && d <= 1) ? dunary : plane_e;
+      p.first_touch = (it == n_iter - 1) ? 1 : 0;
+      // in the last iteration walked the even sweeps leave h planes nobody reads again
+      p.skip_h_store = (it == 0) ? 1 : 0;
       p.idx_min = msg_min_index + (int64_t)it * s->n_dir * N;
       p.idx_norm = msg_norm_index + (int64_t)it * s->n_dir * P;
       // few chains: the wavefront of a chain walks d (odd) and then d - 1 (same pixels, reversed)
       p.fused_pair = (opts.fused_pairs && (d & 1) &&
                       launch_waves(p) <= launch_policy().fused_pair_max_waves) ? 1 : 0;
-      p.skip_h2 = (it == 0) ? 1 : 0;
       launch_bwd(p, false, st);
-      first = false;
       if (p.fused_pair) --d;
+      if (!(d & 1)) a_cur = p.a_out;
     }
   }
   return launch_ok("trwp_backward");

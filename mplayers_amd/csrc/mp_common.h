@@ -502,16 +502,15 @@ struct BackParams {
   int dirs[kMaxDirs];
   int block_prefix[kMaxDirs + 1];
   float rho;
-  // TRWP: g_k = A + h_k.  a_in: plane read as A (dcost_final on the first sweep), a_out: dunary.
+  // TRWP: g_k = A + h_k (mp_bwd.hip).  a_in: the plane both walks of a pair read as A (dcost_final, or
+  // what the even walk of the pair before stored); a_out: where the even walk stores A (plane e of
+  // h, at the end of the call dunary).  Soft TRWP: a_in is dcost_final or dunary, a_out dunary.
   const float* a_in;
   float* a_out;
   float* h;                 // (n_dir_total, N) planes h_k
-  int first_touch;          // h_dir and h_inv have not been written yet: read as zero
-  int inv_from_a;           // h_inv == -A (the previous launch swept the opposite direction)
-  int skip_hd_store;        // h_dir is not read again before it is overwritten (or ever)
-  int skip_hi_store;        // h_inv is never read again (last sweeps of the backward pass)
+  int first_touch;          // this pair's planes of h have not been written yet: read as zero
+  int skip_h_store;         // even walk: nobody reads h_o after it (last iteration walked)
   int fused_pair;           // Gauss-Seidel: every wavefront walks dirs[0] (odd), then dirs[0] ^ 1
-  int skip_h2;              // that second walk stores neither h plane (last iteration walked)
   // ISGMR: gu_in planes (plane stride gu_stride; 0 on the first iteration where gu_k = dcost_final),
   // du_out (n_dir_total, N) receives dU_d in place of gu_d
   const float* gu_in;

@@ -415,31 +415,23 @@ __global__ void __launch_bounds__(kWave) packed_bwd_kernel(const BackParams p) {
 #pragma clang loop unroll(disable)
   for (int half = 0; half < halves; ++half) {
   PackedChains ch = ch0;
-  bool first_touch = p.first_touch != 0, inv_a = p.inv_from_a != 0;
-  bool skip_hd_store = p.skip_hd_store != 0, skip_hi_store = p.skip_hi_store != 0;
-  const float* a_in = p.a_in;
   if (half) {
     ch.dir = ch0.dir ^ 1;
     ch.pix0 = ch0.pix0 + (ch0.n - 1) * ch0.pstep;
     ch.pstep = -ch0.pstep;
-    first_touch = false;
-    inv_a = true;
-    skip_hd_store = skip_hi_store = p.skip_h2 != 0;
-    a_in = p.a_out;
     wait_vmem<0>();
     __syncthreads();
   }
   const int dir = ch.dir;
-  const bool read_h = !JACOBI && !first_touch;
-  const bool inv_from_a = !JACOBI && inv_a;
+  // (which planes the two walks of a pair read and store: mp_bwd.hip)
+  const bool even = !JACOBI && (dir & 1) == 0;
   const int gdir = p.gu_pair_share ? (dir & ~1) : dir;
-  const rsrc_t dA = make_rsrc(JACOBI ? p.gu_in + (int64_t)gdir * p.gu_stride : a_in, plane_bytes);
-  const rsrc_t dAo = make_rsrc(JACOBI ? p.du_out + (int64_t)dir * N : p.a_out, plane_bytes);
+  const rsrc_t dA = make_rsrc(JACOBI ? p.gu_in + (int64_t)gdir * p.gu_stride : p.a_in, plane_bytes);
   float* hbase = JACOBI ? p.du_out : p.h;
-  const rsrc_t dHdIn = make_rsrc(hbase + (int64_t)dir * N, read_h ? plane_bytes : 0);
-  const rsrc_t dHiIn = make_rsrc(hbase + (int64_t)(dir ^ 1) * N, (read_h && !inv_from_a) ? plane_bytes : 0);
-  const rsrc_t dHdOut = make_rsrc(hbase + (int64_t)dir * N, (JACOBI || skip_hd_store) ? 0 : plane_bytes);
-  const rsrc_t dHiOut = make_rsrc(hbase + (int64_t)(dir ^ 1) * N, (JACOBI || skip_hi_store) ? 0 : plane_bytes);
+  const rsrc_t dAo = make_rsrc(even ? p.a_out : hbase + (int64_t)dir * N, plane_bytes);
+  const rsrc_t dHdIn = make_rsrc(hbase + (int64_t)dir * N, (!JACOBI && !p.first_touch) ? plane_bytes : 0);
+  const rsrc_t dHiIn = make_rsrc(hbase + (int64_t)(dir ^ 1) * N, even ? plane_bytes : 0);
+  const rsrc_t dHiOut = make_rsrc(hbase + (int64_t)(dir ^ 1) * N, (even && !p.skip_h_store) ? plane_bytes : 0);
   const rsrc_t dImin = make_rsrc(p.idx_min + (int64_t)dir * N, (int)N);
   const rsrc_t dInorm = make_rsrc(p.idx_norm + (int64_t)dir * P, (int)P);
   const rsrc_t dW = make_rsrc(p.edge + (int64_t)dir * P, (int)(P * 4));
@@ -459,8 +451,7 @@ __global__ void __launch_bounds__(kWave) packed_bwd_kernel(const BackParams p) {
     r.a = ldf(dA, eo);
     if (!JACOBI) {
       r.hd = ldf(dHdIn, eo);
-      r.hi = ldf(dHiIn, eo);
-      if (inv_from_a) r.hi = -r.a;
+      r.hi = ldf(dHiIn, eo);  // (odd walk: reads as zero)
     } else {
       r.hd = r.hi = 0.f;
     }
@@ -477,7 +468,7 @@ __global__ void __launch_bounds__(kWave) packed_bwd_kernel(const BackParams p) {
     return r;
   };
 
-  constexpr int kOps = (JACOBI ? 1 : 3) + 3 + (DE ? 1 : 0) + (JACOBI ? 1 : 3) + (DE ? 1 : 0);
+  constexpr int kOps = (JACOBI ? 1 : 3) + 3 + (DE ? 1 : 0) + (JACOBI ? 1 : 2) + (DE ? 1 : 0);
   constexpr int D = ring_depth(kOps);
   PixPB ring[D];
 #pragma unroll
@@ -500,7 +491,9 @@ __global__ void __launch_bounds__(kWave) packed_bwd_kernel(const BackParams p) {
       ring[u] = load_next();
       // gradient w.r.t. the normalised message of this pixel (none at the chain start, t == 0)
       const bool edge = on && t >= 1;
-      float g = edge ? fmaf(rho, sc, JACOBI ? px.a : px.a + px.hd) : 0.f;
+      const float ap = even ? fmaf(rho, px.hi, px.a) : px.a;
+      const float base = JACOBI ? px.a : ap + (even ? -px.hd - px.hi : px.hd);
+      float g = edge ? fmaf(rho, sc, base) : 0.f;
       const float tot = seg_sum<NQ, EXACT>(xs, sg, g);  // MsgNormNaiveBack, commonCUDA.cuh:131-145
       if (edge && l == px.nidx) g -= tot;
       const int fd = px.fd;
@@ -532,10 +525,8 @@ __global__ void __launch_bounds__(kWave) packed_bwd_kernel(const BackParams p) {
       if (JACOBI) {
         stf(dAo, eo, sc);
       } else {
-        const float an = fmaf(rho, sc, px.a);  // g_k += rho * dU for every k, dunary too
-        stf(dAo, eo, an);
-        stf(dHdOut, eo, -an);          // g_dir = 0 after its sweep
-        stf(dHiOut, eo, px.hi - sc);   // g_inv -= dU
+        stf(dAo, eo, even ? fmaf(rho, sc, ap) : sc);
+        stf(dHiOut, eo, -ap - sc);
       }
       if (DE)
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, px.de + det), dDe,

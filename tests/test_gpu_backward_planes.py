@@ -1,0 +1,34 @@
+"""TRWP backward: the planes the walks of a pair hand to each other and to the next pair.
+
+The two walks of a pair of opposite directions pass on three planes, and the plane a pair reads as
+A is the one the pair before it left in its even direction's slot; the number of pairs, of iterations
+and the way the walks are launched decide which slot that is.  Random argmin labels (any label is a
+valid one) against the fp64 oracle, scratch filled with garbage."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("L", [5, 21, 96, 131, 192])
+@pytest.mark.parametrize("n_dir,n_iter", [(2, 1), (2, 3), (4, 1), (4, 2), (8, 2), (16, 1)])
+def test_planes_of_the_pairs(gpu, oracle, n_dir, n_iter, L):
+  from mplayers_amd import _lib
+  rng = np.random.default_rng(100 * L + 10 * n_dir + n_iter)
+  B, H, W = 2, 9, 37
+  ctx = (np.triu(rng.random((L, L)), 1) if L == 21 else rng.random(L)).astype(np.float32)
+  ew = (0.1 + 0.9 * rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
+  imin = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W, L)).astype(np.uint8)
+  inorm = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W)).astype(np.uint8)
+  ref = oracle.backward("TRWP", ctx.astype(np.float64), ew.astype(np.float64), dcost.astype(np.float64),
+                        imin, inorm, 0.5)
+  routes = [0, _lib.F_FUSED_PAIRS_OFF]
+  if L <= 32:
+    routes += [_lib.F_PACKED_ALWAYS, _lib.F_PACKED_ALWAYS | _lib.F_FUSED_PAIRS_OFF]
+  for flags in routes:
+    print("case", L, n_dir, n_iter, flags, flush=True)
+    got = gpu.gpu_backward("TRWP", ctx, ew, dcost, imin, inorm, 0.5, flags=flags, garbage_scratch=True)
+    for name, g, r in zip(("dunary", "dcontext", "dedge"), got, ref):
+      # the gradient bar of the GPU tests: 1e-4 of the largest entry
+      assert np.abs(g.reshape(r.shape) - r).max() <= 1e-4 * max(1.0, np.abs(r).max()), (name, flags)
