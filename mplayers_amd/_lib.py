@@ -95,6 +95,7 @@ OPT_FUSED_U = 1
 OPT_BELIEF_REBUILD = 2
 OPT_CPU_THREADS = 3
 OPT_DENSE_SPLIT_WAVES = 4
+OPT_TEAM_SCANS = 5
 BELIEF_REBUILD_DEFAULT = -1
 
 

@@ -562,6 +562,7 @@ int labels_per_lane(int L) { return (L + kWave - 1) / kWave; }
 std::atomic<int> g_packed_scans{1};  // MPL_OPT_PACKED_SCANS: 0 off, 1 by chain count, 2 always
 std::atomic<int> g_fused_u{1};       // MPL_OPT_FUSED_U
 std::atomic<int> g_belief_rebuild{MPL_BELIEF_REBUILD_DEFAULT};  // MPL_OPT_BELIEF_REBUILD
+std::atomic<int> g_team_scans{1};    // MPL_OPT_TEAM_SCANS: 0 never, 1 launches with few chains, 2 always
 std::atomic<int> g_split_waves{0};   // MPL_OPT_DENSE_SPLIT_WAVES: 0 = by the model of choose_split
 
 // what one call does, from its flags and the process defaults
@@ -594,6 +595,14 @@ int decide_pack(const mpl_shape* s, const Params& p, const CallOpts& o) {
   const int G = packed_chains_per_wave(s->batch, s->height, s->width, s->n_disp, s->ctx2d != 0,
                                        p.block_prefix[p.n_dirs], o.packed == 2);
   return G >= 2 ? G : 0;
+}
+
+// Four wavefronts per chain in the reverse scans (mp_bwd_team.hip)?
+int decide_team(const BackParams& p) {
+  const int opt = g_team_scans.load(std::memory_order_relaxed);
+  if (p.pack >= 2 || p.ctx2d || opt == 0) return 0;
+  if (opt == 2) return 1;
+  return p.L > kPackedMaxL && p.block_prefix[p.n_dirs] <= launch_policy().team_max_chains ? 1 : 0;
 }
 
 // Wavefronts per chain for the forward scan of a launch whose caller declared a dense 1-D table
@@ -659,6 +668,15 @@ void launch_bwd(const BackParams& p, bool jacobi, hipStream_t st) {
   Timed timed(jacobi ? MPL_KERNEL_BWD_SWEEP_ALL : MPL_KERNEL_BWD_SWEEP, st, p.fused_pair ? 2 : 1);
   if (p.pack >= 2) {
     launch_packed_bwd(p, jacobi, p.pack, st);
+    return;
+  }
+  if (p.team) {
+    switch (labels_per_lane(p.L)) {
+      case 1: launch_team_bwd<1>(p, jacobi, st); break;
+      case 2: launch_team_bwd<2>(p, jacobi, st); break;
+      case 3: launch_team_bwd<3>(p, jacobi, st); break;
+      default: launch_team_bwd<4>(p, jacobi, st); break;
+    }
     return;
   }
   switch (labels_per_lane(p.L)) {
@@ -765,6 +783,7 @@ const LaunchPolicy& launch_policy() {
     pol.packed_min_chains21 = 2 * pol.n_simd + 1;
     pol.packed_min_chains_1d8 = 6 * pol.n_simd + 1;
     pol.packed_min_chains_1d16 = 9 * pol.n_simd + 1;
+    pol.team_max_chains = 3 * pol.n_simd / 4;
     pol.direct_max_chains = 2 * pol.n_simd;
     static std::mutex mu;
     std::lock_guard<std::mutex> lk(mu);
@@ -814,6 +833,11 @@ int mpl_set_option(int option, int value) {
   if (option == MPL_OPT_DENSE_SPLIT_WAVES) {
     if (value < 0 || value > 8) return fail(MPL_EINVAL, "set_option: 0 to 8 wavefronts per chain");
     g_split_waves.store(value, std::memory_order_relaxed);
+    return MPL_OK;
+  }
+  if (option == MPL_OPT_TEAM_SCANS) {
+    if (value < 0 || value > 2) return fail(MPL_EINVAL, "set_option: team scans take 0, 1 or 2");
+    g_team_scans.store(value, std::memory_order_relaxed);
     return MPL_OK;
   }
   return fail(MPL_EINVAL, "set_option: unknown option %d", option);
@@ -1116,6 +1140,7 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
     for (int d = s->n_dir - 1; d >= 0; --d) {  // TRWP_backward.cu:337-424
       fill_dirs(s, d, 1, p.dirs, p.block_prefix, &p.n_dirs);
       p.pack = decide_pack(s, p, opts);
+      p.team = decide_team(p);
       p.a_in = a_cur;
       float* const plane_e = dmsg + (int64_t)(d & ~1) * N;
       p.a_out = (it == 0 && d <= 1) ? dunary : plane_e;
@@ -1180,6 +1205,7 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
   p.same_label = (flags & MPL_F_DCONTEXT_SAME_LABEL) ? 1 : 0;
   fill_dirs(s, 0, s->n_dir, p.dirs, p.block_prefix, &p.n_dirs);
   p.pack = decide_pack(s, p, opts);
+  p.team = decide_team(p);
   for (int it = n_iter - 1; it >= 0; --it) {
     const bool first = (it == n_iter - 1);
     p.gu_in = first ? dcost_final : gu_buf;  // gu_k = dcost_final for every k at the start

@@ -32,3 +32,42 @@ def test_planes_of_the_pairs(gpu, oracle, n_dir, n_iter, L):
     for name, g, r in zip(("dunary", "dcontext", "dedge"), got, ref):
       # the gradient bar of the GPU tests: 1e-4 of the largest entry
       assert np.abs(g.reshape(r.shape) - r).max() <= 1e-4 * max(1.0, np.abs(r).max()), (name, flags)
+
+
+@pytest.mark.parametrize("kind", ["any", "band", "one_far"])
+@pytest.mark.parametrize("mode,n_dir", [("TRWP", 4), ("TRWP", 16), ("ISGMR", 8)])
+@pytest.mark.parametrize("L", [1, 2, 5, 63, 64, 65, 96, 128, 131, 191, 192, 193, 254, 256])
+def test_several_wavefronts_per_chain(gpu, oracle, mode, n_dir, L, kind):
+  """The reverse scan that puts four wavefronts on a chain (MPL_OPT_TEAM_SCANS): label counts at the
+  edges of a lane's labels, chains of 1 to 13 pixels (a block has six), argmin labels anywhere, in the
+  register window or one step outside it with a shared far target (where the two ways of scattering
+  meet), all combinations of wanted gradients."""
+  from mplayers_amd import _lib
+  rng = np.random.default_rng(1000 * L + n_dir)
+  B, H, W, n_iter, rho = 1, 7, 13, 2, (0.5 if mode == "TRWP" else 1.0)
+  ctx = rng.random(L).astype(np.float32)
+  ew = (0.1 + 0.9 * rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
+  imin = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W, L))
+  if kind != "any":
+    reach = 2 if kind == "band" else 3
+    near = np.clip(np.arange(L) + rng.integers(-reach, reach + 1, imin.shape), 0, L - 1)
+    far = np.broadcast_to(imin[..., :1], imin.shape)
+    imin = np.where(rng.random(imin.shape) < 0.6, far, near)
+  imin = imin.astype(np.uint8)
+  inorm = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W)).astype(np.uint8)
+  ref = oracle.backward(mode, ctx.astype(np.float64), ew.astype(np.float64), dcost.astype(np.float64),
+                        imin, inorm, rho, ctx2d=False)
+  _lib.set_option(_lib.OPT_TEAM_SCANS, 2)
+  try:
+    for want_dctx, want_dedge in ((True, True), (False, False), (True, False), (False, True)):
+      if want_dctx and L == 21:
+        continue
+      print("case", mode, n_dir, L, kind, want_dctx, want_dedge, flush=True)
+      got = gpu.gpu_backward(mode, ctx, ew, dcost, imin, inorm, rho, flags=_lib.F_PACKED_OFF,
+                             garbage_scratch=True, want_dctx=want_dctx, want_dedge=want_dedge)
+      for name, g, r in zip(("dunary", "dcontext", "dedge"), got, ref):
+        if g is not None:
+          assert np.abs(g.reshape(r.shape) - r).max() <= 1e-4 * max(1.0, np.abs(r).max()), name
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
