@@ -313,10 +313,20 @@ __global__ void __launch_bounds__(256) label_kernel(const float* __restrict__ un
 // The same for label counts that are a multiple of 4: a group of `group` lanes (a power of two
 // >= L/4) per pixel, 16 bytes per lane and plane, 64/group pixels per wavefront; the argmin is a
 // butterfly over the group on (value, label) pairs.
+// The pass reads what three others read (every message plane and the unary terms), and memory bounds
+// them all, so where one of them is due next its result is stored from here and it is not run:
+//   kLabelSum: the sum itself (cost_final after the last iteration, TRWP's re-summed belief plane),
+//   kLabelU:   ISGMR's U planes of the next iteration over the messages (isgmr_unary_kernel).
+// The sums are formed in the order of those kernels: the same bits.
+constexpr int kLabelOnly = 0, kLabelSum = 1, kLabelU = 2;
+template <int ND, int OUT>
 __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict__ unary,
-                                                         const float* __restrict__ msg, int n_dir,
-                                                         int64_t P, int L, int group, float factor,
-                                                         int min_a_dir, uint8_t* __restrict__ label) {
+                                                         const float* msg, int n_dir_rt, int64_t P,
+                                                         int L, int group, float factor,
+                                                         int min_a_dir, uint8_t* __restrict__ label,
+                                                         float* out, float rho, int pair_share) {
+  static_assert(ND > 0 || OUT != kLabelU, "the U planes need all messages in registers");
+  const int n_dir = ND > 0 ? ND : n_dir_rt;
   const int64_t N = P * L;
   const int sub = threadIdx.x & (group - 1);
   const int64_t pix = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / group;
@@ -325,24 +335,43 @@ __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict
   if (pix < P && sub * 4 < L) {
     const int64_t i = pix * L + sub * 4;
     Pack<4> v = ld_pack<4>(unary + i);
+    Pack<4> m[ND > 0 ? ND : 1];
+    if constexpr (ND > 0) {
+#pragma unroll
+      for (int k = 0; k < ND; ++k) m[k] = ld_pack<4>(msg + (int64_t)k * N + i);
+    }
+    auto message = [&](int k) { return ND > 0 ? m[ND > 0 ? k : 0] : ld_pack<4>(msg + (int64_t)k * N + i); };
 #pragma unroll
     for (int j = 0; j < 4; ++j) v.v[j] *= factor;
-    if (min_a_dir) {
-      Pack<4> mn = ld_pack<4>(msg + i);
+    if (OUT == kLabelOnly && min_a_dir) {
+      Pack<4> mn = message(0);
+#pragma unroll
       for (int k = 1; k < n_dir; ++k) {
-        Pack<4> m = ld_pack<4>(msg + (int64_t)k * N + i);
+        const Pack<4> mk = message(k);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (m.v[j] < mn.v[j]) mn.v[j] = m.v[j];
+          if (mk.v[j] < mn.v[j]) mn.v[j] = mk.v[j];
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) v.v[j] += mn.v[j];
     } else {
-      for (int k = 0; k < n_dir; ++k) {
-        Pack<4> m = ld_pack<4>(msg + (int64_t)k * N + i);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v.v[j] += m.v[j];
+      for (int k = 0; k < n_dir; ++k) {
+        const Pack<4> mk = message(k);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v.v[j] += mk.v[j];
       }
+    }
+    if constexpr (OUT == kLabelSum) st_pack<4>(out + i, v);
+    if constexpr (OUT == kLabelU) {
+#pragma unroll
+      for (int k = 0; k < ND; ++k)
+        if (!(pair_share && (k & 1))) {
+          Pack<4> u;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) u.v[j] = fmaf(v.v[j] - m[k].v[j], rho, -m[k ^ 1].v[j]);
+          st_pack<4>(out + (int64_t)k * N + i, u);  // out == msg: in place
+        }
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -362,20 +391,51 @@ __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict
   if (pix < P && sub == 0) label[pix] = (uint8_t)((arg < L) ? arg : 0);
 }
 
-static void launch_labels(const float* unary, const float* msg, int n_dir, int64_t P, int L,
-                          float factor, int min_a_dir, uint8_t* label, hipStream_t st) {
+// Returns whether `out` has been written (want: what to store there besides the labels).
+static bool launch_labels(const float* unary, const float* msg, int n_dir, int64_t P, int L,
+                          float factor, int min_a_dir, uint8_t* label, hipStream_t st,
+                          int want = kLabelOnly, float* out = nullptr, float rho = 1.f,
+                          int pair_share = 0) {
   const bool aligned = (((uintptr_t)unary | (uintptr_t)msg) & 15) == 0;
-  if ((L & 3) == 0 && aligned) {
-    int group = 1;
-    while (group * 4 < L) group <<= 1;
-    const int64_t blocks = (P * group + 255) / 256;
-    label_quad_kernel<<<(unsigned)blocks, 256, 0, st>>>(unary, msg, n_dir, P, L, group, factor,
-                                                        min_a_dir, label);
-  } else {
+  if ((L & 3) != 0 || !aligned) {
     const int64_t waves = (P < 256 * 64) ? P : 256 * 64;
     label_kernel<<<(int)((waves + 3) / 4), 256, 0, st>>>(unary, msg, n_dir, P, L, factor, min_a_dir,
                                                          label);
+    return false;
   }
+  int group = 1;
+  while (group * 4 < L) group <<= 1;
+  const unsigned blocks = (unsigned)((P * group + 255) / 256);
+  const bool known = n_dir == 4 || n_dir == 8 || n_dir == 16;
+  // (a factor other than one rounds in the product and is left to the pass of its own)
+  if (min_a_dir || factor != 1.f || out == nullptr || ((uintptr_t)out & 15) != 0 ||
+      (want == kLabelU && !known))
+    want = kLabelOnly;
+#define MPL_LABELS(ND, OUT)                                                                          \
+  label_quad_kernel<ND, OUT><<<blocks, 256, 0, st>>>(unary, msg, n_dir, P, L, group, factor, min_a_dir, \
+                                                     label, out, rho, pair_share)
+#define MPL_LABELS_ND(ND)                             \
+  do {                                                \
+    if (want == kLabelU)                              \
+      MPL_LABELS(ND, kLabelU);                        \
+    else if (want == kLabelSum)                       \
+      MPL_LABELS(ND, kLabelSum);                      \
+    else                                              \
+      MPL_LABELS(ND, kLabelOnly);                     \
+  } while (0)
+  switch (n_dir) {
+    case 4: MPL_LABELS_ND(4); break;
+    case 8: MPL_LABELS_ND(8); break;
+    case 16: MPL_LABELS_ND(16); break;
+    default:
+      if (want == kLabelSum)
+        MPL_LABELS(0, kLabelSum);
+      else
+        MPL_LABELS(0, kLabelOnly);
+  }
+#undef MPL_LABELS_ND
+#undef MPL_LABELS
+  return want != kLabelOnly;
 }
 
 // ISGMR: after all directions of an iteration have been scanned back (X_k = dU_k):
@@ -957,8 +1017,11 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
   p.msg_in = msg;
   p.msg_out = msg;
   const int rebuild = belief_rebuild_interval(s->n_dir, n_iter);
+  bool have_belief = false, have_cost = false;  // the pass that writes the labels has stored it
   for (int it = 0; it < n_iter; ++it) {
-    if (rebuild > 0 && it > 0 && it % rebuild == 0) rebuild_belief(s, unary, msg, unary_update, st);
+    if (rebuild > 0 && it > 0 && it % rebuild == 0 && !have_belief)
+      rebuild_belief(s, unary, msg, unary_update, st);
+    have_belief = false;
     for (int d = 0; d < s->n_dir; ++d) {  // Gauss-Seidel over directions: TRWP_forward.cu:440-518
       fill_dirs(s, d, 1, p.dirs, p.block_prefix, &p.n_dirs);
       p.pack = decide_pack(s, p, opts);
@@ -986,10 +1049,15 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
     }
     if (label_all) {
       Timed timed(MPL_KERNEL_LABEL, st);
-      launch_labels(unary, msg, s->n_dir, P, s->n_disp, 1.f, enable_min_a_dir, label_all + it * P, st);
+      // the next pass over the same planes, if one is due: cost_final, the re-summed belief plane
+      const bool last = it + 1 == n_iter;
+      float* out = last ? cost_final : (rebuild > 0 && (it + 1) % rebuild == 0) ? unary_update : nullptr;
+      const bool stored = launch_labels(unary, msg, s->n_dir, P, s->n_disp, 1.f, enable_min_a_dir,
+                                        label_all + it * P, st, kLabelSum, out);
+      (last ? have_cost : have_belief) = stored;
     }
   }
-  {
+  if (!have_cost) {
     Timed timed(MPL_KERNEL_AGGREGATE, st);
     const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
     MPL_EW_LAUNCH(aggregate_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, 1.f,
@@ -1046,6 +1114,7 @@ int mpl_isgmr_forward(const mpl_shape* s, unsigned flags, int enable_sgm, float 
                           p.pack == 0;
   p.belief_zero = unary;
   float* have = msg;  // the buffer that holds the current messages
+  bool have_u = false, have_cost = false;  // the pass that writes the labels has stored it
   for (int it = 0; it < n_iter; ++it) {
     // Jacobi over directions (ISGMR_forward.cu:506-622): every direction reads the old messages,
     // through U; the two buffers alternate instead of being copied.  U normally overwrites the
@@ -1066,6 +1135,9 @@ int mpl_isgmr_forward(const mpl_shape* s, unsigned flags, int enable_sgm, float 
       p.msg_in = have;
       p.u_stride = N;
       p.u_fused = 1;
+    } else if (have_u) {  // over the old messages, as the pass below leaves them
+      p.msg_in = ubuf;
+      p.u_stride = N;
     } else {
       Timed timed(MPL_KERNEL_UNARY_ALL, st);
       const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(msg_update);
@@ -1090,11 +1162,17 @@ int mpl_isgmr_forward(const mpl_shape* s, unsigned flags, int enable_sgm, float 
     p.zero_first = 0;
     if (label_all) {
       Timed timed(MPL_KERNEL_LABEL, st);
-      launch_labels(unary, nxt, s->n_dir, P, s->n_disp, factor, enable_min_a_dir, label_all + it * P, st);
+      // the next pass over the same planes: cost_final, or the U planes of the next iteration in
+      // place of these messages, unless its scans form U themselves
+      const bool last = it + 1 == n_iter;
+      const bool stored = launch_labels(unary, nxt, s->n_dir, P, s->n_disp, factor, enable_min_a_dir,
+                                        label_all + it * P, st, last ? kLabelSum : kLabelU,
+                                        last ? cost_final : fuse_u ? nullptr : nxt, rho, p.u_pair_share);
+      (last ? have_cost : have_u) = stored;
     }
     have = nxt;
   }
-  {
+  if (!have_cost) {
     Timed timed(MPL_KERNEL_AGGREGATE, st);
     const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
     MPL_EW_LAUNCH(aggregate_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, factor,
@@ -1254,8 +1332,11 @@ int mpl_trwp_soft_forward(const mpl_shape* s, unsigned flags, float rho, int n_i
   p.msg_in = msg;
   p.msg_out = msg;
   const int rebuild = belief_rebuild_interval(s->n_dir, n_iter);
+  bool have_belief = false, have_cost = false;  // the pass that writes the labels has stored it
   for (int it = 0; it < n_iter; ++it) {
-    if (rebuild > 0 && it > 0 && it % rebuild == 0) rebuild_belief(s, unary, msg, unary_update, st);
+    if (rebuild > 0 && it > 0 && it % rebuild == 0 && !have_belief)
+      rebuild_belief(s, unary, msg, unary_update, st);
+    have_belief = false;
     for (int d = 0; d < s->n_dir; ++d) {  // TRWP_forward_soft.cu:441-520
       fill_dirs(s, d, 1, p.dirs, p.block_prefix, &p.n_dirs);
       if (train) {
@@ -1271,10 +1352,15 @@ int mpl_trwp_soft_forward(const mpl_shape* s, unsigned flags, float rho, int n_i
     }
     if (label_all) {
       Timed timed(MPL_KERNEL_LABEL, st);
-      launch_labels(unary, msg, s->n_dir, P, s->n_disp, 1.f, 0, label_all + it * P, st);
+      // the next pass over the same planes, if one is due: cost_final, the re-summed belief plane
+      const bool last = it + 1 == n_iter;
+      float* out = last ? cost_final : (rebuild > 0 && (it + 1) % rebuild == 0) ? unary_update : nullptr;
+      const bool stored = launch_labels(unary, msg, s->n_dir, P, s->n_disp, 1.f, 0,
+                                        label_all + it * P, st, kLabelSum, out);
+      (last ? have_cost : have_belief) = stored;
     }
   }
-  {
+  if (!have_cost) {
     Timed timed(MPL_KERNEL_AGGREGATE, st);
     const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
     MPL_EW_LAUNCH(aggregate_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, 1.f, 0,
