@@ -317,7 +317,9 @@ __global__ void __launch_bounds__(256) label_kernel(const float* __restrict__ un
 // them all, so where one of them is due next its result is stored from here and it is not run:
 //   kLabelSum: the sum itself (cost_final after the last iteration, TRWP's re-summed belief plane),
 //   kLabelU:   ISGMR's U planes of the next iteration over the messages (isgmr_unary_kernel).
-// The sums are formed in the order of those kernels: the same bits.
+// The sums are formed in the order of those kernels: the same bits.  50 iterations on 375x450x60 with all
+// labels, passes apart -> together: TRWP, 8 directions 33.2 -> 32.4 ms, 4 directions 15.8 -> 15.4; ISGMR,
+// 8 directions 19.6 -> 16.8 ms (16 labels 7.03 -> 6.39), 4 directions 11.1 -> 10.9 (its scans form U).
 constexpr int kLabelOnly = 0, kLabelSum = 1, kLabelU = 2;
 template <int ND, int OUT>
 __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict__ unary,

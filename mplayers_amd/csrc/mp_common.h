@@ -578,8 +578,8 @@ struct LaunchPolicy {
   // reverse scans with one label per lane: launches of at most this many chains (two wavefronts per
   // SIMD) are taken to be bound by the latency of a step (mp_bwd.hip)
   int direct_max_chains;
-  // Reverse scans with a 1-D table of more than 32 labels and at most this many chains (three to four
-  // SIMDs) put four wavefronts on a chain (mp_bwd_team.hip).  Measured, 4 directions, one wavefront per
+  // Reverse scans with a 1-D table of more than 32 labels and at most this many chains (three for
+  // every four SIMDs) put four wavefronts on a chain (mp_bwd_team.hip).  Measured, 4 directions, one wavefront per
   // chain against four, ms: 192 labels 256 / 512 chains 5.16 / 2.12, 500 / 800 chains 8.9 / 5.9, 1000 chains
   // 8.2 / 7.6, 1400 chains 10.0 / 10.1; 128 labels 250 / 300 chains 2.8 / 1.3, 500 / 600 chains 5.8 / 3.4,
   // 900 / 1000 chains 9.7 / 8.7; 256 labels 600 / 700 chains 10.4 / 7.7, 900 / 1000 chains 15.9 / 15.8; a
