@@ -659,12 +659,44 @@ int decide_pack(const mpl_shape* s, const Params& p, const CallOpts& o) {
   return G >= 2 ? G : 0;
 }
 
-// Four wavefronts per chain in the reverse scans (mp_bwd_team.hip)?
-int decide_team(const BackParams& p) {
+// Four wavefronts per chain in the reverse scans (mp_bwd_team.hip): chains per compute unit up to which
+// a launch takes them, 0 for never.  The time of such a launch steps up with every further chain per
+// compute unit, so the lines lie between those steps, where no kind of call measured slower than with
+// one wavefront per chain.  The table (a band of four labels, or dense) and which gradients are wanted
+// change the ratio but may not change the route: the table is not known here, and dunary is promised to
+// be the same bits whichever gradients are wanted.  Measured, backward of 2 iterations on square images,
+// time with one over time with four wavefronts: dunary alone, on the table that gains less / every
+// gradient, on the table that gains more.
+//   * TRWP, 33 labels: 256 chains 1.08 / 1.63, 512 chains 0.93 / 1.46, 768 chains 0.75 / 1.21, 64x64
+//     with 8 directions 0.90 / 1.32.  49 to 64 labels: 256 chains 1.15 / 1.65, 48x48 and 64x64 with 8
+//     directions 0.98 / 1.35 (32x32: 0.93 / 1.23); 64 labels 320 chains 1.01 / 1.48, 56 labels 640 chains
+//     0.91 / 1.46.  ISGMR, 33 to 64 labels: 0.69 to 1.0 / 0.95 to 1.5 (with one label per lane the step
+//     of mp_bwd.hip is short, and shorter still without the h planes of TRWP).
+//   * TRWP, 768 chains: 65 to 128 labels 1.23 / 2.2, 192 labels 1.42 / 1.77, 256 labels 1.27 / 1.30.
+//     ISGMR (all directions in one launch), 764 and 768 chains: 65 to 128 labels 1.02 / 1.9, 192 labels
+//     1.02 / 1.29, 256 labels 0.96 / 0.99 (640 chains, all gradients, dense table: 0.84), 512 chains
+//     1.15 / 1.48; with 256 labels and the other gradients the LDS of a compute unit holds two chains.
+//   * Labels loaded and stored one by one (their number no multiple of the labels per lane), which gains
+//     less where several chains share a compute unit.  TRWP: 127 labels 768 chains 1.23 / 1.87; 152 / 158
+//     / 190 labels 768 chains 1.04 / 1.65, 0.98 / 1.60, 0.83 / 1.44, 190 labels 512 chains 1.34 / 2.1;
+//     193 labels 512 / 768 chains 1.16 / 2.0 and 0.73 / 1.22; 217 labels 512 chains 1.01 / 1.81; 255 labels
+//     256 / 384 / 512 chains 1.62 / 2.33, 0.99 / 1.71 and 0.78 / 1.45.  ISGMR, 768 chains: 191 labels
+//     1.09 / 1.34; 255 labels 512 chains 0.95 / 1.52.
+int team_chains_per_cu(int L, bool jacobi) {
+  const int R = labels_per_lane(L);
+  const bool whole = L % R == 0;  // every lane has all its labels or none: one access per lane
+  if (R == 1) return !jacobi && L > 48 ? 1 : 0;
+  if (R == 3 && !whole && !jacobi && L > 152) return 2;
+  if (R == 4) return whole ? (jacobi ? 2 : 3) : (L <= 216 ? 2 : 1);
+  return 3;
+}
+
+int decide_team(const BackParams& p, bool jacobi) {
   const int opt = g_team_scans.load(std::memory_order_relaxed);
   if (p.pack >= 2 || p.ctx2d || opt == 0) return 0;
   if (opt == 2) return 1;
-  return p.L > kPackedMaxL && p.block_prefix[p.n_dirs] <= launch_policy().team_max_chains ? 1 : 0;
+  const int cus = launch_policy().n_simd / 4;
+  return p.block_prefix[p.n_dirs] <= team_chains_per_cu(p.L, jacobi) * cus ? 1 : 0;
 }
 
 // Wavefronts per chain for the forward scan of a launch whose caller declared a dense 1-D table
@@ -845,7 +877,6 @@ const LaunchPolicy& launch_policy() {
     pol.packed_min_chains21 = 2 * pol.n_simd + 1;
     pol.packed_min_chains_1d8 = 6 * pol.n_simd + 1;
     pol.packed_min_chains_1d16 = 9 * pol.n_simd + 1;
-    pol.team_max_chains = 3 * pol.n_simd / 4;
     pol.direct_max_chains = 2 * pol.n_simd;
     static std::mutex mu;
     std::lock_guard<std::mutex> lk(mu);
@@ -1220,7 +1251,7 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
     for (int d = s->n_dir - 1; d >= 0; --d) {  // TRWP_backward.cu:337-424
       fill_dirs(s, d, 1, p.dirs, p.block_prefix, &p.n_dirs);
       p.pack = decide_pack(s, p, opts);
-      p.team = decide_team(p);
+      p.team = decide_team(p, false);
       p.a_in = a_cur;
       float* const plane_e = dmsg + (int64_t)(d & ~1) * N;
       p.a_out = (it == 0 && d <= 1) ? dunary : plane_e;
@@ -1285,7 +1316,7 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
   p.same_label = (flags & MPL_F_DCONTEXT_SAME_LABEL) ? 1 : 0;
   fill_dirs(s, 0, s->n_dir, p.dirs, p.block_prefix, &p.n_dirs);
   p.pack = decide_pack(s, p, opts);
-  p.team = decide_team(p);
+  p.team = decide_team(p, true);
   for (int it = n_iter - 1; it >= 0; --it) {
     const bool first = (it == n_iter - 1);
     p.gu_in = first ? dcost_final : gu_buf;  // gu_k = dcost_final for every k at the start

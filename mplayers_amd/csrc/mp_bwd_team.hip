@@ -29,8 +29,8 @@
 // five clocks each, 264 ns by itself), with dedge_weights and dcontext 7.18 -> 3.81, 500x800x192
 // 8.91 -> 5.87; dense table 240x320x96 with dcontext 5.95 -> 3.18.  Two pixels per helper and block, three
 // helpers: one pixel 2.14, four 2.36, seven helpers of one pixel 2.11 (and 6.2 instead of 5.9 ms at
-// 500x800x192).  With every scatter through LDS float adds 3.74 ms.  Where the launch policy draws
-// the line: LaunchPolicy::team_max_chains.
+// 500x800x192).  With every scatter through LDS float adds 3.74 ms.  Which launches take it:
+// team_chains_per_cu (mp_api.hip).
 //
 // Compiled once per R (labels per lane) with -DMPL_INST_R=<R>.
 

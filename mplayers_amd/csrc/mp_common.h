@@ -578,16 +578,6 @@ struct LaunchPolicy {
   // reverse scans with one label per lane: launches of at most this many chains (two wavefronts per
   // SIMD) are taken to be bound by the latency of a step (mp_bwd.hip)
   int direct_max_chains;
-  // Reverse scans with a 1-D table of more than 32 labels and at most this many chains (three for
-  // every four SIMDs) put four wavefronts on a chain (mp_bwd_team.hip).  Measured, 4 directions, one wavefront per
-  // chain against four, ms: 192 labels 256 / 512 chains 5.16 / 2.12, 500 / 800 chains 8.9 / 5.9, 1000 chains
-  // 8.2 / 7.6, 1400 chains 10.0 / 10.1; 128 labels 250 / 300 chains 2.8 / 1.3, 500 / 600 chains 5.8 / 3.4,
-  // 900 / 1000 chains 9.7 / 8.7; 256 labels 600 / 700 chains 10.4 / 7.7, 900 / 1000 chains 15.9 / 15.8; a
-  // dense table of 96 labels 600 chains 8.5 / 7.3, 900 chains 13.6 / 14.1; 60 labels 500 / 600 chains
-  // 2.8 / 2.4; ISGMR (all directions in one launch) 192 labels 656 chains 0.77 / 0.48, 1024 chains
-  // 1.25 / 1.10, 96 labels 1964 chains 0.60 / 0.62.  With 16 labels the step of mp_bwd.hip is short:
-  // 256 chains 0.53 / 0.49, 600 / 700 chains 1.33 / 1.89; 21 labels with a 2-D table 516 chains 0.95 / 1.21.
-  int team_max_chains;
 };
 const LaunchPolicy& launch_policy();  // mp_api.hip
 
