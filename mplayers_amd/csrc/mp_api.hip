@@ -633,6 +633,8 @@ struct CallOpts {
   bool fused_u;
   bool fused_pairs;
   bool dense_table;
+  int split_waves;  // MPL_OPT_DENSE_SPLIT_WAVES
+  int team;         // MPL_OPT_TEAM_SCANS
 };
 
 int read_flags(unsigned flags, const char* what, CallOpts* o) {
@@ -644,6 +646,8 @@ int read_flags(unsigned flags, const char* what, CallOpts* o) {
   o->fused_u = (flags & MPL_F_FUSED_U_OFF) ? false : g_fused_u.load(std::memory_order_relaxed) != 0;
   o->fused_pairs = (flags & MPL_F_FUSED_PAIRS_OFF) == 0;
   o->dense_table = (flags & MPL_F_DENSE_TABLE) != 0;
+  o->split_waves = g_split_waves.load(std::memory_order_relaxed);
+  o->team = g_team_scans.load(std::memory_order_relaxed);
   return MPL_OK;
 }
 
@@ -691,10 +695,9 @@ int team_chains_per_cu(int L, bool jacobi) {
   return 3;
 }
 
-int decide_team(const BackParams& p, bool jacobi) {
-  const int opt = g_team_scans.load(std::memory_order_relaxed);
-  if (p.pack >= 2 || p.ctx2d || opt == 0) return 0;
-  if (opt == 2) return 1;
+int decide_team(const BackParams& p, const CallOpts& o, bool jacobi) {
+  if (p.pack >= 2 || p.ctx2d || o.team == 0) return 0;
+  if (o.team == 2) return 1;
   const int cus = launch_policy().n_simd / 4;
   return p.block_prefix[p.n_dirs] <= team_chains_per_cu(p.L, jacobi) * cus ? 1 : 0;
 }
@@ -718,10 +721,9 @@ template <typename Params>
 int choose_split(const mpl_shape* s, const Params& p, const CallOpts& o, bool train) {
   if (!o.dense_table || s->ctx2d || s->n_disp <= kWave || p.pack >= 2) return 0;
   const int L = s->n_disp, R = labels_per_lane(L);
-  const int forced = g_split_waves.load(std::memory_order_relaxed);
   int w;
-  if (forced > 0) {
-    w = forced;
+  if (o.split_waves > 0) {
+    w = o.split_waves;
   } else {
     const int64_t chains4 = 4 * (int64_t)p.block_prefix[p.n_dirs];  // in quarters of a chain
     const int64_t n_simd = launch_policy().n_simd;
@@ -1251,7 +1253,7 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
     for (int d = s->n_dir - 1; d >= 0; --d) {  // TRWP_backward.cu:337-424
       fill_dirs(s, d, 1, p.dirs, p.block_prefix, &p.n_dirs);
       p.pack = decide_pack(s, p, opts);
-      p.team = decide_team(p, false);
+      p.team = decide_team(p, opts, false);
       p.a_in = a_cur;
       float* const plane_e = dmsg + (int64_t)(d & ~1) * N;
       p.a_out = (it == 0 && d <= 1) ? dunary : plane_e;
@@ -1316,7 +1318,7 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
   p.same_label = (flags & MPL_F_DCONTEXT_SAME_LABEL) ? 1 : 0;
   fill_dirs(s, 0, s->n_dir, p.dirs, p.block_prefix, &p.n_dirs);
   p.pack = decide_pack(s, p, opts);
-  p.team = decide_team(p, true);
+  p.team = decide_team(p, opts, true);
   for (int it = n_iter - 1; it >= 0; --it) {
     const bool first = (it == n_iter - 1);
     p.gu_in = first ? dcost_final : gu_buf;  // gu_k = dcost_final for every k at the start

@@ -48,3 +48,41 @@ def test_launches_with_four_wavefronts_per_chain(gpu, mode, L, per_cu, more, fou
   expected = four_waves if four else one_wave
   assert np.array_equal(dunary(1), expected)
   assert np.array_equal(dunary(1, wanted=True), expected)
+
+
+def test_a_call_reads_the_option_once(gpu):
+  """A thread that sets MPL_OPT_TEAM_SCANS while another one is inside a backward call does not change
+  the kernels of that call half way: its result has the bits of one of the two kernels."""
+  import threading
+  from mplayers_amd import _lib
+  n_iter, n_dir, H, W, L = 4, 16, 6, 7, 70
+  rng = np.random.default_rng(5)
+  ctx = rng.random(L).astype(np.float32)
+  dcost = rng.standard_normal((1, 1, H, W, L)).astype(np.float32)
+  imin = rng.integers(0, L, (n_iter, n_dir, 1, 1, H, W, L)).astype(np.uint8)
+  inorm = rng.integers(0, L, (n_iter, n_dir, 1, 1, H, W)).astype(np.uint8)
+  run = lambda: gpu.gpu_backward("TRWP", ctx, None, dcost, imin, inorm, 0.5, want_dctx=False,
+                                 want_dedge=False)[0]
+  done = threading.Event()
+
+  def toggle():
+    while not done.is_set():
+      _lib.set_option(_lib.OPT_TEAM_SCANS, 0)
+      _lib.set_option(_lib.OPT_TEAM_SCANS, 2)
+
+  pure = []
+  try:
+    for option in (0, 2):
+      _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+      pure.append(run())
+    thread = threading.Thread(target=toggle)
+    thread.start()
+    try:
+      results = [run() for _ in range(200)]
+    finally:
+      done.set()
+      thread.join()
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+  assert not np.array_equal(*pure)
+  assert all(np.array_equal(r, pure[0]) or np.array_equal(r, pure[1]) for r in results)
