@@ -71,3 +71,33 @@ def test_several_wavefronts_per_chain(gpu, oracle, mode, n_dir, L, kind):
           assert np.abs(g.reshape(r.shape) - r).max() <= 1e-4 * max(1.0, np.abs(r).max()), name
   finally:
     _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+
+
+@pytest.mark.parametrize("L", [49, 70, 131, 256])
+def test_every_place_of_the_main_wavefront(gpu, oracle, L):
+  """Which of the four wavefronts of a chain runs the recurrence changes with the workgroup's number
+  over the number of compute units: 7 x 8 x 16 pixels give one ISGMR launch of 8 directions 980 chains,
+  all four places on a device of 256."""
+  import torch
+  from mplayers_amd import _lib
+  B, H, W, n_dir, n_iter = 7, 8, 16, 8, 2
+  chains = sum(B * _lib.load().mpl_n_chains(d, H, W) for d in range(n_dir))
+  assert chains > 3 * torch.cuda.get_device_properties(0).multi_processor_count
+  rng = np.random.default_rng(L)
+  ctx = rng.random(L).astype(np.float32)
+  ew = (0.1 + 0.9 * rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
+  near = np.clip(np.arange(L) + rng.integers(-2, 3, (n_iter, n_dir, B, 1, H, W, L)), 0, L - 1)
+  imin = np.where(rng.random(near.shape) < 0.6, near[..., :1], near).astype(np.uint8)
+  inorm = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W)).astype(np.uint8)
+  ref = oracle.backward("ISGMR", ctx.astype(np.float64), ew.astype(np.float64), dcost.astype(np.float64),
+                        imin, inorm, 1.0, ctx2d=False)
+  print("case", L, chains, flush=True)
+  _lib.set_option(_lib.OPT_TEAM_SCANS, 2)
+  try:
+    got = gpu.gpu_backward("ISGMR", ctx, ew, dcost, imin, inorm, 1.0, garbage_scratch=True)
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+  for name, g, r in zip(("dunary", "dcontext", "dedge"), got, ref):
+    # the gradient bar of the GPU tests: 1e-4 of the largest entry
+    assert np.abs(g.reshape(r.shape) - r).max() <= 1e-4 * max(1.0, np.abs(r).max()), name
