@@ -28,3 +28,14 @@ def gpu():
   _lib.load()
   from tests import _gpu_util
   return _gpu_util
+
+
+@pytest.fixture(params=[1, 0], ids=["by_launch", "one_wavefront"])
+def reverse_scans(request, gpu):
+  """Runs a test twice: with the reverse scans the launch rule takes (images as small as those of the
+  tests put four wavefronts on a chain from 49 or 65 labels on) and with one wavefront per chain, which
+  larger launches take."""
+  from mplayers_amd import _lib
+  _lib.set_option(_lib.OPT_TEAM_SCANS, request.param)
+  yield request.param
+  _lib.set_option(_lib.OPT_TEAM_SCANS, 1)

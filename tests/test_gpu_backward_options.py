@@ -40,6 +40,7 @@ def _problem(oracle, mode, n_dir, B, H, W, L, ctx2d, n_iter=2):
   return rho, ctx, ew, dcost, ref["msg_min_index"], ref["msg_norm_index"]
 
 
+@pytest.mark.usefixtures("reverse_scans")
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("mode,n_dir,B,H,W,L,ctx2d", CASES)
 def test_outputs_switched_off_leave_the_rest_unchanged(gpu, oracle, mode, n_dir, B, H, W, L, ctx2d,
@@ -65,6 +66,7 @@ def test_outputs_switched_off_leave_the_rest_unchanged(gpu, oracle, mode, n_dir,
       assert got[1] is None
 
 
+@pytest.mark.usefixtures("reverse_scans")
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("mode,n_dir,B,H,W,L,ctx2d", [c for c in CASES if c[0] == "TRWP"])
 def test_same_label_flag_matches_oracle(gpu, oracle, mode, n_dir, B, H, W, L, ctx2d, packed):

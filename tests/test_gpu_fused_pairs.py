@@ -56,6 +56,7 @@ def test_fused_pairs_packed_are_bit_identical(gpu, L, n_dir, B, H, W, n_iter, rh
                                      base_flags=_lib.F_PACKED_ALWAYS)
 
 
+@pytest.mark.usefixtures("reverse_scans")
 @pytest.mark.parametrize("L,n_dir,B,H,W,n_iter,rho,train,kind", CASES)
 @pytest.mark.parametrize("start", ["cleared", "uninit", "given"])
 def test_fused_pairs_are_bit_identical(gpu, L, n_dir, B, H, W, n_iter, rho, train, kind, start,

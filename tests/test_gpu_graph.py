@@ -8,6 +8,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.usefixtures("reverse_scans")
 @pytest.mark.parametrize("mode", ["TRWP", "ISGMR"])
 @pytest.mark.parametrize("L,n_dir,B,H,W", [(21, 4, 2, 33, 35), (96, 8, 1, 24, 40), (16, 16, 8, 40, 40)])
 def test_graph_replay_matches_eager(gpu, mode, L, n_dir, B, H, W):

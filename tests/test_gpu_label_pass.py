@@ -35,3 +35,27 @@ def test_pass_with_labels_is_the_passes_apart(gpu, mode, rho, n_dir, L):
           assert np.array_equal(got["label_all"][k], apart[k]["cost_final"].argmin(-1)), (n_iter, k)
   finally:
     _lib.set_option(_lib.OPT_BELIEF_REBUILD, _lib.BELIEF_REBUILD_DEFAULT)
+
+
+@pytest.mark.parametrize("L", [3, 8, 60, 256])
+@pytest.mark.parametrize("n_dir", [2, 4, 6, 8, 16])
+def test_sgm_keeps_the_passes_apart(gpu, n_dir, L):
+  """The one-iteration operator weights the unary terms by the number of directions; its label pass
+  stores nothing else."""
+  rng = np.random.default_rng(10 * L + n_dir)
+  B, H, W = 2, 7, 11
+  unary = rng.random((B, 1, H, W, L)).astype(np.float32)
+  ctx = (0.1 * np.minimum(np.arange(L), 2)).astype(np.float32)
+  ew = (0.1 + 0.9 * rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  print("case", n_dir, L, flush=True)
+  plain, got = (gpu.gpu_forward("ISGMR", unary, ctx, ew, n_dir, 1, 1.0, training=False, enable_sgm=True,
+                                saving_label=labels) for labels in (False, True))
+  for name in ("msg", "cost_final"):
+    assert np.array_equal(got[name], plain[name]), name
+  # six directions: the product with the factor rounds, and either pass may fuse it into its first
+  # sum, so labels are compared where the two smallest costs are further apart than that (a cost is
+  # below 6 + 6 * 0.2, seven roundings of it below 2e-6 in either pass)
+  cost = plain["cost_final"].astype(np.float64)
+  two = np.partition(cost, 1, axis=-1)[..., :2]
+  clear = (two[..., 1] - two[..., 0] > 1e-5) | (n_dir != 6)
+  assert np.array_equal(got["label_all"][0][clear], cost.argmin(-1)[clear])

@@ -148,6 +148,7 @@ def test_negative_edge_weights_take_the_dense_path(gpu, oracle):
                                       2e-5, "msg_min_index")
 
 
+@pytest.mark.usefixtures("reverse_scans")
 @pytest.mark.parametrize("mode,n_dir,B,H,W,L,kind,n_iter", CASES)
 def test_backward_matches_oracle(gpu, oracle, mode, n_dir, B, H, W, L, kind, n_iter):
   rng = np.random.default_rng(_seed(mode, n_dir, L, kind, 1))

@@ -39,6 +39,7 @@ def random_case(seed):
   return mode, n_dir, n_iter, unary, ctx, ew, dcost
 
 
+@pytest.mark.usefixtures("reverse_scans")
 @pytest.mark.parametrize("seed", range(40))
 def test_random_case(gpu, oracle, seed):
   mode, n_dir, n_iter, unary, ctx, ew, dcost = random_case(seed)
@@ -65,6 +66,7 @@ def test_random_case(gpu, oracle, seed):
     assert err <= 1e-4 * max(1.0, np.abs(r).max()), (name, err)
 
 
+@pytest.mark.usefixtures("reverse_scans")
 @pytest.mark.parametrize("mode,rho", [("ISGMR", 0.7), ("ISGMR", 0.5), ("TRWP", 1.0), ("TRWP", 0.3)])
 @pytest.mark.parametrize("L,n_dir", [(21, 8), (96, 4), (7, 16)])
 def test_other_rho_values(gpu, oracle, mode, rho, L, n_dir):
