@@ -666,32 +666,32 @@ int decide_pack(const mpl_shape* s, const Params& p, const CallOpts& o) {
 // Four wavefronts per chain in the reverse scans (mp_bwd_team.hip): chains per compute unit up to which
 // a launch takes them, 0 for never.  The time of such a launch steps up with every further chain per
 // compute unit, so the lines lie between those steps, where no kind of call measured slower than with
-// one wavefront per chain.  The table (a band of four labels, or dense) and which gradients are wanted
-// change the ratio but may not change the route: the table is not known here, and dunary is promised to
-// be the same bits whichever gradients are wanted.  Measured, backward of 2 iterations on square images,
-// time with one over time with four wavefronts: dunary alone, on the table that gains less / every
-// gradient, on the table that gains more.
-//   * TRWP, 33 labels: 256 chains 1.08 / 1.63, 512 chains 0.93 / 1.46, 768 chains 0.75 / 1.21, 64x64
-//     with 8 directions 0.90 / 1.32.  49 to 64 labels: 256 chains 1.15 / 1.65, 48x48 and 64x64 with 8
-//     directions 0.98 / 1.35 (32x32: 0.93 / 1.23); 64 labels 320 chains 1.01 / 1.48, 56 labels 640 chains
-//     0.91 / 1.46.  ISGMR, 33 to 64 labels: 0.69 to 1.0 / 0.95 to 1.5 (with one label per lane the step
-//     of mp_bwd.hip is short, and shorter still without the h planes of TRWP).
-//   * TRWP, 768 chains: 65 to 128 labels 1.23 / 2.2, 192 labels 1.42 / 1.77, 256 labels 1.27 / 1.30.
-//     ISGMR (all directions in one launch), 764 and 768 chains: 65 to 128 labels 1.02 / 1.9, 192 labels
-//     1.02 / 1.29, 256 labels 0.96 / 0.99 (640 chains, all gradients, dense table: 0.84), 512 chains
-//     1.15 / 1.48; with 256 labels and the other gradients the LDS of a compute unit holds two chains.
-//   * Labels loaded and stored one by one (their number no multiple of the labels per lane), which gains
-//     less where several chains share a compute unit.  TRWP: 127 labels 768 chains 1.23 / 1.87; 152 / 158
+// one wavefront per chain.  The table and which gradients are wanted change the ratio but may not change
+// the route: the table is not known here, and dunary is promised to be the same bits whichever gradients
+// are wanted.  Measured, backward of 2 iterations on square images (TRWP: 256, 512 and 768 chains per
+// launch; ISGMR: all directions in one), time with one over time with four wavefronts: the least of
+// dunary alone and of all gradients on a band of four labels, a bent band, a linear and a random table /
+// the greatest.
+//   * up to 64 labels: TRWP 256 chains 0.78 / 1.65, 768 chains with 33 labels 0.75 / 1.2, ISGMR 0.69 / 1.5.
+//     With one label per lane the step of mp_bwd.hip is short, and labels that point anywhere cost this
+//     kernel more (64 labels, dunary alone: 199 ns per pixel and walk there, 245 here).
+//   * TRWP: 65 to 128 labels 768 chains 1.19 / 2.2, 192 labels 1.15 / 1.77, 256 labels 0.98 / 1.5 (576
+//     chains 1.06 / 1.5).
+//   * TRWP, labels loaded and stored one by one (their number no multiple of the labels per lane), which
+//     gains less where several chains share a compute unit: 127 labels 768 chains 1.21 / 1.87; 152 / 158
 //     / 190 labels 768 chains 1.04 / 1.65, 0.98 / 1.60, 0.83 / 1.44, 190 labels 512 chains 1.34 / 2.1;
-//     193 labels 512 / 768 chains 1.16 / 2.0 and 0.73 / 1.22; 217 labels 512 chains 1.01 / 1.81; 255 labels
-//     256 / 384 / 512 chains 1.62 / 2.33, 0.99 / 1.71 and 0.78 / 1.45.  ISGMR, 768 chains: 191 labels
-//     1.09 / 1.34; 255 labels 512 chains 0.95 / 1.52.
+//     193 and 215 labels 512 chains 1.14 / 2.0, 768 chains 0.72 / 1.3; 217 labels 512 chains 1.01 / 1.82;
+//     255 labels 256 / 512 chains 1.62 / 2.33 and 0.78 / 1.84.
+//   * ISGMR: 512 chains with 65 to 192 labels 1.04 / 2.0, 640 to 768 chains 0.87 / 1.9; 256 labels 256
+//     chains 1.31 / 2.2, 512 chains 0.98 / 1.8, 640 chains 0.81 / 1.4.
 int team_chains_per_cu(int L, bool jacobi) {
   const int R = labels_per_lane(L);
-  const bool whole = L % R == 0;  // every lane has all its labels or none: one access per lane
-  if (R == 1) return !jacobi && L > 48 ? 1 : 0;
-  if (R == 3 && !whole && !jacobi && L > 152) return 2;
-  if (R == 4) return whole ? (jacobi ? 2 : 3) : (L <= 216 ? 2 : 1);
+  if (R == 1) return 0;
+  if (jacobi) return R == 4 ? 1 : 2;
+  if (L % R != 0) {  // labels one by one
+    if (R == 4) return L <= 216 ? 2 : 1;
+    if (R == 3 && L > 152) return 2;
+  }
   return 3;
 }
 

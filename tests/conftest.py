@@ -33,7 +33,7 @@ def gpu():
 @pytest.fixture(params=[1, 0], ids=["by_launch", "one_wavefront"])
 def reverse_scans(request, gpu):
   """Runs a test twice: with the reverse scans the launch rule takes (images as small as those of the
-  tests put four wavefronts on a chain from 49 or 65 labels on) and with one wavefront per chain, which
+  tests put four wavefronts on a chain from 65 labels on) and with one wavefront per chain, which
   larger launches take."""
   from mplayers_amd import _lib
   _lib.set_option(_lib.OPT_TEAM_SCANS, request.param)

@@ -72,7 +72,7 @@ def test_several_wavefronts_per_chain(gpu, oracle, mode, n_dir, L, kind):
     _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
 
 
-@pytest.mark.parametrize("L", [64, 96, 131, 192, 254, 256])
+@pytest.mark.parametrize("L", [65, 96, 131, 192, 254, 256])
 def test_kernels_of_a_call_differ_by_direction(gpu, oracle, L):
   """9 x 90 x 5 pixels: 810 rows of 5 pixels, which take one wavefront per chain and both walks of the
   pair in one launch, 45 columns of 90 pixels, which take four, and 846 diagonals; they hand their
