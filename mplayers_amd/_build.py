@@ -2,7 +2,8 @@
 measurement probes (csrc/mp_probe.hip) into libmplayers_probe.so, which only the benchmark and the
 tests load.
 
-The scan kernels are instantiated once per R (labels per lane, 1..4), the forward scans also once
+The scan kernels are instantiated once per R (labels per lane, 1..4; the reverse scans with four
+wavefronts per chain from 2 on), the forward scans also once
 with and once without argmin labels; each instantiation is its own translation unit so that they
 compile in parallel.
 """
@@ -38,7 +39,8 @@ def _units():
       units.append(("mp_fwd_r%d_t%d" % (r, t), "mp_fwd.hip",
                     ["-DMPL_INST_R=%d" % r, "-DMPL_INST_TRAIN=%d" % t]))
     units.append(("mp_bwd_r%d" % r, "mp_bwd.hip", ["-DMPL_INST_R=%d" % r]))
-    units.append(("mp_bwd_team_r%d" % r, "mp_bwd_team.hip", ["-DMPL_INST_R=%d" % r]))
+    if r > 1:
+      units.append(("mp_bwd_team_r%d" % r, "mp_bwd_team.hip", ["-DMPL_INST_R=%d" % r]))
   return units
 
 

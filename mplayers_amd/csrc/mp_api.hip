@@ -624,7 +624,7 @@ int labels_per_lane(int L) { return (L + kWave - 1) / kWave; }
 std::atomic<int> g_packed_scans{1};  // MPL_OPT_PACKED_SCANS: 0 off, 1 by chain count, 2 always
 std::atomic<int> g_fused_u{1};       // MPL_OPT_FUSED_U
 std::atomic<int> g_belief_rebuild{MPL_BELIEF_REBUILD_DEFAULT};  // MPL_OPT_BELIEF_REBUILD
-std::atomic<int> g_team_scans{1};    // MPL_OPT_TEAM_SCANS: 0 never, 1 launches with few chains, 2 always
+std::atomic<int> g_team_scans{1};    // MPL_OPT_TEAM_SCANS: 0 never, 1 launches with few chains, 2 more than 64 labels
 std::atomic<int> g_split_waves{0};   // MPL_OPT_DENSE_SPLIT_WAVES: 0 = by the model of choose_split
 
 // what one call does, from its flags and the process defaults
@@ -674,7 +674,7 @@ int decide_pack(const mpl_shape* s, const Params& p, const CallOpts& o) {
 // the greatest.
 //   * up to 64 labels: TRWP 256 chains 0.78 / 1.65, 768 chains with 33 labels 0.75 / 1.2, ISGMR 0.69 / 1.5.
 //     With one label per lane the step of mp_bwd.hip is short, and labels that point anywhere cost this
-//     kernel more (64 labels, dunary alone: 199 ns per pixel and walk there, 245 here).
+//     kernel more (64 labels, dunary alone: 199 ns per pixel and walk there, 245 here).  Never taken.
 //   * TRWP: 65 to 128 labels 768 chains 1.19 / 2.2, 192 labels 1.15 / 1.77, 256 labels 0.98 / 1.5 (576
 //     chains 1.06 / 1.5).
 //   * TRWP, labels loaded and stored one by one (their number no multiple of the labels per lane), which
@@ -686,7 +686,7 @@ int decide_pack(const mpl_shape* s, const Params& p, const CallOpts& o) {
 //     chains 1.31 / 2.2, 512 chains 0.98 / 1.8, 640 chains 0.81 / 1.4.
 int team_chains_per_cu(int L, bool jacobi) {
   const int R = labels_per_lane(L);
-  if (R == 1) return 0;
+  if (R == 1) return 0;  // (not compiled)
   if (jacobi) return R == 4 ? 1 : 2;
   if (L % R != 0) {  // labels one by one
     if (R == 4) return L <= 216 ? 2 : 1;
@@ -696,7 +696,7 @@ int team_chains_per_cu(int L, bool jacobi) {
 }
 
 int decide_team(const BackParams& p, const CallOpts& o, bool jacobi) {
-  if (p.pack >= 2 || p.ctx2d || o.team == 0) return 0;
+  if (p.pack >= 2 || p.ctx2d || p.L <= kWave || o.team == 0) return 0;
   if (o.team == 2) return 1;
   const int cus = launch_policy().n_simd / 4;
   return p.block_prefix[p.n_dirs] <= team_chains_per_cu(p.L, jacobi) * cus ? 1 : 0;
@@ -768,7 +768,6 @@ void launch_bwd(const BackParams& p, bool jacobi, hipStream_t st) {
   }
   if (p.team) {
     switch (labels_per_lane(p.L)) {
-      case 1: launch_team_bwd<1>(p, jacobi, st); break;
       case 2: launch_team_bwd<2>(p, jacobi, st); break;
       case 3: launch_team_bwd<3>(p, jacobi, st); break;
       default: launch_team_bwd<4>(p, jacobi, st); break;

@@ -1,5 +1,5 @@
-// Reverse scan of TRWP / ISGMR with four wavefronts per chain, for launches with fewer chains than
-// the chip has SIMDs.  The recurrence and what each plane holds: mp_bwd.hip.
+// Reverse scan of TRWP / ISGMR with four wavefronts per chain, for more than 64 labels with a 1-D table
+// in launches with fewer chains than the chip has SIMDs.  The recurrence and what each plane holds: mp_bwd.hip.
 //
 // What bounds such a launch is the length of one pixel's step, not memory: a wavefront that has its
 // SIMD to itself issues one instruction every four clocks, and the step of mp_bwd.hip is some 240
@@ -32,7 +32,7 @@
 // 500x800x192).  With every scatter through LDS float adds 3.74 ms.  Which launches take it:
 // team_chains_per_cu (mp_api.hip).
 //
-// Compiled once per R (labels per lane) with -DMPL_INST_R=<R>.
+// Compiled once per R (labels per lane, 2 to 4) with -DMPL_INST_R=<R>.
 
 #include <type_traits>
 
@@ -51,7 +51,7 @@ constexpr int kWin = 2;                  // labels on either side whose gradient
 // Slot of a pixel, per lane: the gradient of the message without what the recurrence adds and the
 // codes of its labels (one 16-byte read for up to three labels), the argmin labels, dU of the pixel
 // (main wavefront) and A' (even walk).
-constexpr int in_words(int R) { return R == 1 ? 2 : (R == 4 ? 8 : 4); }
+constexpr int in_words(int R) { return R == 4 ? 8 : 4; }
 constexpr int vec_words(int R) { return R == 3 ? 4 : R; }
 template <int R>
 struct alignas(16) Slot {
@@ -189,13 +189,11 @@ __device__ __forceinline__ void lds_get(const float* src, float (&x)[N]) {
     const f32x4 v = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll
     for (int i = 0; i < 4; ++i) x[i] = v[i];
-  } else if constexpr (N == 2) {
+  } else {
+    static_assert(N == 2, "words of a slot come in twos and fours");
     const f32x2 v = *reinterpret_cast<const f32x2*>(src);
     x[0] = v[0];
     x[1] = v[1];
-  } else {
-#pragma unroll
-    for (int i = 0; i < N; ++i) x[i] = src[i];
   }
 }
 template <int N>
@@ -204,10 +202,9 @@ __device__ __forceinline__ void lds_put(float* dst, const float (&x)[N]) {
     *reinterpret_cast<f32x4*>(dst) = f32x4{x[0], x[1], x[2], x[3]};
   } else if constexpr (N == 3) {
     *reinterpret_cast<f32x4*>(dst) = f32x4{x[0], x[1], x[2], 0.f};
-  } else if constexpr (N == 2) {
-    *reinterpret_cast<f32x2*>(dst) = f32x2{x[0], x[1]};
   } else {
-    dst[0] = x[0];
+    static_assert(N == 2, "words of a slot come in twos and fours");
+    *reinterpret_cast<f32x2*>(dst) = f32x2{x[0], x[1]};
   }
 }
 // an R-label vector of a slot (three labels: padded to four words)
@@ -228,7 +225,7 @@ __device__ __forceinline__ void get_in(const float* src, float (&base)[R], int& 
     code = __builtin_bit_cast(int, t[0]);
     rest = __builtin_bit_cast(int, t[1]);
   } else {
-    float t[R == 1 ? 2 : 4];
+    float t[4];
     lds_get(src, t);
 #pragma unroll
     for (int j = 0; j < R; ++j) base[j] = t[j];
@@ -243,9 +240,9 @@ __device__ __forceinline__ void put_in(float* dst, const float (&base)[R], int c
     lds_put(dst, base);
     lds_put(dst + 4, t);
   } else {
-    float t[R == 1 ? 2 : 4];
+    float t[4];
 #pragma unroll
-    for (int j = 0; j < (R == 1 ? 2 : 4); ++j) t[j] = j < R ? base[j < R ? j : 0] : c;
+    for (int j = 0; j < 4; ++j) t[j] = j < R ? base[j < R ? j : 0] : c;
     lds_put(dst, t);
   }
 }
@@ -645,12 +642,13 @@ void launch_vj(const BackParams& p, hipStream_t st) {
 template <int R>
 void launch_team_bwd(const BackParams& p, bool jacobi, hipStream_t st) {
   if (p.block_prefix[p.n_dirs] <= 0) return;
-  if (R == 1 || p.L % R == 0) {
+  static_assert(R > 1, "several labels per lane");
+  if (p.L % R == 0) {
     if (jacobi)
       launch_vj<R, true, true>(p, st);
     else
       launch_vj<R, true, false>(p, st);
-  } else if constexpr (R > 1) {
+  } else {
     if (jacobi)
       launch_vj<R, false, true>(p, st);
     else

@@ -39,10 +39,10 @@ def test_planes_of_the_pairs(gpu, oracle, n_dir, n_iter, L):
 @pytest.mark.parametrize("mode,n_dir", [("TRWP", 4), ("TRWP", 16), ("ISGMR", 8)])
 @pytest.mark.parametrize("L", [1, 2, 5, 63, 64, 65, 96, 128, 131, 191, 192, 193, 254, 256])
 def test_several_wavefronts_per_chain(gpu, oracle, mode, n_dir, L, kind):
-  """The reverse scan that puts four wavefronts on a chain (MPL_OPT_TEAM_SCANS): label counts at the
-  edges of a lane's labels, chains of 1 to 13 pixels (a block has six), argmin labels anywhere, in the
-  register window or one step outside it with a shared far target (where the two ways of scattering
-  meet), all combinations of wanted gradients."""
+  """The reverse scan that puts four wavefronts on a chain (MPL_OPT_TEAM_SCANS; up to 64 labels one
+  wavefront runs whatever the option): label counts at the edges of a lane's labels, chains of 1 to 13
+  pixels (a block has six), argmin labels anywhere, in the register window or one step outside it with
+  a shared far target (where the two ways of scattering meet), all combinations of wanted gradients."""
   from mplayers_amd import _lib
   rng = np.random.default_rng(1000 * L + n_dir)
   B, H, W, n_iter, rho = 1, 7, 13, 2, (0.5 if mode == "TRWP" else 1.0)
@@ -93,7 +93,7 @@ def test_kernels_of_a_call_differ_by_direction(gpu, oracle, L):
     assert np.abs(g.reshape(r.shape) - r).max() <= 1e-4 * max(1.0, np.abs(r).max()), name
 
 
-@pytest.mark.parametrize("L", [49, 70, 131, 256])
+@pytest.mark.parametrize("L", [65, 70, 131, 256])
 def test_every_place_of_the_main_wavefront(gpu, oracle, L):
   """Which of the four wavefronts of a chain runs the recurrence changes with the workgroup's number
   over the number of compute units: 7 x 8 x 16 pixels give one ISGMR launch of 8 directions 980 chains,
