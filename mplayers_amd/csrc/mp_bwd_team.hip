@@ -2,9 +2,9 @@
 // in launches with fewer chains than the chip has SIMDs.  The recurrence and what each plane holds: mp_bwd.hip.
 //
 // What bounds such a launch is the length of one pixel's step, not memory: a wavefront that has its
-// SIMD to itself issues one instruction every four clocks, and the step of mp_bwd.hip is some 240
-// instructions (R = 3; 382 issue slots with its waits), of which the next pixel waits for perhaps a
-// third.  So the work is divided by what the recurrence needs:
+// SIMD to itself issues one instruction every four clocks, and the step of mp_bwd.hip is some 230
+// instructions (R = 3, dunary alone; 374 issue slots with its waits), of which the next pixel waits for
+// perhaps a third.  So the work is divided by what the recurrence needs:
 //   * three helper wavefronts, every third pixel each, load the planes, form the gradient terms that
 //     do not depend on the recurrence and the addresses of the scatter, and put them into an LDS slot
 //     per pixel; two blocks of pixels later they take dU of the pixel from the slot, finish the planes
@@ -21,16 +21,20 @@
 // the ones that share a target (one bit); the main wavefront adds up masked neighbours from registers
 // and sums the others with the wave reduction that the normalisation needs anyway (two interleaved
 // chains of lane shifts).  A pixel with any other argmin label (dense tables) scatters through LDS
-// float adds, which cost some 300 clocks each.  The normalisation (g[norm_index] -= sum g) reaches
+// float adds (R = 3: 447 instead of 242 ns per pixel and walk, R = 2: 365 instead of 211, where every
+// pixel does).  The normalisation (g[norm_index] -= sum g) reaches
 // dU through its argmin label only, and is subtracted there.
 //
 // Measured, TRWP backward on 4 directions, 5 iterations, min(k, 3) table, one wavefront per chain ->
-// this: 256x512x192 5.16 -> 2.12 ms (276 ns per pixel and walk: the main wavefront's 115 instructions,
-// five clocks each, 264 ns by itself), with dedge_weights and dcontext 7.18 -> 3.81, 500x800x192
-// 8.91 -> 5.87; dense table 240x320x96 with dcontext 5.95 -> 3.18.  Two pixels per helper and block, three
-// helpers: one pixel 2.14, four 2.36, seven helpers of one pixel 2.11 (and 6.2 instead of 5.9 ms at
-// 500x800x192).  With every scatter through LDS float adds 3.74 ms.  Which launches take it:
-// team_chains_per_cu (mp_api.hip).
+// this: 256x512x192 5.16 -> 2.12 ms (rows of 256 chains: 645 -> 246 ns per pixel and walk; the main
+// wavefront issues 112 instructions per pixel, some five clocks each), with dedge_weights and dcontext
+// 7.18 -> 3.81, 500x800x192 8.91 -> 5.87; bent table 240x320x96 with dcontext 5.95 -> 3.18.  Two pixels
+// per helper and block, three helpers: one pixel 2.14, four 2.36, seven helpers of one pixel 2.11 (and
+// 6.2 instead of 5.9 ms at 500x800x192).  With every scatter through LDS float adds 3.74 ms.  Errors
+// against 64 bits (argmin labels of the forward scan, 61 problems up to 300x450x192 and 32x2000x192,
+// geometric means of the relative 2-norm, one wavefront -> four): TRWP dunary 1.43e-7 -> 1.40e-7, dcontext
+// 1.07e-6 -> 0.91e-6, dedge_weights 1.41e-7 -> 1.40e-7, ISGMR smaller by a tenth to two fifths.  Which
+// launches take it: team_chains_per_cu (mp_api.hip).
 //
 // Compiled once per R (labels per lane, 2 to 4) with -DMPL_INST_R=<R>.
 
@@ -47,6 +51,13 @@ constexpr int kT = kHelpers * kPer;      // pixels per block
 constexpr int kTeam = (kHelpers + 1) * kWave;
 
 constexpr int kWin = 2;                  // labels on either side whose gradients move in registers
+
+// dcontext of a helper's pixels, in LDS: a word per bin, but for the bins up to kNearBins one per lane
+// (two with four labels per lane).  Most labels of a pixel may lie that near their argmin label; in one
+// word a long chain's sum loses digits, and the adds of a pixel wait for each other.
+constexpr int kNearBins = 3;
+constexpr int near_words(int R) { return R == 4 ? 2 * kWave : kWave; }  // per bin
+constexpr int hist_floats(int R, int n_ctx) { return (kNearBins + 1) * near_words(R) + n_ctx; }
 
 // Slot of a pixel, per lane: the gradient of the message without what the recurrence adds and the
 // codes of its labels (one 16-byte read for up to three labels), the argmin labels, dU of the pixel
@@ -268,7 +279,7 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
   float* ctx_s = acc + kAccFloats;
   const int L = p.L;
   const int n_ctx = L;  // (1-D tables only)
-  float* hist_s = ctx_s + n_ctx;
+  float* hist_s = ctx_s + n_ctx;  // dcontext, one histogram per helper
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   // which wavefront is the main one: workgroups that share a compute unit are as many apart as the chip
@@ -286,11 +297,11 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
   const bool same = p.same_label != 0;
 
   for (int i = tid; i < kAccFloats; i += kTeam) acc[i] = 0.f;
-  if (GR)
-    for (int i = tid; i < n_ctx; i += kTeam) {
-      ctx_s[i] = p.ctx[i];
-      hist_s[i] = 0.f;
-    }
+  const int n_hist = hist_floats(R, n_ctx);
+  if (GR) {
+    for (int i = tid; i < n_ctx; i += kTeam) ctx_s[i] = p.ctx[i];
+    for (int i = tid; i < kHelpers * n_hist; i += kTeam) hist_s[i] = 0.f;
+  }
   __syncthreads();
 
   const int blocks = (n + kT - 1) / kT;
@@ -535,6 +546,7 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
           const int fds = s.fds[lane];
           const int nidx = sv.nidx;
           de_old = sv.de;
+          float* const hist = hist_s + role * n_hist;
 #pragma unroll
           for (int j = 0; j < R; ++j) {
             const int cd = lab0 + j;
@@ -544,7 +556,9 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
             const int ci = fd > cd ? fd - cd : cd - fd;
             if (cd < L) {
               det = fmaf(ctx_s[ci], g, det);
-              if (want_dc && (same || cd != fd)) atomicAdd(&hist_s[ci], w * g);
+              const int near = ci * near_words(R) + (j * kWave) % near_words(R) + lane;
+              const int at = ci <= kNearBins ? near : (kNearBins + 1) * near_words(R) + ci;
+              if (want_dc && (same || cd != fd)) atomicAdd(&hist[at], w * g);
             }
           }
           if (want_de) det = wave_sum_fast(det);
@@ -618,8 +632,21 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
   }
   if (!want_dc) return;
   __syncthreads();
+  if (!is_main) {  // the words of a near bin into its place in the histogram
+    float* const hist = hist_s + role * n_hist;
+#pragma unroll
+    for (int o = 0; o <= kNearBins; ++o) {
+      float v = hist[o * near_words(R) + lane];
+      if (R == 4) v += hist[o * near_words(R) + kWave + lane];
+      v = wave_sum(v);
+      if (lane == 0) hist[(kNearBins + 1) * near_words(R) + o] = v;
+    }
+  }
+  __syncthreads();
   for (int i = tid; i < n_ctx; i += kTeam) {
-    const float v = hist_s[i];
+    float v = 0.f;
+#pragma unroll
+    for (int h = 0; h < kHelpers; ++h) v += hist_s[h * n_hist + (kNearBins + 1) * near_words(R) + i];
     if (v != 0.f) atomicAdd(&p.dctx[i], v);
   }
 }
@@ -630,7 +657,7 @@ void launch_vj(const BackParams& p, hipStream_t st) {
   const bool gr = p.dedge != nullptr || p.dctx != nullptr;
   const int n_cu = launch_policy().n_simd / 4;
   const size_t lds = 2 * kT * (sizeof(Slot<R>) + sizeof(Scalars)) +
-                     sizeof(float) * (kAccFloats + (gr ? 2 * p.L : 0));
+                     sizeof(float) * (kAccFloats + (gr ? p.L + kHelpers * hist_floats(R, p.L) : 0));
   if (gr)
     sweep_bwd_team_kernel<R, VEC, JACOBI, true><<<blocks, kTeam, lds, st>>>(p, n_cu);
   else

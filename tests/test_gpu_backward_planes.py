@@ -121,3 +121,39 @@ def test_every_place_of_the_main_wavefront(gpu, oracle, L):
   for name, g, r in zip(("dunary", "dcontext", "dedge"), got, ref):
     # the gradient bar of the GPU tests: 1e-4 of the largest entry
     assert np.abs(g.reshape(r.shape) - r).max() <= 1e-4 * max(1.0, np.abs(r).max()), name
+
+
+@pytest.mark.parametrize("option", [0, 2])
+@pytest.mark.parametrize("offset", [1, 2, 3])
+@pytest.mark.parametrize("L", [70, 192, 256])
+def test_table_gradient_of_a_long_chain(gpu, L, offset, option):
+  """One entry of the table collects nearly every label of every pixel of a chain of 4000, all terms
+  positive (rho = 0: every gradient is the upstream one; the label that the normalisation makes
+  negative points elsewhere).  A scan sums them in at least a word per lane."""
+  from mplayers_amd import _lib
+  rng = np.random.default_rng(L + offset)
+  n, n_dir = 4000, 2
+  ctx = rng.random(L).astype(np.float32)
+  ew = (0.1 + 0.9 * rng.random((n_dir, 1, 1, 1, n))).astype(np.float32)
+  dcost = (0.5 + 0.5 * rng.random((1, 1, 1, n, L))).astype(np.float32)
+  label = np.arange(L)
+  target = np.where(label + offset < L, label + offset, label)
+  norm = L // 2
+  target[norm] = 0
+  imin = np.broadcast_to(target, (1, n_dir, 1, 1, 1, n, L)).astype(np.uint8)
+  inorm = np.full((1, n_dir, 1, 1, 1, n), norm, np.uint8)
+  # pixels with an incoming edge: all but the first of either direction
+  term = dcost[0, 0, 0].astype(np.float64)[:, (target == label + offset) & (label != norm)].sum(-1)
+  exact = (ew[0, 0, 0, 0, 1:] * term[1:]).sum() + (ew[1, 0, 0, 0, :-1] * term[:-1]).sum()
+  print("case", L, offset, option, flush=True)
+  _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+  try:
+    got = gpu.gpu_backward("ISGMR", ctx, ew, dcost, imin, inorm, 0.0)[1]
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+  # m positive additions into one word round to a relative error of about sqrt(m) * 2^-24 (each rounds
+  # either way); the 64 words of a wavefront average to an eighth of that.  One wavefront adds its
+  # lane's labels first (m = n), each of three helpers every label of a lane (m = n / 3 per label).  A
+  # word for all labels would see m = n L.
+  m = n * (-(-L // 64)) / (3 if option else 1)
+  assert abs(got[offset] - exact) <= m ** 0.5 * 2.0 ** -24 * exact, (got[offset] - exact) / exact
