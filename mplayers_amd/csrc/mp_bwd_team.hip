@@ -20,21 +20,24 @@
 // which of its neighbours up to kWin labels away point at it (five bits) and whether it belongs to
 // the ones that share a target (one bit); the main wavefront adds up masked neighbours from registers
 // and sums the others with the wave reduction that the normalisation needs anyway (two interleaved
-// chains of lane shifts).  A pixel with any other argmin label (dense tables) scatters through LDS
-// float adds (R = 3: 447 instead of 242 ns per pixel and walk, R = 2: 365 instead of 211, where every
-// pixel does).  The normalisation (g[norm_index] -= sum g) reaches
-// dU through its argmin label only, and is subtracted there.
+// chains of lane shifts).  Where labels are left that share a second target (either side of a slope
+// under a linear table) another wave reduction sums them; a pixel with any further argmin label scatters
+// through LDS float adds.  The normalisation (g[norm_index] -= sum g) reaches dU through its argmin label
+// only, and is subtracted there.
 //
 // Measured, TRWP backward on 4 directions, 5 iterations, min(k, 3) table, one wavefront per chain ->
 // this: 256x512x192 5.16 -> 2.12 ms (rows of 256 chains: 645 -> 246 ns per pixel and walk; the main
 // wavefront issues 112 instructions per pixel, some five clocks each), with dedge_weights and dcontext
-// 7.18 -> 3.81, 500x800x192 8.91 -> 5.87; bent table 240x320x96 with dcontext 5.95 -> 3.18.  Two pixels
-// per helper and block, three helpers: one pixel 2.14, four 2.36, seven helpers of one pixel 2.11 (and
-// 6.2 instead of 5.9 ms at 500x800x192).  With every scatter through LDS float adds 3.74 ms.  Errors
-// against 64 bits (argmin labels of the forward scan, 61 problems up to 300x450x192 and 32x2000x192,
-// geometric means of the relative 2-norm, one wavefront -> four): TRWP dunary 1.43e-7 -> 1.40e-7, dcontext
-// 1.07e-6 -> 0.91e-6, dedge_weights 1.41e-7 -> 1.40e-7, ISGMR smaller by a tenth to two fifths.  Which
-// launches take it: team_chains_per_cu (mp_api.hip).
+// 7.18 -> 3.8, 500x800x192 8.91 -> 5.87; bent table 240x320x96 with dcontext 5.95 -> 3.18.  Argmin labels
+// anywhere, so that every pixel scatters through LDS adds, 459 instead of 243 ns with 192 labels.  Two
+// pixels per helper and block, three helpers: one pixel 2.14, four 2.36, seven helpers of one pixel 2.11
+// (and 6.2 instead of 5.9 ms at 500x800x192).  Which launches take it: team_chains_per_cu (mp_api.hip).
+//
+// Errors against 64 bits, one wavefront -> four, geometric means of the relative 2-norm over bands, a bent
+// band, linear and random tables, gradients of a cross entropy, normal and positive ones, 65 to 254
+// labels, images up to 300x450, chains up to 8000 pixels: TRWP dunary 1.47e-7 -> 1.42e-7, dcontext
+// 8.4e-7 -> 6.8e-7, dedge_weights 1.46e-7 both; ISGMR 2.49e-7 -> 2.31e-7, 4.1e-7 -> 3.8e-7, 1.35e-7 ->
+// 1.33e-7; by table and kind of gradient 0.71 to 1.04 times the former.
 //
 // Compiled once per R (labels per lane, 2 to 4) with -DMPL_INST_R=<R>.
 
@@ -80,9 +83,12 @@ struct Scalars {
 constexpr int kPop = 5;    // l points at the shared target,
 constexpr int kIsPop = 6;  // l is the shared target,
 constexpr int kIsNrm = 7;  // l is the argmin label of the normalisation label
-// in every lane's word, with up to three labels (bit 24) or the word after it: some argmin label of the
-// pixel is neither near nor the shared one
-constexpr int kRest = 24;
+// in every lane's word, with up to three labels (from bit 24 on), or the word after it:
+constexpr int kRest = 24;  // some argmin label of the pixel is neither near nor the shared one,
+constexpr int kMore = 31;  // nor the second shared one,
+// and, where kMore is not set, of label j of the lane
+constexpr int pop2_bit(int R) { return R == 4 ? 0 : 25; }    // (+ j) it points at the second shared target,
+constexpr int is_pop2_bit(int R) { return R == 4 ? 4 : 28; }  // (+ j) it is the second shared target
 
 constexpr int kAccFloats = kMaxL + kWave;  // one per label, one spare word per lane
 
@@ -342,12 +348,28 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
           });
           wave_sum2(part, pop);
           float near[R];
-          if (__builtin_expect((__builtin_amdgcn_readfirstlane(rest) & (1 << kRest)) == 0, 1)) {
+          auto near_sums = [&]() __attribute__((always_inline)) {
             float nb[R + 2 * kWin];
             neighbours<R>(g, nb);
             static_for<R>([&](auto jj) __attribute__((always_inline)) {
               constexpr int j = decltype(jj)::value;
               near[j] = window_sum<8 * j>(code, nb[j], nb[j + 1], nb[j + 2], nb[j + 3], nb[j + 4]);
+            });
+          };
+          const int kind = __builtin_amdgcn_readfirstlane(rest);
+          if (__builtin_expect((kind & (1 << kRest)) == 0, 1)) {
+            near_sums();
+          } else if (kind >= 0) {  // (bit kMore) two shared targets
+            near_sums();
+            float pop2 = 0.f;
+            static_for<R>([&](auto jj) __attribute__((always_inline)) {
+              constexpr int j = decltype(jj)::value;
+              pop2 += if_bit<pop2_bit(R) + j>(rest, g[j]);
+            });
+            pop2 = wave_sum_fast(pop2);
+            static_for<R>([&](auto jj) __attribute__((always_inline)) {
+              constexpr int j = decltype(jj)::value;
+              near[j] += if_bit<is_pop2_bit(R) + j>(rest, pop2);
             });
           } else {
             const int fds = s[i].fds[lane];
@@ -487,7 +509,7 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
       int nb[R + 2 * kWin];
       neighbours<R>(src, nb);
       int code = 0;
-      bool left = false;
+      bool left[R];
       float base[R], ap[R];
 #pragma unroll
       for (int j = 0; j < R; ++j) {
@@ -496,7 +518,7 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
 #pragma unroll
         for (int b = 0; b <= 2 * kWin; ++b) c |= nb[j + b] & (1 << b);
         const bool is_pop = out[j] && px.fd[j] == pop;
-        left |= out[j] && !is_pop;
+        left[j] = out[j] && !is_pop;
         c |= is_pop ? 1 << kPop : 0;
         c |= l == pop ? 1 << kIsPop : 0;
         c |= l == fn ? 1 << kIsNrm : 0;
@@ -505,7 +527,30 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
         base[j] = JACOBI ? px.a[j] : ap[j] + (EVEN ? -px.hd[j] - px.hi[j] : px.hd[j]);
         if (l >= L) base[j] = 0.f;
       }
-      put_in<R>(s.in[lane], base, code, ballot(left) != 0 ? 1 << kRest : 0);
+      // of the others, those that point where the last of them does
+      bool any_left = left[0];
+#pragma unroll
+      for (int j = 1; j < R; ++j) any_left |= left[j];
+      int rest = 0;
+      const uint64_t lm = ballot(any_left);
+      if (lm != 0) {
+        const int last = 63 - __builtin_clzll(lm);
+        int fl = 0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) fl = left[j] ? px.fd[j] : fl;
+        const int pop2 = __builtin_amdgcn_readlane(fl, last);
+        bool more = false;
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          const bool is_pop2 = left[j] && px.fd[j] == pop2;
+          more |= left[j] && !is_pop2;
+          rest |= is_pop2 ? 1 << (pop2_bit(R) + j) : 0;
+          rest |= lab0 + j == pop2 ? 1 << (is_pop2_bit(R) + j) : 0;
+        }
+        rest |= 1 << kRest;
+        if (ballot(more) != 0) rest |= 1 << kMore;
+      }
+      put_in<R>(s.in[lane], base, code, rest);
       s.fds[lane] = fds;
       if (EVEN) lds_put(s.ap[lane], ap);
       if (GR) {

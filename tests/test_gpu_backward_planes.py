@@ -35,14 +35,15 @@ def test_planes_of_the_pairs(gpu, oracle, n_dir, n_iter, L):
       assert np.abs(g.reshape(r.shape) - r).max() <= 1e-4 * max(1.0, np.abs(r).max()), (name, flags)
 
 
-@pytest.mark.parametrize("kind", ["any", "band", "one_far"])
+@pytest.mark.parametrize("kind", ["any", "band", "one_far", "two_far"])
 @pytest.mark.parametrize("mode,n_dir", [("TRWP", 4), ("TRWP", 16), ("ISGMR", 8)])
 @pytest.mark.parametrize("L", [1, 2, 5, 63, 64, 65, 96, 128, 131, 191, 192, 193, 254, 256])
 def test_several_wavefronts_per_chain(gpu, oracle, mode, n_dir, L, kind):
   """The reverse scan that puts four wavefronts on a chain (MPL_OPT_TEAM_SCANS; up to 64 labels one
   wavefront runs whatever the option): label counts at the edges of a lane's labels, chains of 1 to 13
   pixels (a block has six), argmin labels anywhere, in the register window or one step outside it with
-  a shared far target (where the two ways of scattering meet), all combinations of wanted gradients."""
+  a shared far target (where the ways of scattering meet) or with two of them, all combinations of
+  wanted gradients."""
   from mplayers_amd import _lib
   rng = np.random.default_rng(1000 * L + n_dir)
   B, H, W, n_iter, rho = 1, 7, 13, 2, (0.5 if mode == "TRWP" else 1.0)
@@ -51,9 +52,11 @@ def test_several_wavefronts_per_chain(gpu, oracle, mode, n_dir, L, kind):
   dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
   imin = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W, L))
   if kind != "any":
-    reach = 2 if kind == "band" else 3
+    reach = 3 if kind == "one_far" else 2
     near = np.clip(np.arange(L) + rng.integers(-reach, reach + 1, imin.shape), 0, L - 1)
     far = np.broadcast_to(imin[..., :1], imin.shape)
+    if kind == "two_far":
+      far = np.where(rng.random(imin.shape) < 0.5, far, imin[..., -1:])
     imin = np.where(rng.random(imin.shape) < 0.6, far, near)
   imin = imin.astype(np.uint8)
   inorm = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W)).astype(np.uint8)
@@ -157,3 +160,37 @@ def test_table_gradient_of_a_long_chain(gpu, L, offset, option):
   # word for all labels would see m = n L.
   m = n * (-(-L // 64)) / (3 if option else 1)
   assert abs(got[offset] - exact) <= m ** 0.5 * 2.0 ** -24 * exact, (got[offset] - exact) / exact
+
+
+@pytest.mark.parametrize("option", [0, 2])
+@pytest.mark.parametrize("L", [128, 192, 256])
+def test_two_targets_share_the_labels(gpu, L, option):
+  """Half of the labels of every pixel point at one label, half at another, as either side of a slope
+  under a linear table.  Chains of two pixels (and the label that the normalisation changes points
+  elsewhere), so a gradient is one sum of random terms and its error shows how it was formed."""
+  from mplayers_amd import _lib
+  rng = np.random.default_rng(L)
+  n_dir, H, W = 2, 400, 2
+  ctx = rng.random(L).astype(np.float32)
+  dcost = rng.standard_normal((1, 1, H, W, L)).astype(np.float32)
+  low, high, norm = L // 4, 3 * L // 4, L // 2
+  target = np.where(np.arange(L) < norm, low, high)
+  target[norm] = norm
+  imin = np.broadcast_to(target, (1, n_dir, 1, 1, H, W, L)).astype(np.uint8)
+  inorm = np.full((1, n_dir, 1, 1, H, W), norm, np.uint8)
+  print("case", L, option, flush=True)
+  _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+  try:
+    got = gpu.gpu_backward("ISGMR", ctx, None, dcost, imin, inorm, 1.0, want_dctx=False, want_dedge=False)[0]
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+  d = dcost[0, 0].astype(np.float64)
+  for label, share in ((low, np.arange(L) < norm), (high, np.arange(L) > norm)):
+    sums = d[:, :, share].sum(-1)
+    exact = d[:, :, label] + sums[:, ::-1]  # a pixel's sum goes to its neighbour
+    err = np.linalg.norm(got[0, 0, :, :, label] - exact) / np.linalg.norm(exact) * 2 ** 24
+    # an addition rounds its sum by some 0.42 * 2^-24 in the root mean square.  In a tree over the lanes
+    # every level's sums have the variance of the whole: nine levels (six of lanes, up to two in a lane, the
+    # upstream gradient) come to 0.42 * 3 = 1.26.  One after the other, 63 to 127 additions of growing
+    # sums come to 0.42 sqrt(n / 2), 2.4 to 3.4
+    assert err <= 1.75, err
