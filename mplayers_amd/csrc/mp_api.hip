@@ -320,6 +320,8 @@ __global__ void __launch_bounds__(256) label_kernel(const float* __restrict__ un
 // The sums are formed in the order of those kernels: the same bits.  50 iterations on 375x450x60 with all
 // labels, passes apart -> together: TRWP, 8 directions 33.2 -> 32.4 ms, 4 directions 15.8 -> 15.4; ISGMR,
 // 8 directions 19.6 -> 16.8 ms (16 labels 7.03 -> 6.39), 4 directions 11.1 -> 10.9 (its scans form U).
+// The loads of all planes going out back to back are not what gives it: 10 iterations, TRWP 6.20 -> 5.99 ms
+// and ISGMR 3.75 -> 3.19, but 6.18 -> 6.14 and 3.76 -> 3.72 with min_a_dir, where nothing is merged.
 constexpr int kLabelOnly = 0, kLabelSum = 1, kLabelU = 2;
 template <int ND, int OUT>
 __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict__ unary,
@@ -409,7 +411,9 @@ static bool launch_labels(const float* unary, const float* msg, int n_dir, int64
   while (group * 4 < L) group <<= 1;
   const unsigned blocks = (unsigned)((P * group + 255) / 256);
   const bool known = n_dir == 4 || n_dir == 8 || n_dir == 16;
-  // (a factor other than one rounds in the product and is left to the pass of its own)
+  // SGM's factor (the number of directions) is left to the pass of its own: it belongs to a single
+  // iteration, and where it is no power of two its product rounds, or not, as either kernel fuses it into
+  // the first sum
   if (min_a_dir || factor != 1.f || out == nullptr || ((uintptr_t)out & 15) != 0 ||
       (want == kLabelU && !known))
     want = kLabelOnly;

@@ -116,7 +116,6 @@ __global__ void __launch_bounds__(kWave) sweep_bwd_kernel(const BackParams p) {
   // even_walk: a constant; which of the two walks of a pair this is (Gauss-Seidel)
   auto walk = [&](const ChainCtx& ch, const auto even_walk) __attribute__((always_inline)) {
   constexpr bool EVEN = !JACOBI && decltype(even_walk)::value;
-  constexpr bool ODD = !JACOBI && !EVEN;
   const int dir = ch.dir;
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t img_p = (int64_t)ch.bv * HW;  // first pixel of this batch item
