@@ -670,33 +670,35 @@ int decide_pack(const mpl_shape* s, const Params& p, const CallOpts& o) {
 // Four wavefronts per chain in the reverse scans (mp_bwd_team.hip): chains per compute unit up to which
 // a launch takes them, 0 for never.  The time of such a launch steps up with every further chain per
 // compute unit, so the lines lie between those steps, where no kind of call measured slower than with
-// one wavefront per chain.  The table and which gradients are wanted change the ratio but may not change
-// the route: the table is not known here, and dunary is promised to be the same bits whichever gradients
-// are wanted.  Measured, backward of 2 iterations on square images (TRWP: 256, 512 and 768 chains per
-// launch; ISGMR: all directions in one), time with one over time with four wavefronts: the least of
-// dunary alone and of all gradients on a band of four labels, a bent band, a linear and a random table /
-// the greatest.
+// one wavefront per chain by more than two runs of it differ.  The table and which gradients are wanted
+// change the ratio but may not change the route: the table is not known here, and dunary is promised to be
+// the same bits whichever gradients are wanted.  Measured, backward of 2 iterations on square images with
+// 4, 8 and 16 directions (TRWP: chains of one direction per launch, ISGMR: of all), time with one over
+// time with four wavefronts: the least of dunary alone and of all gradients on a band of four labels, a
+// bent band, a linear and a random table / the greatest.
 //   * up to 64 labels: TRWP 256 chains 0.78 / 1.65, 768 chains with 33 labels 0.75 / 1.2, ISGMR 0.69 / 1.5.
 //     With one label per lane the step of mp_bwd.hip is short, and labels that point anywhere cost this
 //     kernel more (64 labels, dunary alone: 199 ns per pixel and walk there, 245 here).  Never taken.
-//   * TRWP: 65 to 128 labels 768 chains 1.19 / 2.2, 192 labels 1.15 / 1.77, 256 labels 0.98 / 1.5 (576
-//     chains 1.06 / 1.5).
-//   * TRWP, labels loaded and stored one by one (their number no multiple of the labels per lane), which
-//     gains less where several chains share a compute unit: 127 labels 768 chains 1.21 / 1.87; 152 / 158
-//     / 190 labels 768 chains 1.04 / 1.65, 0.98 / 1.60, 0.83 / 1.44, 190 labels 512 chains 1.34 / 2.1;
-//     193 and 215 labels 512 chains 1.14 / 2.0, 768 chains 0.72 / 1.3; 217 labels 512 chains 1.01 / 1.82;
-//     255 labels 256 / 512 chains 1.62 / 2.33 and 0.78 / 1.84.
-//   * ISGMR: 512 chains with 65 to 192 labels 1.04 / 2.0, 640 to 768 chains 0.87 / 1.9; 256 labels 256
-//     chains 1.31 / 2.2, 512 chains 0.98 / 1.8, 640 chains 0.81 / 1.4.
+//   * TRWP, 768 chains: 65 labels 1.12 / 2.2, 128 labels 1.23 / 2.0, 192 labels 1.17 / 1.84, 224 labels
+//     1.21 / 1.63, 256 labels 1.04 / 1.38; 800 chains: 65 labels 0.95 / 1.8, 256 labels 0.88 / 1.25; 832
+//     chains: 192 labels 0.95 / 1.34.
+//   * Labels loaded and stored one by one (their number no multiple of the labels per lane), which gains
+//     less where several chains share a compute unit.  TRWP: 127 labels 768 chains 1.21 / 1.9; 152 / 158 / 190
+//     labels 768 chains 1.04 / 1.64, 0.99 / 1.59, 0.83 / 1.44, 190 labels 512 chains 1.35 / 2.1; 193 labels
+//     512 / 528 chains 1.14 / 2.0 and 0.89 / 1.31, 215 labels 1.02 / 1.81 and 0.79 / 1.32; 255 labels 256 /
+//     384 / 512 chains 1.59 / 2.3, 0.97 / 1.71 and 0.78 / 1.45.  ISGMR: 191 labels 764 chains 1.05 / 1.37; 193
+//     labels 512 chains 1.18 / 1.71; 255 labels 256 / 512 chains 1.48 / 2.0 and 0.95 / 1.54.
+//   * ISGMR, 688 to 768 chains: 65 labels 0.98 / 1.9, 96 labels 1.06 / 1.6, 128 labels 0.99 / 1.46, 160 labels
+//     1.07 / 1.46, 192 labels 0.98 / 1.32; 988 chains 0.91 / 2.1.  256 labels 512 chains 1.03 / 1.48, 640 chains
+//     0.81 / 1.4; 200 labels 500 chains 1.24 / 1.64.
 int team_chains_per_cu(int L, bool jacobi) {
   const int R = labels_per_lane(L);
   if (R == 1) return 0;  // (not compiled)
-  if (jacobi) return R == 4 ? 1 : 2;
-  if (L % R != 0) {  // labels one by one
+  if (L % R != 0) {      // labels one by one
     if (R == 4) return L <= 216 ? 2 : 1;
-    if (R == 3 && L > 152) return 2;
+    if (R == 3 && !jacobi && L > 152) return 2;
   }
-  return 3;
+  return R == 4 && jacobi ? 2 : 3;
 }
 
 int decide_team(const BackParams& p, const CallOpts& o, bool jacobi) {

@@ -12,13 +12,13 @@ pytestmark = pytest.mark.gpu
 CASES = [
     # mode, labels, chains per compute unit, chains more than that, four wavefronts
     ("TRWP", 33, 1, 0, False), ("TRWP", 64, 1, 0, False), ("ISGMR", 64, 1, 0, False),
-    ("TRWP", 65, 3, 0, True), ("TRWP", 128, 3, 1, False), ("ISGMR", 65, 2, 0, True),
-    ("ISGMR", 128, 2, 2, False), ("TRWP", 152, 3, 0, True), ("TRWP", 154, 2, 0, True),
-    ("TRWP", 154, 2, 1, False), ("ISGMR", 190, 2, 0, True), ("TRWP", 192, 3, 0, True),
-    ("TRWP", 192, 3, 1, False), ("ISGMR", 192, 2, 2, False), ("TRWP", 215, 2, 0, True),
+    ("TRWP", 65, 3, 0, True), ("TRWP", 128, 3, 1, False), ("ISGMR", 65, 3, 0, True),
+    ("ISGMR", 128, 3, 2, False), ("TRWP", 152, 3, 0, True), ("TRWP", 154, 2, 0, True),
+    ("TRWP", 154, 2, 1, False), ("ISGMR", 190, 3, 0, True), ("TRWP", 192, 3, 0, True),
+    ("TRWP", 192, 3, 1, False), ("ISGMR", 192, 3, 2, False), ("TRWP", 215, 2, 0, True),
     ("TRWP", 215, 2, 1, False), ("TRWP", 217, 1, 0, True), ("TRWP", 217, 1, 1, False),
-    ("TRWP", 256, 3, 0, True), ("TRWP", 256, 3, 1, False), ("ISGMR", 256, 1, 0, True),
-    ("ISGMR", 256, 1, 2, False),
+    ("TRWP", 256, 3, 0, True), ("TRWP", 256, 3, 1, False), ("ISGMR", 256, 2, 0, True),
+    ("ISGMR", 256, 2, 2, False), ("ISGMR", 255, 1, 0, True), ("ISGMR", 255, 1, 2, False),
 ]
 
 
