@@ -194,3 +194,36 @@ def test_two_targets_share_the_labels(gpu, L, option):
     # upstream gradient) come to 0.42 * 3 = 1.26.  One after the other, 63 to 127 additions of growing
     # sums come to 0.42 sqrt(n / 2), 2.4 to 3.4
     assert err <= 1.75, err
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("mode,L", [("TRWP", 70), ("ISGMR", 96), ("TRWP", 192), ("ISGMR", 254)])
+def test_non_finite_gradients_reach_the_same_entries(gpu, mode, L, value):
+  """An upstream gradient that is not finite shows in every entry of dunary and dedge_weights that it
+  reaches, and in no fewer entries of dcontext, whichever kernel scans; everywhere else nothing is
+  touched.  (The normalisation gives the other sign to one label of the pixel, so sums may be NaN.)"""
+  from mplayers_amd import _lib
+  rng = np.random.default_rng(L)
+  B, H, W, n_dir, n_iter, rho = 1, 6, 11, 4, 1, (0.5 if mode == "TRWP" else 1.0)
+  for k in range(8):
+    ctx = rng.random(L).astype(np.float32)
+    ew = (0.1 + 0.9 * rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+    dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
+    dcost[0, 0, rng.integers(H), rng.integers(W), rng.integers(L)] = value
+    imin = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W, L))
+    near = np.clip(np.arange(L) + rng.integers(-2, 3, imin.shape), 0, L - 1)
+    imin = np.where(rng.random(imin.shape) < (0.6 if k % 2 else 1.0), imin if k % 4 == 0 else imin[..., :1], near)
+    imin = imin.astype(np.uint8)
+    inorm = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W)).astype(np.uint8)
+    print("case", mode, L, value, k, flush=True)
+    out = []
+    for option in (0, 2):
+      _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+      try:
+        out.append(gpu.gpu_backward(mode, ctx, ew, dcost, imin, inorm, rho, garbage_scratch=True))
+      finally:
+        _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+    one, four = out
+    for i, name in ((0, "dunary"), (2, "dedge")):
+      assert np.array_equal(np.isfinite(one[i]), np.isfinite(four[i])), name
+    assert not np.any(np.isfinite(four[1]) & ~np.isfinite(one[1]))
