@@ -692,11 +692,7 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
     float v = 0.f;
 #pragma unroll
     for (int h = 0; h < kHelpers; ++h) v += hist_s[h * n_hist + (kNearBins + 1) * near_words(R) + i];
-    // NaN, the sum of infinite gradients of either sign, is to be added, too; a comparison of floats, which
-    // the compiler would also make of the integer one if it saw where the bits come from, may take it for zero
-    int bits = __builtin_bit_cast(int, v);
-    asm("" : "+v"(bits));
-    if ((bits & 0x7fffffff) != 0) atomicAdd(&p.dctx[i], v);
+    if (has_value(v)) atomicAdd(&p.dctx[i], v);
   }
 }
 

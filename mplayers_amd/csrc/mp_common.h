@@ -94,6 +94,15 @@ __device__ __forceinline__ float uniform_f(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
 }
 
+// Whether a sum has anything to add to an accumulator in memory: any value but zero, NaN (infinite terms
+// of either sign) included.  A comparison of floats, which the compiler would also make of the integer
+// one if it saw where the bits come from, may take a NaN for zero (-fno-honor-nans).
+__device__ __forceinline__ bool has_value(float v) {
+  int bits = __builtin_bit_cast(int, v);
+  asm("" : "+v"(bits));
+  return (bits & 0x7fffffff) != 0;
+}
+
 // Order-preserving map between the bits of a float and a signed integer (its own inverse):
 // x < y  <=>  float_key(x) < float_key(y), with -0 below +0.
 __device__ __forceinline__ int float_key(int bits) { return bits ^ ((bits >> 31) & 0x7fffffff); }

@@ -370,14 +370,14 @@ __global__ void __launch_bounds__(kWave) soft_bwd_kernel(const BackParams p) {
         if (fd + lane < L) acc += hist[fd * L + fd + lane];
         if (lane > 0 && fd - lane >= 0) acc += hist[fd * L + fd - lane];
       }
-      if (acc != 0.f) atomicAdd(&p.dctx[lane], acc);
+      if (has_value(acc)) atomicAdd(&p.dctx[lane], acc);
     }
   } else {
     for (int i = lane; i < LL; i += kWave) {
       const int fd = i / L, cd = i - fd * L;
       if (cd > fd) continue;  // handled by the (fd, cd) entry
       const float v = hist[i] + (cd < fd ? hist[cd * L + fd] : 0.f);
-      if (v != 0.f) atomicAdd(&p.dctx[cd * L + fd], v);
+      if (has_value(v)) atomicAdd(&p.dctx[cd * L + fd], v);
     }
   }
 }
@@ -900,14 +900,14 @@ __global__ void __launch_bounds__(kWave) soft_split_bwd_kernel(const BackParams 
         if (fd + lane < L) acc += hist[fd * L + fd + lane];
         if (lane > 0 && fd - lane >= 0) acc += hist[fd * L + fd - lane];
       }
-      if (acc != 0.f) atomicAdd(&p.dctx[lane], acc);
+      if (has_value(acc)) atomicAdd(&p.dctx[lane], acc);
     }
   } else {
     for (int i = lane; i < LL; i += kWave) {
       const int fd = i / L, c2 = i - fd * L;
       if (c2 > fd) continue;  // handled by the (fd, cd) entry
       const float v = hist[i] + (c2 < fd ? hist[c2 * L + fd] : 0.f);
-      if (v != 0.f) atomicAdd(&p.dctx[c2 * L + fd], v);
+      if (has_value(v)) atomicAdd(&p.dctx[c2 * L + fd], v);
     }
   }
 }
@@ -1291,7 +1291,7 @@ __global__ void __launch_bounds__(kWave) soft_wide_bwd_kernel(const BackParams p
   if (p.dctx != nullptr) {
 #pragma unroll
     for (int j = 0; j < R; ++j)
-      if (valid[j] && hist[j] != 0.f) atomicAdd(&p.dctx[cd[j]], hist[j]);
+      if (valid[j] && has_value(hist[j])) atomicAdd(&p.dctx[cd[j]], hist[j]);
   }
 }
 

@@ -197,16 +197,20 @@ def test_two_targets_share_the_labels(gpu, L, option):
 
 
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
-@pytest.mark.parametrize("mode,L", [("TRWP", 70), ("ISGMR", 96), ("TRWP", 192), ("ISGMR", 254)])
-def test_non_finite_gradients_reach_the_same_entries(gpu, mode, L, value):
-  """An upstream gradient that is not finite shows in every entry of dunary and dedge_weights that it
-  reaches, and in no fewer entries of dcontext, whichever kernel scans; everywhere else nothing is
-  touched.  (The normalisation gives the other sign to one label of the pixel, so sums may be NaN.)"""
+@pytest.mark.parametrize("mode,L", [("TRWP", 5), ("ISGMR", 21), ("TRWP", 40), ("TRWP", 70), ("ISGMR", 96),
+                                    ("TRWP", 192), ("ISGMR", 254)])
+def test_gradients_that_are_not_finite(gpu, oracle, mode, L, value):
+  """An upstream gradient that is not finite shows in every entry that it reaches and in no other,
+  whichever kernel scans.  (The normalisation gives one label of the pixel the other sign, so a sum over
+  labels may be NaN, the table's gradient among them.)"""
   from mplayers_amd import _lib
   rng = np.random.default_rng(L)
   B, H, W, n_dir, n_iter, rho = 1, 6, 11, 4, 1, (0.5 if mode == "TRWP" else 1.0)
+  routes = [(0, 0), (2, 0)] if L > 64 else [(0, _lib.F_PACKED_OFF)]
+  if L <= 32:
+    routes.append((0, _lib.F_PACKED_ALWAYS))
   for k in range(8):
-    ctx = rng.random(L).astype(np.float32)
+    ctx = (np.triu(rng.random((L, L)), 1) if L == 21 else rng.random(L)).astype(np.float32)
     ew = (0.1 + 0.9 * rng.random((n_dir, B, 1, H, W))).astype(np.float32)
     dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
     dcost[0, 0, rng.integers(H), rng.integers(W), rng.integers(L)] = value
@@ -215,15 +219,14 @@ def test_non_finite_gradients_reach_the_same_entries(gpu, mode, L, value):
     imin = np.where(rng.random(imin.shape) < (0.6 if k % 2 else 1.0), imin if k % 4 == 0 else imin[..., :1], near)
     imin = imin.astype(np.uint8)
     inorm = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W)).astype(np.uint8)
-    print("case", mode, L, value, k, flush=True)
-    out = []
-    for option in (0, 2):
+    ref = oracle.backward(mode, ctx.astype(np.float64), ew.astype(np.float64), dcost.astype(np.float64),
+                          imin, inorm, rho)
+    for option, flags in routes:
+      print("case", mode, L, value, k, option, flags, flush=True)
       _lib.set_option(_lib.OPT_TEAM_SCANS, option)
       try:
-        out.append(gpu.gpu_backward(mode, ctx, ew, dcost, imin, inorm, rho, garbage_scratch=True))
+        got = gpu.gpu_backward(mode, ctx, ew, dcost, imin, inorm, rho, flags=flags, garbage_scratch=True)
       finally:
         _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
-    one, four = out
-    for i, name in ((0, "dunary"), (2, "dedge")):
-      assert np.array_equal(np.isfinite(one[i]), np.isfinite(four[i])), name
-    assert not np.any(np.isfinite(four[1]) & ~np.isfinite(one[1]))
+      for name, g, r in zip(("dunary", "dcontext", "dedge"), got, ref):
+        assert np.array_equal(np.isfinite(g), np.isfinite(r.reshape(g.shape))), (name, option, flags)
