@@ -144,6 +144,40 @@ def test_backward_soft_matches_oracle(gpu, oracle, n_dir, B, H, W, L, kind, n_it
   assert abs(float(dunary.sum()) - float(dcost.sum())) <= 1e-3 * max(1.0, np.abs(dcost).sum())
 
 
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("L,kind", [(5, "tl2"), (21, "dense2d"), (30, "dense1d"), (40, "tl3"), (64, "dense1d"),
+                                    (96, "dense1d"), (200, "tl3")])
+def test_gradients_that_are_not_finite(gpu, oracle, L, kind, value):
+  """An upstream gradient that is not finite shows in every entry that it reaches and in no other.
+  (The normalisation gives one label of the pixel the other sign, so a sum over labels is NaN where
+  it was infinite, the table's gradient among them.)"""
+  import torch
+  from mplayers_amd import lib_stereo
+  rng = np.random.default_rng(L)
+  n_dir, B, H, W, n_iter, rho = 4, 1, 4, 5, 1, 0.5
+  unary = rng.random((B, 1, H, W, L)).astype(np.float32)
+  ctx = make_ctx(kind, L, rng)
+  ew = (0.2 + rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
+  dcost[0, 0, rng.integers(H), rng.integers(W), rng.integers(L)] = value
+  print("case", L, kind, value, flush=True)
+  fwd = oracle.forward_soft(unary, ctx, ew, n_dir, n_iter, rho)
+  refs = oracle.backward_soft(ctx.astype(np.float64), ew.astype(np.float64), dcost.astype(np.float64),
+                              fwd["msg_edge_label"].astype(np.float64), fwd["msg_norm_index"], rho)
+  g = t(dcost)
+  dunary = g.new_zeros(B, 1, H, W, L)
+  dmsg = torch.full((n_dir, B, 1, H, W, L), 3.5, device="cuda")  # scratch: any contents
+  dctx = g.new_zeros(L, L) if L == 21 else g.new_zeros(L)
+  dedge = g.new_zeros(n_dir, B, 1, H, W)
+  lib_stereo.TRWP_hard_soft.backward_soft(rho, g, t(ctx), t(ew), t(fwd["msg_edge_label"]),
+                                          t(fwd["msg_norm_index"]), dunary, dctx, dedge, dmsg,
+                                          g.new_empty(0))
+  torch.cuda.synchronize()
+  for name, got, ref in (("dunary", dunary, refs[0]), ("dcontext", dctx, refs[1]), ("dedge", dedge, refs[2])):
+    print(name, "finite", np.isfinite(ref).mean(), flush=True)
+    assert np.array_equal(np.isfinite(got.cpu().numpy()), np.isfinite(ref.reshape(got.shape))), name
+
+
 @pytest.mark.parametrize("L,train_mode", [(21, "sigmoid"), (9, "")])
 def test_module_soft_forward_backward(gpu, oracle, L, train_mode):
   """MP_module_hard_soft.MPModule with mpnet_enable_soft: five outputs, gradients for the unary
