@@ -277,7 +277,7 @@ __device__ __forceinline__ void lds_order() {  // of this wavefront's own LDS in
 
 // GR: dedge_weights and / or dcontext are wanted
 template <int R, bool VEC, bool JACOBI, bool GR>
-__global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams p, const int n_cu) {
+__global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams p) {
   extern __shared__ __align__(16) char smem_raw[];
   Slot<R>* slots = reinterpret_cast<Slot<R>*>(smem_raw);  // two sets of kT
   Scalars* scal = reinterpret_cast<Scalars*>(slots + 2 * kT);
@@ -288,9 +288,10 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
   float* hist_s = ctx_s + n_ctx;  // dcontext, one histogram per helper
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  // which wavefront is the main one: workgroups that share a compute unit are as many apart as the chip
-  // has compute units, and their main wavefronts should not share a SIMD
-  const int role = uniform_i((tid / kWave + (int)blockIdx.x / n_cu) & 3);  // kHelpers: main
+  // The last wavefront is the main one in every workgroup: the wavefronts of the workgroups that a compute
+  // unit gets one after another start one SIMD further each (read from the hardware-id registers for 2, 3
+  // and 4 workgroups per unit), so the main wavefronts of up to four of them are on SIMDs of their own.
+  const int role = uniform_i(tid / kWave);  // kHelpers: main
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t P = (int64_t)p.B * HW;
   const int64_t N = P * L;
@@ -700,13 +701,12 @@ template <int R, bool VEC, bool JACOBI>
 void launch_vj(const BackParams& p, hipStream_t st) {
   const int blocks = p.block_prefix[p.n_dirs];
   const bool gr = p.dedge != nullptr || p.dctx != nullptr;
-  const int n_cu = launch_policy().n_simd / 4;
   const size_t lds = 2 * kT * (sizeof(Slot<R>) + sizeof(Scalars)) +
                      sizeof(float) * (kAccFloats + (gr ? p.L + kHelpers * hist_floats(R, p.L) : 0));
   if (gr)
-    sweep_bwd_team_kernel<R, VEC, JACOBI, true><<<blocks, kTeam, lds, st>>>(p, n_cu);
+    sweep_bwd_team_kernel<R, VEC, JACOBI, true><<<blocks, kTeam, lds, st>>>(p);
   else
-    sweep_bwd_team_kernel<R, VEC, JACOBI, false><<<blocks, kTeam, lds, st>>>(p, n_cu);
+    sweep_bwd_team_kernel<R, VEC, JACOBI, false><<<blocks, kTeam, lds, st>>>(p);
 }
 
 }  // namespace
