@@ -792,6 +792,7 @@ SweepParams base_fwd_params(const mpl_shape* s, float rho, const float* edge, co
                             const CtxDesc* desc) {
   SweepParams p;
   memset(&p, 0, sizeof(p));
+  p.xcd_group = xcd_group_size(s->n_disp);
   p.B = s->batch;
   p.H = s->height;
   p.W = s->width;
@@ -1241,6 +1242,7 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
 
   BackParams p;
   memset(&p, 0, sizeof(p));
+  p.xcd_group = xcd_group_size(s->n_disp);
   p.B = s->batch;
   p.H = s->height;
   p.W = s->width;
@@ -1309,6 +1311,7 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
 
   BackParams p;
   memset(&p, 0, sizeof(p));
+  p.xcd_group = xcd_group_size(s->n_disp);
   p.B = s->batch;
   p.H = s->height;
   p.W = s->width;
@@ -1427,6 +1430,7 @@ int mpl_trwp_soft_backward(const mpl_shape* s, unsigned flags, float rho, int n_
   const int64_t N = P * s->n_disp;
   BackParams p;
   memset(&p, 0, sizeof(p));
+  p.xcd_group = xcd_group_size(s->n_disp);
   p.B = s->batch;
   p.H = s->height;
   p.W = s->width;

@@ -58,6 +58,7 @@ struct PixB {
 template <int R, bool VEC, bool MASK, bool JACOBI, bool DIRECT, int GRAD>
 __global__ void __launch_bounds__(kWave) sweep_bwd_kernel(const BackParams p) {
   constexpr bool DE = (GRAD & 1) != 0, DC = (GRAD & 2) != 0;
+  constexpr int kLd = load_policy(!MASK);  // (every lane full: whole cache lines)
   extern __shared__ float smem[];
   const int L = p.L;
   // 2-D context tables exist for at most 64 labels, i.e. only with one label per lane
@@ -161,19 +162,19 @@ __global__ void __launch_bounds__(kWave) sweep_bwd_kernel(const BackParams p) {
     const unsigned so = pp * (unsigned)vbytes;
     if constexpr (VEC) {
       const int vo = (int)(lane_ok ? so + (unsigned)foff : kDeadWide);
-      buf_load<R, true>(rA, vo, 0u, r.a);
+      buf_load<R, true, kLd>(rA, vo, 0u, r.a);
       // before the first write of this plane it counts as zero (empty descriptor)
-      if (!JACOBI) buf_load<R, true>(rHdIn, vo, 0u, r.hd);
-      if (EVEN) buf_load<R, true>(rHiIn, vo, 0u, r.hi);
-      buf_load_u8<R, true>(rImin, (int)(lane_ok ? pp * (unsigned)L + (unsigned)lab0 : kDeadWide), 0u,
+      if (!JACOBI) buf_load<R, true, kLd>(rHdIn, vo, 0u, r.hd);
+      if (EVEN) buf_load<R, true, kLd>(rHiIn, vo, 0u, r.hi);
+      buf_load_u8<R, true, kLd>(rImin, (int)(lane_ok ? pp * (unsigned)L + (unsigned)lab0 : kDeadWide), 0u,
                            r.fd);
     } else {
       const int nrec = (int)(so + (unsigned)vbytes);
-      buf_load<R, VEC>(make_rsrc(bA, nrec), foff, so, r.a);
+      buf_load<R, VEC, kLd>(make_rsrc(bA, nrec), foff, so, r.a);
       // before the first write of this plane it counts as zero: an empty descriptor reads 0
-      if (!JACOBI) buf_load<R, VEC>(make_rsrc(bHd, read_h ? nrec : 0), foff, so, r.hd);
-      if (EVEN) buf_load<R, VEC>(make_rsrc(bHi, nrec), foff, so, r.hi);
-      buf_load_u8<R, VEC>(make_rsrc(bImin, (int)(pp * (unsigned)L + (unsigned)L)), lab0,
+      if (!JACOBI) buf_load<R, VEC, kLd>(make_rsrc(bHd, read_h ? nrec : 0), foff, so, r.hd);
+      if (EVEN) buf_load<R, VEC, kLd>(make_rsrc(bHi, nrec), foff, so, r.hi);
+      buf_load_u8<R, VEC, kLd>(make_rsrc(bImin, (int)(pp * (unsigned)L + (unsigned)L)), lab0,
                           pp * (unsigned)L, r.fd);
     }
     // (no arithmetic on what was just loaded in here: it would have to wait for the loads, and the

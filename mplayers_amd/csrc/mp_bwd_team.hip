@@ -439,11 +439,11 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
     };
     auto load_plane = [&](rsrc_t r, bool on, unsigned so, float (&x)[R]) __attribute__((always_inline)) {
       if constexpr (VEC) {
-        buf_load<R, true>(r, vec_off(on, so, 0), 0u, x);
+        buf_load<R, true, load_policy(false)>(r, vec_off(on, so, 0), 0u, x);
       } else {
 #pragma unroll
         for (int j = 0; j < R; ++j)
-          x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, vec_off(on, so, j), 0, MPL_LD_AUX));
+          x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, vec_off(on, so, j), 0, load_policy(false)));
       }
     };
     auto store_plane = [&](rsrc_t r, bool on, unsigned so, const float (&x)[R]) __attribute__((always_inline)) {
@@ -467,12 +467,12 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
       if (!JACOBI) load_plane(rHdIn, on, so, r.hd);
       if (EVEN) load_plane(rHiIn, on, so, r.hi);
       if constexpr (VEC) {
-        buf_load_u8<R, true>(rImin, (int)((on && lane_ok) ? pp * (unsigned)L + (unsigned)lab0 : kDeadWide), 0u, r.fd);
+        buf_load_u8<R, true, load_policy(false)>(rImin, (int)((on && lane_ok) ? pp * (unsigned)L + (unsigned)lab0 : kDeadWide), 0u, r.fd);
       } else {
 #pragma unroll
         for (int j = 0; j < R; ++j)
           r.fd[j] = __builtin_amdgcn_raw_buffer_load_b8(
-              rImin, (int)((on && lab0 + j < L) ? pp * (unsigned)L + (unsigned)(lab0 + j) : kDeadWide), 0, MPL_LD_AUX);
+              rImin, (int)((on && lab0 + j < L) ? pp * (unsigned)L + (unsigned)(lab0 + j) : kDeadWide), 0, load_policy(false));
       }
       r.nidx = __builtin_amdgcn_raw_buffer_load_b8(dInorm, on ? (int)pp : kDeadOffset, 0, 0);
       r.w = r.de = 0.f;

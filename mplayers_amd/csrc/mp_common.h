@@ -274,6 +274,13 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* p, int bytes) {
 #ifndef MPL_ST_AUX
 #define MPL_ST_AUX 2
 #endif
+// Loads of planes whose pixel vectors are not whole cache lines, and of launches of few chains, go without
+// the hint: a line that two pixels share, or that the sweep after this one reads again, is then still
+// there.  Measured, ms per call with the hint / without, neighbouring chains on one die (xcd_group): TRWP
+// 97 labels 300x800 2.83 / 2.46, 150 labels 700x1000 keeping argmin labels 9.09 / 8.08, ISGMR 150 labels
+// 400x600 1.80 / 1.53; whole lines with one wavefront per chain, 96 labels 384x1248 3.65 / 3.68.  (Stores
+// without the hint as well: 2.53, 8.29, 1.61, 3.78.)
+constexpr int load_policy(bool whole_lanes) { return whole_lanes ? MPL_LD_AUX : 0; }
 
 constexpr int kDeadOffset = 0x7ffffff0;  // a vector offset no descriptor covers: access suppressed
 // the same for descriptors that cover a whole image (up to kMaxImageBytes, beyond 2 GiB)
@@ -283,19 +290,19 @@ constexpr int64_t kMaxImageBytes = 0xffffffc0ll;
 // R consecutive floats at vector byte offset `off` (range-checked) + scalar byte offset `so`.
 // VEC: one R-dword access (used when every lane's block lies entirely inside or entirely outside
 // the pixel vector, i.e. L % R == 0); otherwise R single-dword accesses, each checked on its own.
-template <int R, bool VEC>
+template <int R, bool VEC, int AUX = MPL_LD_AUX>
 __device__ __forceinline__ void buf_load(rsrc_t r, int off, unsigned so, float (&x)[R]) {
   if constexpr (VEC && R == 2) {
-    f32x2 t = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)((unsigned)off + so), 0, MPL_LD_AUX));
+    f32x2 t = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)((unsigned)off + so), 0, AUX));
     x[0] = t[0];
     x[1] = t[1];
   } else if constexpr (VEC && R == 3) {
-    f32x3 t = __builtin_bit_cast(f32x3, __builtin_amdgcn_raw_buffer_load_b96(r, (int)((unsigned)off + so), 0, MPL_LD_AUX));
+    f32x3 t = __builtin_bit_cast(f32x3, __builtin_amdgcn_raw_buffer_load_b96(r, (int)((unsigned)off + so), 0, AUX));
     x[0] = t[0];
     x[1] = t[1];
     x[2] = t[2];
   } else if constexpr (VEC && R == 4) {
-    f32x4 t = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)((unsigned)off + so), 0, MPL_LD_AUX));
+    f32x4 t = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)((unsigned)off + so), 0, AUX));
     x[0] = t[0];
     x[1] = t[1];
     x[2] = t[2];
@@ -303,7 +310,7 @@ __device__ __forceinline__ void buf_load(rsrc_t r, int off, unsigned so, float (
   } else {
 #pragma unroll
     for (int j = 0; j < R; ++j)
-      x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)((unsigned)(off + 4 * j) + so), 0, MPL_LD_AUX));
+      x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)((unsigned)(off + 4 * j) + so), 0, AUX));
   }
 }
 
@@ -326,21 +333,21 @@ __device__ __forceinline__ void buf_store(rsrc_t r, int off, unsigned so, const 
 }
 
 // R consecutive uint8 at byte offset `off`
-template <int R, bool VEC>
+template <int R, bool VEC, int AUX = MPL_LD_AUX>
 __device__ __forceinline__ void buf_load_u8(rsrc_t r, int off, unsigned so, int (&x)[R]) {
   if constexpr (VEC && R == 4) {
-    unsigned t = __builtin_amdgcn_raw_buffer_load_b32(r, (int)((unsigned)off + so), 0, MPL_LD_AUX);
+    unsigned t = __builtin_amdgcn_raw_buffer_load_b32(r, (int)((unsigned)off + so), 0, AUX);
     x[0] = t & 0xff;
     x[1] = (t >> 8) & 0xff;
     x[2] = (t >> 16) & 0xff;
     x[3] = t >> 24;
   } else if constexpr (VEC && R == 2) {
-    unsigned t = __builtin_amdgcn_raw_buffer_load_b16(r, (int)((unsigned)off + so), 0, MPL_LD_AUX);
+    unsigned t = __builtin_amdgcn_raw_buffer_load_b16(r, (int)((unsigned)off + so), 0, AUX);
     x[0] = t & 0xff;
     x[1] = (t >> 8) & 0xff;
   } else {
 #pragma unroll
-    for (int j = 0; j < R; ++j) x[j] = __builtin_amdgcn_raw_buffer_load_b8(r, (int)((unsigned)(off + j) + so), 0, MPL_LD_AUX);
+    for (int j = 0; j < R; ++j) x[j] = __builtin_amdgcn_raw_buffer_load_b8(r, (int)((unsigned)(off + j) + so), 0, AUX);
   }
 }
 
@@ -426,13 +433,33 @@ struct ChainCtx {
   int dir;
 };
 
+// Consecutive workgroups go to the eight dies of the chip in turn, each with an L2 of its own.  Where the
+// vector of a pixel is not whole cache lines, the chains beside each other share lines, so xcd_group_size
+// consecutive chains are put on one die: a line is then read once and written whole.  Measured, TRWP
+// forward, ms per call with every chain on another die / in groups of 16: 60 labels 375x450, 8 directions,
+// 1.74 / 1.61 with one wavefront per chain, 1.52 / 1.26 with four (groups of 4, 8, 32: the 50 iterations
+// of the energy minimisation 25.8, 24.8, 25.3 ms, 16: 24.5, none: 29.3); 97 labels 300x800 2.97 / 2.83;
+// vectors of whole lines the same either way.
+constexpr int kXcds = 8;
+constexpr int kLineBytes = 128;
+inline int xcd_group_size(int L) { return (L * 4) % kLineBytes != 0 ? 16 : 0; }
+
 // which (direction, batch item, chain) a workgroup owns
 template <typename Params>
 __device__ __forceinline__ ChainCtx locate_chain(const Params& p) {
+  int block = (int)blockIdx.x;
+  if (p.xcd_group > 0) {  // (whole rounds of eight groups; the workgroups after the last one stay as they are)
+    const int per = kXcds * p.xcd_group;
+    const int base = block / per * per;
+    if (base + per <= (int)gridDim.x) {
+      const int r = block - base;
+      block = base + (r % kXcds) * p.xcd_group + r / kXcds;
+    }
+  }
   int di = 0;
-  while (di + 1 < p.n_dirs && (int)blockIdx.x >= p.block_prefix[di + 1]) ++di;
+  while (di + 1 < p.n_dirs && block >= p.block_prefix[di + 1]) ++di;
   const int dir = p.dirs[di];
-  const int local = (int)blockIdx.x - p.block_prefix[di];
+  const int local = block - p.block_prefix[di];
   const DirGeom g = make_dir(dir, p.H, p.W);
   const int bv = local / g.n_chains;
   const int c = local - bv * g.n_chains;
@@ -482,6 +509,7 @@ struct SweepParams {
                                    // wavefront.  Decided once per launch by the host (mp_api.hip)
   int split;                       // dense 1-D table, several labels per lane, few chains: wavefronts
                                    // per chain that share the front labels of a pixel (0, 1: one)
+  int xcd_group;                   // consecutive chains on one die (0: each on another; locate_chain)
   int pair_q;                      // Gauss-Seidel: belief plane holds Q between the sweeps of a pair
   int skip_s_store;                // Gauss-Seidel: last sweep of the call, nobody reads S after it
   int fused_pair;                  // Gauss-Seidel: every wavefront sweeps dirs[0], then dirs[0] ^ 1
@@ -537,6 +565,7 @@ struct BackParams {
   const float* edge_label;  // soft TRWP: (n_dir_total, P, L, L) duals of this iteration
   int pack;                 // packed scans (mp_pack.hip): chains per wavefront
   int team;                 // four wavefronts per chain (mp_bwd_team.hip)
+  int xcd_group;            // consecutive chains on one die (0: each on another; locate_chain)
 };
 
 // records the message mpl_last_error() returns on this thread and returns `code`

@@ -751,6 +751,8 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
                                               const ChainCtx& ch, float* a_s, const float* ctx_s,
                                               const bool skip_s_store_in, float* xchg = nullptr) {
   constexpr bool SPLIT = (KT == -3);
+  // (every lane full: 64, 128, 192 or 256 labels, whole cache lines)
+  constexpr int kLd = load_policy(!MASK);
   const int L = p.L;
   // The caller's initial messages turned out to be all zero (the usual case: the reference's
   // callers pass a cleared tensor) and this is a sweep that can profit: S = Q = U = unary, so the
@@ -895,25 +897,25 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
     const unsigned so = pp * (unsigned)vbytes;
     if constexpr (VEC) {
       const int vo = (int)(kAddDead ? so + foff_ok : (lane_ok ? so + (unsigned)foff : kDeadWide));
-      buf_load<R, true>(rS, vo, 0u, r.s);
+      buf_load<R, true, kLd>(rS, vo, 0u, r.s);
       if (JACOBI == 0) {
-        buf_load<R, true>(first ? rMd0 : rMd, vo, 0u, r.md);
-        buf_load<R, true>(rMi, vo, 0u, r.mi);
+        buf_load<R, true, kLd>(first ? rMd0 : rMd, vo, 0u, r.md);
+        buf_load<R, true, kLd>(rMi, vo, 0u, r.mi);
       } else if (JACOBI == 2) {
-        buf_load<R, true>(rMd0, vo, 0u, r.md);
-        buf_load<R, true>(rMi, vo, 0u, r.mi);
+        buf_load<R, true, kLd>(rMd0, vo, 0u, r.md);
+        buf_load<R, true, kLd>(rMi, vo, 0u, r.mi);
       }
     } else {
       const int nrec = (int)(so + (unsigned)vbytes);
-      buf_load<R, VEC>(make_rsrc(bS, nrec), foff, so, r.s);
+      buf_load<R, VEC, kLd>(make_rsrc(bS, nrec), foff, so, r.s);
       if (JACOBI == 0) {
         // planes that still hold all-zero initial messages are read through an empty descriptor
-        buf_load<R, VEC>(make_rsrc(bMd, (md_zero || (pair_second && ld_t > 0)) ? 0 : nrec), foff, so,
+        buf_load<R, VEC, kLd>(make_rsrc(bMd, (md_zero || (pair_second && ld_t > 0)) ? 0 : nrec), foff, so,
                          r.md);
-        buf_load<R, VEC>(make_rsrc(bMi, mi_zero ? 0 : nrec), foff, so, r.mi);
+        buf_load<R, VEC, kLd>(make_rsrc(bMi, mi_zero ? 0 : nrec), foff, so, r.mi);
       } else if (JACOBI == 2) {
-        buf_load<R, VEC>(make_rsrc(bMd, nrec), foff, so, r.md);
-        buf_load<R, VEC>(make_rsrc(bMi, nrec), foff, so, r.mi);
+        buf_load<R, VEC, kLd>(make_rsrc(bMd, nrec), foff, so, r.md);
+        buf_load<R, VEC, kLd>(make_rsrc(bMi, nrec), foff, so, r.mi);
       }
     }
     r.w = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(dW, (int)(pp * 4u), 0, 0));
