@@ -329,11 +329,11 @@ const char* mpl_last_error(void);
  * the forward launches that MPL_F_DENSE_TABLE splits, at most 8 and at most what leaves every
  * wavefront a front label (1: never split).  For tests and measurements. */
 #define MPL_OPT_DENSE_SPLIT_WAVES 4
-/* MPL_OPT_TEAM_SCANS (default 1): reverse scans of more than 64 labels with a 1-D table put four
- * wavefronts on a chain in launches with few chains (on an MI355X at most 256 to 768, by label count and
- * operator), one for the recurrence and three that load, prepare, finish and store its pixels; 0: never,
- * 2: every launch of more than 64 labels with a 1-D table.  The results agree to the parity tolerance.
- * For tests and measurements. */
+/* MPL_OPT_TEAM_SCANS (default 1): launches with few chains (on an MI355X at most 256 to 768, by label count
+ * and operator) put four wavefronts on a chain, one for the recurrence and three that load, prepare, finish
+ * and store its pixels: the forward scans of TRWP, whose results are the same bits, and the reverse scans
+ * of more than 64 labels with a 1-D table, whose results agree to the parity tolerance; 0: never, 2: every
+ * such launch whatever its number of chains.  For tests and measurements. */
 #define MPL_OPT_TEAM_SCANS 5
 int mpl_set_option(int option, int value);
 

@@ -628,7 +628,7 @@ int labels_per_lane(int L) { return (L + kWave - 1) / kWave; }
 std::atomic<int> g_packed_scans{1};  // MPL_OPT_PACKED_SCANS: 0 off, 1 by chain count, 2 always
 std::atomic<int> g_fused_u{1};       // MPL_OPT_FUSED_U
 std::atomic<int> g_belief_rebuild{MPL_BELIEF_REBUILD_DEFAULT};  // MPL_OPT_BELIEF_REBUILD
-std::atomic<int> g_team_scans{1};    // MPL_OPT_TEAM_SCANS: 0 never, 1 launches with few chains, 2 more than 64 labels
+std::atomic<int> g_team_scans{1};    // MPL_OPT_TEAM_SCANS: 0 never, 1 launches with few chains, 2 whatever their number
 std::atomic<int> g_split_waves{0};   // MPL_OPT_DENSE_SPLIT_WAVES: 0 = by the model of choose_split
 
 // what one call does, from its flags and the process defaults
@@ -708,6 +708,36 @@ int decide_team(const BackParams& p, const CallOpts& o, bool jacobi) {
   return p.block_prefix[p.n_dirs] <= team_chains_per_cu(p.L, jacobi) * cus ? 1 : 0;
 }
 
+// The same for the forward scans of TRWP (mp_fwd_team.hip; the same bits either way).  Measured on rows of
+// 300 pixels with 192 to 1024 chains, Potts, truncated linear and quadratic, random tables, ns per pixel
+// with one over ns with four wavefronts, the least over the tables / the greatest.  With argmin labels kept,
+// which the helpers find:
+//   * up to 64 labels: 256 chains 1.26 / 1.70, 768 chains 1.16 / 1.35, 1024 chains 0.98 / 1.30;
+//   * up to 128: 256 chains 1.41 / 3.72, 768 chains 1.22 / 2.37, 1024 chains 0.96 / 1.88;
+//   * up to 192: 256 chains 1.36 / 1.94, 768 chains 1.11 / 1.75, 1024 chains 0.66 / 1.05;
+//   * up to 256: 256 chains 2.07 / 2.60, 512 chains 1.38 / 1.81, 768 chains 0.92 / 1.05.
+// Without them:
+//   * up to 64 labels: 768 chains 1.02 / 1.62, 1024 chains 0.89 / 1.37;
+//   * up to 128: 512 chains 1.05 / 1.36, 768 chains 0.86 / 1.12;
+//   * up to 192: 768 chains 1.03 / 1.24;  up to 256: 768 chains 1.05 / 1.08.
+// Labels loaded and stored one by one (their number no multiple of the labels per lane), kept / not: up to 128
+// 768 chains 1.11, 1024 chains 0.88 / 256 chains 1.28, 384 chains 1.02, 512 chains 0.98; up to 192 512
+// chains 1.32, 768 chains 0.92 / 256 chains 1.27, 384 chains 0.76; up to 256 256 chains 1.37, 384 chains
+// 0.89 / 192 chains 0.84.
+int team_fwd_chains_per_cu(int L, bool train) {
+  const int R = labels_per_lane(L);
+  if (L % R == 0) return (R == 4 && train) || (R == 2 && !train) ? 2 : 3;
+  if (train) return 5 - R;
+  return R < 4 ? 1 : 0;
+}
+
+int decide_team_fwd(const SweepParams& p, const CallOpts& o, bool train) {
+  if (p.pack >= 2 || p.split >= 2 || o.team == 0) return 0;
+  if (o.team == 2) return 1;
+  const int per_cu = team_fwd_chains_per_cu(p.L, train);
+  return p.block_prefix[p.n_dirs] <= per_cu * (launch_policy().n_simd / 4) ? 1 : 0;
+}
+
 // Wavefronts per chain for the forward scan of a launch whose caller declared a dense 1-D table
 // (MPL_F_DENSE_TABLE) with several labels per lane: four (one on every SIMD of a compute unit, each
 // scanning a quarter of the front labels of a pixel), two, or one.  A lone wavefront on a SIMD
@@ -756,6 +786,15 @@ void launch_fwd(const SweepParams& p, bool train, bool jacobi, hipStream_t st) {
   Timed timed(jacobi ? MPL_KERNEL_FWD_SWEEP_ALL : MPL_KERNEL_FWD_SWEEP, st, p.fused_pair ? 2 : 1);
   if (p.pack >= 2) {
     launch_packed_fwd(p, train, jacobi, p.pack, st);  // (u_fused is never set together with pack)
+    return;
+  }
+  if (p.team) {
+    switch (labels_per_lane(p.L)) {
+      case 1: launch_team_fwd<1>(p, train, st); break;
+      case 2: launch_team_fwd<2>(p, train, st); break;
+      case 3: launch_team_fwd<3>(p, train, st); break;
+      default: launch_team_fwd<4>(p, train, st); break;
+    }
     return;
   }
   switch (labels_per_lane(p.L)) {
@@ -1067,6 +1106,7 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
       fill_dirs(s, d, 1, p.dirs, p.block_prefix, &p.n_dirs);
       p.pack = decide_pack(s, p, opts);
       p.split = choose_split(s, p, opts, train);
+      p.team = decide_team_fwd(p, opts, train);
       p.first_iter = (it == 0);
       p.pair_q = 1;
       p.belief = (uninit && it == 0 && d <= 1) ? unary : unary_update;

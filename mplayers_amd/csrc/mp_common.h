@@ -509,6 +509,7 @@ struct SweepParams {
                                    // wavefront.  Decided once per launch by the host (mp_api.hip)
   int split;                       // dense 1-D table, several labels per lane, few chains: wavefronts
                                    // per chain that share the front labels of a pixel (0, 1: one)
+  int team;                        // Gauss-Seidel: four wavefronts per chain (mp_fwd_team.hip)
   int xcd_group;                   // consecutive chains on one die (0: each on another; locate_chain)
   int pair_q;                      // Gauss-Seidel: belief plane holds Q between the sweeps of a pair
   int skip_s_store;                // Gauss-Seidel: last sweep of the call, nobody reads S after it
@@ -583,6 +584,15 @@ inline void launch_sweep_fwd(const SweepParams& p, bool train, bool jacobi, hipS
     launch_sweep_fwd_t<R, true>(p, jacobi, st);
   else
     launch_sweep_fwd_t<R, false>(p, jacobi, st);
+}
+template <int R, bool TRAIN>
+void launch_team_fwd_t(const SweepParams& p, hipStream_t st);
+template <int R>
+inline void launch_team_fwd(const SweepParams& p, bool train, hipStream_t st) {
+  if (train)
+    launch_team_fwd_t<R, true>(p, st);
+  else
+    launch_team_fwd_t<R, false>(p, st);
 }
 template <int R>
 void launch_sweep_bwd(const BackParams& p, bool jacobi, hipStream_t st);

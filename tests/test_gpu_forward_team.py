@@ -1,0 +1,91 @@
+"""TRWP's forward scan with four wavefronts per chain (MPL_OPT_TEAM_SCANS): the bits of the scan with
+one wavefront per chain -- messages, costs, labels, both index tensors -- for every kind of table, label
+counts on both sides of a lane's share, chains on both sides of a block of pixels, negative weights,
+given and undefined initial messages, pairs in one launch and in two."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_dense_split import _forward_flags
+
+pytestmark = pytest.mark.gpu
+
+TABLES = {
+    "potts": lambda k, rng: np.minimum(k, 1),
+    "band2": lambda k, rng: np.minimum(k, 2),
+    "band4": lambda k, rng: 0.3 * np.minimum(k, 4) ** 2,
+    "band7": lambda k, rng: 0.1 * np.minimum(k, 7) ** 2,
+    "band14": lambda k, rng: 0.1 * np.minimum(k, 14) ** 2,
+    "band20": lambda k, rng: 0.05 * np.minimum(k, 20) ** 2,
+    "bent": lambda k, rng: np.where(k == 0, 0.2, np.minimum(k, 3) * 0.15),  # entry 0 is not the smallest
+    "linear": lambda k, rng: 0.1 * k,
+    "random": lambda k, rng: np.where(k == 0, 0, rng.random(len(k))),
+}
+
+
+def _run(gpu, option, unary, ctx, ew, n_dir, n_iter, training, flags=0, **kw):
+  from mplayers_amd import _lib
+  _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+  try:
+    return _forward_flags(gpu, "TRWP", unary, ctx, ew, n_dir, n_iter, 0.5, training, flags, **kw)
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+
+
+def _same(a, b, training):
+  for k in ("msg", "cost_final", "label_all") + (("msg_min_index", "msg_norm_index") if training else ()):
+    assert np.array_equal(a[k], b[k]), k
+
+
+def _problem(n_dir, B, H, W, L, table, seed=0, negative=False):
+  rng = np.random.default_rng(1000 * L + 10 * H + W + seed)
+  unary = (rng.random((B, 1, H, W, L)) * 3).astype(np.float32)
+  if table == "2d":
+    ctx = np.triu(rng.random((L, L)), 1).astype(np.float32)
+  else:
+    ctx = TABLES[table](np.arange(L, dtype=np.float64), rng).astype(np.float32)
+  ew = (0.1 + 0.9 * rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  if negative:
+    ew[rng.random(ew.shape) < 0.1] = -0.5
+  return unary, ctx, ew
+
+
+@pytest.mark.parametrize("training", [True, False])
+@pytest.mark.parametrize("L", [2, 16, 21, 33, 64, 65, 96, 127, 130, 192, 193, 256])
+def test_same_bits_for_every_table(gpu, L, training):
+  from mplayers_amd import _lib
+  tables = ["2d"] if L == 21 else [t for t in TABLES if L > 8 or t in ("potts", "random")]
+  for i, table in enumerate(tables):
+    for negative in (False, True):
+      print("case", L, training, table, negative, flush=True)
+      problem = _problem(4, 1, 9, 14, L, table, i, negative)
+      one = _run(gpu, 0, *problem, 4, 2, training, _lib.F_PACKED_OFF)
+      four = _run(gpu, 2, *problem, 4, 2, training, _lib.F_PACKED_OFF)
+      _same(four, one, training)
+
+
+@pytest.mark.parametrize("L,table", [(21, "2d"), (40, "potts"), (96, "band4"), (192, "band4"), (256, "linear")])
+@pytest.mark.parametrize("training", [True, False])
+def test_chain_lengths_and_launches(gpu, L, table, training):
+  """Chains of 1 to 50 pixels, 2 to 16 directions, one and two launches per pair, initial messages that are
+  given, zero and undefined."""
+  from mplayers_amd import _lib
+  for n_dir, B, H, W in ((2, 1, 1, 1), (4, 2, 1, 2), (4, 1, 5, 6), (4, 1, 7, 12), (8, 1, 13, 25), (16, 2, 6, 11),
+                         (4, 1, 3, 50)):
+    problem = _problem(n_dir, B, H, W, L, table, 3)
+    for flags, kw in ((0, {}), (_lib.F_FUSED_PAIRS_OFF, {}), (0, dict(msg_uninit=True))):
+      print("case", L, table, n_dir, B, H, W, flags, kw, flush=True)
+      flags |= _lib.F_PACKED_OFF
+      one = _run(gpu, 0, *problem, n_dir, 3, training, flags, **kw)
+      four = _run(gpu, 2, *problem, n_dir, 3, training, flags, **kw)
+      _same(four, one, training)
+    rng = np.random.default_rng(7)
+    init = rng.random((n_dir, B, 1, H, W, L)).astype(np.float32)
+    got = []
+    for option in (0, 2):
+      _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+      try:
+        got.append(gpu.gpu_forward("TRWP", *problem, n_dir, 2, 0.5, training=training, saving_label=True,
+                                   msg_init=init))
+      finally:
+        _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+    _same(got[1], got[0], training)
