@@ -33,7 +33,7 @@ def _units():
   units = [("mp_api", "mp_api.hip", []), ("mp_edge", "mp_edge.hip", []),
            ("mp_soft", "mp_soft.hip", []), ("mp_pack", "mp_pack.hip", []),
            ("mp_terms", "mp_terms.hip", []), ("mp_probe", "mp_probe.hip", []),
-           ("mp_layout", "mp_layout.hip", [])]
+           ("mp_layout", "mp_layout.hip", []), ("mp_team21", "mp_team21.hip", [])]
   for r in (4, 3, 2, 1):  # (the largest units first)
     for t in (1, 0):
       units.append(("mp_fwd_r%d_t%d" % (r, t), "mp_fwd.hip",

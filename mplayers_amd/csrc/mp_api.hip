@@ -701,8 +701,19 @@ int team_chains_per_cu(int L, bool jacobi) {
   return R == 4 && jacobi ? 2 : 3;
 }
 
+// 21 labels with a 2-D table (mp_team21.hip), one over four wavefronts on images of 129x129, batch 1 / 4 / 8 /
+// 12 (129 / 516 / 1032 / 1548 chains).  Forward, argmin labels kept: 2.05 / 1.95 / 1.51 / 1.48; rows without
+// them 1.51 with 256, 1.46 with 1024, 1.53 with 2048 chains.  Backward, dunary alone: 1.35 / 1.21 / 0.99 /
+// 0.82, with both other gradients 1.85 / 1.47 / 1.08 / 1.21; 65x65, batch 12 (780 chains) 0.85 and 1.11.
+// (More than 2048 chains: the packed scans.)
+constexpr int kTeam21FwdChainsPerCu = 8;
+constexpr int kTeam21BwdChainsPerCu = 3;
+
 int decide_team(const BackParams& p, const CallOpts& o, bool jacobi) {
-  if (p.pack >= 2 || p.ctx2d || p.L <= kWave || o.team == 0) return 0;
+  if (p.pack >= 2 || o.team == 0) return 0;
+  if (p.ctx2d && p.L == 21 && !jacobi)
+    return o.team == 2 || p.block_prefix[p.n_dirs] <= kTeam21BwdChainsPerCu * (launch_policy().n_simd / 4) ? 1 : 0;
+  if (p.ctx2d || p.L <= kWave) return 0;
   if (o.team == 2) return 1;
   const int cus = launch_policy().n_simd / 4;
   return p.block_prefix[p.n_dirs] <= team_chains_per_cu(p.L, jacobi) * cus ? 1 : 0;
@@ -734,7 +745,7 @@ int team_fwd_chains_per_cu(int L, bool train) {
 int decide_team_fwd(const SweepParams& p, const CallOpts& o, bool train) {
   if (p.pack >= 2 || p.split >= 2 || o.team == 0) return 0;
   if (o.team == 2) return 1;
-  const int per_cu = team_fwd_chains_per_cu(p.L, train);
+  const int per_cu = p.ctx2d && p.L == 21 ? kTeam21FwdChainsPerCu : team_fwd_chains_per_cu(p.L, train);
   return p.block_prefix[p.n_dirs] <= per_cu * (launch_policy().n_simd / 4) ? 1 : 0;
 }
 
@@ -788,6 +799,10 @@ void launch_fwd(const SweepParams& p, bool train, bool jacobi, hipStream_t st) {
     launch_packed_fwd(p, train, jacobi, p.pack, st);  // (u_fused is never set together with pack)
     return;
   }
+  if (p.team && p.ctx2d && p.L == 21) {
+    launch_team21_fwd(p, train, st);
+    return;
+  }
   if (p.team) {
     switch (labels_per_lane(p.L)) {
       case 1: launch_team_fwd<1>(p, train, st); break;
@@ -809,6 +824,10 @@ void launch_bwd(const BackParams& p, bool jacobi, hipStream_t st) {
   Timed timed(jacobi ? MPL_KERNEL_BWD_SWEEP_ALL : MPL_KERNEL_BWD_SWEEP, st, p.fused_pair ? 2 : 1);
   if (p.pack >= 2) {
     launch_packed_bwd(p, jacobi, p.pack, st);
+    return;
+  }
+  if (p.team && p.ctx2d) {
+    launch_team21_bwd(p, st);
     return;
   }
   if (p.team) {

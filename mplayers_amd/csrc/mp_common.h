@@ -509,7 +509,7 @@ struct SweepParams {
                                    // wavefront.  Decided once per launch by the host (mp_api.hip)
   int split;                       // dense 1-D table, several labels per lane, few chains: wavefronts
                                    // per chain that share the front labels of a pixel (0, 1: one)
-  int team;                        // Gauss-Seidel: four wavefronts per chain (mp_fwd_team.hip)
+  int team;                        // Gauss-Seidel: four wavefronts per chain (mp_fwd_team.hip, mp_team21.hip)
   int xcd_group;                   // consecutive chains on one die (0: each on another; locate_chain)
   int pair_q;                      // Gauss-Seidel: belief plane holds Q between the sweeps of a pair
   int skip_s_store;                // Gauss-Seidel: last sweep of the call, nobody reads S after it
@@ -565,7 +565,7 @@ struct BackParams {
                             // reference's TRWP_hard_soft build, TRWP_hard_soft/TRWP_backward.cu:104-111)
   const float* edge_label;  // soft TRWP: (n_dir_total, P, L, L) duals of this iteration
   int pack;                 // packed scans (mp_pack.hip): chains per wavefront
-  int team;                 // four wavefronts per chain (mp_bwd_team.hip)
+  int team;                 // four wavefronts per chain (mp_bwd_team.hip, mp_team21.hip)
   int xcd_group;            // consecutive chains on one die (0: each on another; locate_chain)
 };
 
@@ -596,6 +596,9 @@ inline void launch_team_fwd(const SweepParams& p, bool train, hipStream_t st) {
 }
 template <int R>
 void launch_sweep_bwd(const BackParams& p, bool jacobi, hipStream_t st);
+// 21 labels with a 2-D table, TRWP (mp_team21.hip)
+void launch_team21_fwd(const SweepParams& p, bool train, hipStream_t st);
+void launch_team21_bwd(const BackParams& p, hipStream_t st);
 template <int R>
 void launch_team_bwd(const BackParams& p, bool jacobi, hipStream_t st);
 

@@ -1,0 +1,792 @@
+// TRWP scans for 21 labels with a 2-D table (the segmentation layers), four wavefronts per chain.  The
+// recurrences and what each plane holds: mp_fwd.hip, mp_bwd.hip.
+//
+// Such a launch is bound by the length of one pixel's step: planes of a few megabytes, chains of some
+// hundred pixels that a wavefront walks alone, and 21 of its 64 lanes at work.  As in mp_fwd_team.hip
+// three helper wavefronts load the planes, put what the recurrence needs of a pixel into an LDS slot
+// and, two blocks of pixels later, finish and store it; the main wavefront runs the recurrence out of
+// LDS.  Here every wavefront uses both its halves (32 lanes each, label l in lane l and 32 + l):
+//   * a helper has one pixel in each half, so that an instruction serves two pixels,
+//   * the main wavefront holds the recurrence twice and splits what a label sums or searches over: the
+//     lower half takes the source labels 0 .. 10, the upper one 11 .. 20, and one exchange of halves
+//     joins them.  The 11 values reach the lanes as row broadcasts, a lane operand each, from a half's
+//     source labels in lanes 0 .. 10 of both its rows.
+// The forward step is then 11 multiply-adds and 5 minima in place of 21 and 10, and the argmin labels
+// are left to the helpers, who compare the same 21 candidates with the minimum the main wavefront found.
+// The reverse step adds up 11 gradients under masks (1 or 0 per pair of labels, from the helpers).
+//
+// A lone wavefront issues a 32-bit instruction every 4.2 clocks, one in the 64-bit encoding (lane operands
+// among them) every 5.2, an exchange of rows or halves takes 8.2, an LDS access 10 to 14 (measured); by
+// that count the forward step is 290 clocks and the reverse step 250.  Measured, ns per pixel of rows of 256 /
+// 512 chains, one wavefront per chain -> this: 215 / 223 -> 143 / 145 without argmin labels, 340 / 347 -> 171 / 175
+// with them.  4x129x129, 4 directions, 5 iterations, both other gradients wanted: backward 0.96 -> 0.65 ms; of
+// the 0.22 ms that dcontext costs there most is 516 chains adding 441 pairs to one table per launch.
+//
+// Errors of the reverse scan against 64 bits, one wavefront -> four, geometric means of the relative 2-norm
+// over 40 problems (images up to 130x130, 4 and 8 directions, 1 to 5 iterations; normal, positive and cross
+// entropy gradients): dunary 1.52e-7 -> 1.35e-7, dcontext 5.0e-7 both, dedge_weights 1.79e-7 -> 1.63e-7.
+
+#include <type_traits>
+
+#include "mp_fwd_step.h"
+
+namespace mpl {
+namespace {
+
+constexpr int kL = 21;
+constexpr int kHalf = 32;
+constexpr int kSrc = 11;             // source labels per half (the upper half has one that does not exist)
+constexpr int kHelpers = 3;          // one SIMD of the compute unit each, the main one the fourth
+constexpr int kT = 2 * kHelpers;     // pixels per block
+constexpr int kTeam = (kHelpers + 1) * kWave;
+constexpr int kAhead = 2;            // blocks whose loads are in flight (four measure the same)
+constexpr int kRow = 36;             // words between the pixels of a slot read by both halves at once
+
+// workgroup barrier over LDS contents only: global loads in flight stay in flight
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// f(0) .. f(N - 1) with constant arguments
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(const F& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>());
+    static_for<N, I + 1>(f);
+  }
+}
+
+__device__ __forceinline__ int bits(float x) { return __builtin_bit_cast(int, x); }
+__device__ __forceinline__ float flt(int x) { return __builtin_bit_cast(float, x); }
+
+// The scans want the labels of a half's sources in lanes 0 .. 10 of both its rows: the label a lane holds
+// in that order, `source_label`, is an address to what comes from LDS; what is in registers by label (label
+// l in lanes l and 32 + l) gets there by an exchange of rows and two shifts.
+__device__ __forceinline__ int source_label(int lane) { return (lane / kHalf) * kSrc + (lane & 15); }
+
+// Joins the two halves' minima over their source labels (best), and takes the minimum over all labels
+// (nmin, in every lane).  v: the joint minima by label, src: the same by source label.  pad: +inf in the
+// lanes of a row that hold no label 16 .. 20, -inf in the others.  The issue slots that a lane operand
+// needs between its writing and its reading (two) hold the other chain's instructions.
+__device__ __forceinline__ void join_min(float best, float pad, float& v, float& src, float& nmin) {
+  float t, y;
+  asm("v_mov_b32 %3, %0\n\t"
+      "s_nop 1\n\t"
+      "v_permlane32_swap_b32 %0, %3\n\t"
+      "v_min_f32 %0, %0, %3\n\t"
+      "v_mov_b32 %1, %0\n\t"
+      "v_mov_b32 %4, %0\n\t"
+      "s_nop 1\n\t"
+      "v_permlane16_swap_b32 %1, %4\n\t"
+      "v_max_f32 %3, %4, %5\n\t"
+      "v_min_f32 %2, %1, %3\n\t"
+      "v_mov_b32_dpp %1, %1 row_shl:11 row_mask:0xc bank_mask:0xf\n\t"
+      "s_nop 0\n\t"
+      "v_min_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b32_dpp %1, %4 row_shr:5 row_mask:0xc bank_mask:0xf\n\t"
+      "s_nop 0\n\t"
+      "v_min_f32_dpp %2, %2, %2 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_min_f32_dpp %2, %2, %2 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_min_f32_dpp %2, %2, %2 row_ror:1 row_mask:0xf bank_mask:0xf"
+      : "+&v"(best), "=&v"(src), "=&v"(nmin), "=&v"(t), "=&v"(y)
+      : "v"(pad));
+  v = best;
+}
+
+// The reverse step.  m[0 .. 10] are the masks of a lane's label, m[11] is 1 where it is the argmin label of
+// the normalisation's label.  With DC the sums of dcontext by pair of source label and label (pairs: source
+// label q of the half, the lane's label) are kept by the main wavefront: gw, the gradient times the edge
+// weight, under the same masks.  Those multiply-adds stand in the issue slots that the exchanges and lane
+// shifts of the recurrence leave idle, the first four of them a pixel late.
+
+// x by label -> by source label
+template <bool DC>
+__device__ __forceinline__ float to_sources(float x, float gw, const f32x4& m0, float (&pairs)[kSrc]) {
+  float y;
+  if constexpr (DC) {
+    asm("v_mov_b32 %1, %0\n\t"
+        "v_fmac_f32_dpp %2, %6, %7 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %6, %8 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_permlane16_swap_b32 %0, %1\n\t"
+        "v_fmac_f32_dpp %4, %6, %9 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %5, %6, %10 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %0, %0 row_shl:11 row_mask:0xc bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %0, %1 row_shr:5 row_mask:0xc bank_mask:0xf"
+        : "+&v"(x), "=&v"(y), "+&v"(pairs[0]), "+&v"(pairs[1]), "+&v"(pairs[2]), "+&v"(pairs[3])
+        : "v"(gw), "v"(m0[0]), "v"(m0[1]), "v"(m0[2]), "v"(m0[3]));
+  } else {
+    asm("v_mov_b32 %1, %0\n\t"
+        "s_nop 1\n\t"
+        "v_permlane16_swap_b32 %0, %1\n\t"
+        "s_nop 1\n\t"
+        "v_mov_b32_dpp %0, %0 row_shl:11 row_mask:0xc bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %0, %1 row_shr:5 row_mask:0xc bank_mask:0xf"
+        : "+&v"(x), "=&v"(y));
+  }
+  return x;
+}
+
+// Sums the gradients g (by source label) under the masks, less the sum of all of them (tot: of the half's
+// sources) where m[11] says so, over both halves.  src_mask: all ones in the lanes of source labels, zero
+// in the others.
+template <bool DC>
+__device__ __forceinline__ float masked_sums(float g, float gw, const f32x4 (&m)[3], int src_mask, float& tot,
+                                             float (&pairs)[kSrc]) {
+  float x, y;
+#define MPL_SUMS_HEAD \
+  "v_and_b32 %[t], %[k], %[g]\n\ts_nop 0\n\t" \
+  "v_mul_f32_dpp %[x], %[g], %[m0] row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_mul_f32_dpp %[y], %[g], %[m1] row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_add_f32_dpp %[t], %[t], %[t] row_ror:8 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[x], %[g], %[m2] row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[y], %[g], %[m3] row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_add_f32_dpp %[t], %[t], %[t] row_ror:4 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[x], %[g], %[m4] row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[y], %[g], %[m5] row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_add_f32_dpp %[t], %[t], %[t] row_ror:2 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[x], %[g], %[m6] row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[y], %[g], %[m7] row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_add_f32_dpp %[t], %[t], %[t] row_ror:1 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[x], %[g], %[m8] row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[y], %[g], %[m9] row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fmac_f32_dpp %[x], %[g], %[m10] row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t" \
+  "v_fma_f32 %[y], -%[n], %[t], %[y]\n\t" \
+  "v_add_f32 %[x], %[x], %[y]\n\t" \
+  "v_mov_b32 %[y], %[x]\n\t"
+#define MPL_SUMS_IN                                                                                                  \
+  [g] "v"(g), [k] "v"(src_mask), [m0] "v"(m[0][0]), [m1] "v"(m[0][1]), [m2] "v"(m[0][2]), [m3] "v"(m[0][3]),           \
+      [m4] "v"(m[1][0]), [m5] "v"(m[1][1]), [m6] "v"(m[1][2]), [m7] "v"(m[1][3]), [m8] "v"(m[2][0]), [m9] "v"(m[2][1]), \
+      [m10] "v"(m[2][2]), [n] "v"(m[2][3])
+#define MPL_PAIR(N) "v_fmac_f32_dpp %[p" #N "], %[w], %[m" #N "] row_newbcast:" #N " row_mask:0xf bank_mask:0xf\n\t"
+  if constexpr (DC) {
+    asm(MPL_SUMS_HEAD MPL_PAIR(4) MPL_PAIR(5)
+        "v_permlane32_swap_b32 %[x], %[y]\n\t"
+        MPL_PAIR(6) MPL_PAIR(7) MPL_PAIR(8) MPL_PAIR(9) MPL_PAIR(10)
+        "v_add_f32 %[x], %[x], %[y]"
+        : [x] "=&v"(x), [y] "=&v"(y), [t] "=&v"(tot), [p4] "+&v"(pairs[4]), [p5] "+&v"(pairs[5]), [p6] "+&v"(pairs[6]),
+          [p7] "+&v"(pairs[7]), [p8] "+&v"(pairs[8]), [p9] "+&v"(pairs[9]), [p10] "+&v"(pairs[10])
+        : MPL_SUMS_IN, [w] "v"(gw));
+  } else {
+    asm(MPL_SUMS_HEAD "s_nop 1\n\t"
+        "v_permlane32_swap_b32 %[x], %[y]\n\t"
+        "v_add_f32 %[x], %[x], %[y]"
+        : [x] "=&v"(x), [y] "=&v"(y), [t] "=&v"(tot)
+        : MPL_SUMS_IN);
+  }
+#undef MPL_PAIR
+#undef MPL_SUMS_IN
+#undef MPL_SUMS_HEAD
+  return x;
+}
+
+// lane N of every row, in all its lanes
+template <int N>
+__device__ __forceinline__ float row_bcast(float x) {
+  return flt(__builtin_amdgcn_mov_dpp(bits(x), 0x150 + N, 0xf, 0xf, true));
+}
+// lower half of x in both halves, upper half of x in both halves
+__device__ __forceinline__ void halves(float x, float& lower, float& upper) {
+  const auto r = __builtin_amdgcn_permlane32_swap((unsigned)bits(x), (unsigned)bits(x), false, false);
+  lower = flt((int)r[0]);
+  upper = flt((int)r[1]);
+}
+
+// sums over the lanes of each half, in its last lane
+__device__ __forceinline__ float half_sum(float x) {
+#define MPL_ADD_DPP(CTRL) "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 " CTRL " bank_mask:0xf\n\t"
+  asm(MPL_ADD_DPP("row_shr:1 row_mask:0xf") MPL_ADD_DPP("row_shr:2 row_mask:0xf")
+      MPL_ADD_DPP("row_shr:4 row_mask:0xf") MPL_ADD_DPP("row_shr:8 row_mask:0xf")
+      MPL_ADD_DPP("row_bcast:15 row_mask:0xa") "s_nop 0"
+      : "+v"(x));
+#undef MPL_ADD_DPP
+  return x;
+}
+
+// ---- forward ---------------------------------------------------------------------------------------
+struct alignas(16) FwdSlots {   // one set
+  float in[kT][kHalf][2];       // U, edge weight
+  float a[kT][kRow];            // beliefs the pixel's message comes from (argmin labels kept)
+  float out[kT][kHalf][2];      // v and the normalisation minimum; without argmin labels the message
+};
+
+template <bool TRAIN>
+__global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) {
+  extern __shared__ __align__(16) char smem_raw[];
+  FwdSlots* sets = reinterpret_cast<FwdSlots*>(smem_raw);  // two
+  const int tid = threadIdx.x;
+  // (the last wavefront: mp_fwd_team.hip)
+  const int role = uniform_i(tid / kWave);  // kHelpers: main
+  const int lane = tid & (kWave - 1);
+  const int l = lane & (kHalf - 1);
+  const int half = lane / kHalf;
+  const bool ok = l < kL;
+  const ChainCtx ch0 = locate_chain(p);
+  const int n = ch0.n;
+  const float rho = p.rho;
+  const int blocks = (n + kT - 1) / kT;
+  const int iters = (blocks + 2 + kAhead - 1) / kAhead * kAhead;
+  const float floor_l = ok ? -INFINITY : INFINITY;
+  auto table = [&](int fd) __attribute__((always_inline)) {  // ctx(l, fd), TRWP_forward.cu:101-113
+    const int cd = ok ? l : kL - 1, f = fd < kL ? fd : kL - 1;
+    return p.ctx[cd < f ? cd * kL + f : f * kL + cd];
+  };
+
+  auto main_walk = [&]() __attribute__((always_inline)) {
+    float tc[kSrc];
+#pragma unroll
+    for (int i = 0; i < kSrc; ++i) tc[i] = table(half * kSrc + i);
+    const int sl = source_label(lane);
+    const float pad = (lane & 15) < kL - 16 ? -INFINITY : INFINITY;
+    float prev = 0.f, uf = 0.f;  // message and U of the front pixel, by source label
+    for (int k = 0; k < iters; ++k) {
+      if (k >= 1 && k <= blocks) {
+        FwdSlots& s = sets[(k - 1) & 1];
+        f32x2 cur = *reinterpret_cast<const f32x2*>(s.in[0][sl]);
+#pragma unroll
+        for (int i = 0; i < kT; ++i) {
+          f32x2 nxt = cur;
+          if (i + 1 < kT) nxt = *reinterpret_cast<const f32x2*>(s.in[i + 1][sl]);
+          const float a = fmaf(rho, prev, uf);
+          if (TRAIN) s.a[i][sl] = a;
+          float c[kSrc];
+          static_for<kSrc>([&](auto ii) __attribute__((always_inline)) {
+            constexpr int q = decltype(ii)::value;
+            c[q] = fmaf(cur[1], tc[q], row_bcast<q>(a));
+          });
+          const float best = fminf(fminf(fminf(fminf(c[0], c[1]), c[2]), fminf(fminf(c[3], c[4]), c[5])),
+                                   fminf(fminf(fminf(c[6], c[7]), c[8]), fminf(c[9], c[10])));
+          float v, vs, nmin;
+          join_min(best, pad, v, vs, nmin);
+          prev = (i == 0 && k == 1) ? 0.f : vs - nmin;  // (the chain start has no front pixel and no message)
+          if (TRAIN)
+            *reinterpret_cast<f32x2*>(s.out[i][l]) = f32x2{v, nmin};
+          else
+            s.out[i][sl][0] = prev;
+          uf = cur[0];
+          cur = nxt;
+        }
+      }
+      lds_barrier();
+    }
+  };
+
+  const int64_t HW = (int64_t)p.H * p.W;
+  const int64_t P = (int64_t)p.B * HW;
+  const int64_t N = P * kL;
+
+  // even_walk: a constant; the first (even direction) or the second sweep of a pair (run_chain_fwd)
+  auto helper_walk = [&](const ChainCtx& ch, const bool skip_s_in, const auto even_walk)
+      __attribute__((always_inline)) {
+    constexpr bool EVEN = decltype(even_walk)::value;
+    const int dir = ch.dir;
+    const int64_t img_p = (int64_t)ch.bv * HW;
+    const int64_t img_e = img_p * kL;
+    const bool known = p.desc != nullptr && p.desc->msg_nonzero == 0;  // the initial messages are zero
+    const bool zfirst = p.zero_first && known;
+    const bool skip_s = skip_s_in || (EVEN && zfirst);
+    const bool md_zero = p.first_iter && known;
+    const bool mi_zero = md_zero && EVEN;
+    const int img_bytes = (int)(unsigned)(HW * kL * 4);
+    const rsrc_t rS = make_rsrc((zfirst ? p.belief_zero : p.belief) + img_e, img_bytes);
+    const rsrc_t rMd = make_rsrc(p.msg_in + (int64_t)dir * N + img_e, md_zero ? 0 : img_bytes);
+    const rsrc_t rMi = make_rsrc(p.msg_in + (int64_t)(dir ^ 1) * N + img_e, mi_zero ? 0 : img_bytes);
+    const rsrc_t rMo = make_rsrc(p.msg_out + (int64_t)dir * N + img_e, img_bytes);
+    const rsrc_t rSo = make_rsrc(p.belief_out + img_e, skip_s ? 0 : img_bytes);
+    const rsrc_t rImin = make_rsrc(TRAIN ? p.idx_min + (int64_t)dir * N + img_e : nullptr, TRAIN ? (int)(HW * kL) : 0);
+    const rsrc_t rInorm = make_rsrc(TRAIN ? p.idx_norm + (int64_t)dir * P + img_p : nullptr, TRAIN ? (int)HW : 0);
+    const rsrc_t rW = make_rsrc(p.edge + (int64_t)dir * P + img_p, (int)(HW * 4));
+    float tcol[TRAIN ? kL : 1];
+    if constexpr (TRAIN) {
+#pragma unroll
+      for (int fd = 0; fd < kL; ++fd) tcol[fd] = table(fd);
+    }
+    const int i = 2 * role + half;  // the pixel of a block in this half
+    struct Pix {
+      float s, md, mi, w;
+    };
+    auto pixel_off = [&](const int t) __attribute__((always_inline)) { return (unsigned)(ch.pix0 + t * ch.pstep); };
+    auto label_off = [&](const bool on, const unsigned pp) __attribute__((always_inline)) {
+      return (int)((on && ok) ? (pp * (unsigned)kL + (unsigned)l) * 4u : kDeadWide);
+    };
+    auto load = [&](rsrc_t r, int off) __attribute__((always_inline)) {
+      return flt((int)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    };
+    auto store = [&](rsrc_t r, int off, float x) __attribute__((always_inline)) {
+      __builtin_amdgcn_raw_buffer_store_b32((unsigned)bits(x), r, off, 0, 0);
+    };
+    // the loads of chain position t (nothing is read past the end of the chain)
+    auto load_pix = [&](const int t) __attribute__((always_inline)) {
+      Pix r;
+      const bool on = t < n;
+      const unsigned pp = pixel_off(t);
+      const int off = label_off(on, pp);
+      r.s = load(rS, off);
+      r.md = 0.f;
+      if (EVEN) r.md = load(rMd, off);
+      r.mi = load(rMi, off);
+      r.w = load(rW, (int)(on ? pp * 4u : kDeadWide));
+      return r;
+    };
+    // second sweep: the old message of the chain start
+    float md0 = 0.f;
+    if (!EVEN) md0 = load(rMd, label_off(i == 0, pixel_off(0)));
+
+    float tt[2] = {0.f, 0.f}, ww[2] = {0.f, 0.f};
+    auto prepare = [&](const Pix& px, const int t, FwdSlots& s, float& tk, float& wk) __attribute__((always_inline)) {
+      tk = EVEN ? px.s - px.md : px.s + px.mi;
+      const float un = fmaxf(fmaf(tk, rho, -px.mi), floor_l);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
+      wk = px.w;
+      *reinterpret_cast<f32x2*>(s.in[i][l]) = f32x2{un, px.w};
+      // Q of the pixel is known already, whatever its message
+      if (EVEN) store(rSo, label_off(t < n, pixel_off(t)), tk - px.mi);
+    };
+    // what is left of a pixel once its message is known (nothing outside the chain)
+    auto finish = [&](const int t, const FwdSlots& s, const float tk, const float wk) __attribute__((always_inline)) {
+      const bool on = t >= 0 && t < n;
+      const bool step = t > 0 && t < n;
+      const unsigned pp = pixel_off(t);
+      const int off = label_off(on, pp);
+      float m;
+      if constexpr (TRAIN) {
+        const f32x2 o = *reinterpret_cast<const f32x2*>(s.out[i][l]);
+        float val[kL];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(&s.a[i][4 * q]);
+#pragma unroll
+          for (int z = 0; z < 4; ++z) val[4 * q + z] = fmaf(wk, tcol[4 * q + z], x[z]);
+        }
+        val[20] = fmaf(wk, tcol[20], s.a[i][20]);
+        int arg;
+        float unused = 0.f;
+        argmin_and_lane_min_21(val, o[0], unused, arg);
+        const uint64_t at = ballot(ok && o[0] == o[1]);
+        const unsigned lo = (unsigned)at, hi = (unsigned)(at >> 32);
+        const int n0 = lo ? 31 - __builtin_clz(lo) : kL - 1, n1 = hi ? 31 - __builtin_clz(hi) : kL - 1;
+        m = t == 0 ? 0.f : o[0] - o[1];
+        __builtin_amdgcn_raw_buffer_store_b8((unsigned char)arg, rImin,
+                                             (int)((step && ok) ? pp * (unsigned)kL + (unsigned)l : kDeadWide), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b8((unsigned char)(half ? n1 : n0), rInorm,
+                                             (int)((step && l == 0) ? pp : kDeadWide), 0, 0);
+      } else {
+        m = s.out[i][l][0];
+      }
+      // (the reference never writes the chain start)
+      store(rMo, (step || p.zero_start) ? off : (int)kDeadWide, m);
+      if constexpr (!EVEN) store(rSo, off, tk + (t == 0 ? md0 : m));
+    };
+
+    Pix ring[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      ring[q] = load_pix(q * kT + i);
+      MPL_ORDER_LOADS();
+    }
+#pragma clang loop unroll(disable)
+    for (int k0 = 0; k0 < iters; k0 += kAhead) {
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q) {
+        const int k = k0 + q;
+        FwdSlots& s = sets[q & 1];
+        finish((k - 2) * kT + i, s, tt[q & 1], ww[q & 1]);
+        lds_order();
+        prepare(ring[q], k * kT + i, s, tt[q & 1], ww[q & 1]);
+        ring[q] = load_pix((k + kAhead) * kT + i);
+        lds_barrier();
+      }
+    }
+  };
+
+  // the second sweep of a pair reads what the first one's helpers stored: on the same compute unit,
+  // once their stores are complete
+  if (role == kHelpers) {
+    __builtin_amdgcn_s_setprio(3);
+    main_walk();
+    if (!(ch0.dir & 1) && p.fused_pair) {
+      __syncthreads();
+      main_walk();
+    }
+  } else {
+    if (!(ch0.dir & 1)) helper_walk(ch0, p.skip_s_store != 0, std::true_type());
+    if ((ch0.dir & 1) || p.fused_pair) {
+      ChainCtx ch = ch0;
+      bool skip_s = p.skip_s_store != 0;
+      if (!(ch0.dir & 1)) {
+        ch.dir = ch0.dir ^ 1;
+        ch.pix0 = ch0.pix0 + (n - 1) * ch0.pstep;
+        ch.pstep = -ch0.pstep;
+        skip_s = p.skip_s_store2 != 0;
+        wait_vmem<0>();
+        __syncthreads();
+      }
+      helper_walk(ch, skip_s, std::false_type());
+    }
+  }
+}
+
+// ---- backward --------------------------------------------------------------------------------------
+struct alignas(16) BwdSlots {   // one set
+  float mask[kT][2][kL][12];    // per half's sources and label: 1 where the source label points at the
+                                // label, else 0; last: 1 where the normalisation's argmin label is the label
+  float base[kT][kHalf][2];     // gradient of the message without what the recurrence adds; the edge weight,
+                                // 0 where the pixel has no incoming edge
+  float sc[kT][kHalf];          // dU of the pixel (main wavefront)
+  float tot[kT][2];             // sums of the message's gradient over a half's sources (main wavefront)
+  int fd[kT][kHalf];            // argmin labels
+};
+constexpr int kPairs = kL * kL;
+
+// GR: dedge_weights and / or dcontext are wanted; DC: dcontext is
+template <bool GR, bool DC>
+__global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
+  extern __shared__ __align__(16) char smem_raw[];
+  BwdSlots* sets = reinterpret_cast<BwdSlots*>(smem_raw);  // two
+  float* acc = reinterpret_cast<float*>(sets + 2);         // kMaxL
+  float* ctx_s = acc + kMaxL;                              // the table, then dcontext of the chain
+  float* hist_s = ctx_s + kPairs;
+  const int tid = threadIdx.x;
+  const int role = uniform_i(tid / kWave);  // kHelpers: main
+  const int lane = tid & (kWave - 1);
+  const int l = lane & (kHalf - 1);
+  const int half = lane / kHalf;
+  const bool ok = l < kL;
+  const ChainCtx ch0 = locate_chain(p);
+  const int n = ch0.n;
+  const float rho = p.rho;
+  const int blocks = (n + kT - 1) / kT;
+  const int iters = (blocks + 2 + kAhead - 1) / kAhead * kAhead;
+  const bool want_de = GR && p.dedge != nullptr;
+  const bool same = p.same_label != 0;
+  if (tid < kMaxL) acc[tid] = 0.f;
+  if (GR) {
+    for (int i = tid; i < kPairs; i += kTeam) ctx_s[i] = p.ctx[i];
+    for (int i = tid; i < kPairs; i += kTeam) hist_s[i] = 0.f;
+  }
+  __syncthreads();
+
+  float pairs[kSrc];  // (main wavefront) dcontext: source label half * kSrc + q, label l
+#pragma unroll
+  for (int q = 0; q < kSrc; ++q) pairs[q] = 0.f;
+  auto main_walk = [&]() __attribute__((always_inline)) {
+    const int sl = source_label(lane);
+    const int src_mask = (lane & 15) < kSrc && sl < kL ? -1 : 0;
+    const int lm = ok ? l : kL - 1;  // (a lane without a label repeats the last one's sums: nothing reads them)
+    float sc = 0.f;
+    struct In {
+      f32x4 m[3];
+      f32x2 b;
+    };
+    auto get = [&](const BwdSlots& s, const int i) __attribute__((always_inline)) {
+      In x;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) x.m[q] = *reinterpret_cast<const f32x4*>(&s.mask[i][half][lm][4 * q]);
+      x.b = *reinterpret_cast<const f32x2*>(s.base[i][sl]);
+      return x;
+    };
+    // A block of pixels whose gradients are not all finite, one after another: a zero mask does not switch
+    // such a term off, so the gradients go to their labels through LDS.
+    auto careful_block = [&](BwdSlots& s, const int k) __attribute__((always_inline)) {
+#pragma clang loop unroll(disable)
+      for (int i = 0; i < kT; ++i) {
+        const In cur = get(s, i);
+        s.sc[i][l] = sc;
+        float none[kSrc];
+        const float g = fmaf(rho, to_sources<false>(sc, 0.f, cur.m[0], none), cur.b[0]);
+        if (src_mask != 0 && (lane & 16) == 0) atomicAdd(&acc[s.fd[i][sl]], g);
+        lds_order();
+        sc = acc[l];
+        lds_order();
+        acc[lane] = 0.f;
+        lds_order();
+        float tot = src_mask != 0 ? g : 0.f, lower, upper;
+        tot += dpp_f<0x128>(0.f, tot);  // row_ror: 8, 4, 2, 1
+        tot += dpp_f<0x124>(0.f, tot);
+        tot += dpp_f<0x122>(0.f, tot);
+        tot += dpp_f<0x121>(0.f, tot);
+        halves(tot, lower, upper);
+        if (cur.m[2][3] != 0.f) sc -= lower + upper;
+        if (GR) s.tot[i][half] = tot;
+        if (DC && n - 1 - ((k - 1) * kT + i) >= 1) {
+          const float gwi = cur.b[1] * g;
+          static_for<kSrc>([&](auto ii) __attribute__((always_inline)) {
+            constexpr int q = decltype(ii)::value;
+            const float x = row_bcast<q>(gwi);
+            pairs[q] += bits(cur.m[q / 4][q % 4]) != 0 ? x : 0.f;
+          });
+        }
+      }
+    };
+    float gw = 0.f;  // of the pixel before, whose first four pairs are still to be added
+    f32x4 m0 = {0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < iters; ++k) {
+      if (k >= 1 && k <= blocks) {
+        BwdSlots& s = sets[(k - 1) & 1];
+        In cur = get(s, 0);
+        const float sc_was = sc;
+        float pairs_were[kSrc];
+        if (DC) {
+          static_for<4>([&](auto ii) __attribute__((always_inline)) {
+            constexpr int q = decltype(ii)::value;
+            pairs[q] = fmaf(row_bcast<q>(gw), m0[q], pairs[q]);
+          });
+          gw = 0.f;
+#pragma unroll
+          for (int q = 0; q < kSrc; ++q) pairs_were[q] = pairs[q];
+        }
+#pragma unroll
+        for (int i = 0; i < kT; ++i) {
+          In nxt = cur;
+          if (i + 1 < kT) nxt = get(s, i + 1);
+          s.sc[i][l] = sc;
+          // gradient w.r.t. the normalised message of this pixel, including what the previous step
+          // added through the recurrence (dmsg[front] += rho * value, TRWP_backward.cu:108)
+          const float g = fmaf(rho, to_sources<DC>(sc, gw, m0, pairs), cur.b[0]);
+          if (DC) {
+            gw = cur.b[1] * g;
+            m0 = cur.m[0];
+          }
+          float tot;
+          // MsgNormNaiveBack (commonCUDA.cuh:131-145) through the argmin label of its label
+          sc = masked_sums<DC>(g, gw, cur.m, src_mask, tot, pairs);
+          if (GR) s.tot[i][half] = tot;
+          cur = nxt;
+        }
+        // an infinity or a NaN in any gradient makes NaN of every sum of its pixel and of all after it
+        // (tested as an integer: the compiler may take NaN for anything)
+        int probe = uniform_i(bits(sc));
+        asm("" : "+s"(probe));
+        if (__builtin_expect((probe & 0x7f800000) == 0x7f800000, 0)) {
+          sc = sc_was;
+          if (DC) {
+            gw = 0.f;
+#pragma unroll
+            for (int q = 0; q < kSrc; ++q) pairs[q] = pairs_were[q];
+          }
+          careful_block(s, k);
+        }
+      }
+      lds_barrier();
+    }
+    if (DC) {
+      static_for<4>([&](auto ii) __attribute__((always_inline)) {
+        constexpr int q = decltype(ii)::value;
+        pairs[q] = fmaf(row_bcast<q>(gw), m0[q], pairs[q]);
+      });
+    }
+  };
+
+  // even_walk: a constant; which of the two walks of a pair this is (mp_bwd.hip)
+  auto helper_walk = [&](const ChainCtx& ch, const auto even_walk) __attribute__((always_inline)) {
+    constexpr bool EVEN = decltype(even_walk)::value;
+    const int dir = ch.dir;
+    const int64_t HW = (int64_t)p.H * p.W;
+    const int64_t P = (int64_t)p.B * HW;
+    const int64_t N = P * kL;
+    const int64_t img_p = (int64_t)ch.bv * HW;
+    const int64_t img_e = img_p * kL;
+    float* bHd = p.h + (int64_t)dir * N + img_e;
+    float* bHi = p.h + (int64_t)(dir ^ 1) * N + img_e;
+    const int img_bytes = (int)(unsigned)(HW * kL * 4);
+    const rsrc_t rA = make_rsrc(p.a_in + img_e, img_bytes);
+    const rsrc_t rAo = make_rsrc(EVEN ? p.a_out + img_e : bHd, img_bytes);
+    const rsrc_t rHdIn = make_rsrc(bHd, !p.first_touch ? img_bytes : 0);
+    const rsrc_t rHiIn = make_rsrc(bHi, EVEN ? img_bytes : 0);
+    const rsrc_t rHiOut = make_rsrc(bHi, (EVEN && !p.skip_h_store) ? img_bytes : 0);
+    const rsrc_t rImin = make_rsrc(p.idx_min + (int64_t)dir * N + img_e, (int)(HW * kL));
+    const rsrc_t rInorm = make_rsrc(p.idx_norm + (int64_t)dir * P + img_p, (int)HW);
+    const rsrc_t rW = make_rsrc(p.edge + (int64_t)dir * P + img_p, (int)(HW * 4));
+    const rsrc_t rDe = make_rsrc(want_de ? p.dedge + (int64_t)dir * P + img_p : nullptr, want_de ? (int)(HW * 4) : 0);
+    const int p_last = ch.pix0 + (n - 1) * ch.pstep;
+    const int i = 2 * role + half;  // the pixel of a block in this half
+    const int sl = source_label(lane);
+    struct Pix {
+      float a, hd, hi, w, de;
+      int fd, nidx;
+    };
+    auto label_off = [&](const bool on, const unsigned pp) __attribute__((always_inline)) {
+      return (int)((on && ok) ? (pp * (unsigned)kL + (unsigned)l) * 4u : kDeadWide);
+    };
+    auto load = [&](rsrc_t r, int off) __attribute__((always_inline)) {
+      return flt((int)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    };
+    auto store = [&](rsrc_t r, int off, float x) __attribute__((always_inline)) {
+      __builtin_amdgcn_raw_buffer_store_b32((unsigned)bits(x), r, off, 0, 0);
+    };
+    // the loads of walk position s (nothing is read past the end of the chain)
+    auto load_pix = [&](const int s) __attribute__((always_inline)) {
+      Pix r;
+      const bool on = s < n;
+      const unsigned pp = (unsigned)(p_last - s * ch.pstep);
+      const int off = label_off(on, pp);
+      r.a = load(rA, off);
+      r.hd = load(rHdIn, off);
+      r.hi = 0.f;
+      if (EVEN) r.hi = load(rHiIn, off);
+      r.fd = __builtin_amdgcn_raw_buffer_load_b8(rImin, (int)((on && ok) ? pp * (unsigned)kL + (unsigned)l : kDeadWide), 0, 0);
+      r.nidx = __builtin_amdgcn_raw_buffer_load_b8(rInorm, (int)(on ? pp : kDeadWide), 0, 0);
+      r.w = r.de = 0.f;
+      if (GR) {
+        r.w = load(rW, (int)(on ? pp * 4u : kDeadWide));
+        r.de = load(rDe, (int)(on ? pp * 4u : kDeadWide));
+      }
+      return r;
+    };
+    struct Kept {  // of a pixel whose dU is not known yet
+      float ap, base, w, de, cv;
+      int fd, nidx, fn;
+    };
+    // walk position u
+    auto prepare = [&](const Pix& px, const int u, BwdSlots& s, Kept& kp) __attribute__((always_inline)) {
+      kp.ap = EVEN ? fmaf(rho, px.hi, px.a) : px.a;
+      kp.base = ok ? kp.ap + (EVEN ? -px.hd - px.hi : px.hd) : 0.f;
+      kp.w = px.w;
+      kp.de = px.de;
+      kp.fd = px.fd;
+      kp.nidx = px.nidx;
+      *reinterpret_cast<f32x2*>(s.base[i][l]) = f32x2{kp.base, u < n - 1 ? px.w : 0.f};
+      if (GR) {
+        const int lo = l < px.fd ? l : px.fd, hi = l < px.fd ? px.fd : l;
+        kp.cv = ok && px.fd < kL ? ctx_s[lo * kL + hi] : 0.f;
+      }
+      s.fd[i][l] = px.fd;
+      lds_order();
+      const float fl = (float)l;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {  // the pixel of either half
+        const int nidx = __builtin_amdgcn_readlane(px.nidx, h * kHalf);
+        const int fn = __builtin_amdgcn_readlane(px.fd, h * kHalf + (nidx & (kHalf - 1)));
+        // (no label points from a lane without one)
+        const float src = sl < kL ? (float)s.fd[2 * role + h][sl] : -1.f;
+        float m[12];
+        static_for<kSrc>([&](auto ii) __attribute__((always_inline)) {
+          constexpr int q = decltype(ii)::value;
+          const float d = row_bcast<q>(src) - fl;
+          m[q] = __builtin_amdgcn_fmed3f(1.f - __builtin_fabsf(d), 0.f, 1.f);
+        });
+        m[11] = l == fn ? 1.f : 0.f;
+        if (half == h) kp.fn = fn;
+        if (ok) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q)
+            *reinterpret_cast<f32x4*>(&s.mask[2 * role + h][half][l][4 * q]) = f32x4{m[4 * q], m[4 * q + 1], m[4 * q + 2], m[4 * q + 3]};
+        }
+      }
+    };
+    // what is left of a pixel once its dU is known (chain position t; nothing outside the chain)
+    auto finish = [&](const int t, const BwdSlots& s, const Kept& kp) __attribute__((always_inline)) {
+      const bool on = t >= 0 && t < n;
+      const unsigned pp = (unsigned)(ch.pix0 + t * ch.pstep);
+      const int off = label_off(on, pp);
+      const float sc = s.sc[i][l];
+      if constexpr (!EVEN) {
+        store(rAo, off, sc);
+      } else {
+        store(rAo, off, fmaf(rho, sc, kp.ap));  // g_k += rho*dU for every k, dunary too
+        store(rHiOut, off, -kp.ap - sc);        // g_o was 0 after its own walk (h_o = -A'), then g_o -= dU
+      }
+      if constexpr (GR) {
+        const bool edge = t >= 1 && t < n;  // the chain start has no incoming edge
+        const float tot = s.tot[i][0] + s.tot[i][1];
+        float g = fmaf(rho, sc, kp.base);
+        if (l == kp.nidx) g -= tot;
+        float det = ok && edge ? kp.cv * g : 0.f;
+        if (want_de) det = half_sum(det);
+        // what the normalisation adds to dcontext; the gradients themselves are the main wavefront's
+        if (DC && l == 0 && edge && kp.nidx < kL && kp.fn < kL && (same || kp.nidx != kp.fn)) {
+          const int lo = kp.nidx < kp.fn ? kp.nidx : kp.fn, hi = kp.nidx < kp.fn ? kp.fn : kp.nidx;
+          atomicAdd(&hist_s[lo * kL + hi], -kp.w * tot);
+        }
+        // each pixel receives over exactly one edge per direction: plain read-modify-write
+        store(rDe, (int)((edge && l == kHalf - 1) ? pp * 4u : kDeadWide), kp.de + det);
+      }
+    };
+
+    Pix ring[kAhead];
+    Kept kept[2] = {};
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      ring[q] = load_pix(q * kT + i);
+      MPL_ORDER_LOADS();
+    }
+#pragma clang loop unroll(disable)
+    for (int k0 = 0; k0 < iters; k0 += kAhead) {
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q) {
+        const int k = k0 + q;
+        BwdSlots& s = sets[q & 1];
+        finish(n - 1 - ((k - 2) * kT + i), s, kept[q & 1]);
+        lds_order();
+        prepare(ring[q], k * kT + i, s, kept[q & 1]);
+        ring[q] = load_pix((k + kAhead) * kT + i);
+        lds_barrier();
+      }
+    }
+  };
+
+  if (role == kHelpers) {
+    __builtin_amdgcn_s_setprio(3);
+    main_walk();
+    if ((ch0.dir & 1) && p.fused_pair) {
+      __syncthreads();
+      main_walk();
+    }
+  } else {
+    if (ch0.dir & 1) helper_walk(ch0, std::false_type());
+    if (!(ch0.dir & 1) || p.fused_pair) {
+      ChainCtx ch = ch0;
+      if (ch0.dir & 1) {
+        ch.dir = ch0.dir ^ 1;
+        ch.pix0 = ch0.pix0 + (n - 1) * ch0.pstep;
+        ch.pstep = -ch0.pstep;
+        wait_vmem<0>();
+        __syncthreads();
+      }
+      helper_walk(ch, std::true_type());
+    }
+  }
+  if (!DC) return;
+  if (role == kHelpers) {
+#pragma unroll
+    for (int q = 0; q < kSrc; ++q) {
+      const int cd = half * kSrc + q;  // the label that points, at fd = l
+      if (ok && cd < kL && (same || cd != l)) {
+        const int ci = cd < l ? cd * kL + l : l * kL + cd;
+        if (has_value(pairs[q])) atomicAdd(&hist_s[ci], pairs[q]);
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < kPairs; i += kTeam)
+    if (has_value(hist_s[i])) atomicAdd(&p.dctx[i], hist_s[i]);
+}
+
+}  // namespace
+
+void launch_team21_fwd(const SweepParams& p, bool train, hipStream_t st) {
+  const int blocks = p.block_prefix[p.n_dirs];
+  if (blocks <= 0) return;
+  const size_t lds = 2 * sizeof(FwdSlots);
+  if (train)
+    fwd_team21_kernel<true><<<blocks, kTeam, lds, st>>>(p);
+  else
+    fwd_team21_kernel<false><<<blocks, kTeam, lds, st>>>(p);
+}
+
+void launch_team21_bwd(const BackParams& p, hipStream_t st) {
+  const int blocks = p.block_prefix[p.n_dirs];
+  if (blocks <= 0) return;
+  const bool gr = p.dedge != nullptr || p.dctx != nullptr;
+  const size_t lds = 2 * sizeof(BwdSlots) + sizeof(float) * (kMaxL + (gr ? 2 * kPairs : 0));
+  if (p.dctx != nullptr)
+    bwd_team21_kernel<true, true><<<blocks, kTeam, lds, st>>>(p);
+  else if (gr)
+    bwd_team21_kernel<true, false><<<blocks, kTeam, lds, st>>>(p);
+  else
+    bwd_team21_kernel<false, false><<<blocks, kTeam, lds, st>>>(p);
+}
+
+}  // namespace mpl

@@ -1,0 +1,66 @@
+"""TRWP's reverse scan for 21 labels and a 2-D table with four wavefronts per chain (MPL_OPT_TEAM_SCANS)
+against the fp64 oracle: chains around a block of six pixels, both kinds of dcontext, gradients that are left
+out, argmin labels that crowd on one target, terms that are not finite."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+L = 21
+
+
+def _problem(n_dir, n_iter, B, H, W, seed, crowd=False):
+  rng = np.random.default_rng(seed)
+  ctx = np.triu(rng.random((L, L)), 1).astype(np.float32)
+  ew = (rng.random((n_dir, B, 1, H, W)) - 0.2).astype(np.float32)
+  dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
+  imin = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W, L)).astype(np.uint8)
+  if crowd:
+    imin[...] = rng.integers(0, L, imin.shape[:-1] + (1,))
+  inorm = rng.integers(0, L, (n_iter, n_dir, B, 1, H, W)).astype(np.uint8)
+  return ctx, ew, dcost, imin, inorm
+
+
+def _backward(gpu, problem, option=2, **kw):
+  from mplayers_amd import _lib
+  ctx, ew, dcost, imin, inorm = problem
+  _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+  try:
+    return gpu.gpu_backward("TRWP", ctx, ew, dcost, imin, inorm, 0.5, **kw)
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+
+
+@pytest.mark.parametrize("n_dir,B,H,W", [(2, 1, 1, 1), (4, 1, 2, 5), (4, 2, 6, 7), (8, 1, 12, 13), (4, 1, 3, 50),
+                                         (16, 1, 9, 11)])
+@pytest.mark.parametrize("crowd", [False, True])
+def test_backward_against_the_oracle(gpu, oracle, n_dir, B, H, W, crowd):
+  from mplayers_amd import _lib
+  problem = _problem(n_dir, 2, B, H, W, 100 * H + W, crowd)
+  ctx, ew, dcost, imin, inorm = problem
+  for same, flags in ((False, 0), (True, _lib.F_DCONTEXT_SAME_LABEL), (False, _lib.F_FUSED_PAIRS_OFF)):
+    print("case", n_dir, B, H, W, crowd, same, flags, flush=True)
+    ref = oracle.backward("TRWP", ctx.astype(np.float64), ew.astype(np.float64), dcost.astype(np.float64), imin,
+                          inorm, 0.5, same_label=same)
+    got = _backward(gpu, problem, flags=flags | _lib.F_PACKED_OFF)
+    for a, b, what in zip(got, ref, ("dunary", "dcontext", "dedge_weights")):
+      # sums of at most a few thousand products: 1e-4 of the largest entry, as everywhere
+      assert np.abs(a - b).max() <= 1e-4 * max(1.0, float(np.abs(b).max())), what
+    for want_dctx, want_dedge in ((False, False), (True, False), (False, True)):
+      part = _backward(gpu, problem, flags=flags | _lib.F_PACKED_OFF, want_dctx=want_dctx, want_dedge=want_dedge)
+      assert np.array_equal(part[0], got[0])
+      if want_dedge:
+        assert np.array_equal(part[2], got[2])
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_terms_that_are_not_finite(gpu, value):
+  """They reach the entries they reach with one wavefront per chain, and the others are what they are there."""
+  problem = _problem(4, 1, 1, 9, 14, 3)
+  problem[2][0, 0, 4, 5, 7] = value
+  one, four = _backward(gpu, problem, 0), _backward(gpu, problem, 2)
+  for a, b, what in zip(four, one, ("dunary", "dcontext", "dedge_weights")):
+    assert np.array_equal(np.isnan(a), np.isnan(b)), what
+    assert np.array_equal(np.isposinf(a), np.isposinf(b)) and np.array_equal(np.isneginf(a), np.isneginf(b)), what
+    ok = np.isfinite(b)
+    assert np.abs(a[ok] - b[ok]).max() <= 1e-4 * max(1.0, float(np.abs(b[ok]).max())), what
