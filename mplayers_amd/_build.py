@@ -40,6 +40,8 @@ def _units():
                     ["-DMPL_INST_R=%d" % r, "-DMPL_INST_TRAIN=%d" % t]))
       units.append(("mp_fwd_team_r%d_t%d" % (r, t), "mp_fwd_team.hip",
                     ["-DMPL_INST_R=%d" % r, "-DMPL_INST_TRAIN=%d" % t]))
+    if r < 4:
+      units.append(("mp_fwd_dense_r%d" % r, "mp_fwd_dense.hip", ["-DMPL_INST_R=%d" % r]))
     units.append(("mp_bwd_r%d" % r, "mp_bwd.hip", ["-DMPL_INST_R=%d" % r]))
     if r > 1:
       units.append(("mp_bwd_team_r%d" % r, "mp_bwd_team.hip", ["-DMPL_INST_R=%d" % r]))

@@ -786,6 +786,24 @@ int choose_split(const mpl_shape* s, const Params& p, const CallOpts& o, bool tr
   return w >= 2 ? w : 0;
 }
 
+// Four wavefronts per chain for a table declared dense, TRWP forward (mp_fwd_dense.hip), in place of those of
+// choose_split and of mp_fwd_team.hip.  Measured on rows of 300 pixels with a random table, ns per pixel with one
+// wavefront / as choose_split has it / mp_fwd_team.hip / this.  Argmin labels kept, 256 chains: 16 labels 613 / -
+// / 357 / 367, 32 labels 824 / - / 536 / 371, 64 labels 1175 / - / 880 / 414, 96 labels 2324 / 1400 / 1540 / 674,
+// 192 labels 4172 / 2242 / 3079 / 1223; 1248 chains: 16 labels 681 / - / 480 / 563, 32 labels 922 / - / 718 /
+// 563, 96 labels 2858 / 2115 / 2635 / 1555, 192 labels 5568 / 4356 / 6342 / 3742.  Without them, 256 chains: 32
+// labels 551 / - / 498 / 313, 96 labels 1602 / 770 / 1459 / 587, 192 labels 3078 / 1167 / 2962 / 915; 1248
+// chains: 96 labels 2083 / 1486 / 1902 / 1300, 192 labels 4159 / 3701 / 4141 / 2813.
+constexpr int kDenseTeamMinL = 17;
+constexpr int kDenseTeamChainsPerCu = 5;
+int decide_dense_team(const SweepParams& p, const CallOpts& o, bool train) {
+  if (!o.dense_table || p.ctx2d || p.L < kDenseTeamMinL || p.L > kDenseTeamMaxL || p.pack >= 2 || o.team == 0 || o.split_waves > 0) return 0;
+  if (o.team == 2) return 1;
+  // (up to 64 labels the launch that takes any other kind of table is one of mp_fwd_team.hip)
+  const int per_cu = p.L <= kWave ? team_fwd_chains_per_cu(p.L, train) : kDenseTeamChainsPerCu;
+  return p.block_prefix[p.n_dirs] <= per_cu * (launch_policy().n_simd / 4) ? 1 : 0;
+}
+
 // wavefronts of a one-direction launch: one per chain, or one per group of p.pack chains
 template <typename Params>
 int launch_waves(const Params& p) {
@@ -798,6 +816,14 @@ void launch_fwd(const SweepParams& p, bool train, bool jacobi, hipStream_t st) {
   if (p.pack >= 2) {
     launch_packed_fwd(p, train, jacobi, p.pack, st);  // (u_fused is never set together with pack)
     return;
+  }
+  if (p.dense_team) {
+    switch (labels_per_lane(p.L)) {
+      case 1: launch_dense_fwd<1>(p, train, st); break;
+      case 2: launch_dense_fwd<2>(p, train, st); break;
+      default: launch_dense_fwd<3>(p, train, st); break;
+    }
+    if (!p.skip_dense) return;
   }
   if (p.team && p.ctx2d && p.L == 21) {
     launch_team21_fwd(p, train, st);
@@ -1125,7 +1151,9 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
       fill_dirs(s, d, 1, p.dirs, p.block_prefix, &p.n_dirs);
       p.pack = decide_pack(s, p, opts);
       p.split = choose_split(s, p, opts, train);
+      p.dense_team = decide_dense_team(p, opts, train);
       p.team = decide_team_fwd(p, opts, train);
+      p.skip_dense = (p.dense_team && s->n_disp <= kWave) ? 1 : 0;
       p.first_iter = (it == 0);
       p.pair_q = 1;
       p.belief = (uninit && it == 0 && d <= 1) ? unary : unary_update;

@@ -485,6 +485,8 @@ struct CtxDesc {
   int linear;       // c[k] == min(slope * k, c[L-1]) exactly for every k, slope >= 0 (truncated linear)
   float slope;
 };
+// neither a band nor truncated linear (1-D tables; a 2-D table's descriptor says so, too)
+__host__ __device__ inline bool is_dense(const CtxDesc& d) { return d.band_k == 0 && !d.linear; }
 
 // ------------------------------------------------------------------------------------------------
 // kernel parameter blocks
@@ -510,6 +512,9 @@ struct SweepParams {
   int split;                       // dense 1-D table, several labels per lane, few chains: wavefronts
                                    // per chain that share the front labels of a pixel (0, 1: one)
   int team;                        // Gauss-Seidel: four wavefronts per chain (mp_fwd_team.hip, mp_team21.hip)
+  int dense_team;                  // the same for a table declared dense (mp_fwd_dense.hip)
+  int skip_dense;                  // two kernels are launched, mp_fwd_dense.hip for a dense table, the other
+                                   // for any other kind
   int xcd_group;                   // consecutive chains on one die (0: each on another; locate_chain)
   int pair_q;                      // Gauss-Seidel: belief plane holds Q between the sweeps of a pair
   int skip_s_store;                // Gauss-Seidel: last sweep of the call, nobody reads S after it
@@ -594,6 +599,10 @@ inline void launch_team_fwd(const SweepParams& p, bool train, hipStream_t st) {
   else
     launch_team_fwd_t<R, false>(p, st);
 }
+// 1-D tables of 17 to 192 labels declared dense, TRWP (mp_fwd_dense.hip)
+constexpr int kDenseTeamMaxL = 192;
+template <int R>
+void launch_dense_fwd(const SweepParams& p, bool train, hipStream_t st);
 template <int R>
 void launch_sweep_bwd(const BackParams& p, bool jacobi, hipStream_t st);
 // 21 labels with a 2-D table, TRWP (mp_team21.hip)
@@ -649,7 +658,7 @@ void launch_swm_fwd(const float* msg, int n_trees, int L, float* out, uint8_t* m
 void launch_swm_bwd(const float* dout, const float* msg, const uint8_t* min_ind, int n_trees, int L,
                     float* dmsg, hipStream_t st);
 
-// LDS of the forward scan with several labels per lane: after the 1-D table c[0 .. L-1] (padded to
+// LDS of the forward scan with a 1-D table: after the 1-D table c[0 .. L-1] (padded to
 // whole groups of four) stands the table moved down by one entry, c1[i] = c[i + 1], which the dense
 // scan reads four entries at a time up to two trips past the last label
 __host__ __device__ inline int dense_c1_offset(int L) { return (L + 3) & ~3; }
@@ -667,7 +676,7 @@ __host__ __device__ inline int split_share(int L, int R, int waves) {
 __host__ __device__ inline int dense_sym_floats(int R) { return 2 * R * kWave; }
 
 inline size_t fwd_lds_bytes(int L, int ctx2d) {
-  if (ctx2d || L <= kWave) return sizeof(float) * (kMaxL + L * L);
+  if (ctx2d) return sizeof(float) * (kMaxL + L * L);
   const int R = (L + kWave - 1) / kWave;
   return sizeof(float) * (kMaxL + dense_c1_offset(L) + dense_c1_floats(L) + dense_sym_floats(R));
 }

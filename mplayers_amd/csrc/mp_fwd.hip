@@ -136,7 +136,7 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
   // (only where the dense scan is the kernel's step: a kernel compiled for a band or a
   // truncated-linear table meets it at pixels with a negative edge weight and takes
   // dense1d_step_lanes)
-  constexpr bool kDenseMain = R > 1 && (KT == -1 || KT == -3);
+  constexpr bool kDenseMain = KT == -1 || KT == -3;
   float cv0_chain[R];
   if constexpr (kDenseMain) {
 #pragma unroll
@@ -384,7 +384,7 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
         } else {
           nmin = norm_min();
         }
-      } else if (R == 1 && KT < 0 && desc.band_k == 0) {  // (the full table is in LDS then)
+      } else if (R == 1 && KT < 0 && p.ctx2d) {  // (the full table is in LDS then)
         if constexpr (LT > 0) {
           // 21 labels: the scan over front labels fully unrolled, context column in registers.
           // The edge weight stays in a vector register (every lane loaded the same one): a[fd]
@@ -417,7 +417,7 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
           nmin = norm_min();
         }
       } else if (live) {
-        if constexpr (R > 1) {  // (2-D tables exist for one label per lane only)
+        if constexpr (R > 1 || KT < 0) {  // (one label per lane: 1-D tables)
           if constexpr (kDenseMain) {
             dense1d_step<R, TRAIN>(a, w, lab0, a_w, c1_s, cv0_chain, v, fd_idx, fd_lo, fd_hi);
             if constexpr (SPLIT) split_combine<R, TRAIN>(xchg, n_waves, wave, lane, t & 1, v, fd_idx);
@@ -542,7 +542,7 @@ template <int R, bool VEC, bool MASK, bool TRAIN, int JACOBI>
 __global__ void __launch_bounds__(kWave) sweep_fwd_kernel(const SweepParams p) {
   extern __shared__ __align__(16) float smem[];
   float* a_s = smem;            // kMaxL floats
-  float* ctx_s = smem + kMaxL;  // L or L*L floats; several labels per lane: + the table moved down by one
+  float* ctx_s = smem + kMaxL;  // L*L floats, or L and the table moved down by one and around its centre
   const int lane = threadIdx.x;
   const int L = p.L;
   const ChainCtx ch = locate_chain(p);
@@ -560,7 +560,7 @@ __global__ void __launch_bounds__(kWave) sweep_fwd_kernel(const SweepParams p) {
     desc.slope = 0.f;
   }
   // context table into LDS (dense path, run-time band taps, negative-weight fallback)
-  if (R == 1 && desc.band_k == 0) {
+  if (R == 1 && p.ctx2d) {
     // full symmetric table for dense_step_r1: tab[fd * L + cd] = ctx(cd, fd), TRWP_forward.cu:101-113
     for (int i = lane; i < L * L; i += kWave) {
       const int fd = i / L, cd = i - fd * L;
@@ -570,7 +570,7 @@ __global__ void __launch_bounds__(kWave) sweep_fwd_kernel(const SweepParams p) {
   } else {
     const int n_ctx = p.ctx2d ? L * L : L;
     for (int i = lane; i < n_ctx; i += kWave) ctx_s[i] = p.ctx[i];
-    if (R > 1 && desc.band_k == 0) {  // (the dense scan is this kernel's step)
+    if (desc.band_k == 0) {  // (the dense scan is this kernel's step)
       float* c1_s = ctx_s + dense_c1_offset(L);
       for (int i = lane; i < dense_c1_floats(L); i += kWave) c1_s[i] = i + 1 < L ? p.ctx[i + 1] : 0.f;
       if (TRAIN) fill_dense_sym<R>(c1_s + dense_c1_floats(L), p.ctx, L, lane, kWave);
@@ -608,7 +608,7 @@ __global__ void __launch_bounds__(kWave) sweep_fwd_kernel(const SweepParams p) {
     }
     switch (desc.band_k) {
       case 0:
-        if (R == 1 && L == 21)
+        if (R == 1 && L == 21 && p.ctx2d)
           run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, (R == 1 ? -21 : -1)>(p, desc, c, a_s, ctx_s, skip_s);
         else
           run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, -1>(p, desc, c, a_s, ctx_s, skip_s);

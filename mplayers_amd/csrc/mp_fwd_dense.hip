@@ -1,0 +1,395 @@
+// Forward scan of TRWP for tables declared dense (learned ones: every pair of labels counts) with four
+// wavefronts per chain, in launches of few chains.  The recurrence and what each plane holds: mp_fwd.hip;
+// the results are the same bits.
+//
+// Such a launch is bound by the scan over all pairs of labels of one pixel, so the front labels are split
+// over the wavefronts: each holds the chain's state, takes the minimum over its quarter, and the four partial
+// minima meet in LDS (one barrier per pixel).  Next to sweep_fwd_split_kernel, which does the same,
+//   * the table entries a lane needs for its wavefront's front labels stay in registers for the whole chain
+//     (they differ between lanes, but not between pixels), so a front label costs a multiply-add and half a
+//     minimum per label, and of LDS only its belief, four to a broadcast read;
+//   * nothing but the recurrence runs once per pixel.  Loads, the update of the unary terms, argmin
+//     labels and stores wait for the end of a block of kBlock pixels, which the wavefronts then serve two
+//     pixels each; the loads are those of the block after next.
+// The argmin labels take two steps, as in dense1d_step: the scan notes the trip (eight front labels) whose
+// candidates last reached the running minimum; the service evaluates that one trip again.
+//
+// With one label per lane (17 to 64 labels), where the scans of mp_fwd_team.hip take a third to half of this one's
+// time for a band or a truncated linear table, the declaration alone does not decide: both kernels are
+// launched, and the one whose kind of table it is not ends at once (is_dense).
+//
+// Compiled once per R (labels per lane, 1 to 3) with -DMPL_INST_R=<R>.
+
+#include <type_traits>
+
+#include "mp_fwd_step.h"
+
+namespace mpl {
+namespace {
+
+constexpr int kWaves = 4;
+constexpr int kTeam = kWaves * kWave;
+constexpr int kPer = 2;                // pixels of a block that a wavefront serves
+constexpr int kBlock = kWaves * kPer;
+constexpr int kTrip = 8;               // front labels
+
+template <int R>
+struct alignas(16) Slots {
+  float in[kBlock][kWave][R == 1 ? 2 : 4];            // U, edge weight
+  float part[kBlock][kWaves][kWave][R == 1 ? 2 : 4];  // partial minima, the trips they were found in (a byte each)
+  float a[kBlock][kWave * R];                         // beliefs the pixel's message comes from (wavefront 0)
+  float copy[kWaves][kWave * R];                      // each wavefront's own copy of them
+};
+
+// workgroup barrier over LDS contents only: global loads in flight stay in flight
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// R words and one more, of a lane's slot
+template <int R>
+__device__ __forceinline__ void get_slot(const float* src, float (&x)[R], float& extra) {
+  if constexpr (R == 1) {
+    const f32x2 v = *reinterpret_cast<const f32x2*>(src);
+    x[0] = v[0];
+    extra = v[1];
+  } else {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll
+    for (int j = 0; j < R; ++j) x[j] = v[j];
+    extra = v[R];
+  }
+}
+template <int R>
+__device__ __forceinline__ void put_slot(float* dst, const float (&x)[R], float extra) {
+  if constexpr (R == 1)
+    *reinterpret_cast<f32x2*>(dst) = f32x2{x[0], extra};
+  else if constexpr (R == 2)
+    *reinterpret_cast<f32x4*>(dst) = f32x4{x[0], x[1], extra, 0.f};
+  else
+    *reinterpret_cast<f32x4*>(dst) = f32x4{x[0], x[1], x[2], extra};
+}
+
+// NT: trips per wavefront
+template <int R, bool TRAIN, int NT>
+__device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx& ch0, const bool msg_zero,
+                                           Slots<R>& s, const float* csym_s) {
+  constexpr int kShare = NT * kTrip;  // front labels per wavefront
+  const int L = p.L;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = uniform_i((int)threadIdx.x / kWave);
+  const int lab0 = R * lane;
+  const bool whole = L % R == 0;      // every lane's labels exist or none does
+  const int n = ch0.n;
+  const float rho = p.rho;
+  const int64_t HW = (int64_t)p.H * p.W;
+  const int64_t P = (int64_t)p.B * HW;
+  const int64_t N = P * L;
+  const int blocks = (n + kBlock - 1) / kBlock;
+  const int fd_lo = wave * kShare;
+
+  float floor_l[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) floor_l[j] = lab0 + j < L ? -INFINITY : INFINITY;
+  float tab[kShare][R];  // c[|label - front label|]
+#pragma unroll
+  for (int u = 0; u < kShare; ++u)
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int d = lab0 + j - (fd_lo + u);
+      tab[u][j] = csym_s[dense_sym_centre<R>() + (d < -R * kWave ? -R * kWave : d)];
+    }
+  auto norm_min = [&](const float (&v)[R]) __attribute__((always_inline)) {
+    float vm = INFINITY;
+#pragma unroll
+    for (int j = 0; j < R; ++j) vm = fminf(vm, fmaxf(v[j], floor_l[j]));
+    return wave_min_fast(vm);
+  };
+
+  // even_walk: a constant; the first (even direction) or the second sweep of a pair (run_chain_fwd)
+  auto walk = [&](const ChainCtx& ch, const bool skip_s_in, const auto even_walk) __attribute__((always_inline)) {
+    constexpr bool EVEN = decltype(even_walk)::value;
+    const int dir = ch.dir;
+    const int64_t img_p = (int64_t)ch.bv * HW;
+    const int64_t img_e = img_p * L;
+    const bool zfirst = p.zero_first && msg_zero;
+    const bool skip_s = skip_s_in || (EVEN && zfirst);
+    const bool md_zero = p.first_iter && msg_zero;
+    const bool mi_zero = md_zero && EVEN;
+    const int img_bytes = (int)(unsigned)(HW * L * 4);
+    const int img_bytes_p = (int)(HW * 4 > 0x7fffffff ? 0x7fffffff : HW * 4);
+    const rsrc_t rS = make_rsrc((zfirst ? p.belief_zero : p.belief) + img_e, img_bytes);
+    const rsrc_t rMd = make_rsrc(p.msg_in + (int64_t)dir * N + img_e, md_zero ? 0 : img_bytes);
+    const rsrc_t rMi = make_rsrc(p.msg_in + (int64_t)(dir ^ 1) * N + img_e, mi_zero ? 0 : img_bytes);
+    const rsrc_t rMo = make_rsrc(p.msg_out + (int64_t)dir * N + img_e, img_bytes);
+    const rsrc_t rSo = make_rsrc(p.belief_out + img_e, skip_s ? 0 : img_bytes);
+    const rsrc_t rImin = make_rsrc(TRAIN ? p.idx_min + (int64_t)dir * N + img_e : nullptr, TRAIN ? (int)(HW * L) : 0);
+    const rsrc_t dInorm = make_rsrc(TRAIN ? p.idx_norm + (int64_t)dir * P + img_p : nullptr, TRAIN ? (int)HW : 0);
+    const rsrc_t dW = make_rsrc(p.edge + (int64_t)dir * P + img_p, img_bytes_p);
+
+    auto pixel_at = [&](const int t) __attribute__((always_inline)) { return (unsigned)(ch.pix0 + t * ch.pstep); };
+    auto label_off = [&](bool on, unsigned so, int j) __attribute__((always_inline)) {
+      return (int)((on && lab0 + j < L) ? so + (unsigned)(lab0 + j) * 4u : kDeadWide);
+    };
+    // (one access per lane whatever the label count: of a lane with labels and places past the last one, the
+    // places read another pixel's or, past the plane, zero)
+    auto load_plane = [&](rsrc_t r, bool on, unsigned so, float (&x)[R]) __attribute__((always_inline)) {
+      buf_load<R, true, load_policy(false)>(r, label_off(on, so, 0), 0u, x);
+    };
+    auto store_plane = [&](rsrc_t r, bool on, unsigned so, const float (&x)[R]) __attribute__((always_inline)) {
+      if (R == 1 || whole) {
+        buf_store<R, true>(r, label_off(on, so, 0), 0u, x);
+      } else {
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x[j]), r, label_off(on, so, j), 0, MPL_ST_AUX);
+      }
+    };
+    struct Pix {
+      float s[R], md[R], mi[R], w;
+    };
+    // the loads of chain position t (nothing is read past the end of the chain)
+    auto load_pix = [&](const int t) __attribute__((always_inline)) {
+      Pix r;
+      const bool on = t < n;
+      const unsigned pp = pixel_at(t);
+      const unsigned so = pp * (unsigned)L * 4u;
+      load_plane(rS, on, so, r.s);
+      if (EVEN) load_plane(rMd, on, so, r.md);
+      load_plane(rMi, on, so, r.mi);
+      r.w = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(dW, on ? (int)(pp * 4u) : kDeadOffset, 0, 0));
+      return r;
+    };
+    float tt[kPer][R];  // of this wavefront's pixels of the block that is being scanned
+    auto prepare = [&](const Pix& px, const int t, const int i, float (&tk)[R]) __attribute__((always_inline)) {
+      float un[R], q[R];
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        tk[j] = EVEN ? px.s[j] - px.md[j] : px.s[j] + px.mi[j];
+        un[j] = fmaxf(fmaf(tk[j], rho, -px.mi[j]), floor_l[j]);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
+        q[j] = tk[j] - px.mi[j];
+      }
+      put_slot<R>(s.in[i][lane], un, px.w);
+      // Q of the pixel is known already, whatever its message
+      if (EVEN) store_plane(rSo, t < n, pixel_at(t) * (unsigned)L * 4u, q);
+    };
+    float md0[R];  // second sweep: the old message of the chain start (wavefront 0)
+    if (!EVEN) load_plane(rMd, wave == 0, pixel_at(0) * (unsigned)L * 4u, md0);
+
+    // what is left of a pixel of the block that has been scanned
+    auto finish = [&](const int t, const int i, const float (&tk)[R]) __attribute__((always_inline)) {
+      const bool on = t < n;
+      const unsigned pp = pixel_at(t);
+      const unsigned so = pp * (unsigned)L * 4u;
+      float v[R], m[R];
+      int trips = 0;
+#pragma unroll
+      for (int k = 0; k < kWaves; ++k) {
+        float pv[R], pt;
+        get_slot<R>(s.part[i][k][lane], pv, pt);
+        const int theirs = __builtin_bit_cast(int, pt);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          const bool take = k == 0 || pv[j] <= v[j];  // (the later share wins ties)
+          v[j] = take ? pv[j] : v[j];
+          const int byte = 0xff << (8 * j);
+          if (TRAIN) trips = take ? (trips & ~byte) | (theirs & byte) : trips;
+        }
+      }
+      const float nmin = norm_min(v);
+#pragma unroll
+      for (int j = 0; j < R; ++j) m[j] = t == 0 ? 0.f : v[j] - nmin;
+      if constexpr (TRAIN) {
+        float un[R], w;
+        get_slot<R>(s.in[i][lane], un, w);
+        int fd_idx[R];
+        bool pr[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          const int f0 = ((trips >> (8 * j)) & 0xff) * kTrip;
+          const int l = lab0 + j < L ? lab0 + j : L - 1;
+          const f32x4 a0 = *reinterpret_cast<const f32x4*>(&s.a[i][f0]);
+          const f32x4 a1 = *reinterpret_cast<const f32x4*>(&s.a[i][f0 + 4]);
+          const float* cp = csym_s + (dense_sym_centre<R>() + l - f0 - (kTrip - 1));  // entry of front label f0 + kTrip - 1
+          int arg = 0;
+#pragma unroll
+          for (int u = 0; u < kTrip; ++u) {
+            const float val = fmaf(w, cp[kTrip - 1 - u], u < 4 ? a0[u & 3] : a1[u & 3]);
+            arg = val == v[j] ? u : arg;
+          }
+          const int fd = f0 + arg;
+          fd_idx[j] = fd < L ? fd : L - 1;  // (only where no candidate is finite)
+          pr[j] = lab0 + j < L && v[j] == nmin;
+        }
+        const int nidx = last_label<R>(pr, L - 1);
+        const bool idx_on = on && t > 0;
+        const unsigned sob = pp * (unsigned)L;
+        if (R == 1 || whole) {
+          buf_store_u8<R, true>(rImin, (int)((idx_on && lab0 < L) ? sob + (unsigned)lab0 : kDeadWide), 0u, fd_idx);
+        } else {
+#pragma unroll
+          for (int j = 0; j < R; ++j)
+            __builtin_amdgcn_raw_buffer_store_b8((unsigned char)fd_idx[j], rImin,
+                                                 (int)((idx_on && lab0 + j < L) ? sob + (unsigned)(lab0 + j) : kDeadWide), 0, MPL_ST_AUX);
+        }
+        // every lane stores the same byte to the same address
+        __builtin_amdgcn_raw_buffer_store_b8((unsigned char)nidx, dInorm, idx_on ? (int)pp : kDeadOffset, 0, 0);
+      }
+      // (the reference never writes the chain start)
+      store_plane(rMo, on && (t > 0 || p.zero_start), so, m);
+      if constexpr (!EVEN) {
+        float sn[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) sn[j] = tk[j] + (t == 0 ? md0[j] : m[j]);
+        store_plane(rSo, on, so, sn);
+      }
+    };
+
+    float prev[R], uf[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) prev[j] = uf[j] = 0.f;
+    auto scan = [&](const int i, const float w, const bool start) __attribute__((always_inline)) {
+      // (the first wavefront's copy is the one the service reads)
+      float* const mine = wave == 0 ? s.a[i] : s.copy[wave];
+#pragma unroll
+      for (int j = 0; j < R; ++j) mine[lab0 + j] = fmaf(rho, prev[j], uf[j]);
+      lds_order();
+      float v[R];
+      int trip[R];
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        v[j] = INFINITY;
+        trip[j] = wave * NT;
+      }
+#pragma unroll
+      for (int k = 0; k < NT; ++k) {
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(&mine[fd_lo + k * kTrip]);
+        const f32x4 x1 = *reinterpret_cast<const f32x4*>(&mine[fd_lo + k * kTrip + 4]);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          float c[kTrip];
+#pragma unroll
+          for (int u = 0; u < kTrip; ++u) c[u] = fmaf(w, tab[k * kTrip + u][j], u < 4 ? x0[u & 3] : x1[u & 3]);
+          if constexpr (TRAIN) {
+            const float lm = fminf(fminf(fminf(fminf(fminf(c[0], c[1]), c[2]), fminf(fminf(c[3], c[4]), c[5])), c[6]), c[7]);
+            if (k > 0) {
+              const bool take = lm <= v[j];
+              v[j] = fminf(v[j], lm);
+              trip[j] = take ? wave * NT + k : trip[j];
+            } else {
+              v[j] = lm;
+            }
+          } else {
+#pragma unroll
+            for (int u = 0; u < kTrip; u += 2) v[j] = fminf(fminf(v[j], c[u]), c[u + 1]);
+          }
+        }
+      }
+      int trips = 0;
+      if (TRAIN) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) trips |= trip[j] << (8 * j);
+      }
+      put_slot<R>(s.part[i][wave][lane], v, __builtin_bit_cast(float, trips));
+      lds_barrier();
+#pragma unroll
+      for (int k = 1; k < kWaves; ++k) {
+        float pv[R], unused;
+        get_slot<R>(s.part[i][(wave + k) & 3][lane], pv, unused);
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[j] = fminf(v[j], pv[j]);
+      }
+      const float nmin = norm_min(v);
+#pragma unroll
+      for (int j = 0; j < R; ++j) prev[j] = start ? 0.f : v[j] - nmin;  // (the chain start has no front pixel)
+    };
+
+    Pix px[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) px[u] = load_pix(kPer * wave + u);
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      prepare(px[u], kPer * wave + u, kPer * wave + u, tt[u]);
+      px[u] = load_pix(kBlock + kPer * wave + u);
+    }
+    lds_barrier();
+#pragma clang loop unroll(disable)
+    for (int b = 0; b < blocks; ++b) {
+#pragma clang loop unroll(disable)
+      for (int i = 0; i < kBlock; ++i) {
+        float un[R], w;
+        get_slot<R>(s.in[i][lane], un, w);
+        scan(i, w, b == 0 && i == 0);
+#pragma unroll
+        for (int j = 0; j < R; ++j) uf[j] = un[j];
+      }
+      lds_barrier();
+#pragma unroll
+      for (int u = 0; u < kPer; ++u) {
+        const int i = kPer * wave + u;
+        finish(b * kBlock + i, i, tt[u]);
+        lds_order();
+        prepare(px[u], (b + 1) * kBlock + i, i, tt[u]);
+        px[u] = load_pix((b + 2) * kBlock + i);
+      }
+      lds_barrier();
+    }
+  };
+
+  if (!(ch0.dir & 1)) walk(ch0, p.skip_s_store != 0, std::true_type());
+  if ((ch0.dir & 1) || p.fused_pair) {
+    ChainCtx ch = ch0;
+    bool skip_s = p.skip_s_store != 0;
+    if (!(ch0.dir & 1)) {
+      // the second sweep of a pair reads what the first one stored: on the same compute unit, once the
+      // stores are complete
+      ch.dir = ch0.dir ^ 1;
+      ch.pix0 = ch0.pix0 + (n - 1) * ch0.pstep;
+      ch.pstep = -ch0.pstep;
+      skip_s = p.skip_s_store2 != 0;
+      wait_vmem<0>();
+      __syncthreads();
+    }
+    walk(ch, skip_s, std::false_type());
+  }
+}
+
+template <int R, bool TRAIN, int NT>
+__global__ void __launch_bounds__(kTeam) sweep_fwd_dense_kernel(const SweepParams p) {
+  if (R == 1 && p.skip_dense && p.desc != nullptr && !is_dense(*p.desc)) return;
+  extern __shared__ __align__(16) char smem_raw[];
+  Slots<R>* s = reinterpret_cast<Slots<R>*>(smem_raw);
+  float* csym_s = reinterpret_cast<float*>(s + 1);
+  fill_dense_sym<R>(csym_s, p.ctx, p.L, (int)threadIdx.x, kTeam);
+  __syncthreads();
+  const bool msg_zero = p.desc != nullptr && p.desc->msg_nonzero == 0;
+  walk_chain<R, TRAIN, NT>(p, locate_chain(p), msg_zero, *s, csym_s);
+}
+
+}  // namespace
+
+template <int R>
+void launch_dense_fwd(const SweepParams& p, bool train, hipStream_t st) {
+  const int blocks = p.block_prefix[p.n_dirs];
+  if (blocks <= 0) return;
+  const size_t lds = sizeof(Slots<R>) + sizeof(float) * dense_sym_floats(R);
+  constexpr int kFull = 2 * R;  // trips of a wavefront that cover R labels per lane
+  // (one trip fewer covers label counts up to 32 less)
+  if (p.L <= kWaves * kTrip * (kFull - 1)) {
+    if (train)
+      sweep_fwd_dense_kernel<R, true, kFull - 1><<<blocks, kTeam, lds, st>>>(p);
+    else
+      sweep_fwd_dense_kernel<R, false, kFull - 1><<<blocks, kTeam, lds, st>>>(p);
+  } else {
+    if (train)
+      sweep_fwd_dense_kernel<R, true, kFull><<<blocks, kTeam, lds, st>>>(p);
+    else
+      sweep_fwd_dense_kernel<R, false, kFull><<<blocks, kTeam, lds, st>>>(p);
+  }
+}
+
+template void launch_dense_fwd<MPL_INST_R>(const SweepParams&, bool, hipStream_t);
+
+}  // namespace mpl

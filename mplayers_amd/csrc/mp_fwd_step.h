@@ -53,7 +53,7 @@ __device__ __forceinline__ void dense_step(const float (&a)[R], const bool (&val
   lds_order();
 }
 
-// Dense O(L^2) step for 1-D contexts and several labels per lane.  The front labels are visited
+// Dense O(L^2) step for 1-D contexts.  The front labels are visited
 // in ascending order; the context values c[|cd - fd|] of the lane's labels are kept in registers and
 // moved one label up per front label (c[|cd - (fd+1)|] of label cd is c[|(cd-1) - fd|] of label
 // cd - 1; c[fd+1] enters at label 0) with one lane shift.  Both a[fd] and the entering c[fd+1] are
@@ -73,8 +73,10 @@ __device__ __forceinline__ void dense_step(const float (&a)[R], const bool (&val
 // The scan covers the front labels fd_lo .. fd_hi - 1 (fd_lo a multiple of T): all of them, or the
 // share of one wavefront where several scan a pixel together (split_combine below).  cv0: the
 // sliding values at fd_lo, c[|cd - fd_lo|].
+// (one label per lane: two groups of four to a trip, since a group's register is still a sliding value
+// when the next trip would read the same one)
 template <int R>
-constexpr int dense_trip() { return 4 * R; }
+constexpr int dense_trip() { return R == 1 ? 8 : 4 * R; }
 
 template <int R, bool TRAIN>
 __device__ __forceinline__ void dense1d_step(const float (&a)[R], const float w, const int lab0,
@@ -119,7 +121,7 @@ __device__ __forceinline__ void dense1d_step(const float (&a)[R], const float w,
   constexpr int kNext = (T - 3 - R + 3) / 4;  // groups q with 4 q + 3 + R < T
   int fd0 = fd_lo;
 #pragma unroll
-  for (int q = 0; q < R; ++q) read4(a_w + fd0, ba, q);
+  for (int q = 0; q < T / 4; ++q) read4(a_w + fd0, ba, q);
 #pragma unroll
   for (int q = 0; q < kNext; ++q) read4(c1_s + fd0, bc, q);
   for (; fd0 + T <= fd_hi; fd0 += T) {
@@ -155,7 +157,7 @@ __device__ __forceinline__ void dense1d_step(const float (&a)[R], const float w,
   // what is left of the share: fewer than T front labels, one at a time
   if (fd0 < fd_hi) {
 #pragma unroll
-    for (int q = kNext; q < R; ++q) read4(c1_s + fd0, bc, q);
+    for (int q = kNext; q < T / 4; ++q) read4(c1_s + fd0, bc, q);
     float lm[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) lm[j] = INFINITY;
@@ -290,7 +292,7 @@ __device__ __forceinline__ void dense1d_step_lanes(const float (&a)[R], float w,
   }
 }
 
-// Dense step for L <= 64 (one label per lane): a[fd] is broadcast with v_readlane and the context
+// Dense step for 2-D contexts (one label per lane): a[fd] is broadcast with v_readlane and the context
 // comes from a full table tab[fd * L + cd] in LDS, which consecutive lanes read without bank
 // conflicts.  Same scan order as dense_step.
 template <bool TRAIN>

@@ -112,12 +112,12 @@ __device__ __forceinline__ void lds_barrier() {
 template <int R, int KT>
 struct StepCtx {
   int L, lab0, lane, K;
-  bool full_table;            // ctx_s holds the (L, L) table (one label per lane, dense)
+  bool full_table;            // ctx_s holds the (L, L) table (2-D)
   float cmax, slope;
   float floor_l[R];           // -inf, +inf where the lane's label does not exist
   float c_reg[KT > 0 ? KT : 1];
   float tcol[KT == -21 ? 21 : 1];
-  float cv0[R];               // dense 1-D table, several labels per lane: c[label]
+  float cv0[R];               // dense 1-D table: c[label]
   float* a_w;                 // this wavefront's scratch, kMaxL floats
   const float* ctx_s;
   const float* c1_s;
@@ -131,7 +131,7 @@ struct StepCtx {
 template <int R, int KT, bool C0, bool TRAIN, bool PLAIN>
 __device__ __forceinline__ void team_step(const StepCtx<R, KT>& c, const float (&a)[R], const float wv,
                                           float (&v)[R], int (&fd_idx)[R], float& nmin) {
-  constexpr bool kDenseMain = R > 1 && KT == -1;
+  constexpr bool kDenseMain = KT == -1;
   auto norm_min = [&]() __attribute__((always_inline)) {
     float vm = INFINITY;
 #pragma unroll
@@ -207,7 +207,7 @@ __device__ __forceinline__ void team_step(const StepCtx<R, KT>& c, const float (
     if constexpr (kDenseMain) {
       dense1d_step<R, TRAIN>(a, w, c.lab0, c.a_w, c.c1_s, c.cv0, v, fd_idx, 0, L);
       if (TRAIN) dense1d_argmin<R>(v, fd_idx, w, c.lab0, L, c.a_w, c.csym_s, fd_idx);
-    } else if constexpr (R > 1) {
+    } else if constexpr (R > 1 || KT == -2) {
       dense1d_step_lanes<R, TRAIN, false>(a, w, L, c.lab0, c.ctx_s, v, fd_idx, 0, L);
     } else {
       bool valid[R];
@@ -245,7 +245,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
   c.lab0 = lab0;
   c.lane = lane;
   c.K = desc.band_k;
-  c.full_table = desc.band_k == 0;
+  c.full_table = R == 1 && p.ctx2d;
   c.cmax = desc.cmax;
   asm volatile("" : "+v"(c.cmax));
   c.slope = desc.slope;
@@ -264,7 +264,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
 #pragma unroll
     for (int fd = 0; fd < 21; ++fd) c.tcol[fd] = ctx_s[fd * 21 + (lane < 21 ? lane : 20)];
   }
-  if constexpr (R > 1 && KT == -1) {
+  if constexpr (KT == -1) {
 #pragma unroll
     for (int j = 0; j < R; ++j) c.cv0[j] = ctx_s[lab0 + j < L ? lab0 + j : L - 1];
   }
@@ -530,7 +530,7 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
   float* ctx_s = a_s + (kHelpers + 1) * kMaxL;            // as in sweep_fwd_kernel
   const int L = p.L;
   Flags* flags = reinterpret_cast<Flags*>(
-      ctx_s + (p.ctx2d || R == 1 ? L * L : dense_c1_offset(L) + dense_c1_floats(L) + dense_sym_floats(R)));
+      ctx_s + (p.ctx2d ? L * L : dense_c1_offset(L) + dense_c1_floats(L) + dense_sym_floats(R)));
   const int tid = threadIdx.x;
   // The last wavefront is the main one in every workgroup: the wavefronts of the workgroups that a compute
   // unit gets one after another start one SIMD further each (read from the hardware-id registers for 2, 3
@@ -549,7 +549,8 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
     desc.linear = 0;
     desc.slope = 0.f;
   }
-  if (R == 1 && desc.band_k == 0) {
+  if (p.skip_dense && is_dense(desc)) return;  // (mp_fwd_dense.hip runs such a launch)
+  if (R == 1 && p.ctx2d) {
     for (int i = tid; i < L * L; i += kTeam) {
       const int fd = i / L, cd = i - fd * L;
       const int lo = cd < fd ? cd : fd, hi = cd < fd ? fd : cd;
@@ -558,7 +559,7 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
   } else {
     const int n_ctx = p.ctx2d ? L * L : L;
     for (int i = tid; i < n_ctx; i += kTeam) ctx_s[i] = p.ctx[i];
-    if (R > 1 && desc.band_k == 0) {
+    if (desc.band_k == 0) {
       float* c1_s = ctx_s + dense_c1_offset(L);
       for (int i = tid; i < dense_c1_floats(L); i += kTeam) c1_s[i] = i + 1 < L ? p.ctx[i + 1] : 0.f;
       if (TRAIN) fill_dense_sym<R>(c1_s + dense_c1_floats(L), p.ctx, L, tid, kTeam);
@@ -579,10 +580,11 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
   }
   switch (desc.band_k) {
     case 0:
-      if (R == 1 && L == 21)
+      if (R == 1 && L == 21 && p.ctx2d) {
         MPL_WALK((R == 1 ? -21 : -1), false);
-      else
+      } else {
         MPL_WALK(-1, false);
+      }
       break;
     case 1: MPL_WALK(1, true); break;
     case 2: MPL_WALK(2, true); break;
@@ -605,8 +607,8 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
 #undef MPL_WALK
 }
 
-inline size_t team_lds_bytes(int L, int R, size_t slot) {
-  const size_t table = R == 1 ? (size_t)L * L : dense_c1_offset(L) + dense_c1_floats(L) + dense_sym_floats(R);
+inline size_t team_lds_bytes(int L, int R, bool ctx2d, size_t slot) {
+  const size_t table = ctx2d ? (size_t)L * L : dense_c1_offset(L) + dense_c1_floats(L) + dense_sym_floats(R);
   return 2 * kT * slot + sizeof(float) * ((kHelpers + 1) * kMaxL + table) + 2 * sizeof(Flags);
 }
 
@@ -616,7 +618,7 @@ template <int R, bool TRAIN>
 void launch_team_fwd_t(const SweepParams& p, hipStream_t st) {
   const int blocks = p.block_prefix[p.n_dirs];
   if (blocks <= 0) return;
-  const size_t lds = team_lds_bytes(p.L, R, sizeof(Slot<R>));
+  const size_t lds = team_lds_bytes(p.L, R, p.ctx2d != 0, sizeof(Slot<R>));
   if (p.L % R == 0)
     sweep_fwd_team_kernel<R, true, TRAIN><<<blocks, kTeam, lds, st>>>(p);
   else if constexpr (R > 1)

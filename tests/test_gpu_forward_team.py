@@ -89,3 +89,23 @@ def test_chain_lengths_and_launches(gpu, L, table, training):
       finally:
         _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
     _same(got[1], got[0], training)
+
+
+@pytest.mark.parametrize("L", [2, 17, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 191, 192])
+@pytest.mark.parametrize("training", [True, False])
+def test_tables_declared_dense(gpu, L, training):
+  """Four wavefronts that share the front labels: label counts at the edges of a wavefront's trips, of a lane's
+  labels and of the front labels per wavefront; chains around a block of eight pixels."""
+  from mplayers_amd import _lib
+  flags = _lib.F_PACKED_OFF | _lib.F_DENSE_TABLE
+  for H, W, table, negative in ((3, 1, "random", False), (8, 9, "random", True), (7, 16, "random", False),
+                                (17, 25, "linear", False), (2, 40, "potts", True)):
+    problem = _problem(4, 1, H, W, L, table, 5, negative)
+    for more, kw in ((0, {}), (_lib.F_FUSED_PAIRS_OFF, {}), (0, dict(msg_uninit=True))):
+      print("case", L, training, H, W, table, negative, more, kw, flush=True)
+      one = _run(gpu, 0, *problem, 4, 3, training, _lib.F_PACKED_OFF | more, **kw)
+      four = _run(gpu, 2, *problem, 4, 3, training, flags | more, **kw)
+      if table == "linear":  # the label scan and the dense scan differ in the last bits of a tie
+        assert np.abs(four["cost_final"] - one["cost_final"]).max() <= 1e-5 * max(1.0, np.abs(one["cost_final"]).max())
+      else:
+        _same(four, one, training)
