@@ -59,6 +59,7 @@ template <int R, bool VEC, bool MASK, bool JACOBI, bool DIRECT, int GRAD>
 __global__ void __launch_bounds__(kWave) sweep_bwd_kernel(const BackParams p) {
   constexpr bool DE = (GRAD & 1) != 0, DC = (GRAD & 2) != 0;
   constexpr int kLd = load_policy(!MASK);  // (every lane full: whole cache lines)
+  constexpr int kSt = store_policy(R, !MASK);
   extern __shared__ float smem[];
   const int L = p.L;
   // 2-D context tables exist for at most 64 labels, i.e. only with one label per lane
@@ -405,9 +406,9 @@ __global__ void __launch_bounds__(kWave) sweep_bwd_kernel(const BackParams p) {
       const int vo = (int)((lane_ok && t >= 0) ? so + (unsigned)foff : kDeadWide);
       if constexpr (!EVEN) {
         if constexpr (VEC)
-          buf_store<R, true>(rAo, vo, 0u, sc);
+          buf_store<R, true, kSt>(rAo, vo, 0u, sc);
         else
-          buf_store<R, VEC>(make_rsrc(bAo, nrec), foff, so, sc);
+          buf_store<R, VEC, kSt>(make_rsrc(bAo, nrec), foff, so, sc);
       } else {
         float an[R], hin[R];
 #pragma unroll
@@ -416,11 +417,11 @@ __global__ void __launch_bounds__(kWave) sweep_bwd_kernel(const BackParams p) {
           hin[j] = -ap[j] - sc[j];  // g_o was 0 after its own walk (h_o = -A'), then g_o -= dU
         }
         if constexpr (VEC) {
-          buf_store<R, true>(rAo, vo, 0u, an);
-          buf_store<R, true>(rHiOut, vo, 0u, hin);
+          buf_store<R, true, kSt>(rAo, vo, 0u, an);
+          buf_store<R, true, kSt>(rHiOut, vo, 0u, hin);
         } else {
-          buf_store<R, VEC>(make_rsrc(bAo, nrec), foff, so, an);
-          buf_store<R, VEC>(make_rsrc(bHi, p.skip_h_store ? 0 : nrec), foff, so, hin);
+          buf_store<R, VEC, kSt>(make_rsrc(bAo, nrec), foff, so, an);
+          buf_store<R, VEC, kSt>(make_rsrc(bHi, p.skip_h_store ? 0 : nrec), foff, so, hin);
         }
       }
       // each pixel receives over exactly one edge per direction: plain read-modify-write

@@ -281,6 +281,9 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* p, int bytes) {
 // 400x600 1.80 / 1.53; whole lines with one wavefront per chain, 96 labels 384x1248 3.65 / 3.68.  (Stores
 // without the hint as well: 2.53, 8.29, 1.61, 3.78.)
 constexpr int load_policy(bool whole_lanes) { return whole_lanes ? MPL_LD_AUX : 0; }
+// Stores go without it where a vector is no longer than two lines (up to 63 labels: most lines are shared):
+// ISGMR 52 labels 400x600 0.66 / 0.60 with / without, TRWP 60 labels 375x450 the same.
+constexpr int store_policy(int R, bool whole_lanes) { return whole_lanes || R > 1 ? MPL_ST_AUX : 0; }
 
 constexpr int kDeadOffset = 0x7ffffff0;  // a vector offset no descriptor covers: access suppressed
 // the same for descriptors that cover a whole image (up to kMaxImageBytes, beyond 2 GiB)
@@ -314,21 +317,21 @@ __device__ __forceinline__ void buf_load(rsrc_t r, int off, unsigned so, float (
   }
 }
 
-template <int R, bool VEC>
+template <int R, bool VEC, int AUX = MPL_ST_AUX>
 __device__ __forceinline__ void buf_store(rsrc_t r, int off, unsigned so, const float (&x)[R]) {
   if constexpr (VEC && R == 2) {
     f32x2 t = {x[0], x[1]};
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, t), r, (int)((unsigned)off + so), 0, MPL_ST_AUX);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, t), r, (int)((unsigned)off + so), 0, AUX);
   } else if constexpr (VEC && R == 3) {
     f32x3 t = {x[0], x[1], x[2]};
-    __builtin_amdgcn_raw_buffer_store_b96(__builtin_bit_cast(u32x3, t), r, (int)((unsigned)off + so), 0, MPL_ST_AUX);
+    __builtin_amdgcn_raw_buffer_store_b96(__builtin_bit_cast(u32x3, t), r, (int)((unsigned)off + so), 0, AUX);
   } else if constexpr (VEC && R == 4) {
     f32x4 t = {x[0], x[1], x[2], x[3]};
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, t), r, (int)((unsigned)off + so), 0, MPL_ST_AUX);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, t), r, (int)((unsigned)off + so), 0, AUX);
   } else {
 #pragma unroll
     for (int j = 0; j < R; ++j)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x[j]), r, (int)((unsigned)(off + 4 * j) + so), 0, MPL_ST_AUX);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x[j]), r, (int)((unsigned)(off + 4 * j) + so), 0, AUX);
   }
 }
 
@@ -351,18 +354,18 @@ __device__ __forceinline__ void buf_load_u8(rsrc_t r, int off, unsigned so, int 
   }
 }
 
-template <int R, bool VEC>
+template <int R, bool VEC, int AUX = MPL_ST_AUX>
 __device__ __forceinline__ void buf_store_u8(rsrc_t r, int off, unsigned so, const int (&x)[R]) {
   if constexpr (VEC && R == 4) {
     unsigned t = (unsigned)x[0] | ((unsigned)x[1] << 8) | ((unsigned)x[2] << 16) | ((unsigned)x[3] << 24);
-    __builtin_amdgcn_raw_buffer_store_b32(t, r, (int)((unsigned)off + so), 0, MPL_ST_AUX);
+    __builtin_amdgcn_raw_buffer_store_b32(t, r, (int)((unsigned)off + so), 0, AUX);
   } else if constexpr (VEC && R == 2) {
     unsigned short t = (unsigned short)((unsigned)x[0] | ((unsigned)x[1] << 8));
-    __builtin_amdgcn_raw_buffer_store_b16(t, r, (int)((unsigned)off + so), 0, MPL_ST_AUX);
+    __builtin_amdgcn_raw_buffer_store_b16(t, r, (int)((unsigned)off + so), 0, AUX);
   } else {
 #pragma unroll
     for (int j = 0; j < R; ++j)
-      __builtin_amdgcn_raw_buffer_store_b8((unsigned char)x[j], r, (int)((unsigned)(off + j) + so), 0, MPL_ST_AUX);
+      __builtin_amdgcn_raw_buffer_store_b8((unsigned char)x[j], r, (int)((unsigned)(off + j) + so), 0, AUX);
   }
 }
 
@@ -444,18 +447,20 @@ constexpr int kXcds = 8;
 constexpr int kLineBytes = 128;
 inline int xcd_group_size(int L) { return (L * 4) % kLineBytes != 0 ? 16 : 0; }
 
+// workgroup `block` of `blocks` in that order (whole rounds of eight groups; the rest stays as it is)
+__device__ __forceinline__ int xcd_block(int block, int blocks, int group) {
+  if (group <= 0) return block;
+  const int per = kXcds * group;
+  const int base = block / per * per;
+  if (base + per > blocks) return block;
+  const int r = block - base;
+  return base + (r % kXcds) * group + r / kXcds;
+}
+
 // which (direction, batch item, chain) a workgroup owns
 template <typename Params>
 __device__ __forceinline__ ChainCtx locate_chain(const Params& p) {
-  int block = (int)blockIdx.x;
-  if (p.xcd_group > 0) {  // (whole rounds of eight groups; the workgroups after the last one stay as they are)
-    const int per = kXcds * p.xcd_group;
-    const int base = block / per * per;
-    if (base + per <= (int)gridDim.x) {
-      const int r = block - base;
-      block = base + (r % kXcds) * p.xcd_group + r / kXcds;
-    }
-  }
+  const int block = xcd_block((int)blockIdx.x, (int)gridDim.x, p.xcd_group);
   int di = 0;
   while (di + 1 < p.n_dirs && block >= p.block_prefix[di + 1]) ++di;
   const int dir = p.dirs[di];

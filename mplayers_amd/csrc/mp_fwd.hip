@@ -77,6 +77,7 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
   constexpr bool SPLIT = (KT == -3);
   // (every lane full: 64, 128, 192 or 256 labels, whole cache lines)
   constexpr int kLd = load_policy(!MASK);
+  constexpr int kSt = store_policy(R, !MASK);
   const int L = p.L;
   // The caller's initial messages turned out to be all zero (the usual case: the reference's
   // callers pass a cleared tensor) and this is a sweep that can profit: S = Q = U = unary, so the
@@ -279,18 +280,18 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
     const int nrec0 = store_ok ? (int)(so0 + (unsigned)vbytes) : 0;
     if (!JACOBI && p.pair_q && !skip_s_store) {
       if constexpr (VEC)
-        buf_store<R, true>(rSo, vo0, 0u, conv);
+        buf_store<R, true, kSt>(rSo, vo0, 0u, conv);
       else
-        buf_store<R, VEC>(make_rsrc(bSo, nrec0), foff, so0, conv);
+        buf_store<R, VEC, kSt>(make_rsrc(bSo, nrec0), foff, so0, conv);
     }
     if (JACOBI || p.zero_start) {
       float z[R];
 #pragma unroll
       for (int j = 0; j < R; ++j) z[j] = 0.f;
       if constexpr (VEC)
-        buf_store<R, true>(rMo, vo0, 0u, z);
+        buf_store<R, true, kSt>(rMo, vo0, 0u, z);
       else
-        buf_store<R, VEC>(make_rsrc(bMo, nrec0), foff, so0, z);
+        buf_store<R, VEC, kSt>(make_rsrc(bMo, nrec0), foff, so0, z);
     }
   }
 
@@ -456,15 +457,15 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
         const bool on = lane_ok && live && store_ok;  // nothing is stored past the end
         const int vo = (int)(kAddDead ? ((live && store_ok) ? so + foff_ok : kDeadWide)
                                       : (on ? so + (unsigned)foff : kDeadWide));
-        buf_store<R, true>(rMo, vo, 0u, m);
-        if (!JACOBI) buf_store<R, true>(rSo, vo, 0u, sn);
-        if (TRAIN) buf_store_u8<R, true>(rImin, (int)(on ? sob + (unsigned)lab0 : kDeadWide), 0u, fd_idx);
+        buf_store<R, true, kSt>(rMo, vo, 0u, m);
+        if (!JACOBI) buf_store<R, true, kSt>(rSo, vo, 0u, sn);
+        if (TRAIN) buf_store_u8<R, true, kSt>(rImin, (int)(on ? sob + (unsigned)lab0 : kDeadWide), 0u, fd_idx);
       } else {
         const int nrec = (live && store_ok) ? (int)(so + (unsigned)vbytes) : 0;
-        buf_store<R, VEC>(make_rsrc(bMo, nrec), foff, so, m);
-        if (!JACOBI) buf_store<R, VEC>(make_rsrc(bSo, skip_s_store ? 0 : nrec), foff, so, sn);
+        buf_store<R, VEC, kSt>(make_rsrc(bMo, nrec), foff, so, m);
+        if (!JACOBI) buf_store<R, VEC, kSt>(make_rsrc(bSo, skip_s_store ? 0 : nrec), foff, so, sn);
         if (TRAIN)
-          buf_store_u8<R, VEC>(make_rsrc(bImin, (live && store_ok) ? (int)(sob + (unsigned)L) : 0), lab0, sob, fd_idx);
+          buf_store_u8<R, VEC, kSt>(make_rsrc(bImin, (live && store_ok) ? (int)(sob + (unsigned)L) : 0), lab0, sob, fd_idx);
       }
       if (TRAIN) {
         bool pr[R];
