@@ -10,6 +10,7 @@ Tensor layouts (as in the reference):
   MPModule.forward(unary (B, cv, L, H, W), edge_weights (B, n_dir, H, W) or None)
                  -> (cost_final (B, cv, L, H, W), label_context[None], label_all, None, None)
 """
+import numpy as np
 import torch
 import torch.nn as nn
 
@@ -209,6 +210,33 @@ class MPModule(torch.nn.Module):
         create_label_context(self.args, enable_seg=self.args.enable_seg,
                              enable_symmetric=self.args.enable_symmetric)
 
+  def _location_masks(self, label_context):
+    """Masks of label_context_loc and label_context_diag_loc on the table's device, None where a location is
+    a tensor or not a list of entries.  They are formed on the host from the locations of the moment and copied only when they
+    differ from what was copied last."""
+    diag = self.label_context_diag_loc
+    places = [self.label_context_loc, tuple(diag) if isinstance(diag, list) else diag]
+    parts = [part for place in places for part in (place if isinstance(place, tuple) else (place,))]
+    if any(isinstance(part, torch.Tensor) for part in parts):
+      return None
+    host = []
+    for place in places:
+      mask = np.zeros(label_context.shape, bool)
+      as_array = lambda x: np.asarray(x) if isinstance(x, (list, range)) else x
+      index = tuple(map(as_array, place)) if isinstance(place, tuple) else as_array(place)
+      if not host and np.ndim(mask[index]) != 1:
+        return None  # (what takes the values back entry by entry is one-dimensional)
+      mask[index] = True
+      host.append(mask)
+    key = (label_context.device, label_context.shape) + tuple(mask.tobytes() for mask in host)
+    kept = getattr(self, "_kept_masks", None)
+    if kept is None or kept[0] != key:
+      # (copies from pageable memory are complete when they return, for every stream)
+      kept = (key,) + tuple(torch.from_numpy(mask).to(label_context.device) for mask in host)
+      if not (label_context.is_cuda and torch.cuda.is_current_stream_capturing()):
+        self._kept_masks = kept
+    return kept[1:]
+
   def _effective_label_context(self, weight_first=False):
     """Re-parameterisation of the learned context (MP_module.py:207-220).  weight_first: the term
     weight scales the stored parameter before the re-parameterisation instead of the sigmoid's
@@ -216,9 +244,17 @@ class MPModule(torch.nn.Module):
     term_weight = self.args.mpnet_term_weight
     label_context = self.label_context * (term_weight if weight_first else 1)
     mode = self.args.mpnet_smoothness_train
+    scale = 2 if weight_first else 2 * term_weight
+    masks = self._location_masks(label_context) if mode == 'sigmoid' else None
+    if masks is not None:
+      # entry by entry: indexing with the stored locations copies them to the device in every call, waits for
+      # each copy, and sorts them for the gradient
+      learned, pinned = masks
+      valid = label_context.masked_fill(~learned, 0)
+      label_context = torch.where(learned, scale * torch.sigmoid(valid), label_context)
+      return label_context.masked_fill(pinned, self.args.mpnet_diag_value)
     if mode == 'sigmoid':
       valid = label_context[self.label_context_loc].flatten()
-      scale = 2 if weight_first else 2 * term_weight
       label_context[self.label_context_loc] = scale * torch.sigmoid(valid)
     elif mode == 'softmax':
       valid = label_context[self.label_context_loc].flatten()

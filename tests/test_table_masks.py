@@ -1,0 +1,63 @@
+"""The sigmoid re-parameterisation of a learned table under masks: the values and gradients that indexing
+with the stored locations gives (MP_module.py:207-220), for every form the locations take, and after they or
+the table change."""
+import argparse
+
+import numpy as np
+import pytest
+import torch
+
+from mplayers_amd import MPModule
+
+
+def _by_index(table, loc, diag, weight, weight_first, diag_value):
+  label_context = table * (weight if weight_first else 1)
+  label_context[loc] = (2 if weight_first else 2 * weight) * torch.sigmoid(label_context[loc].flatten())
+  label_context[tuple(diag) if isinstance(diag, list) else diag] = diag_value
+  return label_context
+
+
+LOCATIONS = {
+    "triangle": (np.triu_indices(5, k=1), [range(5), range(5)], 2),
+    "tensor": (tuple(torch.from_numpy(i) for i in np.triu_indices(5, k=1)), [range(5), range(5)], 2),
+    "vector": (range(1, 5), range(1), 1),
+    "list": ([1, 3], [0], 1),
+    "slice": (slice(2, None), 0, 1),
+    "negative": (np.array([-1, -2]), range(2), 1),
+    "overlap": (range(0, 5), range(2), 1),
+}
+
+
+@pytest.mark.parametrize("name", sorted(LOCATIONS))
+@pytest.mark.parametrize("weight_first", [False, True])
+def test_masks_give_what_indexing_gives(name, weight_first):
+  loc, diag, dims = LOCATIONS[name]
+  args = argparse.Namespace(mpnet_mrf_mode="TRWP", mpnet_max_iter=1, mpnet_n_dirs=4, n_classes=5,
+                            mpnet_term_weight=1.5, mpnet_smoothness_train="sigmoid", mpnet_diag_value=0.25)
+  module = MPModule(args)
+  gen = torch.Generator().manual_seed(1)
+  for round_ in range(3):  # other values, then other locations
+    table = torch.nn.Parameter(torch.randn((5,) * dims, generator=gen))
+    with torch.no_grad():
+      table[(0,) * dims] = float("inf")  # (pinned or not touched in most of the cases)
+    if round_ == 2 and name == "vector":
+      loc = range(2, 4)
+    module.set_label_context(table, loc, diag)
+    upstream = torch.randn(table.shape, generator=gen)
+    got = module._effective_label_context(weight_first=weight_first)
+    (got_grad,) = torch.autograd.grad(got, table, upstream)
+    want = _by_index(table, loc, diag, 1.5, weight_first, 0.25)
+    (want_grad,) = torch.autograd.grad(want, table, upstream)
+    assert torch.equal(got, want) and torch.equal(got_grad, want_grad)
+
+
+def test_locations_that_are_refused_stay_refused():
+  args = argparse.Namespace(mpnet_mrf_mode="TRWP", mpnet_max_iter=1, mpnet_n_dirs=4, n_classes=5,
+                            mpnet_term_weight=1.0, mpnet_smoothness_train="sigmoid", mpnet_diag_value=0.0)
+  module = MPModule(args)
+  module.set_label_context(torch.nn.Parameter(torch.rand(5, 5)), [0, 3], [range(5), range(5)])
+  with pytest.raises(RuntimeError):
+    module._effective_label_context()
+  module.set_label_context(torch.nn.Parameter(torch.rand(5)), [7], [0])
+  with pytest.raises(IndexError):
+    module._effective_label_context()
