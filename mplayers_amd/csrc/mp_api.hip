@@ -1568,7 +1568,10 @@ int mpl_trwp_soft_backward(const mpl_shape* s, unsigned flags, float rho, int n_
       p.fused_pair = (opts.fused_pairs && s->n_disp <= 32 &&
                       p.block_prefix[p.n_dirs] <= launch_policy().fused_pair_max_waves) ? 1 : 0;
       Timed timed(MPL_KERNEL_BWD_SWEEP, st, p.fused_pair ? 2 : 1);
-      launch_soft_bwd(p, st);
+      if (p.ctx2d && p.L == 21 && decide_team(p, opts, false))
+        launch_team21_bwd(p, st);
+      else
+        launch_soft_bwd(p, st);
       first = false;
       if (p.fused_pair) --d;
     }

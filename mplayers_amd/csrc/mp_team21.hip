@@ -440,8 +440,10 @@ struct alignas(16) BwdSlots {   // one set
 };
 constexpr int kPairs = kL * kL;
 
-// GR: dedge_weights and / or dcontext are wanted; DC: dcontext is
-template <bool GR, bool DC>
+// GR: dedge_weights and / or dcontext are wanted; DC: dcontext is.  SOFT: the soft-weighted operator, whose
+// step has the same form with J[cd][fd] = d message(cd) / d belief(fd) in place of the masks: the helpers
+// read a pixel's duals, take the softmin weights of a label over its front labels and put J into the slot.
+template <bool GR, bool DC, bool SOFT>
 __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
   extern __shared__ __align__(16) char smem_raw[];
   BwdSlots* sets = reinterpret_cast<BwdSlots*>(smem_raw);  // two
@@ -460,7 +462,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
   const int blocks = (n + kT - 1) / kT;
   const int iters = (blocks + 2 + kAhead - 1) / kAhead * kAhead;
   const bool want_de = GR && p.dedge != nullptr;
-  const bool same = p.same_label != 0;
+  const bool same = SOFT || p.same_label != 0;
   if (tid < kMaxL) acc[tid] = 0.f;
   if (GR) {
     for (int i = tid; i < kPairs; i += kTeam) ctx_s[i] = p.ctx[i];
@@ -474,6 +476,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
   auto main_walk = [&]() __attribute__((always_inline)) {
     const int sl = source_label(lane);
     const int src_mask = (lane & 15) < kSrc && sl < kL ? -1 : 0;
+    const int ok_mask = ok ? -1 : 0;
     const int lm = ok ? l : kL - 1;  // (a lane without a label repeats the last one's sums: nothing reads them)
     float sc = 0.f;
     struct In {
@@ -552,14 +555,17 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
           float tot;
           // MsgNormNaiveBack (commonCUDA.cuh:131-145) through the argmin label of its label
           sc = masked_sums<DC>(g, gw, cur.m, src_mask, tot, pairs);
+          // (weights are not masks: what is not finite reaches every label by itself, but not from the
+          // lanes without one)
+          if (SOFT) sc = flt(bits(sc) & ok_mask);
           if (GR) s.tot[i][half] = tot;
           cur = nxt;
         }
         // an infinity or a NaN in any gradient makes NaN of every sum of its pixel and of all after it
         // (tested as an integer: the compiler may take NaN for anything)
-        int probe = uniform_i(bits(sc));
+        int probe = SOFT ? 0 : uniform_i(bits(sc));
         asm("" : "+s"(probe));
-        if (__builtin_expect((probe & 0x7f800000) == 0x7f800000, 0)) {
+        if (!SOFT && __builtin_expect((probe & 0x7f800000) == 0x7f800000, 0)) {
           sc = sc_was;
           if (DC) {
             gw = 0.f;
@@ -580,8 +586,9 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
   };
 
   // even_walk: a constant; which of the two walks of a pair this is (mp_bwd.hip)
-  auto helper_walk = [&](const ChainCtx& ch, const auto even_walk) __attribute__((always_inline)) {
-    constexpr bool EVEN = decltype(even_walk)::value;
+  auto helper_walk = [&](const ChainCtx& ch, const auto even_walk, const float* a_in, const bool first_touch)
+      __attribute__((always_inline)) {
+    constexpr bool EVEN = !SOFT && decltype(even_walk)::value;
     const int dir = ch.dir;
     const int64_t HW = (int64_t)p.H * p.W;
     const int64_t P = (int64_t)p.B * HW;
@@ -591,12 +598,17 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
     float* bHd = p.h + (int64_t)dir * N + img_e;
     float* bHi = p.h + (int64_t)(dir ^ 1) * N + img_e;
     const int img_bytes = (int)(unsigned)(HW * kL * 4);
-    const rsrc_t rA = make_rsrc(p.a_in + img_e, img_bytes);
-    const rsrc_t rAo = make_rsrc(EVEN ? p.a_out + img_e : bHd, img_bytes);
-    const rsrc_t rHdIn = make_rsrc(bHd, !p.first_touch ? img_bytes : 0);
-    const rsrc_t rHiIn = make_rsrc(bHi, EVEN ? img_bytes : 0);
-    const rsrc_t rHiOut = make_rsrc(bHi, (EVEN && !p.skip_h_store) ? img_bytes : 0);
-    const rsrc_t rImin = make_rsrc(p.idx_min + (int64_t)dir * N + img_e, (int)(HW * kL));
+    const rsrc_t rA = make_rsrc(a_in + img_e, img_bytes);
+    const rsrc_t rAo = make_rsrc(EVEN || SOFT ? p.a_out + img_e : bHd, img_bytes);
+    const rsrc_t rHdIn = make_rsrc(bHd, !first_touch ? img_bytes : 0);
+    const rsrc_t rHiIn = make_rsrc(bHi, EVEN || (SOFT && !first_touch) ? img_bytes : 0);
+    const rsrc_t rHdOut = make_rsrc(bHd, SOFT ? img_bytes : 0);
+    const rsrc_t rHiOut = make_rsrc(bHi, SOFT || (EVEN && !p.skip_h_store) ? img_bytes : 0);
+    // the duals of a pixel: even directions [fd][cd], odd ones [cd][fd] (TRWP_forward_soft.cu:64); a lane takes
+    // those of its label and its half's front labels
+    const float* duals = SOFT ? p.edge_label + ((int64_t)dir * P + img_p) * kPairs : nullptr;
+    const bool front_first = (dir & 1) == 0;
+    const rsrc_t rImin = make_rsrc(SOFT ? nullptr : p.idx_min + (int64_t)dir * N + img_e, SOFT ? 0 : (int)(HW * kL));
     const rsrc_t rInorm = make_rsrc(p.idx_norm + (int64_t)dir * P + img_p, (int)HW);
     const rsrc_t rW = make_rsrc(p.edge + (int64_t)dir * P + img_p, (int)(HW * 4));
     const rsrc_t rDe = make_rsrc(want_de ? p.dedge + (int64_t)dir * P + img_p : nullptr, want_de ? (int)(HW * 4) : 0);
@@ -605,6 +617,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
     const int sl = source_label(lane);
     struct Pix {
       float a, hd, hi, w, de;
+      float dual[SOFT ? 2 : 1][kSrc];  // of both halves' pixels
       int fd, nidx;
     };
     auto label_off = [&](const bool on, const unsigned pp) __attribute__((always_inline)) {
@@ -625,8 +638,21 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       r.a = load(rA, off);
       r.hd = load(rHdIn, off);
       r.hi = 0.f;
-      if (EVEN) r.hi = load(rHiIn, off);
-      r.fd = __builtin_amdgcn_raw_buffer_load_b8(rImin, (int)((on && ok) ? pp * (unsigned)kL + (unsigned)l : kDeadWide), 0, 0);
+      if (EVEN || SOFT) r.hi = load(rHiIn, off);
+      if constexpr (SOFT) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int sh = uniform_i(s - half) + h;  // (both halves' positions are consecutive)
+          const unsigned ph = (unsigned)(p_last - sh * ch.pstep);
+          const rsrc_t rD = make_rsrc(duals + (sh < n ? (int64_t)ph * kPairs : 0), sh < n ? kPairs * 4 : 0);
+#pragma unroll
+          for (int q = 0; q < kSrc; ++q) {
+            const int fd = half * kSrc + q;
+            r.dual[h][q] = load(rD, (int)(ok && fd < kL ? (front_first ? fd * kL + l : l * kL + fd) * 4 : (int)kDeadOffset));
+          }
+        }
+      }
+      r.fd = SOFT ? 0 : __builtin_amdgcn_raw_buffer_load_b8(rImin, (int)((on && ok) ? pp * (unsigned)kL + (unsigned)l : kDeadWide), 0, 0);
       r.nidx = __builtin_amdgcn_raw_buffer_load_b8(rInorm, (int)(on ? pp : kDeadWide), 0, 0);
       r.w = r.de = 0.f;
       if (GR) {
@@ -635,8 +661,16 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       }
       return r;
     };
+    float tcol[SOFT ? kSrc : 1];  // ctx(l, front label) of the lane's front labels
+    if constexpr (SOFT && GR) {
+#pragma unroll
+      for (int q = 0; q < kSrc; ++q) {
+        const int fd = half * kSrc + q < kL ? half * kSrc + q : kL - 1, cd = ok ? l : kL - 1;
+        tcol[q] = ctx_s[cd < fd ? cd * kL + fd : fd * kL + cd];
+      }
+    }
     struct Kept {  // of a pixel whose dU is not known yet
-      float ap, base, w, de, cv;
+      float ap, base, w, de, cv, hi;
       int fd, nidx, fn;
     };
     // walk position u
@@ -648,9 +682,62 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       kp.fd = px.fd;
       kp.nidx = px.nidx;
       *reinterpret_cast<f32x2*>(s.base[i][l]) = f32x2{kp.base, u < n - 1 ? px.w : 0.f};
-      if (GR) {
+      if (GR && !SOFT) {
         const int lo = l < px.fd ? l : px.fd, hi = l < px.fd ? px.fd : l;
         kp.cv = ok && px.fd < kL ? ctx_s[lo * kL + hi] : 0.f;
+      }
+      if (SOFT) kp.hi = px.hi;
+      if constexpr (SOFT) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          // softmin over the front labels of this lane's label (TRWP_backward_soft.cu:83-105), both halves
+          const bool two = half * kSrc + kSrc - 1 < kL;  // (the last of the upper half does not exist)
+          float d[kSrc], ex[kSrc], lower, upper;
+#pragma unroll
+          for (int q = 0; q < kSrc; ++q) d[q] = px.dual[h][q];
+          float mn = two ? d[kSrc - 1] : INFINITY;
+#pragma unroll
+          for (int q = 0; q + 1 < kSrc; q += 2) mn = fminf(fminf(mn, d[q]), d[q + 1]);
+          halves(mn, lower, upper);
+          mn = fminf(lower, upper);
+          constexpr float kLog2e = 1.4426950408889634f;
+          const float ml2 = mn * kLog2e;
+          float se = 0.f, sd = 0.f;
+#pragma unroll
+          for (int q = 0; q < kSrc; ++q) {
+            ex[q] = q + 1 < kSrc || two ? __builtin_amdgcn_exp2f(fmaf(d[q], -kLog2e, ml2)) : 0.f;
+            se += ex[q];
+            sd = fmaf(ex[q], d[q], sd);
+          }
+          halves(se, lower, upper);
+          se = lower + upper;
+          halves(sd, lower, upper);
+          sd = lower + upper;
+          const float inv = __builtin_amdgcn_rcpf(se);
+          const float soft1 = fmaf(sd, inv, 1.f);
+          float ev = 0.f;
+#pragma unroll
+          for (int q = 0; q < kSrc; ++q) {
+            const int fd = half * kSrc + q;
+            const float jv = inv * ex[q] * (soft1 - d[q]);  // :110-113
+            if (ok && fd < kL) s.mask[2 * role + h][l / kSrc][fd][l % kSrc] = jv;
+            if (GR) ev = fmaf(tcol[q], ok && fd < kL ? jv : 0.f, ev);
+          }
+          // (the upper half's last source does not exist)
+          if (half == 1 && ok) s.mask[2 * role + h][1][l][kSrc - 1] = 0.f;
+          if (GR) {
+            halves(ev, lower, upper);
+            if (half == h) kp.cv = lower + upper;
+          }
+          lds_order();
+          const int nidx = __builtin_amdgcn_readlane(px.nidx, h * kHalf) & (kHalf - 1);
+          const int nn = nidx < kL ? nidx : kL - 1;
+          if (ok) {
+            const float jn = s.mask[2 * role + h][nn / kSrc][l][nn % kSrc];
+            s.mask[2 * role + h][half][l][kSrc] = nidx < kL ? jn : 0.f;
+          }
+        }
+        return;
       }
       s.fd[i][l] = px.fd;
       lds_order();
@@ -682,7 +769,12 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       const unsigned pp = (unsigned)(ch.pix0 + t * ch.pstep);
       const int off = label_off(on, pp);
       const float sc = s.sc[i][l];
-      if constexpr (!EVEN) {
+      if constexpr (SOFT) {
+        const float an = fmaf(rho, sc, kp.ap);
+        store(rAo, off, an);
+        store(rHdOut, off, -an);
+        store(rHiOut, off, kp.hi - sc);
+      } else if constexpr (!EVEN) {
         store(rAo, off, sc);
       } else {
         store(rAo, off, fmaf(rho, sc, kp.ap));  // g_k += rho*dU for every k, dunary too
@@ -696,7 +788,11 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
         float det = ok && edge ? kp.cv * g : 0.f;
         if (want_de) det = half_sum(det);
         // what the normalisation adds to dcontext; the gradients themselves are the main wavefront's
-        if (DC && l == 0 && edge && kp.nidx < kL && kp.fn < kL && (same || kp.nidx != kp.fn)) {
+        if (SOFT && DC && ok && edge && kp.nidx < kL) {
+          const int lo = l < kp.nidx ? l : kp.nidx, hi = l < kp.nidx ? kp.nidx : l;
+          atomicAdd(&hist_s[lo * kL + hi], -kp.w * tot * s.mask[i][half][l][kSrc]);
+        }
+        if (!SOFT && DC && l == 0 && edge && kp.nidx < kL && kp.fn < kL && (same || kp.nidx != kp.fn)) {
           const int lo = kp.nidx < kp.fn ? kp.nidx : kp.fn, hi = kp.nidx < kp.fn ? kp.fn : kp.nidx;
           atomicAdd(&hist_s[lo * kL + hi], -kp.w * tot);
         }
@@ -735,7 +831,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       main_walk();
     }
   } else {
-    if (ch0.dir & 1) helper_walk(ch0, std::false_type());
+    if (ch0.dir & 1) helper_walk(ch0, std::false_type(), p.a_in, p.first_touch != 0);
     if (!(ch0.dir & 1) || p.fused_pair) {
       ChainCtx ch = ch0;
       if (ch0.dir & 1) {
@@ -745,7 +841,8 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
         wait_vmem<0>();
         __syncthreads();
       }
-      helper_walk(ch, std::true_type());
+      const bool second = (ch0.dir & 1) != 0;
+      helper_walk(ch, std::true_type(), SOFT && second ? p.a_out : p.a_in, (SOFT && second) ? false : p.first_touch != 0);
     }
   }
   if (!DC) return;
@@ -781,12 +878,14 @@ void launch_team21_bwd(const BackParams& p, hipStream_t st) {
   if (blocks <= 0) return;
   const bool gr = p.dedge != nullptr || p.dctx != nullptr;
   const size_t lds = 2 * sizeof(BwdSlots) + sizeof(float) * (kMaxL + (gr ? 2 * kPairs : 0));
-  if (p.dctx != nullptr)
-    bwd_team21_kernel<true, true><<<blocks, kTeam, lds, st>>>(p);
-  else if (gr)
-    bwd_team21_kernel<true, false><<<blocks, kTeam, lds, st>>>(p);
-  else
-    bwd_team21_kernel<false, false><<<blocks, kTeam, lds, st>>>(p);
+  auto kernel = p.edge_label != nullptr
+                    ? (p.dctx != nullptr ? bwd_team21_kernel<true, true, true>
+                       : gr              ? bwd_team21_kernel<true, false, true>
+                                         : bwd_team21_kernel<false, false, true>)
+                    : (p.dctx != nullptr ? bwd_team21_kernel<true, true, false>
+                       : gr              ? bwd_team21_kernel<true, false, false>
+                                         : bwd_team21_kernel<false, false, false>);
+  kernel<<<blocks, kTeam, lds, st>>>(p);
 }
 
 }  // namespace mpl
