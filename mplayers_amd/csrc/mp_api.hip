@@ -729,6 +729,8 @@ int team_chains_per_cu(int L, bool jacobi) {
 // 12 (129 / 516 / 1032 / 1548 chains).  Forward, argmin labels kept: 2.05 / 1.95 / 1.51 / 1.48; rows without
 // them 1.51 with 256, 1.46 with 1024, 1.53 with 2048 chains.  Backward, dunary alone: 1.35 / 1.21 / 0.99 /
 // 0.82, with both other gradients 1.85 / 1.47 / 1.08 / 1.21; 65x65, batch 12 (780 chains) 0.85 and 1.11.
+// Soft-weighted, forward (one wavefront on both sides) and backward, ms: 135 chains 1.85 -> 1.53, 258 chains
+// 3.85 -> 3.10, 516 chains 4.97 -> 4.02, 516 / 660 chains 5.74 -> 4.70.
 // (More than 2048 chains: the packed scans.)
 constexpr int kTeam21FwdChainsPerCu = 8;
 constexpr int kTeam21BwdChainsPerCu = 3;

@@ -64,3 +64,34 @@ def test_terms_that_are_not_finite(gpu, value):
     assert np.array_equal(np.isposinf(a), np.isposinf(b)) and np.array_equal(np.isneginf(a), np.isneginf(b)), what
     ok = np.isfinite(b)
     assert np.abs(a[ok] - b[ok]).max() <= 1e-4 * max(1.0, float(np.abs(b[ok]).max())), what
+
+
+@pytest.mark.parametrize("n_dir,B,H,W", [(4, 1, 1, 1), (4, 1, 2, 5), (4, 2, 6, 7), (8, 1, 12, 13), (4, 1, 3, 50)])
+@pytest.mark.parametrize("pairs", [True, False])
+def test_soft_backward_against_the_oracle(gpu, oracle, n_dir, B, H, W, pairs):
+  """Soft-weighted TRWP: the same scan with the softmin's stored parts in the place of the argmin labels."""
+  import torch
+  from mplayers_amd import _lib, lib_stereo
+  rng = np.random.default_rng(100 * H + W)
+  unary = rng.random((B, 1, H, W, L)).astype(np.float32)
+  ctx = np.triu(rng.random((L, L)), 1).astype(np.float32)
+  ew = (0.2 + rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
+  fwd = oracle.forward_soft(unary, ctx, ew, n_dir, 2, 0.5)
+  ref = oracle.backward_soft(ctx.astype(np.float64), ew.astype(np.float64), dcost.astype(np.float64),
+                             fwd["msg_edge_label"].astype(np.float64), fwd["msg_norm_index"], 0.5)
+  up = lambda a: torch.as_tensor(np.ascontiguousarray(a)).cuda()
+  print("case", n_dir, B, H, W, pairs, flush=True)
+  try:
+    for option in (0, 2):
+      _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+      g = up(dcost)
+      got = g.new_zeros(B, 1, H, W, L), g.new_zeros(L, L), g.new_zeros(n_dir, B, 1, H, W)
+      lib_stereo.TRWP_hard_soft.backward_soft(0.5, g, up(ctx), up(ew), up(fwd["msg_edge_label"]),
+                                              up(fwd["msg_norm_index"]), *got, g.new_full((n_dir, B, 1, H, W, L), 3.5),
+                                              g.new_empty(0), flags=0 if pairs else _lib.F_FUSED_PAIRS_OFF)
+      for a, b, what in zip(got, ref, ("dunary", "dcontext", "dedge_weights")):
+        # sums of at most a few thousand products: 1e-4 of the largest entry, as everywhere
+        assert np.abs(a.cpu().numpy() - b).max() <= 1e-4 * max(1.0, float(np.abs(b).max())), (option, what)
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
