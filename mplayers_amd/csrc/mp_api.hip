@@ -699,7 +699,8 @@ int chains_at_once(const Params& p) {
 // the same bits whichever gradients are wanted.  Measured, backward of 2 iterations on square images with
 // 4, 8 and 16 directions (TRWP: chains of one direction per launch, ISGMR: of all), time with one over
 // time with four wavefronts: the least of dunary alone and of all gradients on a band of four labels, a
-// bent band, a linear and a random table / the greatest.
+// bent band, a linear and a random table / the greatest.  (Taken while the main wavefronts of a unit's chains
+// shared a SIMD, which cost this side where there are two or three: 150 labels 300x500 2.68 -> 2.20 ms since.)
 //   * up to 64 labels: TRWP 256 chains 0.78 / 1.65, 768 chains with 33 labels 0.75 / 1.2, ISGMR 0.69 / 1.5.
 //     With one label per lane the step of mp_bwd.hip is short, and labels that point anywhere cost this
 //     kernel more (64 labels, dunary alone: 199 ns per pixel and walk there, 245 here).  Never taken.
@@ -729,11 +730,15 @@ int team_chains_per_cu(int L, bool jacobi) {
 // 12 (129 / 516 / 1032 / 1548 chains).  Forward, argmin labels kept: 2.05 / 1.95 / 1.51 / 1.48; rows without
 // them 1.51 with 256, 1.46 with 1024, 1.53 with 2048 chains.  Backward, dunary alone: 1.35 / 1.21 / 0.99 /
 // 0.82, with both other gradients 1.85 / 1.47 / 1.08 / 1.21; 65x65, batch 12 (780 chains) 0.85 and 1.11.
-// Soft-weighted, forward (one wavefront on both sides) and backward, ms: 135 chains 1.85 -> 1.53, 258 chains
-// 3.85 -> 3.10, 516 chains 4.97 -> 4.02, 516 / 660 chains 5.74 -> 4.70.
+// Soft-weighted, five iterations forward and backward, ms with the reverse scan on one -> on four wavefronts, the
+// forward scan on one: 135 chains 1.85 -> 1.53, 258 chains 3.85 -> 3.10, 516 chains 4.97 -> 4.02, 516 / 660
+// chains 5.74 -> 4.70.
 // (More than 2048 chains: the packed scans.)
 constexpr int kTeam21FwdChainsPerCu = 8;
 constexpr int kTeam21BwdChainsPerCu = 3;
+// Its forward scan, two iterations on images of 129x129, one over four wavefronts, duals kept / not: 129 chains 1.65
+// / 1.32, 516 chains 1.57 / 1.35, 774 chains 1.16 / 1.22, 1032 chains 1.07 / 1.00, 2064 chains 1.07 / 0.89.
+constexpr int kTeam21SoftFwdChainsPerCu = 4;
 
 int decide_team(const BackParams& p, const CallOpts& o, bool jacobi) {
   if (p.pack >= 2 || o.team == 0) return 0;
@@ -775,6 +780,11 @@ int decide_team_fwd(const SweepParams& p, const CallOpts& o, bool train) {
   if (o.team == 2) return 1;
   const int per_cu = p.ctx2d && p.L == 21 ? kTeam21FwdChainsPerCu : team_fwd_chains_per_cu(p.L, train);
   return chains_at_once(p) <= per_cu * (launch_policy().n_simd / 4) ? 1 : 0;
+}
+
+bool decide_team21_soft_fwd(const SweepParams& p, const CallOpts& o) {
+  if (o.team == 0) return false;
+  return o.team == 2 || chains_at_once(p) <= kTeam21SoftFwdChainsPerCu * (launch_policy().n_simd / 4);
 }
 
 // Wavefronts per chain for the forward scan of a launch whose caller declared a dense 1-D table
@@ -1505,7 +1515,10 @@ int mpl_trwp_soft_forward(const mpl_shape* s, unsigned flags, float rho, int n_i
       p.fused_pair = (opts.fused_pairs && s->n_disp <= 32 &&
                       p.block_prefix[p.n_dirs] <= launch_policy().fused_pair_max_waves) ? 1 : 0;
       Timed timed(MPL_KERNEL_FWD_SWEEP, st, p.fused_pair ? 2 : 1);
-      launch_soft_fwd(p, train, st);
+      if (p.ctx2d && p.L == 21 && decide_team21_soft_fwd(p, opts))
+        launch_team21_soft_fwd(p, st);
+      else
+        launch_soft_fwd(p, train, st);
       if (p.fused_pair) ++d;
     }
     if (label_all) {

@@ -612,6 +612,7 @@ template <int R>
 void launch_sweep_bwd(const BackParams& p, bool jacobi, hipStream_t st);
 // 21 labels with a 2-D table, TRWP (mp_team21.hip)
 void launch_team21_fwd(const SweepParams& p, bool train, hipStream_t st);
+void launch_team21_soft_fwd(const SweepParams& p, hipStream_t st);  // (p.edge_label: the duals are kept)
 void launch_team21_bwd(const BackParams& p, hipStream_t st);
 template <int R>
 void launch_team_bwd(const BackParams& p, bool jacobi, hipStream_t st);

@@ -26,8 +26,11 @@
 // over 40 problems (images up to 130x130, 4 and 8 directions, 1 to 5 iterations; normal, positive and cross
 // entropy gradients): dunary 1.52e-7 -> 1.35e-7, dcontext 5.0e-7 both, dedge_weights 1.79e-7 -> 1.63e-7.
 // Soft-weighted, 30 problems up to 100x100, 4 directions: 9.6e-8 -> 8.8e-8, 2.7e-7 both, 2.55e-7 -> 2.44e-7
-// (dedge_weights 2.9e-7 to 3.6e-7 while the expected dual's own rounding was left in).  Its reverse scan,
-// 2x129x129, five iterations: 2.0 -> 1.3 ms, bound by the helpers' softmin weights (441 exponentials a pixel).
+// (dedge_weights 2.9e-7 to 3.6e-7 while the expected dual's own rounding was left in).  Its scans,
+// 2x129x129, five iterations, duals kept: forward 1.44 -> 0.87 ms, bound by the main wavefront (11 exponentials and
+// three exchanges of halves a pixel), reverse 2.03 -> 1.30 ms, by the helpers' softmin weights.  Forward errors
+// over 24 problems: messages 5.0e-7 -> 4.7e-7, costs 1.11e-7 -> 1.06e-7, duals 7.7e-8 ->
+// 7.5e-8.
 
 #include <type_traits>
 
@@ -43,6 +46,7 @@ constexpr int kHelpers = 3;          // one SIMD of the compute unit each, the m
 constexpr int kT = 2 * kHelpers;     // pixels per block
 constexpr int kTeam = (kHelpers + 1) * kWave;
 constexpr int kAhead = 2;            // blocks whose loads are in flight (four measure the same)
+constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kRow = 36;             // words between the pixels of a slot read by both halves at once
 
 // workgroup barrier over LDS contents only: global loads in flight stay in flight
@@ -98,6 +102,29 @@ __device__ __forceinline__ void join_min(float best, float pad, float& v, float&
       : "+&v"(best), "=&v"(src), "=&v"(nmin), "=&v"(t), "=&v"(y)
       : "v"(pad));
   v = best;
+}
+
+// The same from the softmin messages by label, which are +inf in the lanes without one.
+__device__ __forceinline__ void spread_min(float v, float& src, float& nmin) {
+  float y;
+  asm("v_mov_b32 %0, %3\n\t"
+      "v_mov_b32 %2, %3\n\t"
+      "s_nop 1\n\t"
+      "v_permlane16_swap_b32 %0, %2\n\t"
+      "v_min_f32 %1, %0, %2\n\t"
+      "s_nop 0\n\t"
+      "v_mov_b32_dpp %0, %0 row_shl:11 row_mask:0xc bank_mask:0xf\n\t"
+      "s_nop 0\n\t"
+      "v_min_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b32_dpp %0, %2 row_shr:5 row_mask:0xc bank_mask:0xf\n\t"
+      "s_nop 0\n\t"
+      "v_min_f32_dpp %1, %1, %1 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_min_f32_dpp %1, %1, %1 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_min_f32_dpp %1, %1, %1 row_ror:1 row_mask:0xf bank_mask:0xf"
+      : "=&v"(src), "=&v"(nmin), "=&v"(y)
+      : "v"(v));
 }
 
 // The reverse step.  m[0 .. 10] are the masks of a lane's label, m[11] is 1 where it is the argmin label of
@@ -216,7 +243,10 @@ struct alignas(16) FwdSlots {   // one set
   float out[kT][kHalf][2];      // v and the normalisation minimum; without argmin labels the message
 };
 
-template <bool TRAIN>
+// SOFT: the soft-weighted operator.  The main wavefront takes each half's softmin sums around the joint
+// minimum; where the duals are kept (TRAIN) the helpers form a pixel's block again from its beliefs, 64
+// entries to a store.
+template <bool TRAIN, bool SOFT>
 __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) {
   extern __shared__ __align__(16) char smem_raw[];
   FwdSlots* sets = reinterpret_cast<FwdSlots*>(smem_raw);  // two
@@ -260,12 +290,35 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
             constexpr int q = decltype(ii)::value;
             c[q] = fmaf(cur[1], tc[q], row_bcast<q>(a));
           });
+          float v, vs, nmin;
+          if (SOFT) c[kSrc - 1] = half ? c[0] : c[kSrc - 1];  // (the upper half's last source does not exist)
           const float best = fminf(fminf(fminf(fminf(c[0], c[1]), c[2]), fminf(fminf(c[3], c[4]), c[5])),
                                    fminf(fminf(fminf(c[6], c[7]), c[8]), fminf(c[9], c[10])));
-          float v, vs, nmin;
-          join_min(best, pad, v, vs, nmin);
+          if constexpr (SOFT) {
+            // TRWP_forward_soft.cu:81-97, the duals relative to the least one
+            float lower, upper;
+            halves(best, lower, upper);
+            const float mn = fminf(lower, upper);
+            float se[2] = {0.f, 0.f}, sd[2] = {0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < kSrc; ++q) {
+              const float d = c[q] - mn;
+              float e = __builtin_amdgcn_exp2f(d * -kLog2e);
+              if (q == kSrc - 1) e = half ? 0.f : e;
+              se[q & 1] += e;
+              sd[q & 1] = fmaf(e, d, sd[q & 1]);
+            }
+            float se_l, se_u;
+            halves(se[0] + se[1], se_l, se_u);
+            halves(sd[0] + sd[1], lower, upper);
+            v = fmaf(lower + upper, __builtin_amdgcn_rcpf(se_l + se_u), mn);
+            v = ok ? v : INFINITY;
+            spread_min(v, vs, nmin);
+          } else {
+            join_min(best, pad, v, vs, nmin);
+          }
           prev = (i == 0 && k == 1) ? 0.f : vs - nmin;  // (the chain start has no front pixel and no message)
-          if (TRAIN)
+          if (TRAIN || SOFT)
             *reinterpret_cast<f32x2*>(s.out[i][l]) = f32x2{v, nmin};
           else
             s.out[i][sl][0] = prev;
@@ -284,7 +337,7 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
   // even_walk: a constant; the first (even direction) or the second sweep of a pair (run_chain_fwd)
   auto helper_walk = [&](const ChainCtx& ch, const bool skip_s_in, const auto even_walk)
       __attribute__((always_inline)) {
-    constexpr bool EVEN = decltype(even_walk)::value;
+    constexpr bool EVEN = SOFT || decltype(even_walk)::value;  // (soft-weighted: every sweep stores S)
     const int dir = ch.dir;
     const int64_t img_p = (int64_t)ch.bv * HW;
     const int64_t img_e = img_p * kL;
@@ -299,11 +352,27 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
     const rsrc_t rMi = make_rsrc(p.msg_in + (int64_t)(dir ^ 1) * N + img_e, mi_zero ? 0 : img_bytes);
     const rsrc_t rMo = make_rsrc(p.msg_out + (int64_t)dir * N + img_e, img_bytes);
     const rsrc_t rSo = make_rsrc(p.belief_out + img_e, skip_s ? 0 : img_bytes);
-    const rsrc_t rImin = make_rsrc(TRAIN ? p.idx_min + (int64_t)dir * N + img_e : nullptr, TRAIN ? (int)(HW * kL) : 0);
+    constexpr bool ARGMIN = TRAIN && !SOFT;
+    const rsrc_t rImin = make_rsrc(ARGMIN ? p.idx_min + (int64_t)dir * N + img_e : nullptr, ARGMIN ? (int)(HW * kL) : 0);
     const rsrc_t rInorm = make_rsrc(TRAIN ? p.idx_norm + (int64_t)dir * P + img_p : nullptr, TRAIN ? (int)HW : 0);
     const rsrc_t rW = make_rsrc(p.edge + (int64_t)dir * P + img_p, (int)(HW * 4));
-    float tcol[TRAIN ? kL : 1];
-    if constexpr (TRAIN) {
+    // the entries lane + 64 j of a block of duals, [front label][label] in even directions, [label][front label] in
+    // odd ones (TRWP_forward_soft.cu:64): the table is symmetric, so they differ in whose belief they add
+    constexpr int kEntries = (kL * kL + kWave - 1) / kWave;
+    float tblk[SOFT && TRAIN ? kEntries : 1];
+    int ablk[SOFT && TRAIN ? kEntries : 1];
+    float* const duals = SOFT && TRAIN ? p.edge_label + ((int64_t)dir * P + img_p) * (kL * kL) : nullptr;
+    if constexpr (SOFT && TRAIN) {
+#pragma unroll
+      for (int j = 0; j < kEntries; ++j) {
+        const int e = lane + kWave * j < kL * kL ? lane + kWave * j : kL * kL - 1;
+        const int row = e / kL, col = e - row * kL;
+        tblk[j] = p.ctx[row < col ? row * kL + col : col * kL + row];
+        ablk[j] = (dir & 1) ? col : row;
+      }
+    }
+    float tcol[ARGMIN ? kL : 1];
+    if constexpr (ARGMIN) {
 #pragma unroll
       for (int fd = 0; fd < kL; ++fd) tcol[fd] = table(fd);
     }
@@ -341,11 +410,12 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
     float tt[2] = {0.f, 0.f}, ww[2] = {0.f, 0.f};
     auto prepare = [&](const Pix& px, const int t, FwdSlots& s, float& tk, float& wk) __attribute__((always_inline)) {
       tk = EVEN ? px.s - px.md : px.s + px.mi;
-      const float un = fmaxf(fmaf(tk, rho, -px.mi), floor_l);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
+      float un = fmaf(tk, rho, -px.mi);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
+      if (!SOFT) un = fmaxf(un, floor_l);
       wk = px.w;
       *reinterpret_cast<f32x2*>(s.in[i][l]) = f32x2{un, px.w};
       // Q of the pixel is known already, whatever its message
-      if (EVEN) store(rSo, label_off(t < n, pixel_off(t)), tk - px.mi);
+      if (EVEN && !SOFT) store(rSo, label_off(t < n, pixel_off(t)), tk - px.mi);
     };
     // what is left of a pixel once its message is known (nothing outside the chain)
     auto finish = [&](const int t, const FwdSlots& s, const float tk, const float wk) __attribute__((always_inline)) {
@@ -354,7 +424,27 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
       const unsigned pp = pixel_off(t);
       const int off = label_off(on, pp);
       float m;
-      if constexpr (TRAIN) {
+      if constexpr (SOFT) {
+        const f32x2 o = *reinterpret_cast<const f32x2*>(s.out[i][l]);
+        m = o[0] - o[1];
+        if constexpr (TRAIN) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {  // the pixel of either half
+            const int th = uniform_i(t - half) + h;
+            const bool live = th > 0 && th < n;
+            const float w = flt(__builtin_amdgcn_readlane(bits(wk), h * kHalf));
+            const rsrc_t rBlk = make_rsrc(duals + (live ? (int64_t)pixel_off(th) * (kL * kL) : 0), live ? kL * kL * 4 : 0);
+#pragma unroll
+            for (int j = 0; j < kEntries; ++j)
+              store(rBlk, (lane + kWave * j) * 4, fmaf(w, tblk[j], s.a[2 * role + h][ablk[j]]));
+          }
+          const uint64_t at = ballot(ok && o[0] == o[1]);
+          const unsigned lo = (unsigned)at, hi = (unsigned)(at >> 32);
+          const int n0 = lo ? 31 - __builtin_clz(lo) : kL - 1, n1 = hi ? 31 - __builtin_clz(hi) : kL - 1;
+          __builtin_amdgcn_raw_buffer_store_b8((unsigned char)(half ? n1 : n0), rInorm,
+                                               (int)((step && l == 0) ? pp : kDeadWide), 0, 0);
+        }
+      } else if constexpr (TRAIN) {
         const f32x2 o = *reinterpret_cast<const f32x2*>(s.out[i][l]);
         float val[kL];
 #pragma unroll
@@ -379,7 +469,8 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
         m = s.out[i][l][0];
       }
       // (the reference never writes the chain start)
-      store(rMo, (step || p.zero_start) ? off : (int)kDeadWide, m);
+      store(rMo, (step || (!SOFT && p.zero_start)) ? off : (int)kDeadWide, m);
+      if constexpr (SOFT) store(rSo, step ? off : (int)kDeadWide, tk + m);
       if constexpr (!EVEN) store(rSo, off, tk + (t == 0 ? md0 : m));
     };
 
@@ -704,7 +795,6 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
           halves(mn, lower, upper);
           mn = fminf(lower, upper);
           // relative to the least dual: the sums keep the bits that its size would cost them
-          constexpr float kLog2e = 1.4426950408889634f;
           float se2[2] = {0.f, 0.f}, sd2[2] = {0.f, 0.f};
 #pragma unroll
           for (int q = 0; q < kSrc; ++q) {
@@ -886,9 +976,19 @@ void launch_team21_fwd(const SweepParams& p, bool train, hipStream_t st) {
   if (blocks <= 0) return;
   const size_t lds = 2 * sizeof(FwdSlots);
   if (train)
-    fwd_team21_kernel<true><<<blocks, kTeam, lds, st>>>(p);
+    fwd_team21_kernel<true, false><<<blocks, kTeam, lds, st>>>(p);
   else
-    fwd_team21_kernel<false><<<blocks, kTeam, lds, st>>>(p);
+    fwd_team21_kernel<false, false><<<blocks, kTeam, lds, st>>>(p);
+}
+
+void launch_team21_soft_fwd(const SweepParams& p, hipStream_t st) {
+  const int blocks = p.block_prefix[p.n_dirs];
+  if (blocks <= 0) return;
+  const size_t lds = 2 * sizeof(FwdSlots);
+  if (p.edge_label != nullptr)
+    fwd_team21_kernel<true, true><<<blocks, kTeam, lds, st>>>(p);
+  else
+    fwd_team21_kernel<false, true><<<blocks, kTeam, lds, st>>>(p);
 }
 
 void launch_team21_bwd(const BackParams& p, hipStream_t st) {

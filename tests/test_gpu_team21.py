@@ -1,6 +1,6 @@
 """TRWP's reverse scan for 21 labels and a 2-D table with four wavefronts per chain (MPL_OPT_TEAM_SCANS)
 against the fp64 oracle: chains around a block of six pixels, both kinds of dcontext, gradients that are left
-out, argmin labels that crowd on one target, terms that are not finite."""
+out, argmin labels that crowd on one target, terms that are not finite; both soft-weighted scans."""
 import numpy as np
 import pytest
 
@@ -95,3 +95,51 @@ def test_soft_backward_against_the_oracle(gpu, oracle, n_dir, B, H, W, pairs):
         assert np.abs(a.cpu().numpy() - b).max() <= 1e-4 * max(1.0, float(np.abs(b).max())), (option, what)
   finally:
     _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+
+
+@pytest.mark.parametrize("n_dir,B,H,W", [(4, 1, 1, 1), (4, 1, 2, 5), (4, 2, 6, 7), (8, 1, 12, 13), (4, 1, 3, 50)])
+@pytest.mark.parametrize("train", [True, False])
+def test_soft_forward_against_the_oracle(gpu, oracle, n_dir, B, H, W, train):
+  """Soft-weighted TRWP forward, one and four wavefronts, pairs in one launch and in two."""
+  import torch
+  from mplayers_amd import _lib, lib_stereo
+  rng = np.random.default_rng(100 * H + W + 1)
+  unary = rng.random((B, 1, H, W, L)).astype(np.float32)
+  ctx = np.triu(rng.random((L, L)), 1).astype(np.float32)
+  ew = (0.2 + rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  start = rng.random((n_dir, B, 1, H, W, L)).astype(np.float32)  # what the scans leave alone shows
+  up = lambda a: torch.as_tensor(np.ascontiguousarray(a)).cuda()
+  u8 = dict(dtype=torch.uint8, device="cuda")
+
+  def forward(option, flags, u=unary, m0=start):
+    u = up(u)
+    msg, cost, scratch = up(m0), torch.zeros_like(u), torch.zeros_like(u)
+    duals = u.new_full((2, n_dir, B, 1, H, W, L, L), 7.0) if train else torch.empty(0)
+    norm = torch.full((2, n_dir, B, 1, H, W), 77, **u8) if train else torch.empty(0, dtype=torch.uint8)
+    _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+    try:
+      lib_stereo.TRWP_hard_soft.forward_soft(0.5, 2, u, up(ctx), up(ew), msg, duals, norm, cost, scratch,
+                                             torch.empty(0, **u8), flags=flags)
+      torch.cuda.synchronize()
+    finally:
+      _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+    return [x.cpu().numpy() for x in ((msg, cost, duals, norm) if train else (msg, cost))]
+
+  print("case", n_dir, B, H, W, train, flush=True)
+  ref = oracle.forward_soft(unary, ctx, ew, n_dir, 2, 0.5)
+  got = forward(2, 0, m0=np.zeros_like(start))
+  scale = max(1.0, float(np.abs(ref["cost_final"]).max()))
+  assert np.abs(got[0] - ref["msg"]).max() <= 2e-5 * scale
+  assert np.abs(got[1] - ref["cost_final"]).max() <= 2e-5 * scale
+  one, pairs, single = forward(0, 0), forward(2, 0), forward(2, _lib.F_FUSED_PAIRS_OFF)
+  for a, b, c in zip(one, pairs, single):
+    assert np.array_equal(b, c)
+    if a.dtype != np.uint8:
+      assert np.abs(a - b).max() <= 2e-5 * scale
+    else:  # (labels whose softmin messages are closer than the tolerance aside)
+      assert (a != b).mean() <= 0.02 and np.array_equal(a == 77, b == 77)
+  for value in (np.inf, -np.inf, np.nan):
+    bad = unary.copy()
+    bad[0, 0, H // 2, W // 2, 18] = value
+    for a, b in zip(forward(0, 0, bad)[:2], forward(2, 0, bad)[:2]):
+      assert np.array_equal(np.isfinite(a), np.isfinite(b)), value
