@@ -231,8 +231,10 @@ class MPModule(torch.nn.Module):
     key = (label_context.device, label_context.shape) + tuple(mask.tobytes() for mask in host)
     kept = getattr(self, "_kept_masks", None)
     if kept is None or kept[0] != key:
-      # (copies from pageable memory are complete when they return, for every stream)
-      kept = (key,) + tuple(torch.from_numpy(mask).to(label_context.device) for mask in host)
+      # (copies from pageable memory are complete when they return, for every stream; tensors of inference
+      # mode could not be saved for a later call's backward pass)
+      with torch.inference_mode(False):
+        kept = (key,) + tuple(torch.from_numpy(mask).to(label_context.device) for mask in host)
       if not (label_context.is_cuda and torch.cuda.is_current_stream_capturing()):
         self._kept_masks = kept
     return kept[1:]

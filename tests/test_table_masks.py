@@ -51,6 +51,35 @@ def test_masks_give_what_indexing_gives(name, weight_first):
     assert torch.equal(got, want) and torch.equal(got_grad, want_grad)
 
 
+def _module(loc, diag, dims, **more):
+  args = argparse.Namespace(**dict(dict(mpnet_mrf_mode="TRWP", mpnet_max_iter=1, mpnet_n_dirs=4, n_classes=5,
+                                        mpnet_term_weight=1.5, mpnet_smoothness_train="sigmoid",
+                                        mpnet_diag_value=0.25), **more))
+  module = MPModule(args)
+  table = torch.nn.Parameter(torch.randn((5,) * dims, generator=torch.Generator().manual_seed(2)))
+  module.set_label_context(table, loc, diag)
+  return module
+
+
+def _check(module):
+  """Value and gradient of the module's table are those of indexing."""
+  table = module.label_context
+  upstream = torch.arange(1., 1. + table.numel()).reshape(table.shape)
+  got = module._effective_label_context()
+  want = _by_index(table, module.label_context_loc, module.label_context_diag_loc, 1.5, False,
+                   module.args.mpnet_diag_value)
+  assert type(got) is torch.Tensor and torch.equal(got, want)
+  assert torch.equal(torch.autograd.grad(got, table, upstream)[0], torch.autograd.grad(want, table, upstream)[0])
+
+
+def test_a_first_call_under_inference_mode():
+  """An evaluation before training leaves nothing that autograd cannot save."""
+  module = _module(*LOCATIONS["triangle"])
+  with torch.inference_mode():
+    module._effective_label_context()
+  _check(module)
+
+
 def test_locations_that_are_refused_stay_refused():
   args = argparse.Namespace(mpnet_mrf_mode="TRWP", mpnet_max_iter=1, mpnet_n_dirs=4, n_classes=5,
                             mpnet_term_weight=1.0, mpnet_smoothness_train="sigmoid", mpnet_diag_value=0.0)
