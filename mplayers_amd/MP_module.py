@@ -212,8 +212,8 @@ class MPModule(torch.nn.Module):
 
   def _location_masks(self, label_context):
     """Masks of label_context_loc and label_context_diag_loc on the table's device, None where a location is
-    a tensor or not a list of entries.  They are formed on the host from the locations of the moment and copied only when they
-    differ from what was copied last."""
+    a tensor or not a list of different entries.  They are formed on the host from the locations of the moment
+    and copied only when they differ from what was copied last."""
     diag = self.label_context_diag_loc
     places = [self.label_context_loc, tuple(diag) if isinstance(diag, list) else diag]
     parts = [part for place in places for part in (place if isinstance(place, tuple) else (place,))]
@@ -224,9 +224,12 @@ class MPModule(torch.nn.Module):
       mask = np.zeros(label_context.shape, bool)
       as_array = lambda x: np.asarray(x) if isinstance(x, (list, range)) else x
       index = tuple(map(as_array, place)) if isinstance(place, tuple) else as_array(place)
-      if not host and np.ndim(mask[index]) != 1:
+      taken = mask[index]
+      if not host and np.ndim(taken) != 1:
         return None  # (what takes the values back entry by entry is one-dimensional)
       mask[index] = True
+      if not host and np.count_nonzero(mask) != np.size(taken):
+        return None  # (an entry named twice has its gradient twice)
       host.append(mask)
     key = (label_context.device, label_context.shape) + tuple(mask.tobytes() for mask in host)
     kept = getattr(self, "_kept_masks", None)

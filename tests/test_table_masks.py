@@ -25,6 +25,10 @@ LOCATIONS = {
     "slice": (slice(2, None), 0, 1),
     "negative": (np.array([-1, -2]), range(2), 1),
     "overlap": (range(0, 5), range(2), 1),
+    "repeated": ([1, 3, 3], [0], 1),
+    "two names of one entry": ([-1, 4], [0], 1),
+    "repeated, 2-D": ((np.array([0, 0, 1]), np.array([1, 1, 2])), [range(5), range(5)], 2),
+    "pinned twice": ([1, 3], [[0, 0, -5]], 1),
 }
 
 
