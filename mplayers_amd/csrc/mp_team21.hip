@@ -641,7 +641,11 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
           s.sc[i][l] = sc;
           // gradient w.r.t. the normalised message of this pixel, including what the previous step
           // added through the recurrence (dmsg[front] += rho * value, TRWP_backward.cu:108)
-          const float g = fmaf(rho, to_sources<DC>(sc, gw, m0, pairs), cur.b[0]);
+          float g = fmaf(rho, to_sources<DC>(sc, gw, m0, pairs), cur.b[0]);
+          // The chain start has no message, and neither have the places of the block past it: without a gradient
+          // there, the sums and dcontext stay what they are (a zero weight would not do: zero times what is
+          // not finite)
+          if (SOFT) g = flt(bits(g) & ((k - 1) * kT + i < n - 1 ? -1 : 0));
           if (DC) {
             gw = cur.b[1] * g;
             m0 = cur.m[0];
@@ -738,7 +742,8 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
         for (int h = 0; h < 2; ++h) {
           const int sh = uniform_i(s - half) + h;  // (both halves' positions are consecutive)
           const unsigned ph = (unsigned)(p_last - sh * ch.pstep);
-          const rsrc_t rD = make_rsrc(duals + (sh < n ? (int64_t)ph * kPairs : 0), sh < n ? kPairs * 4 : 0);
+          const bool edge = sh < n - 1;  // (nobody writes the duals of a chain start)
+          const rsrc_t rD = make_rsrc(duals + (edge ? (int64_t)ph * kPairs : 0), edge ? kPairs * 4 : 0);
 #pragma unroll
           for (int q = 0; q < kSrc; ++q) {
             const int fd = half * kSrc + q;

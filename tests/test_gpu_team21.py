@@ -53,17 +53,20 @@ def test_backward_against_the_oracle(gpu, oracle, n_dir, B, H, W, crowd):
         assert np.array_equal(part[2], got[2])
 
 
-@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
-def test_terms_that_are_not_finite(gpu, value):
-  """They reach the entries they reach with one wavefront per chain, and the others are what they are there."""
-  problem = _problem(4, 1, 1, 9, 14, 3)
-  problem[2][0, 0, 4, 5, 7] = value
-  one, four = _backward(gpu, problem, 0), _backward(gpu, problem, 2)
+def _same_where_not_finite(four, one):
   for a, b, what in zip(four, one, ("dunary", "dcontext", "dedge_weights")):
     assert np.array_equal(np.isnan(a), np.isnan(b)), what
     assert np.array_equal(np.isposinf(a), np.isposinf(b)) and np.array_equal(np.isneginf(a), np.isneginf(b)), what
     ok = np.isfinite(b)
     assert np.abs(a[ok] - b[ok]).max() <= 1e-4 * max(1.0, float(np.abs(b[ok]).max())), what
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_terms_that_are_not_finite(gpu, value):
+  """They reach the entries they reach with one wavefront per chain, and the others are what they are there."""
+  problem = _problem(4, 1, 1, 9, 14, 3)
+  problem[2][0, 0, 4, 5, 7] = value
+  _same_where_not_finite(_backward(gpu, problem, 2), _backward(gpu, problem, 0))
 
 
 @pytest.mark.parametrize("n_dir,B,H,W", [(4, 1, 1, 1), (4, 1, 2, 5), (4, 2, 6, 7), (8, 1, 12, 13), (4, 1, 3, 50)])
@@ -95,6 +98,65 @@ def test_soft_backward_against_the_oracle(gpu, oracle, n_dir, B, H, W, pairs):
         assert np.abs(a.cpu().numpy() - b).max() <= 1e-4 * max(1.0, float(np.abs(b).max())), (option, what)
   finally:
     _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+
+
+def _soft_backward(option, dcost, ctx, ew, duals, norm, flags=0, **kw):
+  import torch
+  from mplayers_amd import _lib, lib_stereo
+  up = lambda a: torch.as_tensor(np.ascontiguousarray(a)).cuda()
+  _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+  try:
+    g = up(dcost)
+    got = g.new_zeros(dcost.shape), g.new_zeros(L, L), g.new_zeros(ew.shape)
+    lib_stereo.TRWP_hard_soft.backward_soft(0.5, g, up(ctx), up(ew), up(duals), up(norm), *got,
+                                            g.new_full(ew.shape + (L,), 3.5), g.new_empty(0), flags=flags)
+    return [x.cpu().numpy() for x in got]
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+
+
+@pytest.mark.parametrize("n_dir,B,H,W", [(4, 1, 1, 1), (4, 1, 6, 7), (8, 1, 12, 13), (4, 1, 3, 50)])
+@pytest.mark.parametrize("value", [np.nan, np.inf, 3e38])
+def test_soft_backward_reads_no_duals_of_chain_starts(gpu, oracle, n_dir, B, H, W, value):
+  """The forward scan does not write them (a chain start has no message): whatever is in that memory reaches no
+  gradient, whether the scan has one wavefront per chain or four."""
+  from mplayers_amd import _lib
+  rng = np.random.default_rng(100 * H + W + 2)
+  unary = (0.1 + rng.random((B, 1, H, W, L))).astype(np.float32)
+  ctx = np.triu(rng.random((L, L)), 1).astype(np.float32)
+  ew = (0.2 + rng.random((n_dir, B, 1, H, W))).astype(np.float32)
+  dcost = rng.standard_normal((B, 1, H, W, L)).astype(np.float32)
+  fwd = oracle.forward_soft(unary, ctx, ew, n_dir, 2, 0.5)
+  duals, norm = fwd["msg_edge_label"].astype(np.float32), fwd["msg_norm_index"]
+  ref = oracle.backward_soft(ctx.astype(np.float64), ew.astype(np.float64), dcost.astype(np.float64),
+                             fwd["msg_edge_label"].astype(np.float64), norm, 0.5)
+  starts = (duals == 0).all(axis=(-1, -2))  # (the oracle leaves them at zero; the others are positive)
+  assert starts.any()
+  duals[starts] = value
+  duals[starts, ::2] *= -1
+  for option in (0, 2):
+    for flags in (0, _lib.F_FUSED_PAIRS_OFF):
+      print("case", n_dir, B, H, W, value, option, flags, flush=True)
+      for a, b, what in zip(_soft_backward(option, dcost, ctx, ew, duals, norm, flags), ref,
+                            ("dunary", "dcontext", "dedge_weights")):
+        # sums of at most a few thousand products: 1e-4 of the largest entry, as everywhere
+        assert np.abs(a - b).max() <= 1e-4 * max(1.0, float(np.abs(b).max())), (option, what)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_soft_backward_of_one_pixel(gpu, value):
+  """An image of one pixel has chain starts only: its gradient, finite or not, reaches neither the table nor the
+  edge weights."""
+  rng = np.random.default_rng(5)
+  ctx = np.triu(rng.random((L, L)), 1).astype(np.float32)
+  ew = np.ones((4, 1, 1, 1, 1), np.float32)
+  dcost = rng.standard_normal((1, 1, 1, 1, L)).astype(np.float32)
+  dcost[..., 7] = value
+  for option in (0, 2):
+    print("case", value, option, flush=True)
+    _, dctx, dedge = _soft_backward(option, dcost, ctx, ew, np.zeros((2, 4, 1, 1, 1, 1, L, L), np.float32),
+                                    np.zeros((2, 4, 1, 1, 1, 1), np.uint8))
+    assert not dctx.any() and not dedge.any()
 
 
 @pytest.mark.parametrize("n_dir,B,H,W", [(4, 1, 1, 1), (4, 1, 2, 5), (4, 2, 6, 7), (8, 1, 12, 13), (4, 1, 3, 50)])
