@@ -138,7 +138,10 @@ template <bool DC>
 __device__ __forceinline__ float to_sources(float x, float gw, const f32x4& m0, float (&pairs)[kSrc]) {
   float y;
   if constexpr (DC) {
+    // (a lane operand may be read two issue slots after it was written, and the compiler does not look into
+    // the block for it: the first two instructions leave gw alone)
     asm("v_mov_b32 %1, %0\n\t"
+        "s_nop 0\n\t"
         "v_fmac_f32_dpp %2, %6, %7 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
         "v_fmac_f32_dpp %3, %6, %8 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
         "v_permlane16_swap_b32 %0, %1\n\t"
