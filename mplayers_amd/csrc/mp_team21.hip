@@ -133,23 +133,23 @@ __device__ __forceinline__ void spread_min(float v, float& src, float& nmin) {
 // weight, under the same masks.  Those multiply-adds stand in the issue slots that the exchanges and lane
 // shifts of the recurrence leave idle, the first four of them a pixel late.
 
-// x by label -> by source label
+// x by label -> by source label.  zero: becomes NaN where gw is not finite
 template <bool DC>
-__device__ __forceinline__ float to_sources(float x, float gw, const f32x4& m0, float (&pairs)[kSrc]) {
+__device__ __forceinline__ float to_sources(float x, float gw, const f32x4& m0, float (&pairs)[kSrc], float& zero) {
   float y;
   if constexpr (DC) {
     // (a lane operand may be read two issue slots after it was written, and the compiler does not look into
-    // the block for it: the first two instructions leave gw alone)
+    // the block for it: the first two instructions leave that of gw alone)
     asm("v_mov_b32 %1, %0\n\t"
-        "s_nop 0\n\t"
-        "v_fmac_f32_dpp %2, %6, %7 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f32_dpp %3, %6, %8 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32 %6, 0, %7\n\t"
+        "v_fmac_f32_dpp %2, %7, %8 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %7, %9 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
         "v_permlane16_swap_b32 %0, %1\n\t"
-        "v_fmac_f32_dpp %4, %6, %9 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f32_dpp %5, %6, %10 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %4, %7, %10 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %5, %7, %11 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
         "v_mov_b32_dpp %0, %0 row_shl:11 row_mask:0xc bank_mask:0xf\n\t"
         "v_mov_b32_dpp %0, %1 row_shr:5 row_mask:0xc bank_mask:0xf"
-        : "+&v"(x), "=&v"(y), "+&v"(pairs[0]), "+&v"(pairs[1]), "+&v"(pairs[2]), "+&v"(pairs[3])
+        : "+&v"(x), "=&v"(y), "+&v"(pairs[0]), "+&v"(pairs[1]), "+&v"(pairs[2]), "+&v"(pairs[3]), "+&v"(zero)
         : "v"(gw), "v"(m0[0]), "v"(m0[1]), "v"(m0[2]), "v"(m0[3]));
   } else {
     asm("v_mov_b32 %1, %0\n\t"
@@ -587,15 +587,17 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       x.b = *reinterpret_cast<const f32x2*>(s.base[i][sl]);
       return x;
     };
-    // A block of pixels whose gradients are not all finite, one after another: a zero mask does not switch
-    // such a term off, so the gradients go to their labels through LDS.
+    // A block of pixels whose gradients, or their products with the edge weight, are not all finite, one after
+    // another: a zero mask does not switch such a term off, so the gradients go to their labels through LDS.
+    // (What the normalisation takes off stays a term of its own: where the weight is not finite, that entry of
+    // dcontext can be NaN here and infinite with one wavefront per chain.)
     auto careful_block = [&](BwdSlots& s, const int k) __attribute__((always_inline)) {
 #pragma clang loop unroll(disable)
       for (int i = 0; i < kT; ++i) {
         const In cur = get(s, i);
         s.sc[i][l] = sc;
-        float none[kSrc];
-        const float g = fmaf(rho, to_sources<false>(sc, 0.f, cur.m[0], none), cur.b[0]);
+        float none[kSrc], nothing;
+        const float g = fmaf(rho, to_sources<false>(sc, 0.f, cur.m[0], none, nothing), cur.b[0]);
         if (src_mask != 0 && (lane & 16) == 0) atomicAdd(&acc[s.fd[i][sl]], g);
         lds_order();
         sc = acc[l];
@@ -627,7 +629,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
         BwdSlots& s = sets[(k - 1) & 1];
         In cur = get(s, 0);
         const float sc_was = sc;
-        float pairs_were[kSrc];
+        float pairs_were[kSrc], zero = 0.f;
         if (DC) {
           static_for<4>([&](auto ii) __attribute__((always_inline)) {
             constexpr int q = decltype(ii)::value;
@@ -644,7 +646,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
           s.sc[i][l] = sc;
           // gradient w.r.t. the normalised message of this pixel, including what the previous step
           // added through the recurrence (dmsg[front] += rho * value, TRWP_backward.cu:108)
-          float g = fmaf(rho, to_sources<DC>(sc, gw, m0, pairs), cur.b[0]);
+          float g = fmaf(rho, to_sources<DC>(sc, gw, m0, pairs, zero), cur.b[0]);
           // The chain start has no message, and neither have the places of the block past it: without a gradient
           // there, the sums and dcontext stay what they are (a zero weight would not do: zero times what is
           // not finite)
@@ -666,7 +668,14 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
         // (tested as an integer: the compiler may take NaN for anything)
         int probe = SOFT ? 0 : uniform_i(bits(sc));
         asm("" : "+s"(probe));
-        if (!SOFT && __builtin_expect((probe & 0x7f800000) == 0x7f800000, 0)) {
+        bool odd_sums = !SOFT && (probe & 0x7f800000) == 0x7f800000;
+        if constexpr (!SOFT && DC) {
+          // ... and so does one in a gradient times the edge weight with the pairs' sums (an integer, again)
+          int z = bits(zero);
+          asm("v_fmac_f32 %0, 0, %1" : "+v"(z) : "v"(gw));
+          odd_sums |= ballot(z != 0) != 0;
+        }
+        if (!SOFT && __builtin_expect(odd_sums, 0)) {
           sc = sc_was;
           if (DC) {
             gw = 0.f;

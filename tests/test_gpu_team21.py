@@ -69,6 +69,23 @@ def test_terms_that_are_not_finite(gpu, value):
   _same_where_not_finite(_backward(gpu, problem, 2), _backward(gpu, problem, 0))
 
 
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 1e38])
+@pytest.mark.parametrize("y,x", [(4, 5), (0, 0), (8, 13), (4, 12)])
+def test_edge_weights_that_are_not_finite(gpu, value, y, x):
+  """The same for an edge weight, and for one whose product with a gradient overflows: only dcontext has it as
+  a factor, in the entries that the argmin labels of its pixel point at."""
+  problem = _problem(4, 1, 1, 9, 14, 4)
+  problem[1][:, 0, 0, y, x] = value
+  if np.isfinite(value):
+    problem[2][0, 0, y, x] *= 1e10
+  one, four = _backward(gpu, problem, 0), _backward(gpu, problem, 2)
+  bad = ~np.isfinite(one[1])
+  assert bad.any() and not bad.all()
+  assert np.array_equal(~np.isfinite(four[1]), bad)
+  four[1][bad] = one[1][bad]  # (infinities that meet in another order)
+  _same_where_not_finite(four, one)
+
+
 @pytest.mark.parametrize("n_dir,B,H,W", [(4, 1, 1, 1), (4, 1, 2, 5), (4, 2, 6, 7), (8, 1, 12, 13), (4, 1, 3, 50)])
 @pytest.mark.parametrize("pairs", [True, False])
 def test_soft_backward_against_the_oracle(gpu, oracle, n_dir, B, H, W, pairs):
