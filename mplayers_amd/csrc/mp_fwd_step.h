@@ -208,7 +208,9 @@ __device__ __forceinline__ void dense1d_argmin(const float (&v)[R], const int (&
   constexpr int T = dense_trip<R>();
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const int t0 = trip0[j];
+    // (no trip is noted where no candidate is a number, and no label found there: the last one, as the
+    // reference's scan has it)
+    const int t0 = max(trip0[j], 0);
     const int l = lab0 + j < L ? lab0 + j : L - 1;
     float af[T];
 #pragma unroll
@@ -218,14 +220,14 @@ __device__ __forceinline__ void dense1d_argmin(const float (&v)[R], const int (&
       for (int i = 0; i < 4; ++i) af[4 * q + i] = x[i];
     }
     const float* cp = csym_s + (dense_sym_centre<R>() + l - t0 - (T - 1));  // entry of front label t0 + T - 1
-    int arg = 0;
+    int arg = kMaxL;
 #pragma unroll
     for (int u = 0; u < T; ++u) {
       const float val = fmaf(w, cp[T - 1 - u], af[u]);
       arg = val == v[j] ? u : arg;
     }
     const int fd = t0 + arg;
-    fd_idx[j] = fd < L ? fd : L - 1;  // (only where no candidate is finite)
+    fd_idx[j] = fd < L ? fd : L - 1;
   }
 }
 

@@ -109,3 +109,23 @@ def test_tables_declared_dense(gpu, L, training):
         assert np.abs(four["cost_final"] - one["cost_final"]).max() <= 1e-5 * max(1.0, np.abs(one["cost_final"]).max())
       else:
         _same(four, one, training)
+
+
+@pytest.mark.parametrize("L", [2, 7, 8, 33, 64, 65, 96, 130, 192, 256])
+@pytest.mark.parametrize("mode", ["TRWP", "ISGMR"])
+def test_argmin_labels_exist_where_no_candidate_is_a_number(gpu, L, mode):
+  """An edge weight that is NaN leaves a dense table's scan without a candidate to compare: whichever label is kept,
+  it is one, and the reverse scan does not look outside its tables for it."""
+  from mplayers_amd import _lib
+  unary, ctx, ew = _problem(4, 1, 7, 9, L, "random", 9)
+  ew[:, 0, 0, 3, 4] = np.nan
+  for option, flags in ((0, 0), (2, 0), (2, _lib.F_DENSE_TABLE)):
+    print("case", L, mode, option, flags, flush=True)
+    _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+    try:
+      got = _forward_flags(gpu, mode, unary, ctx, ew, 4, 2, 0.5 if mode == "TRWP" else 1.0, True,
+                           flags | _lib.F_PACKED_OFF)
+    finally:
+      _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+    assert got["msg_min_index"].max() < L and got["msg_norm_index"].max() < L
+    assert not np.isfinite(got["msg"][:, 0, 0, 3, 4]).any()
