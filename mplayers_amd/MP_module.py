@@ -161,6 +161,21 @@ class ISGMRFunction(torch.autograd.Function):
             buf["dedge_weights"] if need_edge_weights else None, None)
 
 
+def _entries(place):
+  """`place` as an index that numpy reads as torch does, None for one that it may read otherwise (bytes, which
+  torch takes as a mask, floats and short integers, negative steps, lists of lists) and for tensors."""
+  if isinstance(place, tuple):
+    parts = tuple(None if isinstance(part, tuple) else _entries(part) for part in place)
+    return None if any(part is None for part in parts) else parts
+  if isinstance(place, range) or (isinstance(place, list) and all(type(i) is int for i in place)):
+    return np.array(place, np.int64)
+  if isinstance(place, np.ndarray):
+    return place if place.dtype in (np.bool_, np.int32, np.int64) else None
+  if isinstance(place, slice):
+    return place if place.step is None or place.step > 0 else None
+  return place if type(place) is int else None
+
+
 class MPModule(torch.nn.Module):
   """nn.Module wrapper (MP_module.py:164-234).
 
@@ -212,18 +227,15 @@ class MPModule(torch.nn.Module):
 
   def _location_masks(self, label_context):
     """Masks of label_context_loc and label_context_diag_loc on the table's device, None where a location is
-    a tensor or not a list of different entries.  They are formed on the host from the locations of the moment
-    and copied only when they differ from what was copied last."""
+    not a list of different entries that numpy reads as torch does, or more than one value is pinned.  They are
+    formed on the host from the locations of the moment and copied only when they differ from what was copied last."""
     diag = self.label_context_diag_loc
-    places = [self.label_context_loc, tuple(diag) if isinstance(diag, list) else diag]
-    parts = [part for place in places for part in (place if isinstance(place, tuple) else (place,))]
-    if any(isinstance(part, torch.Tensor) for part in parts):
+    places = [_entries(self.label_context_loc), _entries(tuple(diag) if isinstance(diag, list) else diag)]
+    if any(place is None for place in places) or not isinstance(self.args.mpnet_diag_value, (int, float)):
       return None
     host = []
-    for place in places:
+    for index in places:
       mask = np.zeros(label_context.shape, bool)
-      as_array = lambda x: np.asarray(x) if isinstance(x, (list, range)) else x
-      index = tuple(map(as_array, place)) if isinstance(place, tuple) else as_array(place)
       taken = mask[index]
       if not host and np.ndim(taken) != 1:
         return None  # (what takes the values back entry by entry is one-dimensional)

@@ -29,6 +29,13 @@ LOCATIONS = {
     "two names of one entry": ([-1, 4], [0], 1),
     "repeated, 2-D": ((np.array([0, 0, 1]), np.array([1, 1, 2])), [range(5), range(5)], 2),
     "pinned twice": ([1, 3], [[0, 0, -5]], 1),
+    "no entry": ([], [0], 1),
+    "empty range": (range(1, 1), [0], 1),
+    "bytes as a mask": (np.array([0, 1, 1, 0, 0], np.uint8), [0], 1),
+    "booleans": (np.array([False, True, True, False, False]), [True, False, False, False, False], 1),
+    "floats": (np.array([1., 2.]), [0], 1),
+    "rows": (np.triu_indices(5, k=1), np.array([[0, 1], [2, 3]]), 2),
+    "all": ([1, 3], Ellipsis, 1),
 }
 
 
@@ -94,3 +101,21 @@ def test_locations_that_are_refused_stay_refused():
   module.set_label_context(torch.nn.Parameter(torch.rand(5)), [7], [0])
   with pytest.raises(IndexError):
     module._effective_label_context()
+  for loc, diag, error in ((slice(None, None, -1), [0], ValueError), ([1, 3], slice(2, None, -1), ValueError),
+                           ([1, 3], np.array([1, 0, 0, 0, 1], np.uint8), RuntimeError),
+                           (np.array([1, 3], np.int16), [0], IndexError)):
+    module.set_label_context(torch.nn.Parameter(torch.rand(5)), loc, diag)
+    with pytest.raises(error):
+      module._effective_label_context()
+
+
+@pytest.mark.parametrize("value", [1, 0.25, True, np.float64(0.5), torch.tensor(0.5), torch.tensor([0.5]),
+                                   torch.arange(5.)])
+def test_pinned_values(value):
+  """One number, or a tensor that indexing spreads over the pinned entries."""
+  _check(_module(*LOCATIONS["triangle"], mpnet_diag_value=value))
+
+
+def test_a_pinned_value_that_is_refused_stays_refused():
+  with pytest.raises(TypeError):
+    _module(*LOCATIONS["triangle"], mpnet_diag_value=np.float32(0.5))._effective_label_context()
