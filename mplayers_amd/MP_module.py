@@ -176,6 +176,15 @@ def _entries(place):
   return place if type(place) is int else None
 
 
+def _runs_now(tensor):
+  """Whether operations on `tensor` run as they are called: no trace, transform, dispatch mode or stream capture
+  that could hold on to a tensor kept between calls, or leave one of its own in its place."""
+  return (type(tensor) is torch.Tensor and torch._C._len_torch_dispatch_stack() == 0 and
+          torch._C._functorch.peek_interpreter_stack() is None and not torch.jit.is_tracing() and
+          not torch.compiler.is_compiling() and
+          not (tensor.is_cuda and torch.cuda.is_current_stream_capturing()))
+
+
 class MPModule(torch.nn.Module):
   """nn.Module wrapper (MP_module.py:164-234).
 
@@ -227,8 +236,11 @@ class MPModule(torch.nn.Module):
 
   def _location_masks(self, label_context):
     """Masks of label_context_loc and label_context_diag_loc on the table's device, None where a location is
-    not a list of different entries that numpy reads as torch does, or more than one value is pinned.  They are
-    formed on the host from the locations of the moment and copied only when they differ from what was copied last."""
+    not a list of different entries that numpy reads as torch does, or more than one value is pinned, and in
+    traces, transforms and captures.  They are formed on the host from the locations of the moment and copied
+    only when they differ from what was copied last."""
+    if not _runs_now(label_context):
+      return None
     diag = self.label_context_diag_loc
     places = [_entries(self.label_context_loc), _entries(tuple(diag) if isinstance(diag, list) else diag)]
     if any(place is None for place in places) or not isinstance(self.args.mpnet_diag_value, (int, float)):
@@ -250,8 +262,7 @@ class MPModule(torch.nn.Module):
       # mode could not be saved for a later call's backward pass)
       with torch.inference_mode(False):
         kept = (key,) + tuple(torch.from_numpy(mask).to(label_context.device) for mask in host)
-      if not (label_context.is_cuda and torch.cuda.is_current_stream_capturing()):
-        self._kept_masks = kept
+      self._kept_masks = kept
     return kept[1:]
 
   def _effective_label_context(self, weight_first=False):

@@ -119,3 +119,52 @@ def test_pinned_values(value):
 def test_a_pinned_value_that_is_refused_stays_refused():
   with pytest.raises(TypeError):
     _module(*LOCATIONS["triangle"], mpnet_diag_value=np.float32(0.5))._effective_label_context()
+
+
+def _fake(f, table):
+  from torch._subclasses.fake_tensor import FakeTensorMode
+  with FakeTensorMode(allow_non_fake_inputs=True):
+    f(table)
+
+
+def _export(f, table):
+  module = type("Module", (torch.nn.Module,), dict(forward=lambda self, x: f(x)))()
+  return torch.export.export(module, (table,)).module()(2 * table)
+
+
+def _make_fx(f, table):
+  from torch.fx.experimental.proxy_tensor import make_fx
+  return make_fx(f)(table)(2 * table)
+
+
+TRANSFORMS = {
+    "fake tensors": _fake, "export": _export, "make_fx": _make_fx,
+    "trace": lambda f, table: torch.jit.trace(f, (table,), check_trace=False)(2 * table),
+    "vmap": lambda f, table: torch.func.vmap(f)(torch.stack([2 * table, table]))[0],
+    "vmap of others": lambda f, table: torch.func.vmap(lambda x: f(2 * table) * x)(torch.ones(3, 1, 1))[1],
+    "jvp": lambda f, table: torch.func.jvp(f, (2 * table,), (table,))[0],
+    "grad of others": lambda f, table: torch.func.grad(lambda x: (f(2 * table) * x).sum())(torch.ones(5, 5)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(TRANSFORMS))
+@pytest.mark.parametrize("warm", [False, True])
+def test_traces_and_transforms(name, warm):
+  """They see the table's own values, take nothing that another call kept, and leave nothing behind for the next."""
+  loc, diag, _ = LOCATIONS["triangle"]
+  table = torch.randn(5, 5, generator=torch.Generator().manual_seed(3))
+  module = _module(loc, diag, 2)
+  if warm:
+    module._effective_label_context()
+  parameter = module.label_context
+  del module.label_context
+
+  def effective(x):
+    module.label_context = x
+    return module._effective_label_context()
+
+  got = TRANSFORMS[name](effective, table)
+  if got is not None:
+    assert torch.equal(got, _by_index(2 * table, loc, diag, 1.5, False, 0.25))
+  module.label_context = parameter
+  _check(module)
