@@ -256,14 +256,19 @@ class MPModule(torch.nn.Module):
         return None  # (an entry named twice has its gradient twice)
       host.append(mask)
     key = (label_context.device, label_context.shape) + tuple(mask.tobytes() for mask in host)
+    stream = torch.cuda.current_stream(label_context.device) if label_context.is_cuda else None
     kept = getattr(self, "_kept_masks", None)
     if kept is None or kept[0] != key:
       # (copies from pageable memory are complete when they return, for every stream; tensors of inference
       # mode could not be saved for a later call's backward pass)
       with torch.inference_mode(False):
-        kept = (key,) + tuple(torch.from_numpy(mask).to(label_context.device) for mask in host)
+        kept = (key, stream, [torch.from_numpy(mask).to(label_context.device) for mask in host])
       self._kept_masks = kept
-    return kept[1:]
+    if stream != kept[1]:
+      # (their memory goes back to the stream they were formed on when other locations take their place)
+      for mask in kept[2]:
+        mask.record_stream(stream)
+    return kept[2]
 
   def _effective_label_context(self, weight_first=False):
     """Re-parameterisation of the learned context (MP_module.py:207-220).  weight_first: the term

@@ -168,3 +168,28 @@ def test_traces_and_transforms(name, warm):
     assert torch.equal(got, _by_index(2 * table, loc, diag, 1.5, False, 0.25))
   module.label_context = parameter
   _check(module)
+
+
+@pytest.mark.gpu
+def test_masks_on_another_stream(gpu, monkeypatch):
+  """A call on another stream than the one the masks were formed on holds their memory until it is through, also
+  when other locations have taken their place."""
+  loc, diag, _ = LOCATIONS["triangle"]
+  table = torch.nn.Parameter(torch.randn(5, 5, generator=torch.Generator().manual_seed(3)).cuda())
+  module = _module(loc, diag, 2)
+  module.label_context = table
+  held = []
+  record = torch.Tensor.record_stream
+  monkeypatch.setattr(torch.Tensor, "record_stream", lambda self, stream: (held.append(stream), record(self, stream)))
+  first = module._effective_label_context()
+  assert not held
+  side = torch.cuda.Stream()
+  side.wait_stream(torch.cuda.current_stream())
+  with torch.cuda.stream(side):
+    second = module._effective_label_context()
+  assert held == [side, side]
+  module.set_label_context(table, (np.array([0]), np.array([1])), diag)
+  module._effective_label_context()
+  torch.cuda.synchronize()
+  want = _by_index(table.detach().cpu(), loc, diag, 1.5, False, 0.25)
+  assert torch.allclose(first.detach().cpu(), want) and torch.equal(first, second)
