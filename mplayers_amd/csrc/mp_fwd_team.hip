@@ -112,11 +112,10 @@ __device__ __forceinline__ void lds_barrier() {
 template <int R, int KT>
 struct StepCtx {
   int L, lab0, lane, K;
-  bool full_table;            // ctx_s holds the (L, L) table (2-D)
+  bool full_table;            // ctx_s holds the (L, L) table (2-D; 21 labels: mp_team21.hip)
   float cmax, slope;
   float floor_l[R];           // -inf, +inf where the lane's label does not exist
   float c_reg[KT > 0 ? KT : 1];
-  float tcol[KT == -21 ? 21 : 1];
   float cv0[R];               // dense 1-D table: c[label]
   float* a_w;                 // this wavefront's scratch, kMaxL floats
   const float* ctx_s;
@@ -180,28 +179,8 @@ __device__ __forceinline__ void team_step(const StepCtx<R, KT>& c, const float (
         nmin = norm_min();
     }
   } else if (R == 1 && KT < 0 && c.full_table) {
-    if constexpr (KT == -21) {
-      float af[21], val[21];
-#pragma unroll
-      for (int fd = 0; fd < 21; ++fd) af[fd] = readlane_f(a[0], fd);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int fd = 0; fd < 21; ++fd) val[fd] = fmaf(wv, c.tcol[fd], af[fd]);
-      float best = val[20];
-#pragma unroll
-      for (int fd = 19; fd >= 1; fd -= 2) best = fminf(fminf(val[fd], val[fd - 1]), best);
-      v[0] = best;
-      if (TRAIN) {
-        float red = fmaxf(best, c.floor_l[0]);
-        argmin_and_lane_min_21(val, best, red, fd_idx[0]);
-        nmin = readlane_f(red, 31);
-      } else {
-        nmin = norm_min();
-      }
-    } else {
-      dense_step_r1<TRAIN>(a[0], L, uniform_f(wv), c.lane, c.ctx_s, v[0], fd_idx[0]);
-      nmin = norm_min();
-    }
+    dense_step_r1<TRAIN>(a[0], L, uniform_f(wv), c.lane, c.ctx_s, v[0], fd_idx[0]);
+    nmin = norm_min();
   } else {
     const float w = uniform_f(wv);
     if constexpr (kDenseMain) {
@@ -259,10 +238,6 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
   if constexpr (KT > 0) {
 #pragma unroll
     for (int k = 0; k < KT; ++k) c.c_reg[k] = p.ctx[k];
-  }
-  if constexpr (KT == -21) {
-#pragma unroll
-    for (int fd = 0; fd < 21; ++fd) c.tcol[fd] = ctx_s[fd * 21 + (lane < 21 ? lane : 20)];
   }
   if constexpr (KT == -1) {
 #pragma unroll
@@ -579,13 +554,7 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
     return;
   }
   switch (desc.band_k) {
-    case 0:
-      if (R == 1 && L == 21 && p.ctx2d) {
-        MPL_WALK((R == 1 ? -21 : -1), false);
-      } else {
-        MPL_WALK(-1, false);
-      }
-      break;
+    case 0: MPL_WALK(-1, false); break;
     case 1: MPL_WALK(1, true); break;
     case 2: MPL_WALK(2, true); break;
     case 3: MPL_WALK(3, true); break;

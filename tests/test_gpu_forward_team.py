@@ -129,3 +129,36 @@ def test_argmin_labels_exist_where_no_candidate_is_a_number(gpu, L, mode):
       _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
     assert got["msg_min_index"].max() < L and got["msg_norm_index"].max() < L
     assert not np.isfinite(got["msg"][:, 0, 0, 3, 4]).any()
+
+
+@pytest.mark.parametrize("L,ctx2d", [(2, 1), (20, 1), (22, 1), (33, 1), (64, 1), (21, 0)])
+@pytest.mark.parametrize("training", [True, False])
+def test_tables_the_operators_do_not_pass(gpu, L, ctx2d, training):
+  """2-D tables of other label counts than 21, and 21 labels with a 1-D one, which the library takes."""
+  import torch
+  from mplayers_amd import _lib
+  rng = np.random.default_rng(L)
+  n_dir, n_iter, shape = 4, 2, (1, 1, 9, 14, L)
+  table = np.triu(rng.random((L, L)), 1) if ctx2d else rng.random(L)
+  unary, ctx, ew = gpu._t(3 * rng.random(shape)), gpu._t(table), gpu._t(rng.random((n_dir,) + shape[:4]) - 0.1)
+  out = []
+  for option in (0, 2):
+    msg, cost, scratch = unary.new_zeros((n_dir,) + shape), torch.zeros_like(unary), torch.zeros_like(unary)
+    u8 = dict(dtype=torch.uint8, device=unary.device)
+    imin = torch.zeros((n_iter, n_dir) + shape, **u8)
+    inorm, label = torch.zeros((n_iter, n_dir) + shape[:4], **u8), torch.zeros((n_iter,) + shape[:4], **u8)
+    ptr = lambda t: t.data_ptr()
+    print("case", L, ctx2d, training, option, flush=True)
+    _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+    try:
+      rc = _lib.load().mpl_trwp_forward(_lib.Shape(n_dir, 1, 9, 14, L, ctx2d), _lib.F_PACKED_OFF, 0.5, n_iter, 0,
+                                        ptr(unary), ptr(ctx), ptr(ew), ptr(msg), ptr(cost), ptr(imin) if training else None,
+                                        ptr(inorm) if training else None, ptr(scratch), ptr(label), None)
+      torch.cuda.synchronize()
+    finally:
+      _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+    _lib.check(rc, "trwp_forward")
+    out.append([t.cpu().numpy() for t in (msg, cost, imin, inorm, label)])
+  assert out[0][0].any() and (not training or out[0][2].any())
+  for a, b in zip(*out):
+    assert np.array_equal(a, b)
