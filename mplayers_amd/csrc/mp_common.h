@@ -457,10 +457,13 @@ __device__ __forceinline__ int xcd_block(int block, int blocks, int group) {
   return base + (r % kXcds) * group + r / kXcds;
 }
 
-// which (direction, batch item, chain) a workgroup owns
-template <typename Params>
+// which (direction, batch item, chain) a workgroup owns.  GROUPS false: the soft-weighted scans of mp_soft.hip,
+// which are bound by their exponentials and their blocks of duals; the groups brought them nothing, and the
+// instructions in front of their loops cost 5 % of the forward scan of 33 to 64 labels (48 labels 46x54, batch
+// 2: 2192 -> 2316 us) and 1 % of the reverse scans of up to 32.
+template <bool GROUPS = true, typename Params>
 __device__ __forceinline__ ChainCtx locate_chain(const Params& p) {
-  const int block = xcd_block((int)blockIdx.x, (int)gridDim.x, p.xcd_group);
+  const int block = GROUPS ? xcd_block((int)blockIdx.x, (int)gridDim.x, p.xcd_group) : (int)blockIdx.x;
   int di = 0;
   while (di + 1 < p.n_dirs && block >= p.block_prefix[di + 1]) ++di;
   const int dir = p.dirs[di];

@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(kWave) soft_fwd_kernel(const SweepParams p) {
   float* tab = smem;        // LL floats
   float* tile = smem + LL;  // max(LL, 64 * T) floats: the pixel's block of duals
   const int lane = threadIdx.x;
-  const ChainCtx ch = locate_chain(p);
+  const ChainCtx ch = locate_chain<false>(p);
   if (ch.n < 2) return;  // nothing to write
   fill_table(p.ctx, L, p.ctx2d, lane, tab);
   __syncthreads();
@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(kWave) soft_bwd_kernel(const BackParams p) {
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t P = (int64_t)p.B * HW;
   const int64_t N = P * L;
-  const ChainCtx ch = locate_chain(p);
+  const ChainCtx ch = locate_chain<false>(p);
   const int dir = ch.dir;
   const int n = ch.n;
 
@@ -479,7 +479,7 @@ __global__ void __launch_bounds__(kWave) soft_split_fwd_kernel(const SweepParams
   float* tile = smem;              // 256 * NT4 floats (training): the pixel's block as it is stored
   float* tab = smem + (TRAIN ? 256 * NT4 : 0);  // LL floats (training: and a spare word per lane)
   const int lane = threadIdx.x;
-  const ChainCtx ch0 = locate_chain(p);
+  const ChainCtx ch0 = locate_chain<false>(p);
   if (ch0.n < 2) return;  // nothing to write
   fill_table(p.ctx, L, p.ctx2d, lane, tab);
   __syncthreads();
@@ -689,7 +689,7 @@ __global__ void __launch_bounds__(kWave) soft_split_bwd_kernel(const BackParams 
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t P = (int64_t)p.B * HW;
   const int64_t N = P * L;
-  const ChainCtx ch0 = locate_chain(p);
+  const ChainCtx ch0 = locate_chain<false>(p);
   const int n = ch0.n;
 
   fill_table(p.ctx, L, p.ctx2d, lane, tab);
@@ -981,7 +981,7 @@ __global__ void __launch_bounds__(kWave) soft_wide_fwd_kernel(const SweepParams 
   float* ctx_s = a_s + kMaxL;     // kMaxL
   float* tile = ctx_s + kMaxL;    // L * kTs (training, odd directions)
   const int lane = threadIdx.x;
-  const ChainCtx ch = locate_chain(p);
+  const ChainCtx ch = locate_chain<false>(p);
   if (ch.n < 2) return;  // nothing to write
   for (int i = lane; i < L; i += kWave) ctx_s[i] = p.ctx[i];
   __syncthreads();
@@ -1121,7 +1121,7 @@ __global__ void __launch_bounds__(kWave) soft_wide_bwd_kernel(const BackParams p
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t P = (int64_t)p.B * HW;
   const int64_t N = P * L;
-  const ChainCtx ch = locate_chain(p);
+  const ChainCtx ch = locate_chain<false>(p);
   const int dir = ch.dir;
   const bool even = (dir & 1) == 0;
   const int n = ch.n;
