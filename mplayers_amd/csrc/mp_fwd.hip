@@ -385,7 +385,7 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
         } else {
           nmin = norm_min();
         }
-      } else if (R == 1 && KT < 0 && p.ctx2d) {  // (the full table is in LDS then)
+      } else if (R == 1 && KT < 0 && (p.ctx2d || (KT == -1 && L < kSlidingMinL))) {  // (the full table is in LDS then)
         if constexpr (LT > 0) {
           // 21 labels: the scan over front labels fully unrolled, context column in registers.
           // The edge weight stays in a vector register (every lane loaded the same one): a[fd]
@@ -561,7 +561,7 @@ __global__ void __launch_bounds__(kWave) sweep_fwd_kernel(const SweepParams p) {
     desc.slope = 0.f;
   }
   // context table into LDS (dense path, run-time band taps, negative-weight fallback)
-  if (R == 1 && p.ctx2d) {
+  if (R == 1 && (p.ctx2d || (is_dense(desc) && L < kSlidingMinL))) {
     // full symmetric table for dense_step_r1: tab[fd * L + cd] = ctx(cd, fd), TRWP_forward.cu:101-113
     for (int i = lane; i < L * L; i += kWave) {
       const int fd = i / L, cd = i - fd * L;

@@ -112,7 +112,7 @@ __device__ __forceinline__ void lds_barrier() {
 template <int R, int KT>
 struct StepCtx {
   int L, lab0, lane, K;
-  bool full_table;            // ctx_s holds the (L, L) table (2-D; 21 labels: mp_team21.hip)
+  bool full_table;            // ctx_s holds the (L, L) table (2-D, or few labels; 21 labels: mp_team21.hip)
   float cmax, slope;
   float floor_l[R];           // -inf, +inf where the lane's label does not exist
   float c_reg[KT > 0 ? KT : 1];
@@ -224,7 +224,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
   c.lab0 = lab0;
   c.lane = lane;
   c.K = desc.band_k;
-  c.full_table = R == 1 && p.ctx2d;
+  c.full_table = R == 1 && (p.ctx2d || (KT == -1 && L < kSlidingMinL));
   c.cmax = desc.cmax;
   asm volatile("" : "+v"(c.cmax));
   c.slope = desc.slope;
@@ -525,7 +525,7 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
     desc.slope = 0.f;
   }
   if (p.skip_dense && is_dense(desc)) return;  // (mp_fwd_dense.hip runs such a launch)
-  if (R == 1 && p.ctx2d) {
+  if (R == 1 && (p.ctx2d || (is_dense(desc) && L < kSlidingMinL))) {
     for (int i = tid; i < L * L; i += kTeam) {
       const int fd = i / L, cd = i - fd * L;
       const int lo = cd < fd ? cd : fd, hi = cd < fd ? fd : cd;

@@ -162,3 +162,26 @@ def test_tables_the_operators_do_not_pass(gpu, L, ctx2d, training):
   assert out[0][0].any() and (not training or out[0][2].any())
   for a, b in zip(*out):
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("L", [3, 7, 8, 9])
+@pytest.mark.parametrize("mode", ["TRWP", "ISGMR"])
+@pytest.mark.parametrize("option", [0, 2])
+def test_dense_tables_of_few_labels(gpu, oracle, L, mode, option):
+  """Both sides of the label count from which a dense 1-D table is scanned with sliding entries, one and four
+  wavefronts per chain, against the oracle."""
+  from mplayers_amd import _lib
+  unary, ctx, ew = _problem(4, 1, 9, 14, L, "random", 2, negative=True)
+  rho = 0.5 if mode == "TRWP" else 1.0
+  print("case", L, mode, option, flush=True)
+  ref = oracle.forward(mode, unary, ctx, ew, 4, 2, rho)
+  _lib.set_option(_lib.OPT_TEAM_SCANS, option)
+  try:
+    got = _forward_flags(gpu, mode, unary, ctx, ew, 4, 2, rho, True, _lib.F_PACKED_OFF)
+  finally:
+    _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
+  scale = float(np.abs(ref["cost_final"]).max())
+  for k in ("msg", "cost_final"):
+    assert np.abs(got[k] - ref[k]).max() <= 1e-5 * scale, k
+  # (labels whose candidates are closer than that aside)
+  assert (got["msg_min_index"] != ref["msg_min_index"]).mean() <= 1e-3
