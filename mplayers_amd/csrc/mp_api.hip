@@ -747,8 +747,10 @@ int decide_team(const BackParams& p, const CallOpts& o, bool jacobi) {
   if (p.ctx2d || p.L <= kWave) return 0;
   if (o.team == 2) return 1;
   const int cus = launch_policy().n_simd / 4;
-  // (a Jacobi launch holds every direction; its lines were measured in chains of all of them)
-  const int chains = jacobi ? p.block_prefix[p.n_dirs] : chains_at_once(p);
+  // (A Jacobi launch holds every direction; its lines were measured in chains of all of them.  With four labels
+  // per lane the LDS holds two workgroups of a unit and every chain counts, however early it ends: 200 labels
+  // 32x34, batch 12, 8 directions, min(k, 14)^2, 780 diagonals, all directions 0.69 ms so, 0.74 by chains_at_once.)
+  const int chains = jacobi || labels_per_lane(p.L) == 4 ? p.block_prefix[p.n_dirs] : chains_at_once(p);
   return chains <= team_chains_per_cu(p.L, jacobi) * cus ? 1 : 0;
 }
 

@@ -277,7 +277,7 @@ __device__ __forceinline__ void lds_order() {  // of this wavefront's own LDS in
 
 // GR: dedge_weights and / or dcontext are wanted
 template <int R, bool VEC, bool JACOBI, bool GR>
-__global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams p) {
+__global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams p, const int turn_every) {
   extern __shared__ __align__(16) char smem_raw[];
   Slot<R>* slots = reinterpret_cast<Slot<R>*>(smem_raw);  // two sets of kT
   Scalars* scal = reinterpret_cast<Scalars*>(slots + 2 * kT);
@@ -291,7 +291,8 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
   // The last wavefront is the main one in every workgroup: the wavefronts of the workgroups that a compute
   // unit gets one after another start one SIMD further each (read from the hardware-id registers for 2, 3
   // and 4 workgroups per unit), so the main wavefronts of up to four of them are on SIMDs of their own.
-  const int role = uniform_i(tid / kWave);  // kHelpers: main
+  // turn_every > 0 (launch_vj): it moves on by one every so many workgroups.
+  const int role = uniform_i((tid / kWave + (turn_every > 0 ? (int)blockIdx.x / turn_every : 0)) & 3);  // kHelpers: main
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t P = (int64_t)p.B * HW;
   const int64_t N = P * L;
@@ -703,10 +704,17 @@ void launch_vj(const BackParams& p, hipStream_t st) {
   const bool gr = p.dedge != nullptr || p.dctx != nullptr;
   const size_t lds = 2 * kT * (sizeof(Slot<R>) + sizeof(Scalars)) +
                      sizeof(float) * (kAccFloats + (gr ? p.L + kHelpers * hist_floats(R, p.L) : 0));
+  // With four labels per lane the LDS holds two workgroups of a unit, and a launch of more runs in rounds.  When
+  // both end together the next ones are placed in pairs again and the last round takes as long as the first;
+  // with the main wavefronts of a unit's workgroups on one SIMD they do not.  Measured, 760 rows of 300 pixels,
+  // 2 iterations, ms on SIMDs of their own / on one: 256 labels, min(k, 4) 1.38 / 1.25, linear 3.07 / 2.50, random 3.38 / 2.75;
+  // 500 rows 0.710 / 0.723, 1.55 / 1.60, 1.72 / 1.78.
+  const int n_cu = launch_policy().n_simd / 4;
+  const int turn_every = R == 4 && blocks > 2 * n_cu ? n_cu : 0;
   if (gr)
-    sweep_bwd_team_kernel<R, VEC, JACOBI, true><<<blocks, kTeam, lds, st>>>(p);
+    sweep_bwd_team_kernel<R, VEC, JACOBI, true><<<blocks, kTeam, lds, st>>>(p, turn_every);
   else
-    sweep_bwd_team_kernel<R, VEC, JACOBI, false><<<blocks, kTeam, lds, st>>>(p);
+    sweep_bwd_team_kernel<R, VEC, JACOBI, false><<<blocks, kTeam, lds, st>>>(p, turn_every);
 }
 
 }  // namespace
