@@ -1369,7 +1369,6 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
 
   BackParams p;
   memset(&p, 0, sizeof(p));
-  p.xcd_group = xcd_group_size(s->n_disp);
   p.B = s->batch;
   p.H = s->height;
   p.W = s->width;
@@ -1438,7 +1437,6 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
 
   BackParams p;
   memset(&p, 0, sizeof(p));
-  p.xcd_group = xcd_group_size(s->n_disp);
   p.B = s->batch;
   p.H = s->height;
   p.W = s->width;
@@ -1560,7 +1558,6 @@ int mpl_trwp_soft_backward(const mpl_shape* s, unsigned flags, float rho, int n_
   const int64_t N = P * s->n_disp;
   BackParams p;
   memset(&p, 0, sizeof(p));
-  p.xcd_group = xcd_group_size(s->n_disp);
   p.B = s->batch;
   p.H = s->height;
   p.W = s->width;

@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(kWave) sweep_bwd_kernel(const BackParams p) {
   const int lane = threadIdx.x;
   const int64_t P = (int64_t)p.B * p.H * p.W;
   const int64_t N = P * L;
-  const ChainCtx ch0 = locate_chain(p);
+  const ChainCtx ch0 = locate_chain<false>(p);
   const int n = ch0.n;
 
   const bool same = DC && p.same_label != 0;

@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t P = (int64_t)p.B * HW;
   const int64_t N = P * L;
-  const ChainCtx ch0 = locate_chain(p);
+  const ChainCtx ch0 = locate_chain<false>(p);
   const int n = ch0.n;
   const int lab0 = R * lane;
   const bool lane_ok = lab0 < L;

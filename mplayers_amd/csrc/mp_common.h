@@ -457,13 +457,17 @@ __device__ __forceinline__ int xcd_block(int block, int blocks, int group) {
   return base + (r % kXcds) * group + r / kXcds;
 }
 
-// which (direction, batch item, chain) a workgroup owns.  GROUPS false: the soft-weighted scans of mp_soft.hip,
-// which are bound by their exponentials and their blocks of duals; the groups brought them nothing, and the
-// instructions in front of their loops cost 5 % of the forward scan of 33 to 64 labels (48 labels 46x54, batch
-// 2: 2192 -> 2316 us) and 1 % of the reverse scans of up to 32.
+// which (direction, batch item, chain) a workgroup owns.  GROUPS false:
+//   * the soft-weighted scans of mp_soft.hip, which are bound by their exponentials and their blocks of duals;
+//     the groups brought them nothing, and the instructions in front of their loops cost 5 % of the forward scan
+//     of 33 to 64 labels (48 labels 46x54, batch 2: 2192 -> 2316 us) and 1 % of the reverse scans of up to 32;
+//   * the reverse scans: us without / with groups, ISGMR 60 labels
+//     43x49, 8 directions 59 / 63, 150 labels 100x140, 8 directions 457 / 469, TRWP 60 labels 375x450, 8 directions
+//     2359 / 2377, 150 labels 700x1000 5260 / 5283; ISGMR 52 labels 400x600 1178 / 1168.
 template <bool GROUPS = true, typename Params>
 __device__ __forceinline__ ChainCtx locate_chain(const Params& p) {
-  const int block = GROUPS ? xcd_block((int)blockIdx.x, (int)gridDim.x, p.xcd_group) : (int)blockIdx.x;
+  int block = (int)blockIdx.x;
+  if constexpr (GROUPS) block = xcd_block(block, (int)gridDim.x, p.xcd_group);
   int di = 0;
   while (di + 1 < p.n_dirs && block >= p.block_prefix[di + 1]) ++di;
   const int dir = p.dirs[di];
@@ -579,7 +583,6 @@ struct BackParams {
   const float* edge_label;  // soft TRWP: (n_dir_total, P, L, L) duals of this iteration
   int pack;                 // packed scans (mp_pack.hip): chains per wavefront
   int team;                 // four wavefronts per chain (mp_bwd_team.hip, mp_team21.hip)
-  int xcd_group;            // consecutive chains on one die (0: each on another; locate_chain)
 };
 
 // records the message mpl_last_error() returns on this thread and returns `code`

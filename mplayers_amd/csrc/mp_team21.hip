@@ -553,7 +553,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
   const int l = lane & (kHalf - 1);
   const int half = lane / kHalf;
   const bool ok = l < kL;
-  const ChainCtx ch0 = locate_chain(p);
+  const ChainCtx ch0 = locate_chain<false>(p);
   const int n = ch0.n;
   const float rho = p.rho;
   const int blocks = (n + kT - 1) / kT;
