@@ -234,6 +234,13 @@ class MPModule(torch.nn.Module):
         create_label_context(self.args, enable_seg=self.args.enable_seg,
                              enable_symmetric=self.args.enable_symmetric)
 
+  def __getstate__(self):
+    """What copies and files hold of the module: not the masks of this process, whose stream cannot be pickled and
+    whose device may be another one after loading."""
+    state = self.__dict__.copy()
+    state.pop("_kept_masks", None)
+    return state
+
   def _location_masks(self, label_context):
     """Masks of label_context_loc and label_context_diag_loc on the table's device, None where a location is
     not a list of different entries that numpy reads as torch does, or more than one value is pinned, and in

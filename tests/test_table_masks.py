@@ -2,6 +2,8 @@
 with the stored locations gives (MP_module.py:207-220), for every form the locations take, and after they or
 the table change."""
 import argparse
+import copy
+import io
 
 import numpy as np
 import pytest
@@ -193,3 +195,21 @@ def test_masks_on_another_stream(gpu, monkeypatch):
   torch.cuda.synchronize()
   want = _by_index(table.detach().cpu(), loc, diag, 1.5, False, 0.25)
   assert torch.allclose(first.detach().cpu(), want) and torch.equal(first, second)
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_copies_and_files_of_the_module(device):
+  """They hold no masks, nor the stream those were formed on, and work wherever they are loaded."""
+  loc, diag, _ = LOCATIONS["triangle"]
+  module = _module(loc, diag, 2).to(device)
+  want = module._effective_label_context().detach().cpu()
+  assert "_kept_masks" in module.__dict__
+  file = io.BytesIO()
+  torch.save(module, file)
+  file.seek(0)
+  # (the module of this test, written above)
+  loaded = torch.load(file, map_location="cpu", weights_only=False)
+  for other in (copy.deepcopy(module), loaded):
+    assert "_kept_masks" not in other.__dict__
+    assert torch.allclose(other._effective_label_context().detach().cpu(), want)
+  assert torch.allclose(loaded.to(device)._effective_label_context().detach().cpu(), want)
