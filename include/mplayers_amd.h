@@ -331,8 +331,9 @@ const char* mpl_last_error(void);
 #define MPL_OPT_DENSE_SPLIT_WAVES 4
 /* MPL_OPT_TEAM_SCANS (default 1): launches with few chains (on an MI355X at most 256 to 768, by label count
  * and operator) put four wavefronts on a chain, one for the recurrence and three that load, prepare, finish
- * and store its pixels: the forward scans of TRWP (with 21 labels and a 2-D table up to 2048 chains), whose
- * results are the same bits, the reverse scans of more than 64 labels with a 1-D table, TRWP's of 21 labels with
+ * and store its pixels: the forward scans of TRWP (with 21 labels and a 2-D table up to 2048 chains, with 65 to
+ * 192 labels and MPL_F_DENSE_TABLE up to 1280), whose results are the same bits but for linear tables under that flag,
+ * which agree to the parity tolerance, the reverse scans of more than 64 labels with a 1-D table, TRWP's of 21 labels with
  * a 2-D table and both soft-weighted scans of those (the forward one up to 1024 chains), whose results agree to
  * the parity tolerance; 0: never, 2: every such launch whatever its number of chains.  For tests and
  * measurements. */

@@ -274,14 +274,16 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* p, int bytes) {
 #ifndef MPL_ST_AUX
 #define MPL_ST_AUX 2
 #endif
-// Loads of planes whose pixel vectors are not whole cache lines, and of launches of few chains, go without
-// the hint: a line that two pixels share, or that the sweep after this one reads again, is then still
-// there.  Measured, ms per call with the hint / without, neighbouring chains on one die (xcd_group): TRWP
-// 97 labels 300x800 2.83 / 2.46, 150 labels 700x1000 keeping argmin labels 9.09 / 8.08, ISGMR 150 labels
-// 400x600 1.80 / 1.53; whole lines with one wavefront per chain, 96 labels 384x1248 3.65 / 3.68.  (Stores
+// Loads of planes with idle lanes (whole_lanes false: a label count that is no multiple of 64), and of launches of
+// few chains, go without the hint: a line that two pixels share, or that the sweep after this one reads again, is
+// then still there.  Label counts that fill whole lines but not all lanes (32, 96, 160, 224) go with the others, a
+// variant per line size being more code than the 1 % below.  Measured, ms per call with the hint / without,
+// neighbouring chains on one die (xcd_group): TRWP 97 labels 300x800 2.83 / 2.46, 150 labels 700x1000 keeping argmin
+// labels 9.09 / 8.08, ISGMR 150 labels 400x600 1.80 / 1.53; whole lines with one wavefront per chain, 96 labels 384x1248 3.65 / 3.68.  (Stores
 // without the hint as well: 2.53, 8.29, 1.61, 3.78.)
 constexpr int load_policy(bool whole_lanes) { return whole_lanes ? MPL_LD_AUX : 0; }
-// Stores go without it where a vector is no longer than two lines (up to 63 labels: most lines are shared):
+// Stores of the scans with one wavefront per chain go without it where a vector is no longer than two lines (up to
+// 63 labels: most lines are shared; mp_fwd_team.hip and mp_fwd_dense.hip store with it at every label count):
 // ISGMR 52 labels 400x600 0.66 / 0.60 with / without, TRWP 60 labels 375x450 the same.
 constexpr int store_policy(int R, bool whole_lanes) { return whole_lanes || R > 1 ? MPL_ST_AUX : 0; }
 

@@ -1,6 +1,7 @@
 // Forward scan of TRWP for tables declared dense (learned ones: every pair of labels counts) with four
 // wavefronts per chain, in launches of few chains.  The recurrence and what each plane holds: mp_fwd.hip;
-// the results are the same bits.
+// the results are the same bits, but for a linear table of 65 labels or more, which takes the scan over all pairs
+// of labels here and the minima from both sides there: they agree to the parity tolerance.
 //
 // Such a launch is bound by the scan over all pairs of labels of one pixel, so the front labels are split
 // over the wavefronts: each holds the chain's state, takes the minimum over its quarter, and the four partial

@@ -25,6 +25,10 @@
 // Errors of the reverse scan against 64 bits, one wavefront -> four, geometric means of the relative 2-norm
 // over 40 problems (images up to 130x130, 4 and 8 directions, 1 to 5 iterations; normal, positive and cross
 // entropy gradients): dunary 1.52e-7 -> 1.35e-7, dcontext 5.0e-7 both, dedge_weights 1.79e-7 -> 1.63e-7.
+// With longer chains, 36 problems of up to 2000 pixels a chain, by kind of gradient (normal / positive / cross
+// entropy): dunary 1.23 / 1.07 / 1.07e-7 -> 1.17 / 0.96 / 1.10e-7, dcontext 6.1 / 4.7 / 5.7e-7 -> 5.4 / 4.7 / 4.9e-7,
+// dedge_weights 1.28 / 1.19 / 1.32e-7 -> 1.24 / 1.09 / 1.34e-7; soft-weighted dunary 8.1 / 12.1 / 6.4e-8 -> 7.3 / 8.8 /
+// 6.0e-8, dcontext 7.4 / 5.4 / 6.7e-7 -> 7.2 / 5.2 / 6.4e-7, dedge_weights 4.5 / 3.0 / 7.2e-7 -> 3.4 / 2.3 / 5.3e-7.
 // Soft-weighted, 30 problems up to 100x100, 4 directions: 9.6e-8 -> 8.8e-8, 2.7e-7 both, 2.55e-7 -> 2.44e-7
 // (dedge_weights 2.9e-7 to 3.6e-7 while the expected dual's own rounding was left in).  Its scans,
 // 2x129x129, five iterations, duals kept: forward 1.44 -> 0.87 ms, bound by the main wavefront (11 exponentials and
