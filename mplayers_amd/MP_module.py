@@ -179,9 +179,10 @@ def _entries(place):
 def _runs_now(tensor):
   """Whether operations on `tensor` run as they are called: no trace, transform, dispatch mode or stream capture
   that could hold on to a tensor kept between calls, or leave one of its own in its place."""
-  return (type(tensor) is torch.Tensor and torch._C._len_torch_dispatch_stack() == 0 and
+  # (compiling first: the compiler refuses the questions after it)
+  return (not torch.compiler.is_compiling() and
+          type(tensor) is torch.Tensor and torch._C._len_torch_dispatch_stack() == 0 and
           torch._C._functorch.peek_interpreter_stack() is None and not torch.jit.is_tracing() and
-          not torch.compiler.is_compiling() and
           not (tensor.is_cuda and torch.cuda.is_current_stream_capturing()))
 
 

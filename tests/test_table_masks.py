@@ -141,6 +141,7 @@ def _make_fx(f, table):
 
 TRANSFORMS = {
     "fake tensors": _fake, "export": _export, "make_fx": _make_fx,
+    "compile": lambda f, table: torch.compile(f, backend="eager", fullgraph=True)(2 * table),
     "trace": lambda f, table: torch.jit.trace(f, (table,), check_trace=False)(2 * table),
     "vmap": lambda f, table: torch.func.vmap(f)(torch.stack([2 * table, table]))[0],
     "vmap of others": lambda f, table: torch.func.vmap(lambda x: f(2 * table) * x)(torch.ones(3, 1, 1))[1],
