@@ -291,8 +291,9 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
   // The last wavefront is the main one in every workgroup: the wavefronts of the workgroups that a compute
   // unit gets one after another start one SIMD further each (read from the hardware-id registers for 2, 3
   // and 4 workgroups per unit), so the main wavefronts of up to four of them are on SIMDs of their own.
-  // turn_every > 0 (launch_vj): it moves on by one every so many workgroups.
-  const int role = uniform_i((tid / kWave + (turn_every > 0 ? (int)blockIdx.x / turn_every : 0)) & 3);  // kHelpers: main
+  // With four labels per lane and turn_every > 0 (launch_vj) it moves on by one every so many workgroups.
+  const int turn = R == 4 && turn_every > 0 ? (int)blockIdx.x / turn_every : 0;
+  const int role = uniform_i((tid / kWave + turn) & 3);  // kHelpers: main
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t P = (int64_t)p.B * HW;
   const int64_t N = P * L;
