@@ -221,7 +221,10 @@ __device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx&
             arg = val == v[j] ? u : arg;
           }
           const int fd = f0 + arg;
-          fd_idx[j] = fd < L ? fd : L - 1;  // (only where no candidate is finite)
+          // (the last label where no candidate is a number, as in the other scans: a test of the bits, which the
+          // compiler may not take for false)
+          const bool none = (__builtin_bit_cast(unsigned, v[j]) & 0x7fffffffu) > 0x7f800000u;
+          fd_idx[j] = fd < L && !none ? fd : L - 1;
           pr[j] = lab0 + j < L && v[j] == nmin;
         }
         const int nidx = last_label<R>(pr, L - 1);

@@ -114,8 +114,8 @@ def test_tables_declared_dense(gpu, L, training):
 @pytest.mark.parametrize("L", [2, 7, 8, 33, 64, 65, 96, 130, 192, 256])
 @pytest.mark.parametrize("mode", ["TRWP", "ISGMR"])
 def test_argmin_labels_exist_where_no_candidate_is_a_number(gpu, L, mode):
-  """An edge weight that is NaN leaves a dense table's scan without a candidate to compare: whichever label is kept,
-  it is one, and the reverse scan does not look outside its tables for it."""
+  """An edge weight that is NaN leaves a dense table's scan without a candidate to compare: the last label is kept,
+  whichever scan takes the launch, and the reverse scan does not look outside its tables for it."""
   from mplayers_amd import _lib
   unary, ctx, ew = _problem(4, 1, 7, 9, L, "random", 9)
   ew[:, 0, 0, 3, 4] = np.nan
@@ -129,6 +129,8 @@ def test_argmin_labels_exist_where_no_candidate_is_a_number(gpu, L, mode):
       _lib.set_option(_lib.OPT_TEAM_SCANS, 1)
     assert got["msg_min_index"].max() < L and got["msg_norm_index"].max() < L
     assert not np.isfinite(got["msg"][:, 0, 0, 3, 4]).any()
+    if L > 2:  # (two entries are a band, whose scan keeps the label itself)
+      assert (got["msg_min_index"][:, :, 0, 0, 3, 4] == L - 1).all()
 
 
 @pytest.mark.parametrize("L,ctx2d", [(2, 1), (20, 1), (22, 1), (33, 1), (64, 1), (21, 0)])
