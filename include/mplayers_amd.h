@@ -81,7 +81,12 @@ typedef struct mpl_shape {
  * without the flag; a wider truncated linear table loses its O(L) label scan, whose values may
  * differ from the dense step's in the last bits where the table is not integer-valued, both within
  * the tolerance of the parity tests. */
-#define MPL_F_ALL 0x7fu
+#define MPL_F_DCONTEXT_COPIES 0x80u
+/* backward calls that want dcontext: dunary_update holds mpl_dcontext_copies() tables of dcontext's size one
+ * after another, cleared by the caller, which the chains of a launch take turns on; dcontext is
+ * OVERWRITTEN with their sum (it need not be cleared).  Without the flag, and where that number is 0,
+ * every chain adds to dcontext itself, all of them to the same few cache lines. */
+#define MPL_F_ALL 0xffu
 
 /* Replaces lib_*.TRWP.forward: MPLayers/TRWP/TRWP.cpp:245-283 (Forward) -> TRWP_forward.cu:378-560.
  * msg: initial messages in, final normalised messages out.  msg_min_index/msg_norm_index NULL =>
@@ -95,8 +100,8 @@ int mpl_trwp_forward(const mpl_shape* shape, unsigned flags, float rho, int n_it
 
 /* Replaces lib_*.TRWP.backward: MPLayers/TRWP/TRWP.cpp:285-318 -> TRWP_backward.cu:277-433.
  * dunary receives the gradient; dcontext and dedge_weights (zero-filled) accumulate; dmsg is
- * scratch (n_dir planes, any contents); dunary_update is accepted and unused.
- * dcontext and / or dedge_weights may be NULL when the caller has no use for that gradient (a fixed
+ * scratch (n_dir planes, any contents); dunary_update is accepted and unused but for
+ * MPL_F_DCONTEXT_COPIES.  dcontext and / or dedge_weights may be NULL when the caller has no use for that gradient (a fixed
  * pairwise table, edge weights that are not learned): the reverse scans then leave that part of
  * their step out; dunary is the same bit for bit. */
 int mpl_trwp_backward(const mpl_shape* shape, unsigned flags, float rho, int n_iter,
@@ -116,7 +121,8 @@ int mpl_isgmr_forward(const mpl_shape* shape, unsigned flags, int enable_sgm, fl
 
 /* Replaces lib_*.ISGMR.backward: MPLayers/ISGMR/ISGMR.cpp:344-379 -> ISGMR_backward.cu:290-493.
  * dmsg_update and dmsg are scratch (n_dir planes each, any contents); dmsg may be NULL (the pass
- * then works in place in dmsg_update and moves somewhat more data); dunary_update is unused.
+ * then works in place in dmsg_update and moves somewhat more data); dunary_update is unused but for
+ * MPL_F_DCONTEXT_COPIES.
  * dcontext and / or dedge_weights may be NULL, as for mpl_trwp_backward. */
 int mpl_isgmr_backward(const mpl_shape* shape, unsigned flags, int enable_sgm, float rho,
                        int n_iter, const float* context, const float* edge_weights,
@@ -208,6 +214,11 @@ int mpl_profile_end(mpl_kernel_stat* stats, int n_stats);
  * counts trees of the two-pixel steps that never enter the image).  Host-only helper; -1 for a
  * direction outside the table. */
 int mpl_n_chains(int dir, int height, int width);
+
+/* How many tables MPL_F_DCONTEXT_COPIES wants in dunary_update for a backward call of this shape: a power of
+ * two, or 0 where the call has so few chains that adding to dcontext itself is as fast; -1 for a shape
+ * the backward calls refuse.  Host-only helper, no counterpart in the reference. */
+int mpl_dcontext_copies(const mpl_shape* shape, int n_iter);
 
 /* Whether the forward scans take their O(L^2) step on the 1-D pairwise table `context` (n_disp
  * floats in HOST memory): 1 when it has neither a constant tail from entry 32 at the latest with no

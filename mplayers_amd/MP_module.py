@@ -72,13 +72,26 @@ def _backward_buffers(dcost_final, message_index, with_message_tmp, need_context
     buf["dedge_weights"] = dcost_final.new_empty(0)
   if with_message_tmp:
     buf["dmessage_tmp"] = dcost_final.new_empty(n_dir, batch, cv, h, w, n_disp)
-  if not need_context:
-    buf["dlabel_context"] = dcost_final.new_empty(0)
-  elif n_disp == 21:
-    buf["dlabel_context"] = dcost_final.new_zeros(n_disp, n_disp)
+  buf["flags"] = 0
+  if need_context:
+    buf["dlabel_context"], buf["dunary_update"], buf["flags"] = _context_gradient(
+        dcost_final, n_iter, n_dir, batch * cv, h, w, n_disp,
+        (n_disp, n_disp) if n_disp == 21 else (n_disp,))
   else:
-    buf["dlabel_context"] = dcost_final.new_zeros(n_disp)
+    buf["dlabel_context"] = dcost_final.new_empty(0)
   return buf
+
+
+def _context_gradient(like, n_iter, n_dir, batch, h, w, n_disp, size):
+  """dlabel_context, the operators' scratch tensor and their flags: with many chains these take turns on
+  tables of their own in the scratch (MPL_F_DCONTEXT_COPIES), whose sum overwrites dlabel_context."""
+  ctx2d = n_disp == 21  # (what the operators take the table for)
+  copies = 0
+  if like.is_cuda and len(size) == (2 if ctx2d else 1):
+    copies = _lib.dcontext_copies(_lib.Shape(n_dir, batch, h, w, n_disp, int(ctx2d)), n_iter)
+  if copies == 0:
+    return like.new_zeros(size), like.new_empty(0), 0
+  return like.new_empty(size), like.new_zeros((copies,) + size), _lib.F_DCONTEXT_COPIES
 
 
 def _table_flags(args):
@@ -118,7 +131,8 @@ class TRWPFunction(torch.autograd.Function):
     buf = _backward_buffers(dcost_final, message_index, False, need_context, need_edge_weights)
     _ops_for(n_disp).TRWP.backward(rho, label_context, edge_weights, dcost_final, message_index,
                                    cost_index, buf["dunary"], buf["dlabel_context"],
-                                   buf["dedge_weights"], buf["dmessage"], buf["dunary_update"])
+                                   buf["dedge_weights"], buf["dmessage"], buf["dunary_update"],
+                                   flags=buf["flags"])
     return (buf["dunary"], buf["dlabel_context"] if need_context else None,
             buf["dedge_weights"] if need_edge_weights else None, None)
 
@@ -156,7 +170,7 @@ class ISGMRFunction(torch.autograd.Function):
     _ops_for(n_disp).ISGMR.backward(int(enable_sgm), rho, label_context, edge_weights,
                                     dcost_final, message_index, cost_index, buf["dunary"],
                                     buf["dlabel_context"], buf["dedge_weights"], buf["dmessage"],
-                                    buf["dunary_update"], buf["dmessage_tmp"])
+                                    buf["dunary_update"], buf["dmessage_tmp"], flags=buf["flags"])
     return (buf["dunary"], buf["dlabel_context"] if need_context else None,
             buf["dedge_weights"] if need_edge_weights else None, None)
 

@@ -7,7 +7,7 @@ LIB_PATH = os.environ.get("MPLAYERS_HIP_LIB", os.path.join(HERE, "libmplayers_hi
 
 SYMBOLS = ("mpl_trwp_forward", "mpl_trwp_backward", "mpl_isgmr_forward", "mpl_isgmr_backward",
            "mpl_trwp_forward_cpu", "mpl_isgmr_forward_cpu",
-           "mpl_profile_begin", "mpl_profile_end", "mpl_n_chains", "mpl_table_is_dense",
+           "mpl_profile_begin", "mpl_profile_end", "mpl_n_chains", "mpl_dcontext_copies", "mpl_table_is_dense",
            "mpl_last_error", "mpl_version", "mpl_edge_shift", "mpl_edge_shift_static",
            "mpl_trwp_soft_forward",
            "mpl_trwp_soft_backward", "mpl_soft_weighted_message", "mpl_soft_weighted_message_back", "mpl_set_option",
@@ -31,6 +31,7 @@ F_FUSED_U_OFF = 0x08
 F_DCONTEXT_SAME_LABEL = 0x10
 F_FUSED_PAIRS_OFF = 0x20
 F_DENSE_TABLE = 0x40
+F_DCONTEXT_COPIES = 0x80
 
 
 class KernelStat(ctypes.Structure):
@@ -71,6 +72,7 @@ def load():
   lib.mpl_mrf_energy.argtypes = [sp, ci, vp, vp, vp, vp, vp, vp]
   lib.mpl_transpose.argtypes = [vp, vp, ci, ctypes.c_int64, ctypes.c_int64, vp]
   lib.mpl_n_chains.argtypes = [ci, ci, ci]
+  lib.mpl_dcontext_copies.argtypes = [sp, ci]
   lib.mpl_table_is_dense.argtypes = [vp, ci]
   lib.mpl_profile_begin.argtypes = []
   lib.mpl_profile_end.argtypes = [ctypes.POINTER(KernelStat), ci]
@@ -125,6 +127,13 @@ def table_is_dense(table):
   if rc < 0:
     raise ValueError("table_is_dense: an empty table")
   return bool(rc)
+
+
+def dcontext_copies(shape, n_iter):
+  """mpl_dcontext_copies: tables that a backward call with F_DCONTEXT_COPIES wants, 0 for none."""
+  copies = load().mpl_dcontext_copies(shape, int(n_iter))
+  check(min(copies, 0), "dcontext_copies")
+  return copies
 
 
 def check(rc, what):

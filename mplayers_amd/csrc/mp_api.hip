@@ -501,6 +501,14 @@ __global__ void __launch_bounds__(256) isgmr_combine_kernel(const float* X, floa
 // ------------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------------
+// Tables the reverse scans take turns on for dcontext, and the chains of a call, over all its iterations, from
+// which they pay for the pass that sums them (mpl_dcontext_copies).  Measured, backward with all gradients, us per
+// call without and with 8 tables (16, 32 and 64 are the same): 21 labels, a 2-D table, TRWP 2 directions 205x129
+// (4100 chains) 491 -> 465, 4x129x129 680 -> 611, ISGMR 2x65x65 164 -> 136, 12x65x65 560 -> 436, 12x129x129 1525 ->
+// 1251; 1-D tables, 64 labels TRWP 103x103 1484 -> 1475, 96 labels ISGMR 240x320 1812 -> 1630, TRWP 1477 both.
+constexpr int kDctxCopies = 8;
+constexpr int64_t kDctxMinChains = 4096;
+
 thread_local char g_err[512] = "";
 
 // Optional per-kernel timing with HIP events on the launch stream (off unless mpl_profile_begin
@@ -974,6 +982,39 @@ void rebuild_belief(const mpl_shape* s, const float* unary, const float* msg, fl
   MPL_EW_LAUNCH(belief_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, S, (int*)nullptr);
 }
 
+// dcontext = the sum of the tables the reverse scans added to (MPL_F_DCONTEXT_COPIES), always in the same order
+__global__ void __launch_bounds__(kWave) dcontext_fold_kernel(const float* __restrict__ tables, int entries,
+                                                              float* __restrict__ dcontext) {
+  const int i = (int)blockIdx.x * kWave + (int)threadIdx.x;
+  if (i >= entries) return;
+  float x[kDctxCopies];
+#pragma unroll
+  for (int k = 0; k < kDctxCopies; ++k) x[k] = tables[k * entries + i];
+#pragma unroll
+  for (int w = kDctxCopies / 2; w > 0; w /= 2)
+#pragma unroll
+    for (int k = 0; k < w; ++k) x[k] += x[k + w];
+  dcontext[i] = x[0];
+}
+
+// Where the reverse scans of a backward call add their parts of dcontext: the caller's tensor, or tables in its
+// scratch tensor that fold_dcontext sums at the end of the call.  False: no scratch to take.
+bool place_dcontext(const mpl_shape* s, unsigned flags, int n_iter, float* dcontext, float* scratch, BackParams* p) {
+  p->dctx = dcontext;
+  p->dctx_mask = 0;
+  if ((flags & MPL_F_DCONTEXT_COPIES) == 0 || dcontext == nullptr || mpl_dcontext_copies(s, n_iter) == 0) return true;
+  if (scratch == nullptr) return false;
+  p->dctx = scratch;
+  p->dctx_mask = kDctxCopies - 1;
+  return true;
+}
+void fold_dcontext(const BackParams& p, float* dcontext, hipStream_t st) {
+  if (p.dctx_mask == 0) return;
+  Timed timed(MPL_KERNEL_OTHER, st);
+  const int entries = p.ctx2d ? p.L * p.L : p.L;
+  dcontext_fold_kernel<<<(entries + kWave - 1) / kWave, kWave, 0, st>>>(p.dctx, entries, dcontext);
+}
+
 // cost_final is not written before the final aggregation, so its first bytes carry the context
 // descriptor during the sweeps (no allocation, no state shared between streams).
 const CtxDesc* make_desc(const mpl_shape* s, const float* ctx, float* cost_final, hipStream_t st) {
@@ -1124,6 +1165,13 @@ int mpl_table_is_dense(const float* context, int n_disp) {
   const bool band = last_ne + 1 <= kMaxBandK;
   const bool linear = L >= 2 && c0 == 0.f && slope >= 0.f && lin;
   return (band || linear) ? 0 : 1;
+}
+
+int mpl_dcontext_copies(const mpl_shape* s, int n_iter) {
+  if (check_shape(s, n_iter) != MPL_OK) return -1;
+  int64_t chains = 0;
+  for (int d = 0; d < s->n_dir; ++d) chains += (int64_t)s->batch * make_dir(d, s->height, s->width).n_chains;
+  return chains * n_iter >= kDctxMinChains ? kDctxCopies : 0;
 }
 
 int mpl_n_chains(int dir, int height, int width) {
@@ -1354,7 +1402,6 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
                       const uint8_t* msg_min_index, const uint8_t* msg_norm_index, float* dunary,
                       float* dcontext, float* dedge_weights, float* dmsg, float* dunary_update,
                       void* stream) {
-  (void)dunary_update;
   int rc = check_shape(s, n_iter);
   if (rc) return rc;
   CallOpts opts;
@@ -1379,7 +1426,8 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
   p.edge = edge_weights;
   p.ctx = context;
   p.dedge = dedge_weights;
-  p.dctx = dcontext;
+  if (!place_dcontext(s, flags, n_iter, dcontext, dunary_update, &p))
+    return fail(MPL_EINVAL, "MPL_F_DCONTEXT_COPIES needs the tables in dunary_update");
   p.same_label = (flags & MPL_F_DCONTEXT_SAME_LABEL) ? 1 : 0;
   const float* a_cur = dcost_final;  // CostAggregateKernelBack: every g_k starts as dcost
   for (int it = n_iter - 1; it >= 0; --it) {
@@ -1403,6 +1451,7 @@ int mpl_trwp_backward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
       if (!(d & 1)) a_cur = p.a_out;
     }
   }
+  fold_dcontext(p, dcontext, st);
   return launch_ok("trwp_backward");
 }
 
@@ -1411,7 +1460,6 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
                        const uint8_t* msg_min_index, const uint8_t* msg_norm_index, float* dunary,
                        float* dcontext, float* dedge_weights, float* dmsg, float* dunary_update,
                        float* dmsg_update, void* stream) {
-  (void)dunary_update;
   int rc = check_shape(s, n_iter);
   if (rc) return rc;
   CallOpts opts;
@@ -1447,7 +1495,8 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
   p.edge = edge_weights;
   p.ctx = context;
   p.dedge = dedge_weights;
-  p.dctx = dcontext;
+  if (!place_dcontext(s, flags, n_iter, dcontext, dunary_update, &p))
+    return fail(MPL_EINVAL, "MPL_F_DCONTEXT_COPIES needs the tables in dunary_update");
   p.same_label = (flags & MPL_F_DCONTEXT_SAME_LABEL) ? 1 : 0;
   fill_dirs(s, 0, s->n_dir, p.dirs, p.block_prefix, &p.n_dirs);
   p.pack = decide_pack(s, p, opts);
@@ -1466,6 +1515,7 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
     MPL_EW_LAUNCH(isgmr_combine_kernel, v4, s->n_dir, N, st, dmsg_update, gu_buf, s->n_dir, N, rho,
                   dcost_final, factor, first ? 1 : 0, it > 0 ? 1 : 0, pair_share, dunary);
   }
+  fold_dcontext(p, dcontext, st);
   return launch_ok("isgmr_backward");
 }
 
@@ -1545,7 +1595,6 @@ int mpl_trwp_soft_backward(const mpl_shape* s, unsigned flags, float rho, int n_
                            const float* edge_weights, const float* msg_edge_label,
                            const uint8_t* msg_norm_index, float* dunary, float* dcontext,
                            float* dedge_weights, float* dmsg, float* dunary_update, void* stream) {
-  (void)dunary_update;
   int rc = check_shape(s, n_iter);
   if (rc) return rc;
   CallOpts opts;
@@ -1569,7 +1618,8 @@ int mpl_trwp_soft_backward(const mpl_shape* s, unsigned flags, float rho, int n_
   p.edge = edge_weights;
   p.ctx = context;
   p.dedge = dedge_weights;
-  p.dctx = dcontext;
+  if (!place_dcontext(s, flags, n_iter, dcontext, dunary_update, &p))
+    return fail(MPL_EINVAL, "MPL_F_DCONTEXT_COPIES needs the tables in dunary_update");
   bool first = true;
   for (int it = n_iter - 1; it >= 0; --it) {
     for (int d = s->n_dir - 1; d >= 0; --d) {  // TRWP_backward_soft.cu:454-538
@@ -1590,6 +1640,7 @@ int mpl_trwp_soft_backward(const mpl_shape* s, unsigned flags, float rho, int n_
       if (p.fused_pair) --d;
     }
   }
+  fold_dcontext(p, dcontext, st);
   return launch_ok("trwp_soft_backward");
 }
 

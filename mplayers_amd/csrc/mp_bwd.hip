@@ -468,25 +468,26 @@ __global__ void __launch_bounds__(kWave) sweep_bwd_kernel(const BackParams p) {
     }
   }
   if (!DC) return;
+  float* const dctx = dctx_table(p);
   __syncthreads();
   for (int i = lane; i < n_ctx; i += kWave) {
     float v = hist_s[i];
-    if (has_value(v)) atomicAdd(&p.dctx[i], v);
+    if (has_value(v)) atomicAdd(&dctx[i], v);
   }
   if (!ctx2d) {
 #pragma unroll
     for (int j = 0; j < R; ++j)
-      if (valid[j] && lab0 + j >= 1 && has_value(hist_reg[j])) atomicAdd(&p.dctx[lab0 + j], hist_reg[j]);
+      if (valid[j] && lab0 + j >= 1 && has_value(hist_reg[j])) atomicAdd(&dctx[lab0 + j], hist_reg[j]);
 #pragma unroll
     for (int k = 1; k <= kNear; ++k) {
       const float v = wave_sum(near_acc[k]);
-      if (lane == 0 && k < L && has_value(v)) atomicAdd(&p.dctx[k], v);
+      if (lane == 0 && k < L && has_value(v)) atomicAdd(&dctx[k], v);
     }
     if (same) {
       // bin 0: the popular labels that point at themselves were gathered twice into the
       // accumulator of label 0 (x + x, exact), the others were summed per lane
       const float v = wave_sum(near_acc[0] + (lane == 0 ? 0.5f * hist_reg[0] : 0.f));
-      if (lane == 0 && has_value(v)) atomicAdd(&p.dctx[0], v);
+      if (lane == 0 && has_value(v)) atomicAdd(&dctx[0], v);
     }
   }
 }

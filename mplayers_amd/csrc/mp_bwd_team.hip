@@ -691,11 +691,12 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
     }
   }
   __syncthreads();
+  float* const dctx = dctx_table(p);
   for (int i = tid; i < n_ctx; i += kTeam) {
     float v = 0.f;
 #pragma unroll
     for (int h = 0; h < kHelpers; ++h) v += hist_s[h * n_hist + (kNearBins + 1) * near_words(R) + i];
-    if (has_value(v)) atomicAdd(&p.dctx[i], v);
+    if (has_value(v)) atomicAdd(&dctx[i], v);
   }
 }
 

@@ -580,12 +580,21 @@ struct BackParams {
   const uint8_t* idx_norm;  // (n_dir_total, P)
   float* dedge;             // (n_dir_total, P) accumulates; null: not wanted, that part of the step is left out
   float* dctx;              // accumulates; null: not wanted
+  int dctx_mask;            // number of tables at dctx less one (MPL_F_DCONTEXT_COPIES; a power of two)
   int same_label;           // dctx also collects the pairs with cd == fd (the hard operator of the
                             // reference's TRWP_hard_soft build, TRWP_hard_soft/TRWP_backward.cu:104-111)
   const float* edge_label;  // soft TRWP: (n_dir_total, P, L, L) duals of this iteration
   int pack;                 // packed scans (mp_pack.hip): chains per wavefront
   int team;                 // four wavefronts per chain (mp_bwd_team.hip, mp_team21.hip)
 };
+
+// The table of dctx this workgroup adds to.  All chains of a launch end at about the same time and add to the same
+// few cache lines, whose atomics the eight dies take one after another, 10 to 18 ns each.  With a table per die
+// (consecutive workgroups go to the dies in turn) they stay in that die's L2, and dcontext_fold_kernel (mp_api.hip)
+// sums the tables once per call.
+__device__ __forceinline__ float* dctx_table(const BackParams& p) {
+  return p.dctx + ((int)blockIdx.x & p.dctx_mask) * (p.ctx2d ? p.L * p.L : p.L);
+}
 
 // records the message mpl_last_error() returns on this thread and returns `code`
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));

@@ -544,6 +544,7 @@ __global__ void __launch_bounds__(kWave) packed_bwd_kernel(const BackParams p) {
   }
   }  // both walks of a fused pair
   if (!DC) return;
+  float* const dctx = dctx_table(p);
   __syncthreads();
   // fold the pair tables of all chain slots into dcontext's bins (the pairs with cd == fd were
   // only collected when the caller asked for them)
@@ -555,7 +556,7 @@ __global__ void __launch_bounds__(kWave) packed_bwd_kernel(const BackParams p) {
           if (c + lane < L) acc += pairs[g2 * L * L + c * L + c + lane];
           if (lane >= 1 && c - lane >= 0) acc += pairs[g2 * L * L + c * L + c - lane];
         }
-      if (has_value(acc)) atomicAdd(&p.dctx[lane], acc);
+      if (has_value(acc)) atomicAdd(&dctx[lane], acc);
     }
   } else {
     for (int i = lane; i < L * L; i += kWave) {
@@ -564,7 +565,7 @@ __global__ void __launch_bounds__(kWave) packed_bwd_kernel(const BackParams p) {
       float v = 0.f;
       for (int g2 = 0; g2 < G; ++g2)
         v += pairs[g2 * L * L + i] + (c < f ? pairs[g2 * L * L + f * L + c] : 0.f);
-      if (has_value(v)) atomicAdd(&p.dctx[i], v);
+      if (has_value(v)) atomicAdd(&dctx[i], v);
     }
   }
 }

@@ -360,6 +360,7 @@ __global__ void __launch_bounds__(kWave) soft_bwd_kernel(const BackParams p) {
     }
   }
   if (p.dctx == nullptr) return;
+  float* const dctx = dctx_table(p);
   __syncthreads();
   // fold the pair table into dcontext's bins: |cd - fd| (1-D) or [min, max] (2-D), the diagonal
   // included (TRWP_backward_soft.cu:116-126)
@@ -370,14 +371,14 @@ __global__ void __launch_bounds__(kWave) soft_bwd_kernel(const BackParams p) {
         if (fd + lane < L) acc += hist[fd * L + fd + lane];
         if (lane > 0 && fd - lane >= 0) acc += hist[fd * L + fd - lane];
       }
-      if (has_value(acc)) atomicAdd(&p.dctx[lane], acc);
+      if (has_value(acc)) atomicAdd(&dctx[lane], acc);
     }
   } else {
     for (int i = lane; i < LL; i += kWave) {
       const int fd = i / L, cd = i - fd * L;
       if (cd > fd) continue;  // handled by the (fd, cd) entry
       const float v = hist[i] + (cd < fd ? hist[cd * L + fd] : 0.f);
-      if (has_value(v)) atomicAdd(&p.dctx[cd * L + fd], v);
+      if (has_value(v)) atomicAdd(&dctx[cd * L + fd], v);
     }
   }
 }
@@ -881,6 +882,7 @@ __global__ void __launch_bounds__(kWave) soft_split_bwd_kernel(const BackParams 
   }
   }  // both walks of a fused pair
   if (p.dctx == nullptr) return;
+  float* const dctx = dctx_table(p);
   {
     const int F = (L + G - 1) / G;
     const bool valid = lane < G * L;
@@ -900,14 +902,14 @@ __global__ void __launch_bounds__(kWave) soft_split_bwd_kernel(const BackParams 
         if (fd + lane < L) acc += hist[fd * L + fd + lane];
         if (lane > 0 && fd - lane >= 0) acc += hist[fd * L + fd - lane];
       }
-      if (has_value(acc)) atomicAdd(&p.dctx[lane], acc);
+      if (has_value(acc)) atomicAdd(&dctx[lane], acc);
     }
   } else {
     for (int i = lane; i < LL; i += kWave) {
       const int fd = i / L, c2 = i - fd * L;
       if (c2 > fd) continue;  // handled by the (fd, cd) entry
       const float v = hist[i] + (c2 < fd ? hist[c2 * L + fd] : 0.f);
-      if (has_value(v)) atomicAdd(&p.dctx[c2 * L + fd], v);
+      if (has_value(v)) atomicAdd(&dctx[c2 * L + fd], v);
     }
   }
 }
@@ -1289,9 +1291,10 @@ __global__ void __launch_bounds__(kWave) soft_wide_bwd_kernel(const BackParams p
     if (t >= 1 && bDe != nullptr && lane == 0) bDe[pix] += det;
   }
   if (p.dctx != nullptr) {
+    float* const dctx = dctx_table(p);
 #pragma unroll
     for (int j = 0; j < R; ++j)
-      if (valid[j] && has_value(hist[j])) atomicAdd(&p.dctx[cd[j]], hist[j]);
+      if (valid[j] && has_value(hist[j])) atomicAdd(&dctx[cd[j]], hist[j]);
   }
 }
 

@@ -986,8 +986,9 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
     }
   }
   __syncthreads();
+  float* const dctx = dctx_table(p);
   for (int i = tid; i < kPairs; i += kTeam)
-    if (has_value(hist_s[i])) atomicAdd(&p.dctx[i], hist_s[i]);
+    if (has_value(hist_s[i])) atomicAdd(&dctx[i], hist_s[i]);
 }
 
 }  // namespace

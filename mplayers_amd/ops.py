@@ -44,6 +44,14 @@ def _context_numel(L, ctx2d):
   return L * L if ctx2d else L
 
 
+def _check_tables(dcontext, tables, shape, n_iter, flags):
+  """The scratch of MPL_F_DCONTEXT_COPIES: dunary_update holds the tables, cleared by the caller."""
+  if (int(flags) & _lib.F_DCONTEXT_COPIES) and _wanted(dcontext):
+    copies = _lib.dcontext_copies(shape, n_iter)
+    if copies > 0:
+      _check("dunary_update", tables, torch.float32, copies * _context_numel(shape.n_disp, shape.ctx2d))
+
+
 def _wanted(t):
   """An output gradient the caller has no use for is passed as None or as an empty tensor, the
   reference's way of switching an output off (TRWP_forward.cu:406-408)."""
@@ -167,6 +175,7 @@ class TRWP(object):
     _check("dunary", dunary, f32, N)
     if _wanted(dcontext):
       _check("dcontext", dcontext, f32, _context_numel(L, ctx2d))
+    _check_tables(dcontext, dunary_update, shape, n_iter, flags)
     if _wanted(dedge_weights):
       _check("dedge_weights", dedge_weights, f32, shape.n_dir * P)
     _check("dmsg", dmsg, f32, shape.n_dir * N)
@@ -224,6 +233,7 @@ class ISGMR(object):
     _check("dunary", dunary, f32, N)
     if _wanted(dcontext):
       _check("dcontext", dcontext, f32, _context_numel(L, ctx2d))
+    _check_tables(dcontext, dunary_update, shape, n_iter, flags)
     if _wanted(dedge_weights):
       _check("dedge_weights", dedge_weights, f32, shape.n_dir * P)
     _check("dmsg_update", dmsg_update, f32, shape.n_dir * N)
@@ -306,6 +316,7 @@ class TRWP_hard_soft(object):
     _check("dunary", dunary, f32, N)
     if _wanted(dcontext):
       _check("dcontext", dcontext, f32, _context_numel(L, ctx2d))
+    _check_tables(dcontext, dunary_update, shape, n_iter, flags)
     if _wanted(dedge_weights):
       _check("dedge_weights", dedge_weights, f32, n_dir * P)
     _check("dmsg", dmsg, f32, n_dir * N)
