@@ -86,7 +86,10 @@ typedef struct mpl_shape {
  * after another, cleared by the caller, which the chains of a launch take turns on; dcontext is
  * OVERWRITTEN with their sum (it need not be cleared).  Without the flag, and where that number is 0,
  * every chain adds to dcontext itself, all of them to the same few cache lines. */
-#define MPL_F_ALL 0xffu
+#define MPL_F_CHAIN_STARTS 0x100u
+/* mpl_trwp_soft_forward: the blocks of duals and the normalisation indices of chain-start pixels are
+ * written too, with zeros, so that nothing of msg_edge_label and msg_norm_index need be cleared. */
+#define MPL_F_ALL 0x1ffu
 
 /* Replaces lib_*.TRWP.forward: MPLayers/TRWP/TRWP.cpp:245-283 (Forward) -> TRWP_forward.cu:378-560.
  * msg: initial messages in, final normalised messages out.  msg_min_index/msg_norm_index NULL =>
@@ -156,7 +159,7 @@ int mpl_isgmr_forward_cpu(const mpl_shape* shape, int enable_sgm, float rho, int
  * stereo build (TRWP.cpp:336-340); 2-D context tables up to 64 labels.
  *   msg_edge_label (n_iter, n_dir, B, H, W, L, L) fp32: every dual of every pixel, kept for the
  *   backward pass (even directions [fd][cd], odd ones [cd][fd]); blocks of chain-start pixels are
- *   not written.  NULL together with msg_norm_index => inference. */
+ *   not written without MPL_F_CHAIN_STARTS.  NULL together with msg_norm_index => inference. */
 int mpl_trwp_soft_forward(const mpl_shape* shape, unsigned flags, float rho, int n_iter,
                           const float* unary, const float* context, const float* edge_weights,
                           float* msg, float* msg_edge_label, uint8_t* msg_norm_index,

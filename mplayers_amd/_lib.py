@@ -32,6 +32,7 @@ F_DCONTEXT_SAME_LABEL = 0x10
 F_FUSED_PAIRS_OFF = 0x20
 F_DENSE_TABLE = 0x40
 F_DCONTEXT_COPIES = 0x80
+F_CHAIN_STARTS = 0x100
 
 
 class KernelStat(ctypes.Structure):

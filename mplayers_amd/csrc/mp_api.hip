@@ -956,6 +956,22 @@ void zero_fill(float* dst, int64_t n, hipStream_t st) {
     zero_fill_kernel<1><<<elementwise_blocks(n), 256, 0, st>>>(dst, n);
 }
 
+// Zeros in the blocks of duals and the normalisation indices of chain-start pixels (MPL_F_CHAIN_STARTS), of all
+// iterations and directions: grid.x the chains of p's directions, grid.y the iterations.  The rest of both tensors
+// is the scans' to write, so nothing else needs clearing: 2x129x129, 21 labels, 4 directions, 5 iterations 156 us
+// (a fill of 1.17 GB) -> 5 us.
+__global__ void __launch_bounds__(256) chain_starts_kernel(const SweepParams p, int n_iter, float* __restrict__ duals,
+                                                           uint8_t* __restrict__ norm) {
+  const ChainCtx ch = locate_chain<false>(p);
+  const int64_t P = (int64_t)p.B * p.H * p.W;
+  const int block = p.L * p.L;
+  for (int64_t it = blockIdx.y; it < n_iter; it += gridDim.y) {
+    const int64_t pix = (it * p.n_dirs + ch.dir) * P + (int64_t)ch.bv * p.H * p.W + ch.pix0;
+    for (int i = threadIdx.x; i < block; i += 256) duals[pix * block + i] = 0.f;
+    if (threadIdx.x == 0) norm[pix] = 0;
+  }
+}
+
 // The sweeps keep the belief plane up to date by differences, S <- (S - m_old) + m_new, where the
 // reference re-sums unary + sum_k m_k before every sweep (UpdateUnaryKernel, TRWP_forward.cu:60-80):
 // the rounding of each update stays in the plane.  Between two iterations the plane holds S itself,
@@ -1537,6 +1553,13 @@ int mpl_trwp_soft_forward(const mpl_shape* s, unsigned flags, float rho, int n_i
   const int64_t P = (int64_t)s->batch * s->height * s->width;
   const int64_t N = P * s->n_disp;
   const bool train = msg_edge_label != nullptr;
+  if (train && (flags & MPL_F_CHAIN_STARTS)) {
+    Timed timed(MPL_KERNEL_OTHER, st);
+    SweepParams p = base_fwd_params(s, rho, edge_weights, context, nullptr);
+    fill_dirs(s, 0, s->n_dir, p.dirs, p.block_prefix, &p.n_dirs);
+    const dim3 grid((unsigned)p.block_prefix[p.n_dirs], (unsigned)std::min(n_iter, 65535));
+    chain_starts_kernel<<<grid, 256, 0, st>>>(p, n_iter, msg_edge_label, msg_norm_index);
+  }
   if (flags & MPL_F_MSG_UNINIT) zero_fill(msg, (int64_t)s->n_dir * N, st);
   {
     Timed timed(MPL_KERNEL_BELIEF, st);
