@@ -19,8 +19,8 @@
 // among them) every 5.2, an exchange of rows or halves takes 8.2, an LDS access 10 to 14 (measured); by
 // that count the forward step is 290 clocks and the reverse step 250.  Measured, ns per pixel of rows of 256 /
 // 512 chains, one wavefront per chain -> this: 215 / 223 -> 143 / 145 without argmin labels, 340 / 347 -> 171 / 175
-// with them.  4x129x129, 4 directions, 5 iterations, both other gradients wanted: backward 0.96 -> 0.65 ms; of
-// the 0.22 ms that dcontext costs there most is 516 chains adding 441 pairs to one table per launch.
+// with them.  4x129x129, 4 directions, 5 iterations, both other gradients wanted: backward 0.96 -> 0.65 ms, 0.59
+// with a table of dcontext per die (dctx_table).
 //
 // Errors of the reverse scan against 64 bits, one wavefront -> four, geometric means of the relative 2-norm
 // over 40 problems (images up to 130x130, 4 and 8 directions, 1 to 5 iterations; normal, positive and cross
@@ -32,7 +32,8 @@
 // Soft-weighted, 30 problems up to 100x100, 4 directions: 9.6e-8 -> 8.8e-8, 2.7e-7 both, 2.55e-7 -> 2.44e-7
 // (dedge_weights 2.9e-7 to 3.6e-7 while the expected dual's own rounding was left in).  Its scans,
 // 2x129x129, five iterations, duals kept: forward 1.44 -> 0.87 ms, bound by the main wavefront (11 exponentials and
-// three exchanges of halves a pixel), reverse 2.03 -> 1.30 ms, by the helpers' softmin weights.  Forward errors
+// three exchanges of halves a pixel), reverse 2.03 -> 1.10 ms, by the helpers' softmin weights, 540 instructions for two
+// pixels (650 while every weight was stored under a mask of its own, and the loads were waited for: keep).  Forward errors
 // over 24 problems: messages 5.0e-7 -> 4.7e-7, costs 1.11e-7 -> 1.06e-7, duals 7.7e-8 ->
 // 7.5e-8.
 
@@ -67,6 +68,17 @@ __device__ __forceinline__ void static_for(const F& f) {
     f(std::integral_constant<int, I>());
     static_for<N, I + 1>(f);
   }
+}
+
+// A loaded value in a register of its own, moved there where it is first used.  The helpers keep some of what they
+// load for a pixel until the pixel is finished; left to the compiler the two share a register and change places
+// once per two blocks, with moves right behind the loads of the block after next that wait for all of them: the
+// whole latency of memory, every twelve pixels.
+template <typename T>
+__device__ __forceinline__ T keep(T x) {
+  T y;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
+  return y;
 }
 
 __device__ __forceinline__ int bits(float x) { return __builtin_bit_cast(int, x); }
@@ -374,7 +386,7 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
       for (int j = 0; j < kEntries; ++j) {
         const int e = lane + kWave * j < kL * kL ? lane + kWave * j : kL * kL - 1;
         const int row = e / kL, col = e - row * kL;
-        tblk[j] = p.ctx[row < col ? row * kL + col : col * kL + row];
+        tblk[j] = keep(p.ctx[row < col ? row * kL + col : col * kL + row]);  // (waited for here, not in the loop)
         ablk[j] = (dir & 1) ? col : row;
       }
     }
@@ -419,7 +431,7 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
       tk = EVEN ? px.s - px.md : px.s + px.mi;
       float un = fmaf(tk, rho, -px.mi);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
       if (!SOFT) un = fmaxf(un, floor_l);
-      wk = px.w;
+      wk = SOFT && TRAIN ? keep(px.w) : px.w;
       *reinterpret_cast<f32x2*>(s.in[i][l]) = f32x2{un, px.w};
       // Q of the pixel is known already, whatever its message
       if (EVEN && !SOFT) store(rSo, label_off(t < n, pixel_off(t)), tk - px.mi);
@@ -530,6 +542,7 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
 }
 
 // ---- backward --------------------------------------------------------------------------------------
+template <int kT>
 struct alignas(16) BwdSlots {   // one set
   float mask[kT][2][kL][12];    // per half's sources and label: 1 where the source label points at the
                                 // label, else 0; last: 1 where the normalisation's argmin label is the label
@@ -541,18 +554,27 @@ struct alignas(16) BwdSlots {   // one set
 };
 constexpr int kPairs = kL * kL;
 
+// Helpers of the soft-weighted scan where every chain has a compute unit to itself: the fourth SIMD, the main
+// wavefront's in the other launches, takes two of them.  More chains fill the SIMDs with three each.  Rows of 129 pixels,
+// all gradients, us per pair of walks with three / six: 128 chains 90 / 76, 256 chains 95 / 81, 258 chains 111 / 145, 512 chains 117 / 153.
+constexpr int kSoftHelpersAlone = 6;
+
 // GR: dedge_weights and / or dcontext are wanted; DC: dcontext is.  SOFT: the soft-weighted operator, whose
 // step has the same form with J[cd][fd] = d message(cd) / d belief(fd) in place of the masks: the helpers
 // read a pixel's duals, take the softmin weights of a label over its front labels and put J into the slot.
-template <bool GR, bool DC, bool SOFT>
-__global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
+template <bool GR, bool DC, bool SOFT, int kHelpers>
+__global__ void __launch_bounds__((kHelpers + 1) * kWave) bwd_team21_kernel(const BackParams p) {
+  constexpr int kT = 2 * kHelpers, kTeam = (kHelpers + 1) * kWave;
+  using Slots = BwdSlots<kT>;
   extern __shared__ __align__(16) char smem_raw[];
-  BwdSlots* sets = reinterpret_cast<BwdSlots*>(smem_raw);  // two
+  Slots* sets = reinterpret_cast<Slots*>(smem_raw);  // two
   float* acc = reinterpret_cast<float*>(sets + 2);         // kMaxL
   float* ctx_s = acc + kMaxL;                              // the table, then dcontext of the chain
   float* hist_s = ctx_s + kPairs;
   const int tid = threadIdx.x;
-  const int role = uniform_i(tid / kWave);  // kHelpers: main
+  // kHelpers: main, the fourth wavefront (the last of four: mp_fwd_team.hip; of seven the one whose SIMD has no other)
+  const int wave = uniform_i(tid / kWave);
+  const int role = wave == 3 ? kHelpers : wave - (wave > 3 ? 1 : 0);
   const int lane = tid & (kWave - 1);
   const int l = lane & (kHalf - 1);
   const int half = lane / kHalf;
@@ -584,7 +606,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       f32x4 m[3];
       f32x2 b;
     };
-    auto get = [&](const BwdSlots& s, const int i) __attribute__((always_inline)) {
+    auto get = [&](const Slots& s, const int i) __attribute__((always_inline)) {
       In x;
 #pragma unroll
       for (int q = 0; q < 3; ++q) x.m[q] = *reinterpret_cast<const f32x4*>(&s.mask[i][half][lm][4 * q]);
@@ -595,7 +617,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
     // another: a zero mask does not switch such a term off, so the gradients go to their labels through LDS.
     // (What the normalisation takes off stays a term of its own: where the weight is not finite, that entry of
     // dcontext can be NaN here and infinite with one wavefront per chain.)
-    auto careful_block = [&](BwdSlots& s, const int k) __attribute__((always_inline)) {
+    auto careful_block = [&](Slots& s, const int k) __attribute__((always_inline)) {
 #pragma clang loop unroll(disable)
       for (int i = 0; i < kT; ++i) {
         const In cur = get(s, i);
@@ -630,7 +652,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
     f32x4 m0 = {0.f, 0.f, 0.f, 0.f};
     for (int k = 0; k < iters; ++k) {
       if (k >= 1 && k <= blocks) {
-        BwdSlots& s = sets[(k - 1) & 1];
+        Slots& s = sets[(k - 1) & 1];
         In cur = get(s, 0);
         const float sc_was = sc;
         float pairs_were[kSrc], zero = 0.f;
@@ -744,8 +766,9 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       __builtin_amdgcn_raw_buffer_store_b32((unsigned)bits(x), r, off, 0, 0);
     };
     // the loads of walk position s (nothing is read past the end of the chain)
-    auto load_pix = [&](const int s) __attribute__((always_inline)) {
+    auto load_pix = [&](const int s0) __attribute__((always_inline)) {  // (of the lower half's pixel)
       Pix r;
+      const int s = s0 + half;
       const bool on = s < n;
       const unsigned pp = (unsigned)(p_last - s * ch.pstep);
       const int off = label_off(on, pp);
@@ -756,7 +779,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       if constexpr (SOFT) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const int sh = uniform_i(s - half) + h;  // (both halves' positions are consecutive)
+          const int sh = s0 + h;
           const unsigned ph = (unsigned)(p_last - sh * ch.pstep);
           const bool edge = sh < n - 1;  // (nobody writes the duals of a chain start)
           const rsrc_t rD = make_rsrc(duals + (edge ? (int64_t)ph * kPairs : 0), edge ? kPairs * 4 : 0);
@@ -781,27 +804,29 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
 #pragma unroll
       for (int q = 0; q < kSrc; ++q) {
         const int fd = half * kSrc + q < kL ? half * kSrc + q : kL - 1, cd = ok ? l : kL - 1;
-        tcol[q] = ctx_s[cd < fd ? cd * kL + fd : fd * kL + cd];
+        const float x = ctx_s[cd < fd ? cd * kL + fd : fd * kL + cd];
+        tcol[q] = ok && half * kSrc + q < kL ? x : 0.f;
       }
     }
     struct Kept {  // of a pixel whose dU is not known yet
       float ap, base, w, de, cv, hi;
-      int fd, nidx, fn;
+      int nidx, fn;
     };
     // walk position u
-    auto prepare = [&](const Pix& px, const int u, BwdSlots& s, Kept& kp) __attribute__((always_inline)) {
-      kp.ap = EVEN ? fmaf(rho, px.hi, px.a) : px.a;
+    auto prepare = [&](const Pix& px, const int u, Slots& s, Kept& kp) __attribute__((always_inline)) {
+      kp.ap = EVEN ? fmaf(rho, px.hi, px.a) : SOFT ? keep(px.a) : px.a;
       kp.base = ok ? kp.ap + (EVEN ? -px.hd - px.hi : px.hd) : 0.f;
-      kp.w = px.w;
-      kp.de = px.de;
-      kp.fd = px.fd;
-      kp.nidx = px.nidx;
+      if (GR) {
+        kp.w = keep(px.w);
+        kp.de = keep(px.de);
+        kp.nidx = keep(px.nidx);
+      }
       *reinterpret_cast<f32x2*>(s.base[i][l]) = f32x2{kp.base, u < n - 1 ? px.w : 0.f};
       if (GR && !SOFT) {
         const int lo = l < px.fd ? l : px.fd, hi = l < px.fd ? px.fd : l;
         kp.cv = ok && px.fd < kL ? ctx_s[lo * kL + hi] : 0.f;
       }
-      if (SOFT) kp.hi = px.hi;
+      if (SOFT) kp.hi = keep(px.hi);
       if constexpr (SOFT) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -843,17 +868,21 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
           }
           halves(left2[0] + left2[1], lower, upper);
           const float left = (lower + upper) * inv;
-          float ev2[2] = {0.f, 0.f};
+          float jv[kSrc], ev2[2] = {0.f, 0.f};
 #pragma unroll
           for (int q = 0; q < kSrc; ++q) {
-            const int fd = half * kSrc + q;
             const float w = inv * ex[q];
-            const float jv = fmaf(w, d[q] - left, w);  // :110-113
-            if (ok && fd < kL) s.mask[2 * role + h][l / kSrc][fd][l % kSrc] = jv;
-            if (GR) ev2[q & 1] = fmaf(tcol[q], ok && fd < kL ? jv : 0.f, ev2[q & 1]);
+            jv[q] = fmaf(w, d[q] - left, w);  // :110-113
+            if (GR) ev2[q & 1] = fmaf(tcol[q], jv[q], ev2[q & 1]);  // (tcol: zero where there is no entry)
           }
-          // (the upper half's last source does not exist)
-          if (half == 1 && ok) s.mask[2 * role + h][1][l][kSrc - 1] = 0.f;
+          if (ok) {
+            float* const row = &s.mask[2 * role + h][l / kSrc][half * kSrc][l % kSrc];
+#pragma unroll
+            for (int q = 0; q + 1 < kSrc; ++q) row[q * 12] = jv[q];
+            // (the upper half's last source does not exist: a zero where it would be read)
+            float* const last = two ? row + (kSrc - 1) * 12 : &s.mask[2 * role + h][1][l][kSrc - 1];
+            *last = two ? jv[kSrc - 1] : 0.f;
+          }
           if (GR) {
             halves(ev2[0] + ev2[1], lower, upper);
             if (half == h) kp.cv = lower + upper;
@@ -862,7 +891,8 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
           const int nidx = __builtin_amdgcn_readlane(px.nidx, h * kHalf) & (kHalf - 1);
           const int nn = nidx < kL ? nidx : kL - 1;
           if (ok) {
-            const float jn = s.mask[2 * role + h][nn / kSrc][l][nn % kSrc];
+            const int upper_src = nn >= kSrc ? 1 : 0;
+            const float jn = s.mask[2 * role + h][upper_src][l][nn - upper_src * kSrc];
             s.mask[2 * role + h][half][l][kSrc] = nidx < kL ? jn : 0.f;
           }
         }
@@ -893,7 +923,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
       }
     };
     // what is left of a pixel once its dU is known (chain position t; nothing outside the chain)
-    auto finish = [&](const int t, const BwdSlots& s, const Kept& kp) __attribute__((always_inline)) {
+    auto finish = [&](const int t, const Slots& s, const Kept& kp) __attribute__((always_inline)) {
       const bool on = t >= 0 && t < n;
       const unsigned pp = (unsigned)(ch.pix0 + t * ch.pstep);
       const int off = label_off(on, pp);
@@ -934,7 +964,7 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
     Kept kept[2] = {};
 #pragma unroll
     for (int q = 0; q < kAhead; ++q) {
-      ring[q] = load_pix(q * kT + i);
+      ring[q] = load_pix(q * kT + 2 * role);
       MPL_ORDER_LOADS();
     }
 #pragma clang loop unroll(disable)
@@ -942,11 +972,11 @@ __global__ void __launch_bounds__(kTeam) bwd_team21_kernel(const BackParams p) {
 #pragma unroll
       for (int q = 0; q < kAhead; ++q) {
         const int k = k0 + q;
-        BwdSlots& s = sets[q & 1];
+        Slots& s = sets[q & 1];
         finish(n - 1 - ((k - 2) * kT + i), s, kept[q & 1]);
         lds_order();
         prepare(ring[q], k * kT + i, s, kept[q & 1]);
-        ring[q] = load_pix((k + kAhead) * kT + i);
+        ring[q] = load_pix((k + kAhead) * kT + 2 * role);
         lds_barrier();
       }
     }
@@ -1017,15 +1047,22 @@ void launch_team21_bwd(const BackParams& p, hipStream_t st) {
   const int blocks = p.block_prefix[p.n_dirs];
   if (blocks <= 0) return;
   const bool gr = p.dedge != nullptr || p.dctx != nullptr;
-  const size_t lds = 2 * sizeof(BwdSlots) + sizeof(float) * (kMaxL + (gr ? 2 * kPairs : 0));
-  auto kernel = p.edge_label != nullptr
-                    ? (p.dctx != nullptr ? bwd_team21_kernel<true, true, true>
-                       : gr              ? bwd_team21_kernel<true, false, true>
-                                         : bwd_team21_kernel<false, false, true>)
-                    : (p.dctx != nullptr ? bwd_team21_kernel<true, true, false>
-                       : gr              ? bwd_team21_kernel<true, false, false>
-                                         : bwd_team21_kernel<false, false, false>);
-  kernel<<<blocks, kTeam, lds, st>>>(p);
+  const auto launch = [&](auto kernel, int helpers, size_t set) {
+    const size_t lds = 2 * set + sizeof(float) * (kMaxL + (gr ? 2 * kPairs : 0));
+    kernel<<<blocks, (helpers + 1) * kWave, lds, st>>>(p);
+  };
+#define MPL_BWD21(SOFT, N)                                                                                       \
+  launch(p.dctx != nullptr ? bwd_team21_kernel<true, true, SOFT, N>                                              \
+         : gr              ? bwd_team21_kernel<true, false, SOFT, N>                                             \
+                           : bwd_team21_kernel<false, false, SOFT, N>,                                           \
+         N, sizeof(BwdSlots<2 * N>))
+  if (p.edge_label == nullptr)
+    MPL_BWD21(false, kHelpers);
+  else if (blocks <= launch_policy().n_simd / 4)
+    MPL_BWD21(true, kSoftHelpersAlone);
+  else
+    MPL_BWD21(true, kHelpers);
+#undef MPL_BWD21
 }
 
 }  // namespace mpl
