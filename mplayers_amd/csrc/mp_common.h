@@ -287,6 +287,21 @@ constexpr int load_policy(bool whole_lanes) { return whole_lanes ? MPL_LD_AUX : 
 // ISGMR 52 labels 400x600 0.66 / 0.60 with / without, TRWP 60 labels 375x450 the same.
 constexpr int store_policy(int R, bool whole_lanes) { return whole_lanes || R > 1 ? MPL_ST_AUX : 0; }
 
+// ISGMR's launches scan all directions and hand every line they write to the next pass: with both message buffers
+// larger than the 256 MB of the last-level cache, stores of whole lines that go through the dies' L2 at once (sc1, no
+// hint) leave it to the lines that are read.  Measured on whole lanes (64, 128, 192, 256 labels), 8 directions unless said,
+// this over the hint: inference, 256 labels 4 directions 256x256 0.89, 180x240 0.86, 150x200 (123 MB of messages) 0.99,
+// 140x170 (98 MB) 1.03, 512x512 0.99; 192 labels 256x512 0.92, 120x140 (103 MB) 0.94, 1000x1500 1.00; 128 labels 180x400
+// 0.86, 375x1242 0.97; 64 labels 300x400 0.88, 100x150 (31 MB) 1.03.  Argmin labels kept: 64 labels 0.90, 128 labels 0.89
+// and 0.98, but 192 labels 1.10 to 1.24 and 256 labels 1.00 (their bytes come three or four to a lane).  Not for vectors
+// that share lines: 96 labels 1.04, 150 labels 1.04, 61 labels 1.06.  (Neither hint nor sc1: 256x256 0.93, 256x512 0.94.)
+constexpr int kStoreThrough = 16;
+constexpr int64_t kStoreThroughBytes = (int64_t)128 << 20;
+template <typename Params>
+inline bool store_through(const Params& p) {
+  return (int64_t)p.n_dirs * p.B * p.H * p.W * p.L * 4 >= kStoreThroughBytes;
+}
+
 constexpr int kDeadOffset = 0x7ffffff0;  // a vector offset no descriptor covers: access suppressed
 // the same for descriptors that cover a whole image (up to kMaxImageBytes, beyond 2 GiB)
 constexpr unsigned kDeadWide = 0xfffffff0u;

@@ -70,14 +70,15 @@ __device__ __forceinline__ void split_combine(float* xchg, int n_waves, int wave
 // VEC: L % R == 0 (vector accesses).  MASK: some lanes own labels >= L.
 // C0: the table's entry 0 is its smallest (band steps only; CtxDesc::c0_is_min), which gives the
 // normalisation minimum without a second reduction.
-template <int R, bool VEC, bool MASK, bool TRAIN, int JACOBI, int KT, bool C0 = false>
+// THROUGH: store_through (mp_common.h).
+template <int R, bool VEC, bool MASK, bool TRAIN, int JACOBI, int KT, bool C0 = false, bool THROUGH = false>
 __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDesc& desc,
                                               const ChainCtx& ch, float* a_s, const float* ctx_s,
                                               const bool skip_s_store_in, float* xchg = nullptr) {
   constexpr bool SPLIT = (KT == -3);
   // (every lane full: 64, 128, 192 or 256 labels, whole cache lines)
   constexpr int kLd = load_policy(!MASK);
-  constexpr int kSt = store_policy(R, !MASK);
+  constexpr int kSt = THROUGH ? kStoreThrough : store_policy(R, !MASK);
   const int L = p.L;
   // The caller's initial messages turned out to be all zero (the usual case: the reference's
   // callers pass a cleared tensor) and this is a sweep that can profit: S = Q = U = unary, so the
@@ -539,7 +540,7 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
   }
 }
 
-template <int R, bool VEC, bool MASK, bool TRAIN, int JACOBI>
+template <int R, bool VEC, bool MASK, bool TRAIN, int JACOBI, bool THROUGH = false>
 __global__ void __launch_bounds__(kWave) sweep_fwd_kernel(const SweepParams p) {
   extern __shared__ __align__(16) float smem[];
   float* a_s = smem;            // kMaxL floats
@@ -598,25 +599,25 @@ __global__ void __launch_bounds__(kWave) sweep_fwd_kernel(const SweepParams p) {
     }
     // wide truncated-linear contexts: two label scans instead of 2K-1 taps or the dense scan
     if (desc.linear && !p.ctx2d && (desc.band_k == 0 || desc.band_k > 4)) {
-      run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, -2>(p, desc, c, a_s, ctx_s, skip_s);
+      run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, -2, false, THROUGH>(p, desc, c, a_s, ctx_s, skip_s);
       continue;
     }
     // (a band whose entry 0 is not its smallest -- no Potts, linear or quadratic table -- takes the
     // taps at run time and reduces for the normalisation minimum)
     if (desc.band_k > 0 && !desc.c0_is_min) {
-      run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 0, false>(p, desc, c, a_s, ctx_s, skip_s);
+      run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 0, false, THROUGH>(p, desc, c, a_s, ctx_s, skip_s);
       continue;
     }
     switch (desc.band_k) {
       case 0:
         if (R == 1 && L == 21 && p.ctx2d)
-          run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, (R == 1 ? -21 : -1)>(p, desc, c, a_s, ctx_s, skip_s);
+          run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, (R == 1 ? -21 : -1), false, THROUGH>(p, desc, c, a_s, ctx_s, skip_s);
         else
-          run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, -1>(p, desc, c, a_s, ctx_s, skip_s);
+          run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, -1, false, THROUGH>(p, desc, c, a_s, ctx_s, skip_s);
         break;
-      case 2: run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 2, true>(p, desc, c, a_s, ctx_s, skip_s); break;
-      case 3: run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 3, true>(p, desc, c, a_s, ctx_s, skip_s); break;
-      case 4: run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 4, true>(p, desc, c, a_s, ctx_s, skip_s); break;
+      case 2: run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 2, true, THROUGH>(p, desc, c, a_s, ctx_s, skip_s); break;
+      case 3: run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 3, true, THROUGH>(p, desc, c, a_s, ctx_s, skip_s); break;
+      case 4: run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 4, true, THROUGH>(p, desc, c, a_s, ctx_s, skip_s); break;
       default:
         // wider bands with the taps in registers: the table is constant from band_k on, so the
         // taps between band_k and the compiled width are the dense scan's own candidates
@@ -624,15 +625,15 @@ __global__ void __launch_bounds__(kWave) sweep_fwd_kernel(const SweepParams p) {
         // and pay for the larger kernel)
         if constexpr (R >= 2) {
           if (desc.band_k <= 8) {
-            run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 8, true>(p, desc, c, a_s, ctx_s, skip_s);
+            run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 8, true, THROUGH>(p, desc, c, a_s, ctx_s, skip_s);
             break;
           }
           if (desc.band_k <= 16) {
-            run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 16, true>(p, desc, c, a_s, ctx_s, skip_s);
+            run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 16, true, THROUGH>(p, desc, c, a_s, ctx_s, skip_s);
             break;
           }
         }
-        run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 0, true>(p, desc, c, a_s, ctx_s, skip_s);
+        run_chain_fwd<R, VEC, MASK, TRAIN, JACOBI, 0, true, THROUGH>(p, desc, c, a_s, ctx_s, skip_s);
         break;
     }
   }
@@ -711,6 +712,15 @@ void launch_vm(const SweepParams& p, bool jacobi, hipStream_t st) {
   const int blocks = p.block_prefix[p.n_dirs];
   const size_t lds = fwd_lds_bytes(p.L, p.ctx2d);
   const int mode = jacobi ? (p.u_fused ? 2 : 1) : 0;
+  if constexpr (!MASK && (!TRAIN || R <= 2)) {
+    if (jacobi && store_through(p)) {
+      if (mode == 2)
+        sweep_fwd_kernel<R, VEC, MASK, TRAIN, 2, true><<<blocks, kWave, lds, st>>>(p);
+      else
+        sweep_fwd_kernel<R, VEC, MASK, TRAIN, 1, true><<<blocks, kWave, lds, st>>>(p);
+      return;
+    }
+  }
   if (mode == 2)
     sweep_fwd_kernel<R, VEC, MASK, TRAIN, 2><<<blocks, kWave, lds, st>>>(p);
   else if (mode == 1)
