@@ -76,29 +76,27 @@ __global__ void __launch_bounds__(kWave) analyze_context_kernel(const float* __r
 // plane size is a multiple of 4, else 1); ND: number of directions when it is one of the usual ones
 // (loads of all planes are then issued back to back), 0: run-time loop.
 // ------------------------------------------------------------------------------------------------
-#ifndef MPL_EW_NT
-#define MPL_EW_NT 1  // planes are streamed once: non-temporal loads and stores
-#endif
+// NT: the non-temporal hint on loads and stores (planes are streamed once; ew_hint).
 template <int V>
 struct Pack {
   float v[V];
 };
-template <int V>
+template <int V, bool NT>
 __device__ __forceinline__ Pack<V> ld_pack(const float* p) {
   Pack<V> r;
   if constexpr (V == 4) {
-    const f32x4 t = MPL_EW_NT ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p))
+    const f32x4 t = NT ? __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p))
                               : *reinterpret_cast<const f32x4*>(p);
     r.v[0] = t.x;
     r.v[1] = t.y;
     r.v[2] = t.z;
     r.v[3] = t.w;
   } else {
-    r.v[0] = MPL_EW_NT ? __builtin_nontemporal_load(p) : *p;
+    r.v[0] = NT ? __builtin_nontemporal_load(p) : *p;
   }
   return r;
 }
-template <int V>
+template <int V, bool NT>
 __device__ __forceinline__ void st_pack(float* p, const Pack<V>& r) {
   if constexpr (V == 4) {
     f32x4 t;
@@ -106,12 +104,12 @@ __device__ __forceinline__ void st_pack(float* p, const Pack<V>& r) {
     t.y = r.v[1];
     t.z = r.v[2];
     t.w = r.v[3];
-    if (MPL_EW_NT)
+    if (NT)
       __builtin_nontemporal_store(t, reinterpret_cast<f32x4*>(p));
     else
       *reinterpret_cast<f32x4*>(p) = t;
   } else {
-    if (MPL_EW_NT)
+    if (NT)
       __builtin_nontemporal_store(r.v[0], p);
     else
       *p = r.v[0];
@@ -119,7 +117,7 @@ __device__ __forceinline__ void st_pack(float* p, const Pack<V>& r) {
 }
 
 // S = unary + sum_k m_k  (k ascending, as UpdateUnaryKernel sums, TRWP_forward.cu:70-73)
-template <int V, int ND>
+template <int V, int ND, bool NT>
 __global__ void __launch_bounds__(256) belief_kernel(const float* __restrict__ unary,
                                                      const float* __restrict__ msg, int n_dir_rt,
                                                      int64_t N, float* __restrict__ S,
@@ -130,11 +128,11 @@ __global__ void __launch_bounds__(256) belief_kernel(const float* __restrict__ u
   bool any = false;  // some message of this thread's elements is not zero
   for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V; i < N;
        i += (int64_t)gridDim.x * blockDim.x * V) {
-    Pack<V> v = ld_pack<V>(unary + i);
+    Pack<V> v = ld_pack<V, NT>(unary + i);
     if constexpr (ND > 0) {
       Pack<V> m[ND];
 #pragma unroll
-      for (int k = 0; k < ND; ++k) m[k] = ld_pack<V>(msg + (int64_t)k * N + i);
+      for (int k = 0; k < ND; ++k) m[k] = ld_pack<V, NT>(msg + (int64_t)k * N + i);
 #pragma unroll
       for (int k = 0; k < ND; ++k)
 #pragma unroll
@@ -144,7 +142,7 @@ __global__ void __launch_bounds__(256) belief_kernel(const float* __restrict__ u
         }
     } else {
       for (int k = 0; k < n_dir; ++k) {
-        const Pack<V> m = ld_pack<V>(msg + (int64_t)k * N + i);
+        const Pack<V> m = ld_pack<V, NT>(msg + (int64_t)k * N + i);
 #pragma unroll
         for (int j = 0; j < V; ++j) {
           v.v[j] += m.v[j];
@@ -152,7 +150,7 @@ __global__ void __launch_bounds__(256) belief_kernel(const float* __restrict__ u
         }
       }
     }
-    st_pack<V>(S + i, v);
+    st_pack<V, NT>(S + i, v);
   }
   if (nonzero_flag != nullptr && any) *nonzero_flag = 1;  // every writer stores the same value
 }
@@ -160,7 +158,7 @@ __global__ void __launch_bounds__(256) belief_kernel(const float* __restrict__ u
 // Sets *flag when some element of the n_dir message planes is not zero (every writer stores the
 // same value).  The reference's callers pass cleared message tensors; knowing that on the device
 // lets the first sweeps read the unary terms in place of planes that would have to be built first.
-template <int V, int ND>
+template <int V, int ND, bool NT>
 __global__ void __launch_bounds__(256) check_nonzero_kernel(const float* __restrict__ msg,
                                                             int n_dir_rt, int64_t N, int* flag) {
   const int n_dir = ND > 0 ? ND : n_dir_rt;
@@ -170,14 +168,14 @@ __global__ void __launch_bounds__(256) check_nonzero_kernel(const float* __restr
     if constexpr (ND > 0) {
       Pack<V> m[ND];
 #pragma unroll
-      for (int k = 0; k < ND; ++k) m[k] = ld_pack<V>(msg + (int64_t)k * N + i);
+      for (int k = 0; k < ND; ++k) m[k] = ld_pack<V, NT>(msg + (int64_t)k * N + i);
 #pragma unroll
       for (int k = 0; k < ND; ++k)
 #pragma unroll
         for (int j = 0; j < V; ++j) any = any || (m[k].v[j] != 0.f);
     } else {
       for (int k = 0; k < n_dir; ++k) {
-        const Pack<V> m = ld_pack<V>(msg + (int64_t)k * N + i);
+        const Pack<V> m = ld_pack<V, NT>(msg + (int64_t)k * N + i);
 #pragma unroll
         for (int j = 0; j < V; ++j) any = any || (m.v[j] != 0.f);
       }
@@ -190,7 +188,7 @@ __global__ void __launch_bounds__(256) check_nonzero_kernel(const float* __restr
 //   U_d = rho * (unary + sum_k m_k - m_d) - m_{d^1}      (UpdateUnaryKernel, ISGMR_forward.cu:101-121)
 // so U_d is stored once per iteration (in place of m_d, or into the other message buffer) before
 // the sweeps: a sweep then reads one plane per pixel, not three.
-template <int V, int ND>
+template <int V, int ND, bool NT>
 __global__ void __launch_bounds__(256) isgmr_unary_kernel(const float* __restrict__ unary,
                                                           const float* msg, float* out,
                                                           int n_dir_rt, int64_t N, float rho,
@@ -200,12 +198,12 @@ __global__ void __launch_bounds__(256) isgmr_unary_kernel(const float* __restric
   const int n_dir = ND > 0 ? ND : n_dir_rt;
   for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V; i < N;
        i += (int64_t)gridDim.x * blockDim.x * V) {
-    Pack<V> S = ld_pack<V>(unary + i);
+    Pack<V> S = ld_pack<V, NT>(unary + i);
     Pack<V> m[KD];
 #pragma unroll
     for (int k = 0; k < KD; ++k) {
       if (k < n_dir) {
-        m[k] = ld_pack<V>(msg + (int64_t)k * N + i);
+        m[k] = ld_pack<V, NT>(msg + (int64_t)k * N + i);
       } else {
 #pragma unroll
         for (int j = 0; j < V; ++j) m[k].v[j] = 0.f;
@@ -225,7 +223,7 @@ __global__ void __launch_bounds__(256) isgmr_unary_kernel(const float* __restric
         Pack<V> u;
 #pragma unroll
         for (int j = 0; j < V; ++j) u.v[j] = fmaf(S.v[j] - m[k].v[j], rho, -m[k ^ 1].v[j]);
-        st_pack<V>(out + (int64_t)k * N + i, u);  // out == msg: in place
+        st_pack<V, NT>(out + (int64_t)k * N + i, u);  // out == msg: in place
       }
     }
   }
@@ -233,7 +231,7 @@ __global__ void __launch_bounds__(256) isgmr_unary_kernel(const float* __restric
 
 // cost = factor*unary + sum_k m_k  (or + min_k m_k): CostAggregateKernel, TRWP_forward.cu:31-58,
 // ISGMR_forward.cu:69-99.
-template <int V, int ND>
+template <int V, int ND, bool NT>
 __global__ void __launch_bounds__(256) aggregate_kernel(const float* __restrict__ unary,
                                                         const float* __restrict__ msg, int n_dir_rt,
                                                         int64_t N, float factor, int min_a_dir,
@@ -241,7 +239,7 @@ __global__ void __launch_bounds__(256) aggregate_kernel(const float* __restrict_
   const int n_dir = ND > 0 ? ND : n_dir_rt;
   for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V; i < N;
        i += (int64_t)gridDim.x * blockDim.x * V) {
-    Pack<V> v = ld_pack<V>(unary + i);
+    Pack<V> v = ld_pack<V, NT>(unary + i);
 #pragma unroll
     for (int j = 0; j < V; ++j) v.v[j] *= factor;
     Pack<V> mn;  // min_a_dir only
@@ -259,17 +257,17 @@ __global__ void __launch_bounds__(256) aggregate_kernel(const float* __restrict_
     if constexpr (ND > 0) {
       Pack<V> m[ND];
 #pragma unroll
-      for (int k = 0; k < ND; ++k) m[k] = ld_pack<V>(msg + (int64_t)k * N + i);
+      for (int k = 0; k < ND; ++k) m[k] = ld_pack<V, NT>(msg + (int64_t)k * N + i);
 #pragma unroll
       for (int k = 0; k < ND; ++k) fold(k, m[k]);
     } else {
-      for (int k = 0; k < n_dir; ++k) fold(k, ld_pack<V>(msg + (int64_t)k * N + i));
+      for (int k = 0; k < n_dir; ++k) fold(k, ld_pack<V, NT>(msg + (int64_t)k * N + i));
     }
     if (min_a_dir) {
 #pragma unroll
       for (int j = 0; j < V; ++j) v.v[j] += mn.v[j];
     }
-    st_pack<V>(cost + i, v);
+    st_pack<V, NT>(cost + i, v);
   }
 }
 
@@ -325,7 +323,7 @@ __global__ void __launch_bounds__(256) label_kernel(const float* __restrict__ un
 // The loads of all planes going out back to back are not what gives it: 10 iterations, TRWP 6.20 -> 5.99 ms
 // and ISGMR 3.75 -> 3.19, but 6.18 -> 6.14 and 3.76 -> 3.72 with min_a_dir, where nothing is merged.
 constexpr int kLabelOnly = 0, kLabelSum = 1, kLabelU = 2;
-template <int ND, int OUT>
+template <int ND, int OUT, bool NT>
 __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict__ unary,
                                                          const float* msg, int n_dir_rt, int64_t P,
                                                          int L, int group, float factor,
@@ -340,13 +338,13 @@ __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict
   int arg = 0x7fffffff;
   if (pix < P && sub * 4 < L) {
     const int64_t i = pix * L + sub * 4;
-    Pack<4> v = ld_pack<4>(unary + i);
+    Pack<4> v = ld_pack<4, NT>(unary + i);
     Pack<4> m[ND > 0 ? ND : 1];
     if constexpr (ND > 0) {
 #pragma unroll
-      for (int k = 0; k < ND; ++k) m[k] = ld_pack<4>(msg + (int64_t)k * N + i);
+      for (int k = 0; k < ND; ++k) m[k] = ld_pack<4, NT>(msg + (int64_t)k * N + i);
     }
-    auto message = [&](int k) { return ND > 0 ? m[ND > 0 ? k : 0] : ld_pack<4>(msg + (int64_t)k * N + i); };
+    auto message = [&](int k) { return ND > 0 ? m[ND > 0 ? k : 0] : ld_pack<4, NT>(msg + (int64_t)k * N + i); };
 #pragma unroll
     for (int j = 0; j < 4; ++j) v.v[j] *= factor;
     if (OUT == kLabelOnly && min_a_dir) {
@@ -368,7 +366,7 @@ __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict
         for (int j = 0; j < 4; ++j) v.v[j] += mk.v[j];
       }
     }
-    if constexpr (OUT == kLabelSum) st_pack<4>(out + i, v);
+    if constexpr (OUT == kLabelSum) st_pack<4, NT>(out + i, v);
     if constexpr (OUT == kLabelU) {
 #pragma unroll
       for (int k = 0; k < ND; ++k)
@@ -376,7 +374,7 @@ __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict
           Pack<4> u;
 #pragma unroll
           for (int j = 0; j < 4; ++j) u.v[j] = fmaf(v.v[j] - m[k].v[j], rho, -m[k ^ 1].v[j]);
-          st_pack<4>(out + (int64_t)k * N + i, u);  // out == msg: in place
+          st_pack<4, NT>(out + (int64_t)k * N + i, u);  // out == msg: in place
         }
     }
 #pragma unroll
@@ -400,7 +398,7 @@ __global__ void __launch_bounds__(256) label_quad_kernel(const float* __restrict
 // Returns whether `out` has been written (want: what to store there besides the labels).
 static bool launch_labels(const float* unary, const float* msg, int n_dir, int64_t P, int L,
                           float factor, int min_a_dir, uint8_t* label, hipStream_t st,
-                          int want = kLabelOnly, float* out = nullptr, float rho = 1.f,
+                          bool nt, int want = kLabelOnly, float* out = nullptr, float rho = 1.f,
                           int pair_share = 0) {
   const bool aligned = (((uintptr_t)unary | (uintptr_t)msg) & 15) == 0;
   if ((L & 3) != 0 || !aligned) {
@@ -420,8 +418,8 @@ static bool launch_labels(const float* unary, const float* msg, int n_dir, int64
       (want == kLabelU && !known))
     want = kLabelOnly;
 #define MPL_LABELS(ND, OUT)                                                                          \
-  label_quad_kernel<ND, OUT><<<blocks, 256, 0, st>>>(unary, msg, n_dir, P, L, group, factor, min_a_dir, \
-                                                     label, out, rho, pair_share)
+  (nt ? label_quad_kernel<ND, OUT, true> : label_quad_kernel<ND, OUT, false>)<<<blocks, 256, 0, st>>>( \
+      unary, msg, n_dir, P, L, group, factor, min_a_dir, label, out, rho, pair_share)
 #define MPL_LABELS_ND(ND)                             \
   do {                                                \
     if (want == kLabelU)                              \
@@ -449,7 +447,7 @@ static bool launch_labels(const float* unary, const float* msg, int n_dir, int64
 // ISGMR: after all directions of an iteration have been scanned back (X_k = dU_k):
 //   dunary += rho * sum_k X_k ;  gu_k = rho * (sum - X_k) - X_{k^1}   (written to G)
 // (UpdateUnaryKernelBack summed over directions + SumMsgKernel, ISGMR_backward.cu:39-60, 482-483)
-template <int V, int ND>
+template <int V, int ND, bool NT>
 __global__ void __launch_bounds__(256) isgmr_combine_kernel(const float* X, float* G, int n_dir_rt,
                                                             int64_t N, float rho,
                                                             const float* __restrict__ dcost,
@@ -464,13 +462,13 @@ __global__ void __launch_bounds__(256) isgmr_combine_kernel(const float* X, floa
 #pragma unroll
     for (int k = 0; k < KD; ++k) {
       if (k < n_dir) {
-        x[k] = ld_pack<V>(X + (int64_t)k * N + i);
+        x[k] = ld_pack<V, NT>(X + (int64_t)k * N + i);
       } else {
 #pragma unroll
         for (int j = 0; j < V; ++j) x[k].v[j] = 0.f;
       }
     }
-    Pack<V> du = init_dunary ? ld_pack<V>(dcost + i) : ld_pack<V>(dunary + i);
+    Pack<V> du = init_dunary ? ld_pack<V, NT>(dcost + i) : ld_pack<V, NT>(dunary + i);
     Pack<V> sum;
 #pragma unroll
     for (int j = 0; j < V; ++j) {
@@ -481,7 +479,7 @@ __global__ void __launch_bounds__(256) isgmr_combine_kernel(const float* X, floa
       if (init_dunary) du.v[j] *= factor;
       du.v[j] = fmaf(rho, sum.v[j], du.v[j]);
     }
-    st_pack<V>(dunary + i, du);
+    st_pack<V, NT>(dunary + i, du);
     if (write_gu) {
 #pragma unroll
       for (int k = 0; k < KD; ++k) {
@@ -491,7 +489,7 @@ __global__ void __launch_bounds__(256) isgmr_combine_kernel(const float* X, floa
           Pack<V> g;
 #pragma unroll
           for (int j = 0; j < V; ++j) g.v[j] = fmaf(rho, sum.v[j] - x[k].v[j], -x[k ^ 1].v[j]);
-          st_pack<V>(G + (int64_t)k * N + i, g);
+          st_pack<V, NT>(G + (int64_t)k * N + i, g);
         }
       }
     }
@@ -604,22 +602,42 @@ int elementwise_blocks(int64_t n) {
   return (int)b;
 }
 
+// Whether the element-wise passes over the planes carry the non-temporal hint: not where the messages fit the
+// last-level cache (256 MB) and the label vectors share lines, whose scans read and write without it (load_policy).
+// Measured, ISGMR with 8 directions, without over with, forward / keeping argmin labels / backward: 21 labels
+// 12x65x65 (34 MB of messages) 0.98 / 0.98 / 0.98, 12x129x129 (134 MB) 0.92 / 0.99 / 1.01; 60 labels 100x150 0.93 / 0.97 /
+// 0.99, 200x250 0.91 / 0.97 / 1.00, 300x400 (220 MiB) 1.09 / 1.09 / 1.05; 150 labels 180x250 (206 MiB) 0.94 / 0.93 / 0.99,
+// 300x400 1.03 / 1.01 / 1.04; 100 labels 200x300 0.93 / 0.94 / 0.98.  Whole lines: 64 labels 100x150 1.04, 300x400 1.03;
+// 96 labels 384x1248 1.04.
+constexpr int64_t kCachedMessages = (int64_t)208 << 20;
+bool ew_hint(const mpl_shape* s) {
+  const int64_t messages = (int64_t)s->n_dir * s->batch * s->height * s->width * s->n_disp * 4;
+  return (s->n_disp * 4) % kLineBytes == 0 || messages > kCachedMessages;
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Picks the instantiation of an element-wise kernel: 4 floats per access when the planes allow it,
 // the direction count as a compile-time constant when it is 4, 8 or 16.
-#define MPL_EW_LAUNCH(KERNEL, VEC4, NDIR, N, ST, ...)                                            \
+#define MPL_EW_LAUNCH(KERNEL, VEC4, NT, NDIR, N, ST, ...)                                         \
+  do {                                                                                           \
+    if (NT)                                                                                      \
+      MPL_EW_LAUNCH_NT(KERNEL, VEC4, true, NDIR, N, ST, __VA_ARGS__);                            \
+    else                                                                                         \
+      MPL_EW_LAUNCH_NT(KERNEL, VEC4, false, NDIR, N, ST, __VA_ARGS__);                           \
+  } while (0)
+#define MPL_EW_LAUNCH_NT(KERNEL, VEC4, NT, NDIR, N, ST, ...)                                      \
   do {                                                                                           \
     const int blocks_ = elementwise_blocks((VEC4) ? (N) / 4 : (N));                              \
     if (VEC4) {                                                                                  \
       switch (NDIR) {                                                                            \
-        case 4: KERNEL<4, 4><<<blocks_, 256, 0, ST>>>(__VA_ARGS__); break;                       \
-        case 8: KERNEL<4, 8><<<blocks_, 256, 0, ST>>>(__VA_ARGS__); break;                       \
-        case 16: KERNEL<4, 16><<<blocks_, 256, 0, ST>>>(__VA_ARGS__); break;                     \
-        default: KERNEL<4, 0><<<blocks_, 256, 0, ST>>>(__VA_ARGS__); break;                      \
+        case 4: KERNEL<4, 4, NT><<<blocks_, 256, 0, ST>>>(__VA_ARGS__); break;                   \
+        case 8: KERNEL<4, 8, NT><<<blocks_, 256, 0, ST>>>(__VA_ARGS__); break;                   \
+        case 16: KERNEL<4, 16, NT><<<blocks_, 256, 0, ST>>>(__VA_ARGS__); break;                 \
+        default: KERNEL<4, 0, NT><<<blocks_, 256, 0, ST>>>(__VA_ARGS__); break;                  \
       }                                                                                          \
     } else {                                                                                     \
-      KERNEL<1, 0><<<blocks_, 256, 0, ST>>>(__VA_ARGS__);                                        \
+      KERNEL<1, 0, NT><<<blocks_, 256, 0, ST>>>(__VA_ARGS__);                                    \
     }                                                                                            \
   } while (0)
 
@@ -946,7 +964,7 @@ __global__ void __launch_bounds__(256) zero_fill_kernel(float* __restrict__ dst,
   for (int j = 0; j < V; ++j) z.v[j] = 0.f;
   for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V; i < n;
        i += (int64_t)gridDim.x * blockDim.x * V)
-    st_pack<V>(dst + i, z);
+    st_pack<V, true>(dst + i, z);
 }
 
 void zero_fill(float* dst, int64_t n, hipStream_t st) {
@@ -995,7 +1013,7 @@ void rebuild_belief(const mpl_shape* s, const float* unary, const float* msg, fl
   Timed timed(MPL_KERNEL_BELIEF, st);
   const int64_t N = (int64_t)s->batch * s->height * s->width * s->n_disp;
   const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(S);
-  MPL_EW_LAUNCH(belief_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, S, (int*)nullptr);
+  MPL_EW_LAUNCH(belief_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, S, (int*)nullptr);
 }
 
 // dcontext = the sum of the tables the reverse scans added to (MPL_F_DCONTEXT_COPIES), always in the same order
@@ -1232,11 +1250,11 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
     const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(unary_update);
     int* flag = desc != nullptr ? &const_cast<CtxDesc*>(desc)->msg_nonzero : nullptr;
     if (probe_zero) {
-      MPL_EW_LAUNCH(check_nonzero_kernel, v4, s->n_dir, N, st, msg, s->n_dir, N, flag);
-      MPL_EW_LAUNCH(belief_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, unary_update,
+      MPL_EW_LAUNCH(check_nonzero_kernel, v4, ew_hint(s), s->n_dir, N, st, msg, s->n_dir, N, flag);
+      MPL_EW_LAUNCH(belief_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, unary_update,
                     (int*)nullptr, (const int*)flag);
     } else {
-      MPL_EW_LAUNCH(belief_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, unary_update, flag);
+      MPL_EW_LAUNCH(belief_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, unary_update, flag);
     }
   }
 
@@ -1285,14 +1303,14 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
       const bool last = it + 1 == n_iter;
       float* out = last ? cost_final : (rebuild > 0 && (it + 1) % rebuild == 0) ? unary_update : nullptr;
       const bool stored = launch_labels(unary, msg, s->n_dir, P, s->n_disp, 1.f, enable_min_a_dir,
-                                        label_all + it * P, st, kLabelSum, out);
+                                        label_all + it * P, st, ew_hint(s), kLabelSum, out);
       (last ? have_cost : have_belief) = stored;
     }
   }
   if (!have_cost) {
     Timed timed(MPL_KERNEL_AGGREGATE, st);
     const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
-    MPL_EW_LAUNCH(aggregate_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, 1.f,
+    MPL_EW_LAUNCH(aggregate_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, 1.f,
                   enable_min_a_dir, cost_final);
   }
   return launch_ok("trwp_forward");
@@ -1376,11 +1394,11 @@ int mpl_isgmr_forward(const mpl_shape* s, unsigned flags, int enable_sgm, float 
       const int* only_if = nullptr;
       if (probe_zero && it == 0) {
         int* flag = &const_cast<CtxDesc*>(desc)->msg_nonzero;
-        MPL_EW_LAUNCH(check_nonzero_kernel, v4, s->n_dir, N, st, have, s->n_dir, N, flag);
+        MPL_EW_LAUNCH(check_nonzero_kernel, v4, ew_hint(s), s->n_dir, N, st, have, s->n_dir, N, flag);
         only_if = flag;
         p.zero_first = 1;
       }
-      MPL_EW_LAUNCH(isgmr_unary_kernel, v4, s->n_dir, N, st, unary, have, ubuf, s->n_dir, N, rho,
+      MPL_EW_LAUNCH(isgmr_unary_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, have, ubuf, s->n_dir, N, rho,
                     p.u_pair_share, only_if);
       p.msg_in = ubuf;
       p.u_stride = N;
@@ -1398,7 +1416,7 @@ int mpl_isgmr_forward(const mpl_shape* s, unsigned flags, int enable_sgm, float 
       // place of these messages, unless its scans form U themselves
       const bool last = it + 1 == n_iter;
       const bool stored = launch_labels(unary, nxt, s->n_dir, P, s->n_disp, factor, enable_min_a_dir,
-                                        label_all + it * P, st, last ? kLabelSum : kLabelU,
+                                        label_all + it * P, st, ew_hint(s), last ? kLabelSum : kLabelU,
                                         last ? cost_final : fuse_u ? nullptr : nxt, rho, p.u_pair_share);
       (last ? have_cost : have_u) = stored;
     }
@@ -1407,7 +1425,7 @@ int mpl_isgmr_forward(const mpl_shape* s, unsigned flags, int enable_sgm, float 
   if (!have_cost) {
     Timed timed(MPL_KERNEL_AGGREGATE, st);
     const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
-    MPL_EW_LAUNCH(aggregate_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, factor,
+    MPL_EW_LAUNCH(aggregate_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, factor,
                   enable_min_a_dir, cost_final);
   }
   return launch_ok("isgmr_forward");
@@ -1528,7 +1546,7 @@ int mpl_isgmr_backward(const mpl_shape* s, unsigned flags, int enable_sgm, float
     Timed timed(MPL_KERNEL_COMBINE, st);
     const bool v4 = (N % 4 == 0) && aligned16(dmsg_update) && aligned16(gu_buf) &&
                     aligned16(dcost_final) && aligned16(dunary);
-    MPL_EW_LAUNCH(isgmr_combine_kernel, v4, s->n_dir, N, st, dmsg_update, gu_buf, s->n_dir, N, rho,
+    MPL_EW_LAUNCH(isgmr_combine_kernel, v4, ew_hint(s), s->n_dir, N, st, dmsg_update, gu_buf, s->n_dir, N, rho,
                   dcost_final, factor, first ? 1 : 0, it > 0 ? 1 : 0, pair_share, dunary);
   }
   fold_dcontext(p, dcontext, st);
@@ -1564,7 +1582,7 @@ int mpl_trwp_soft_forward(const mpl_shape* s, unsigned flags, float rho, int n_i
   {
     Timed timed(MPL_KERNEL_BELIEF, st);
     const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(unary_update);
-    MPL_EW_LAUNCH(belief_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, unary_update,
+    MPL_EW_LAUNCH(belief_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, unary_update,
                   (int*)nullptr);
   }
   SweepParams p = base_fwd_params(s, rho, edge_weights, context, nullptr);
@@ -1600,14 +1618,14 @@ int mpl_trwp_soft_forward(const mpl_shape* s, unsigned flags, float rho, int n_i
       const bool last = it + 1 == n_iter;
       float* out = last ? cost_final : (rebuild > 0 && (it + 1) % rebuild == 0) ? unary_update : nullptr;
       const bool stored = launch_labels(unary, msg, s->n_dir, P, s->n_disp, 1.f, 0,
-                                        label_all + it * P, st, kLabelSum, out);
+                                        label_all + it * P, st, ew_hint(s), kLabelSum, out);
       (last ? have_cost : have_belief) = stored;
     }
   }
   if (!have_cost) {
     Timed timed(MPL_KERNEL_AGGREGATE, st);
     const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
-    MPL_EW_LAUNCH(aggregate_kernel, v4, s->n_dir, N, st, unary, msg, s->n_dir, N, 1.f, 0,
+    MPL_EW_LAUNCH(aggregate_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, 1.f, 0,
                   cost_final);
   }
   return launch_ok("trwp_soft_forward");
