@@ -859,7 +859,9 @@ int choose_split(const mpl_shape* s, const Params& p, const CallOpts& o, bool tr
 // 192 labels 4172 / 2242 / 3079 / 1223; 1248 chains: 16 labels 681 / - / 480 / 563, 32 labels 922 / - / 718 /
 // 563, 96 labels 2858 / 2115 / 2635 / 1555, 192 labels 5568 / 4356 / 6342 / 3742.  Without them, 256 chains: 32
 // labels 551 / - / 498 / 313, 96 labels 1602 / 770 / 1459 / 587, 192 labels 3078 / 1167 / 2962 / 915; 1248
-// chains: 96 labels 2083 / 1486 / 1902 / 1300, 192 labels 4159 / 3701 / 4141 / 2813.
+// chains: 96 labels 2083 / 1486 / 1902 / 1300, 192 labels 4159 / 3701 / 4141 / 2813.  (The last column before it had
+// servers; with them, kept / not, 256 chains: 17 and 32 labels 287 / 285, 64 labels 327 / 322, 96 labels 458 / 447, 192
+// labels 838 / 789; 1248 chains: 96 labels 1454 / 1411, 192 labels, which have none there, 3705 / 2856.)
 constexpr int kDenseTeamMinL = 17;
 constexpr int kDenseTeamChainsPerCu = 5;
 int decide_dense_team(const SweepParams& p, const CallOpts& o, bool train) {
