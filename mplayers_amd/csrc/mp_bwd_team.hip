@@ -5,8 +5,8 @@
 // SIMD to itself issues one instruction every four clocks, and the step of mp_bwd.hip is some 230
 // instructions (R = 3, dunary alone; 374 issue slots with its waits), of which the next pixel waits for
 // perhaps a third.  So the work is divided by what the recurrence needs:
-//   * three helper wavefronts, every third pixel each, load the planes, form the gradient terms that
-//     do not depend on the recurrence and the addresses of the scatter, and put them into an LDS slot
+//   * three helper wavefronts, every third pixel each (six and every sixth: launch_vj), load the planes, form the
+//     gradient terms that do not depend on the recurrence and the addresses of the scatter, and put them into an LDS slot
 //     per pixel; two blocks of pixels later they take dU of the pixel from the slot, finish the planes
 //     it goes into, store them, and add to dedge_weights and dcontext,
 //   * the main wavefront touches LDS only: gradient of the message, its sum (the normalisation), the
@@ -29,9 +29,8 @@
 // this: 256x512x192 5.16 -> 2.12 ms (rows of 256 chains: 645 -> 246 ns per pixel and walk; the main
 // wavefront issues 112 instructions per pixel, some five clocks each), with dedge_weights and dcontext
 // 7.18 -> 3.8, 500x800x192 8.91 -> 5.87; bent table 240x320x96 with dcontext 5.95 -> 3.18.  Argmin labels
-// anywhere, so that every pixel scatters through LDS adds, 459 instead of 243 ns with 192 labels.  Two
-// pixels per helper and block, three helpers: one pixel 2.14, four 2.36, seven helpers of one pixel 2.11
-// (and 6.2 instead of 5.9 ms at 500x800x192).  Which launches take it: team_chains_per_cu (mp_api.hip).
+// anywhere, so that every pixel scatters through LDS adds, 459 instead of 243 ns with 192 labels.  Three helpers with
+// two pixels each of a block; with one pixel 2.14, with four 2.36; six helpers of one pixel: launch_vj.  Which launches take it: team_chains_per_cu (mp_api.hip).
 //
 // Errors against 64 bits, one wavefront -> four, geometric means of the relative 2-norm over bands, a bent
 // band, linear and random tables, gradients of a cross entropy, normal and positive ones, 65 to 254
@@ -48,10 +47,7 @@
 namespace mpl {
 namespace {
 
-constexpr int kHelpers = 3;              // one SIMD of the compute unit each, the main one the fourth
-constexpr int kPer = 2;                  // pixels of a block per helper
-constexpr int kT = kHelpers * kPer;      // pixels per block
-constexpr int kTeam = (kHelpers + 1) * kWave;
+constexpr int kT = 6;                    // pixels per block, shared out among three or six helpers (launch_vj)
 
 constexpr int kWin = 2;                  // labels on either side whose gradients move in registers
 
@@ -276,8 +272,10 @@ __device__ __forceinline__ void lds_order() {  // of this wavefront's own LDS in
 }
 
 // GR: dedge_weights and / or dcontext are wanted
-template <int R, bool VEC, bool JACOBI, bool GR>
-__global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams p, const int turn_every) {
+template <int R, bool VEC, bool JACOBI, bool GR, int kHelpers>
+__global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_bwd_team_kernel(const BackParams p, const int turn_every) {
+  constexpr int kPer = kT / kHelpers;  // pixels of a block per helper
+  constexpr int kTeam = (kHelpers + 1) * kWave;
   extern __shared__ __align__(16) char smem_raw[];
   Slot<R>* slots = reinterpret_cast<Slot<R>*>(smem_raw);  // two sets of kT
   Scalars* scal = reinterpret_cast<Scalars*>(slots + 2 * kT);
@@ -293,7 +291,9 @@ __global__ void __launch_bounds__(kTeam) sweep_bwd_team_kernel(const BackParams 
   // and 4 workgroups per unit), so the main wavefronts of up to four of them are on SIMDs of their own.
   // With four labels per lane and turn_every > 0 (launch_vj) it moves on by one every so many workgroups.
   const int turn = R == 4 && turn_every > 0 ? (int)blockIdx.x / turn_every : 0;
-  const int role = uniform_i((tid / kWave + turn) & 3);  // kHelpers: main
+  // (of seven wavefronts the main one is the fourth, whose SIMD has only one of them)
+  const int wave = uniform_i(tid / kWave);
+  const int role = kHelpers == 3 ? (wave + turn) & 3 : wave == 3 ? kHelpers : wave - (wave > 3 ? 1 : 0);  // kHelpers: main
   const int64_t HW = (int64_t)p.H * p.W;
   const int64_t P = (int64_t)p.B * HW;
   const int64_t N = P * L;
@@ -704,8 +704,11 @@ template <int R, bool VEC, bool JACOBI>
 void launch_vj(const BackParams& p, hipStream_t st) {
   const int blocks = p.block_prefix[p.n_dirs];
   const bool gr = p.dedge != nullptr || p.dctx != nullptr;
-  const size_t lds = 2 * kT * (sizeof(Slot<R>) + sizeof(Scalars)) +
-                     sizeof(float) * (kAccFloats + (gr ? p.L + kHelpers * hist_floats(R, p.L) : 0));
+  const auto launch = [&](auto kernel, int helpers, int turn_every) {
+    const size_t lds = 2 * kT * (sizeof(Slot<R>) + sizeof(Scalars)) +
+                       sizeof(float) * (kAccFloats + (gr ? p.L + helpers * hist_floats(R, p.L) : 0));
+    kernel<<<blocks, (helpers + 1) * kWave, lds, st>>>(p, turn_every);
+  };
   // With four labels per lane the LDS holds two workgroups of a unit, and a launch of more runs in rounds.  When
   // both end together the next ones are placed in pairs again and the last round takes as long as the first;
   // with the main wavefronts of a unit's workgroups on one SIMD they do not.  Measured, 760 rows of 300 pixels,
@@ -713,10 +716,20 @@ void launch_vj(const BackParams& p, hipStream_t st) {
   // 500 rows 0.710 / 0.723, 1.55 / 1.60, 1.72 / 1.78.
   const int n_cu = launch_policy().n_simd / 4;
   const int turn_every = R == 4 && blocks > 2 * n_cu ? n_cu : 0;
-  if (gr)
-    sweep_bwd_team_kernel<R, VEC, JACOBI, true><<<blocks, kTeam, lds, st>>>(p, turn_every);
-  else
-    sweep_bwd_team_kernel<R, VEC, JACOBI, false><<<blocks, kTeam, lds, st>>>(p, turn_every);
+  // Six helpers where the launch has at most three chains per unit: what they do for a pixel bounds the scan wherever
+  // dcontext or dedge_weights are wanted, and three of them on a SIMD of their own each issue less than half of the
+  // time.  Over three helpers, dunary alone / with dedge_weights / with both, rows of 129: 192 labels, min(k, 3), 256
+  // chains 0.95 / 0.81 / 0.82, 512 chains 0.98 / 0.84 / 0.92, 768 chains 1.00 / 0.92 / 0.98; 96 labels, a random table, 256
+  // chains 0.98 / 0.96 / 0.99, 768 chains 0.99 / 0.98 / 0.99; 65 labels 768 chains 0.93 / 0.83 / 0.85; labels one by one,
+  // 191 labels 256 chains 0.92 / 0.72 / 0.79; ISGMR 96 labels 96x96 0.99 / 1.00 / 0.99, 192 labels 64x64 0.97 / 0.91 / 0.86;
+  // 500x700, 192 labels, 1199 diagonals 1.04 / 0.94 / 1.04.
+  if constexpr (R < 4) {
+    if (blocks <= 3 * n_cu) {
+      launch(gr ? sweep_bwd_team_kernel<R, VEC, JACOBI, true, 6> : sweep_bwd_team_kernel<R, VEC, JACOBI, false, 6>, 6, 0);
+      return;
+    }
+  }
+  launch(gr ? sweep_bwd_team_kernel<R, VEC, JACOBI, true, 3> : sweep_bwd_team_kernel<R, VEC, JACOBI, false, 3>, 3, turn_every);
 }
 
 }  // namespace

@@ -5,7 +5,8 @@
 // to itself issues one instruction every four clocks or more, and of the instructions of a step the next
 // pixel waits for the beliefs, the minimum over front labels and the normalisation only.  So the work is
 // divided by what the recurrence needs:
-//   * three helper wavefronts, every third pixel each, load the planes, form U of the pixel and put it
+//   * three helper wavefronts (six where argmin labels are kept and chains are few: launch_v), every third (sixth)
+//     pixel each, load the planes, form U of the pixel and put it
 //     into an LDS slot; two blocks of pixels later they take the message from the slot and store the
 //     planes.  Where argmin labels are kept they take the beliefs from the slot instead and run the
 //     whole step again, with the labels: the same operations on the same operands, so the same message,
@@ -16,7 +17,7 @@
 //
 // Measured, ns per pixel of rows of 256 / 512 chains, one wavefront per chain -> this: 60 labels, Potts, no
 // argmin labels 150 / 158 -> 95 / 103; 96 labels, min(k, 3), kept 418 / 439 -> 204 / 241; 192 labels 469 / 500 ->
-// 241 / 364, where the planes move at 4.7 TB/s.  The main wavefront of the first issues 29 instructions per
+// 241 / 364 (with six helpers 183 / 236 and 228 / 385 on rows of 129), where the planes move at 4.7 TB/s.  The main wavefront of the first issues 29 instructions per
 // pixel, of the last 57.  Which launches take it: team_fwd_chains_per_cu (mp_api.hip).
 //
 // Compiled once per R (labels per lane) with -DMPL_INST_R=<R>.
@@ -28,10 +29,7 @@
 namespace mpl {
 namespace {
 
-constexpr int kHelpers = 3;          // one SIMD of the compute unit each, the main one the fourth
-constexpr int kPer = 2;              // pixels of a block per helper
-constexpr int kT = kHelpers * kPer;  // pixels per block
-constexpr int kTeam = (kHelpers + 1) * kWave;
+constexpr int kT = 6;                // pixels per block, shared out among three or six helpers (launch_h)
 
 constexpr int kAhead = 2;            // blocks of pixels whose loads are in flight (four and six measure the same)
 
@@ -203,10 +201,11 @@ struct PixT {
   float s[R], md[R], mi[R];
 };
 
-template <int R, bool VEC, bool TRAIN, int KT, bool C0>
+template <int R, bool VEC, bool TRAIN, int KT, bool C0, int kHelpers>
 __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& desc, const ChainCtx& ch0,
                                           Slot<R>* slots, Flags* flags, float* a_s, const float* ctx_s,
                                           const int role) {
+  constexpr int kPer = kT / kHelpers;  // pixels of a block per helper
   const int L = p.L;
   const int lane = threadIdx.x & (kWave - 1);
   const int lab0 = R * lane;
@@ -228,7 +227,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
   c.cmax = desc.cmax;
   asm volatile("" : "+v"(c.cmax));
   c.slope = desc.slope;
-  c.a_w = a_s + (role & 3) * kMaxL;
+  c.a_w = a_s + role * kMaxL;
   c.ctx_s = ctx_s;
   c.c1_s = ctx_s + dense_c1_offset(L);
   c.csym_s = c.c1_s + dense_c1_floats(L);
@@ -497,8 +496,9 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
   }
 }
 
-template <int R, bool VEC, bool TRAIN>
-__global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams p) {
+template <int R, bool VEC, bool TRAIN, int kHelpers>
+__global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_fwd_team_kernel(const SweepParams p) {
+  constexpr int kTeam = (kHelpers + 1) * kWave;
   extern __shared__ __align__(16) char smem_raw[];
   Slot<R>* slots = reinterpret_cast<Slot<R>*>(smem_raw);  // two sets of kT
   float* a_s = reinterpret_cast<float*>(slots + 2 * kT);  // kMaxL floats per wavefront
@@ -510,7 +510,9 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
   // The last wavefront is the main one in every workgroup: the wavefronts of the workgroups that a compute
   // unit gets one after another start one SIMD further each (read from the hardware-id registers for 2, 3
   // and 4 workgroups per unit), so the main wavefronts of up to four of them are on SIMDs of their own.
-  const int role = uniform_i(tid / kWave);  // kHelpers: main
+  // (Of seven wavefronts the main one is the fourth, whose SIMD has only one of them.)
+  const int wave = uniform_i(tid / kWave);
+  const int role = wave == 3 ? kHelpers : wave - (wave > 3 ? 1 : 0);  // kHelpers: main
   const ChainCtx ch = locate_chain(p);
 
   CtxDesc desc;
@@ -543,7 +545,7 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
   __syncthreads();
   if (role == kHelpers) __builtin_amdgcn_s_setprio(3);
 
-#define MPL_WALK(KT, C0) team_walk<R, VEC, TRAIN, KT, C0>(p, desc, ch, slots, flags, a_s, ctx_s, role)
+#define MPL_WALK(KT, C0) team_walk<R, VEC, TRAIN, KT, C0, kHelpers>(p, desc, ch, slots, flags, a_s, ctx_s, role)
   // (the choice of the step: sweep_fwd_kernel)
   if (desc.linear && !p.ctx2d && (desc.band_k == 0 || desc.band_k > 4)) {
     MPL_WALK(-2, false);
@@ -576,22 +578,42 @@ __global__ void __launch_bounds__(kTeam) sweep_fwd_team_kernel(const SweepParams
 #undef MPL_WALK
 }
 
-inline size_t team_lds_bytes(int L, int R, bool ctx2d, size_t slot) {
+inline size_t team_lds_bytes(int L, int R, bool ctx2d, size_t slot, int helpers) {
   const size_t table = ctx2d ? (size_t)L * L : dense_c1_offset(L) + dense_c1_floats(L) + dense_sym_floats(R);
-  return 2 * kT * slot + sizeof(float) * ((kHelpers + 1) * kMaxL + table) + 2 * sizeof(Flags);
+  return 2 * kT * slot + sizeof(float) * ((helpers + 1) * kMaxL + table) + 2 * sizeof(Flags);
+}
+
+template <int R, bool VEC, bool TRAIN, int kHelpers>
+void launch_h(const SweepParams& p, hipStream_t st) {
+  const size_t lds = team_lds_bytes(p.L, R, p.ctx2d != 0, sizeof(Slot<R>), kHelpers);
+  sweep_fwd_team_kernel<R, VEC, TRAIN, kHelpers><<<p.block_prefix[p.n_dirs], (kHelpers + 1) * kWave, lds, st>>>(p);
+}
+
+template <int R, bool VEC, bool TRAIN>
+void launch_v(const SweepParams& p, hipStream_t st) {
+  // Where argmin labels are kept the helpers run every step again, and three of them bound a scan of up to two chains per
+  // unit (with four labels per lane, one).  Six helpers over three, rows of 129: 60 labels, min(k, 3), 256 chains 0.78,
+  // Potts 256 / 400 / 768 chains 0.84 / 0.89 / 0.97; 96 labels 256 / 512 / 768 chains 0.76 / 0.85 / 1.03; 192 labels 0.77 /
+  // 0.95 / 1.07, a linear table 0.96 / 0.99; 256 labels 256 / 512 chains 0.82 / 1.03; labels one by one, 127 and 191 labels
+  // 256 chains 0.73, 0.79.  Without argmin labels the main wavefront bounds it (0.99 to 1.07).
+  if constexpr (TRAIN) {
+    if (p.block_prefix[p.n_dirs] <= (R == 4 ? 1 : 2) * (launch_policy().n_simd / 4)) {
+      launch_h<R, VEC, TRAIN, 6>(p, st);
+      return;
+    }
+  }
+  launch_h<R, VEC, TRAIN, 3>(p, st);
 }
 
 }  // namespace
 
 template <int R, bool TRAIN>
 void launch_team_fwd_t(const SweepParams& p, hipStream_t st) {
-  const int blocks = p.block_prefix[p.n_dirs];
-  if (blocks <= 0) return;
-  const size_t lds = team_lds_bytes(p.L, R, p.ctx2d != 0, sizeof(Slot<R>));
+  if (p.block_prefix[p.n_dirs] <= 0) return;
   if (p.L % R == 0)
-    sweep_fwd_team_kernel<R, true, TRAIN><<<blocks, kTeam, lds, st>>>(p);
+    launch_v<R, true, TRAIN>(p, st);
   else if constexpr (R > 1)
-    sweep_fwd_team_kernel<R, false, TRAIN><<<blocks, kTeam, lds, st>>>(p);
+    launch_v<R, false, TRAIN>(p, st);
 }
 
 template void launch_team_fwd_t<MPL_INST_R, (MPL_INST_TRAIN != 0)>(const SweepParams&, hipStream_t);
