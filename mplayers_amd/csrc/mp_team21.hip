@@ -557,7 +557,9 @@ constexpr int kPairs = kL * kL;
 // Helpers of the soft-weighted scan where every chain has a compute unit to itself: the fourth SIMD, the main
 // wavefront's in the other launches, takes two of them.  More chains fill the SIMDs with three each.  Rows of 129 pixels,
 // all gradients, us per pair of walks with three / six: 128 chains 90 / 76, 256 chains 95 / 81, 258 chains 111 / 145, 512 chains 117 / 153.
-constexpr int kSoftHelpersAlone = 6;
+// The hard scan gains where dcontext is wanted and the LDS holds every chain of a unit: 128 chains 47.5 / 43.7, 256 chains
+// 46.5 / 42.7, 400 chains 50 / 47, 512 chains 51 / 47, 516 chains 59 / 82; without dcontext 0.97 to 1.05 of the time.
+constexpr int kManyHelpers = 6;
 
 // GR: dedge_weights and / or dcontext are wanted; DC: dcontext is.  SOFT: the soft-weighted operator, whose
 // step has the same form with J[cd][fd] = d message(cd) / d belief(fd) in place of the masks: the helpers
@@ -1056,10 +1058,13 @@ void launch_team21_bwd(const BackParams& p, hipStream_t st) {
          : gr              ? bwd_team21_kernel<true, false, SOFT, N>                                             \
                            : bwd_team21_kernel<false, false, SOFT, N>,                                           \
          N, sizeof(BwdSlots<2 * N>))
-  if (p.edge_label == nullptr)
+  const int cus = launch_policy().n_simd / 4;
+  if (p.edge_label == nullptr && p.dctx != nullptr && blocks <= 2 * cus)
+    launch(bwd_team21_kernel<true, true, false, kManyHelpers>, kManyHelpers, sizeof(BwdSlots<2 * kManyHelpers>));
+  else if (p.edge_label == nullptr)
     MPL_BWD21(false, kHelpers);
-  else if (blocks <= launch_policy().n_simd / 4)
-    MPL_BWD21(true, kSoftHelpersAlone);
+  else if (blocks <= cus)
+    MPL_BWD21(true, kManyHelpers);
   else
     MPL_BWD21(true, kHelpers);
 #undef MPL_BWD21
