@@ -89,7 +89,10 @@ typedef struct mpl_shape {
 #define MPL_F_CHAIN_STARTS 0x100u
 /* mpl_trwp_soft_forward: the blocks of duals and the normalisation indices of chain-start pixels are
  * written too, with zeros, so that nothing of msg_edge_label and msg_norm_index need be cleared. */
-#define MPL_F_ALL 0x1ffu
+#define MPL_F_COST_LABELS_FIRST 0x200u
+/* forward calls: cost_final is written as (batch, n_disp, height, width), the layout of the network around the
+ * layer, by the pass that sums it, instead of (batch, height, width, n_disp). */
+#define MPL_F_ALL 0x3ffu
 
 /* Replaces lib_*.TRWP.forward: MPLayers/TRWP/TRWP.cpp:245-283 (Forward) -> TRWP_forward.cu:378-560.
  * msg: initial messages in, final normalised messages out.  msg_min_index/msg_norm_index NULL =>

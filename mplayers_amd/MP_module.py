@@ -16,7 +16,7 @@ import torch.nn as nn
 
 from . import _lib, lib_seg, lib_stereo
 from .label_context import create_label_context
-from .layout import labels_first, labels_last
+from .layout import gradient_labels_last, labels_first, labels_last
 
 
 def _ops_for(n_disp):
@@ -28,7 +28,7 @@ def _ops_for(n_disp):
 _EMPTY_U8 = dict(dtype=torch.uint8)
 
 
-def _forward_buffers(unary, args, n_dir, n_iter, with_message_tmp):
+def _forward_buffers(unary, args, n_dir, n_iter, with_message_tmp, cost_labels_first=False):
   """Allocates what the operators fill in place (MP_module.py:26-45, 97-118).  Nothing is
   zero-filled: the library writes every element that is ever read (index bytes of chain-start
   pixels stay unwritten and are never used), and the operators are told that the messages start
@@ -37,7 +37,7 @@ def _forward_buffers(unary, args, n_dir, n_iter, with_message_tmp):
   batch, cv, h, w, n_disp = unary.size()
   buf = dict(
       message=unary.new_empty(n_dir, batch, cv, h, w, n_disp),
-      cost_final=unary.new_empty(batch, cv, h, w, n_disp),
+      cost_final=unary.new_empty((batch, cv, n_disp, h, w) if cost_labels_first else (batch, cv, h, w, n_disp)),
       unary_update=unary.new_empty(batch, cv, h, w, n_disp))
   if with_message_tmp:
     buf["message_tmp"] = unary.new_empty(n_dir, batch, cv, h, w, n_disp)
@@ -94,6 +94,12 @@ def _context_gradient(like, n_iter, n_dir, batch, h, w, n_disp, size):
   return like.new_empty(size), like.new_zeros((copies,) + size), _lib.F_DCONTEXT_COPIES
 
 
+def _sums_labels_first(unary, args):
+  """Whether the operators are to write the costs in the network's layout themselves (not in the reference).  Where
+  labels are saved, the pass that finds the last ones stores the costs in the kernels' layout."""
+  return unary.is_cuda and unary.dtype == torch.float32 and not args.enable_saving_label
+
+
 def _table_flags(args):
   """MPL_F_DENSE_TABLE when the module says its pairwise table is dense (not in the reference: the
   kind of the table is only known on the device otherwise, see include/mplayers_amd.h)."""
@@ -104,17 +110,20 @@ class TRWPFunction(torch.autograd.Function):
   """Tree-reweighted message passing, Gauss-Seidel over directions (MP_module.py:17-86)."""
 
   @staticmethod
-  def forward(ctx, unary, label_context, edge_weights, args):
+  def forward(ctx, unary, label_context, edge_weights, args, cost_labels_first=False):
+    # cost_labels_first: cost_final comes as (batch, cv, labels, H, W), as the module returns it
     n_disp = unary.size(4)
     rho, n_iter, n_dir = args.rho, int(args.mpnet_max_iter), int(args.mpnet_n_dirs)
-    buf = _forward_buffers(unary, args, n_dir, n_iter, with_message_tmp=False)
+    buf = _forward_buffers(unary, args, n_dir, n_iter, False, cost_labels_first)
     enable_edge_weights = edge_weights is not None
     if not enable_edge_weights:
       edge_weights = unary.new_ones((n_dir,) + tuple(unary.shape[:4]))
     _ops_for(n_disp).TRWP.forward(rho, n_iter, int(args.enable_min_a_dir), unary, label_context,
                                   edge_weights, buf["message"], buf["cost_final"],
                                   buf["message_index"], buf["cost_index"], buf["unary_update"],
-                                  buf["label_all"], msg_uninit=True, flags=_table_flags(args))
+                                  buf["label_all"], msg_uninit=True,
+                                  flags=_table_flags(args) | (_lib.F_COST_LABELS_FIRST if cost_labels_first else 0))
+    ctx.cost_labels_first = cost_labels_first
     ctx.intermediate_results = (rho, buf["message_index"], buf["cost_index"], label_context,
                                 edge_weights, enable_edge_weights)
     return buf["cost_final"], buf["label_all"]
@@ -124,7 +133,7 @@ class TRWPFunction(torch.autograd.Function):
     rho, message_index, cost_index, label_context, edge_weights, enable_edge_weights = \
         ctx.intermediate_results
     del ctx.intermediate_results
-    dcost_final = dcost_final.contiguous()
+    dcost_final = gradient_labels_last(dcost_final) if ctx.cost_labels_first else dcost_final.contiguous()
     n_disp = message_index.size(6)
     need_context = ctx.needs_input_grad[1]
     need_edge_weights = enable_edge_weights and ctx.needs_input_grad[2]
@@ -134,17 +143,17 @@ class TRWPFunction(torch.autograd.Function):
                                    buf["dedge_weights"], buf["dmessage"], buf["dunary_update"],
                                    flags=buf["flags"])
     return (buf["dunary"], buf["dlabel_context"] if need_context else None,
-            buf["dedge_weights"] if need_edge_weights else None, None)
+            buf["dedge_weights"] if need_edge_weights else None, None, None)
 
 
 class ISGMRFunction(torch.autograd.Function):
   """Iterative semi-global matching revised, Jacobi over directions (MP_module.py:89-161)."""
 
   @staticmethod
-  def forward(ctx, unary, label_context, edge_weights, args):
+  def forward(ctx, unary, label_context, edge_weights, args, cost_labels_first=False):
     n_disp = unary.size(4)
     rho, n_iter, n_dir = args.rho, int(args.mpnet_max_iter), int(args.mpnet_n_dirs)
-    buf = _forward_buffers(unary, args, n_dir, n_iter, with_message_tmp=True)
+    buf = _forward_buffers(unary, args, n_dir, n_iter, True, cost_labels_first)
     enable_edge_weights = edge_weights is not None
     if not enable_edge_weights:
       edge_weights = unary.new_ones((n_dir,) + tuple(unary.shape[:4]))
@@ -152,7 +161,9 @@ class ISGMRFunction(torch.autograd.Function):
                                    unary, label_context, edge_weights, buf["message"],
                                    buf["cost_final"], buf["message_index"], buf["cost_index"],
                                    buf["unary_update"], buf["message_tmp"], buf["label_all"],
-                                   msg_uninit=True, flags=_table_flags(args))
+                                   msg_uninit=True,
+                                   flags=_table_flags(args) | (_lib.F_COST_LABELS_FIRST if cost_labels_first else 0))
+    ctx.cost_labels_first = cost_labels_first
     ctx.intermediate_results = (args.enable_sgm, rho, buf["message_index"], buf["cost_index"],
                                 label_context, edge_weights, enable_edge_weights)
     return buf["cost_final"], buf["label_all"]
@@ -162,7 +173,7 @@ class ISGMRFunction(torch.autograd.Function):
     enable_sgm, rho, message_index, cost_index, label_context, edge_weights, \
         enable_edge_weights = ctx.intermediate_results
     del ctx.intermediate_results
-    dcost_final = dcost_final.contiguous()
+    dcost_final = gradient_labels_last(dcost_final) if ctx.cost_labels_first else dcost_final.contiguous()
     n_disp = message_index.size(6)
     need_context = ctx.needs_input_grad[1]
     need_edge_weights = enable_edge_weights and ctx.needs_input_grad[2]
@@ -172,7 +183,7 @@ class ISGMRFunction(torch.autograd.Function):
                                     buf["dlabel_context"], buf["dedge_weights"], buf["dmessage"],
                                     buf["dunary_update"], buf["dmessage_tmp"], flags=buf["flags"])
     return (buf["dunary"], buf["dlabel_context"] if need_context else None,
-            buf["dedge_weights"] if need_edge_weights else None, None)
+            buf["dedge_weights"] if need_edge_weights else None, None, None)
 
 
 def _entries(place):
@@ -336,11 +347,13 @@ class MPModule(torch.nn.Module):
     if dense is None:
       dense = self.label_context.requires_grad or self._fixed_table_is_dense(label_context)
     self.args.dense_table = bool(dense)
+    turned = _sums_labels_first(unary, self.args)
     if self.args.mpnet_mrf_mode in {'ISGMR', 'SGM'}:
-      cost_final, cost_all = ISGMRFunction.apply(unary, label_context, edge_weights, self.args)
+      cost_final, cost_all = ISGMRFunction.apply(unary, label_context, edge_weights, self.args, turned)
     elif self.args.mpnet_mrf_mode == 'TRWP':
-      cost_final, cost_all = TRWPFunction.apply(unary, label_context, edge_weights, self.args)
+      cost_final, cost_all = TRWPFunction.apply(unary, label_context, edge_weights, self.args, turned)
     else:
       assert False
-    cost_final = labels_first(cost_final)
+    if not turned:
+      cost_final = labels_first(cost_final)
     return cost_final, label_context.unsqueeze(0), cost_all, None, None

@@ -33,6 +33,7 @@ F_FUSED_PAIRS_OFF = 0x20
 F_DENSE_TABLE = 0x40
 F_DCONTEXT_COPIES = 0x80
 F_CHAIN_STARTS = 0x100
+F_COST_LABELS_FIRST = 0x200
 
 
 class KernelStat(ctypes.Structure):

@@ -271,6 +271,79 @@ __global__ void __launch_bounds__(256) aggregate_kernel(const float* __restrict_
   }
 }
 
+// The same with the labels first in the result (MPL_F_COST_LABELS_FIRST): a workgroup sums `tile` consecutive pixels of
+// an image, one run of memory in every plane whatever the label count, and turns them over through LDS (an odd row
+// stride), so the sums are not stored and read once more to change their layout.  Bound by HBM.  Tiles beside each other
+// share lines of the result where a row of it is no whole number of them: groups of tiles go to one die, as the
+// transposes' do (mp_layout.hip), and only whole lines carry the hint (NT_ST).  Measured, us, sum and transpose -> this:
+// 128 labels 375x1242, 8 directions 414 + 131 -> 416; 96 labels 384x1248, 4 directions 180 + 90 -> 186; 21 labels
+// 12x65x65, 8 directions 8.4 + 11 -> 8.4 (32 with tiles of 128 pixels, too few of them), 4x129x129, 4 directions 7 + 14 -> 6.
+template <int V, int ND, bool NT, bool NT_ST>
+__global__ void __launch_bounds__(256) aggregate_first_kernel(const float* __restrict__ unary,
+                                                              const float* __restrict__ msg, int n_dir_rt,
+                                                              int64_t N, int HW, int L, int tile_log, float factor,
+                                                              int min_a_dir, float* __restrict__ cost) {
+  extern __shared__ float turn[];  // [pixel][L | 1]
+  const int n_dir = ND > 0 ? ND : n_dir_rt;
+  const int tile = 1 << tile_log, stride = L | 1;
+  const int p0 = xcd_block((int)blockIdx.x, (int)gridDim.x, 8) << tile_log;
+  const int pixels = HW - p0 < tile ? HW - p0 : tile;
+  for (int64_t b = blockIdx.y; b * HW * L < N; b += gridDim.y) {
+    const int64_t first = (b * HW + p0) * L;
+    for (int e = (int)threadIdx.x * V; e < pixels * L; e += 256 * V) {
+      const int64_t i = first + e;
+      Pack<V> v = ld_pack<V, NT>(unary + i);
+#pragma unroll
+      for (int j = 0; j < V; ++j) v.v[j] *= factor;
+      Pack<V> mn;  // min_a_dir only
+      auto fold = [&](int k, const Pack<V>& m) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          if (!min_a_dir)
+            v.v[j] += m.v[j];  // ((unary + m_0) + m_1) + ... as the reference adds
+          else if (k == 0)
+            mn.v[j] = m.v[j];
+          else
+            mn.v[j] = (m.v[j] < mn.v[j]) ? m.v[j] : mn.v[j];
+        }
+      };
+      if constexpr (ND > 0) {
+        Pack<V> m[ND];
+#pragma unroll
+        for (int k = 0; k < ND; ++k) m[k] = ld_pack<V, NT>(msg + (int64_t)k * N + i);
+#pragma unroll
+        for (int k = 0; k < ND; ++k) fold(k, m[k]);
+      } else {
+        for (int k = 0; k < n_dir; ++k) fold(k, ld_pack<V, NT>(msg + (int64_t)k * N + i));
+      }
+      if (min_a_dir) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) v.v[j] += mn.v[j];
+      }
+      int p = e / L, l = e - p * L;
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        turn[p * stride + l] = v.v[j];
+        if (++l == L) {
+          l = 0;
+          ++p;
+        }
+      }
+    }
+    __syncthreads();
+    float* const out = cost + b * HW * L + p0;
+    for (int x = threadIdx.x; x < L << tile_log; x += 256) {
+      const int l = x >> tile_log, p = x & (tile - 1);
+      if (p >= pixels) continue;
+      if (NT_ST)
+        __builtin_nontemporal_store(turn[p * stride + l], out + (int64_t)l * HW + p);
+      else
+        out[(int64_t)l * HW + p] = turn[p * stride + l];
+    }
+    __syncthreads();
+  }
+}
+
 // label = argmin_l cost(l), smallest label on ties: CalLabelKernel, TRWP_forward.cu:8-29, with the
 // cost of CostAggregateKernel recomputed on the fly.  One wave per pixel.
 __global__ void __launch_bounds__(256) label_kernel(const float* __restrict__ unary,
@@ -1051,6 +1124,46 @@ void fold_dcontext(const BackParams& p, float* dcontext, hipStream_t st) {
   dcontext_fold_kernel<<<(entries + kWave - 1) / kWave, kWave, 0, st>>>(p.dctx, entries, dcontext);
 }
 
+// cost_final from the unary terms and the messages, in either layout.
+void aggregate(const mpl_shape* s, unsigned flags, const float* unary, const float* msg, float factor, int min_a_dir,
+               float* cost_final, hipStream_t st) {
+  Timed timed(MPL_KERNEL_AGGREGATE, st);
+  const int L = s->n_disp, n_dir = s->n_dir;
+  const int64_t HW = (int64_t)s->height * s->width, N = s->batch * HW * L;
+  const bool nt = ew_hint(s);
+  if ((flags & MPL_F_COST_LABELS_FIRST) == 0) {
+    const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
+    MPL_EW_LAUNCH(aggregate_kernel, v4, nt, n_dir, N, st, unary, msg, n_dir, N, factor, min_a_dir, cost_final);
+    return;
+  }
+  // some 32 KB of LDS at most, a run of a few KB per plane; one line of the result, where that is not enough to go round
+  int tile_log = L <= 32 ? 7 : L <= 128 ? 6 : 5;
+  while (tile_log > 5 && (((HW - 1) >> tile_log) + 1) * s->batch < 2 * launch_policy().n_simd) --tile_log;
+  const bool v4 = (HW * L) % 4 == 0 && aligned16(unary) && aligned16(msg);
+  const bool lines = (HW * (int64_t)sizeof(float)) % kLineBytes == 0 && ((uintptr_t)cost_final & (kLineBytes - 1)) == 0;
+  const dim3 grid((unsigned)(((HW - 1) >> tile_log) + 1), (unsigned)std::min(s->batch, 65535));
+  const size_t lds = sizeof(float) * ((size_t)(L | 1) << tile_log);
+  const auto launch = [&](auto kernel) {
+    kernel<<<grid, 256, lds, st>>>(unary, msg, n_dir, N, (int)HW, L, tile_log, factor, min_a_dir, cost_final);
+  };
+#define MPL_FIRST(V, ND)                                                                                             \
+  launch(nt ? (lines ? aggregate_first_kernel<V, ND, true, true> : aggregate_first_kernel<V, ND, true, false>)       \
+            : (lines ? aggregate_first_kernel<V, ND, false, true> : aggregate_first_kernel<V, ND, false, false>))
+  if (v4 && n_dir == 4)
+    MPL_FIRST(4, 4);
+  else if (v4 && n_dir == 8)
+    MPL_FIRST(4, 8);
+  else if (v4)
+    MPL_FIRST(4, 0);
+  else if (n_dir == 4)
+    MPL_FIRST(1, 4);
+  else if (n_dir == 8)
+    MPL_FIRST(1, 8);
+  else
+    MPL_FIRST(1, 0);
+#undef MPL_FIRST
+}
+
 // cost_final is not written before the final aggregation, so its first bytes carry the context
 // descriptor during the sweeps (no allocation, no state shared between streams).
 const CtxDesc* make_desc(const mpl_shape* s, const float* ctx, float* cost_final, hipStream_t st) {
@@ -1267,6 +1380,7 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
   p.msg_out = msg;
   const int rebuild = belief_rebuild_interval(s->n_dir, n_iter);
   bool have_belief = false, have_cost = false;  // the pass that writes the labels has stored it
+  float* const cost_plane = (flags & MPL_F_COST_LABELS_FIRST) ? nullptr : cost_final;  // (where it can)
   for (int it = 0; it < n_iter; ++it) {
     if (rebuild > 0 && it > 0 && it % rebuild == 0 && !have_belief)
       rebuild_belief(s, unary, msg, unary_update, st);
@@ -1303,18 +1417,13 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
       Timed timed(MPL_KERNEL_LABEL, st);
       // the next pass over the same planes, if one is due: cost_final, the re-summed belief plane
       const bool last = it + 1 == n_iter;
-      float* out = last ? cost_final : (rebuild > 0 && (it + 1) % rebuild == 0) ? unary_update : nullptr;
+      float* out = last ? cost_plane : (rebuild > 0 && (it + 1) % rebuild == 0) ? unary_update : nullptr;
       const bool stored = launch_labels(unary, msg, s->n_dir, P, s->n_disp, 1.f, enable_min_a_dir,
                                         label_all + it * P, st, ew_hint(s), kLabelSum, out);
       (last ? have_cost : have_belief) = stored;
     }
   }
-  if (!have_cost) {
-    Timed timed(MPL_KERNEL_AGGREGATE, st);
-    const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
-    MPL_EW_LAUNCH(aggregate_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, 1.f,
-                  enable_min_a_dir, cost_final);
-  }
+  if (!have_cost) aggregate(s, flags, unary, msg, 1.f, enable_min_a_dir, cost_final, st);
   return launch_ok("trwp_forward");
 }
 
@@ -1367,6 +1476,7 @@ int mpl_isgmr_forward(const mpl_shape* s, unsigned flags, int enable_sgm, float 
   p.belief_zero = unary;
   float* have = msg;  // the buffer that holds the current messages
   bool have_u = false, have_cost = false;  // the pass that writes the labels has stored it
+  float* const cost_plane = (flags & MPL_F_COST_LABELS_FIRST) ? nullptr : cost_final;  // (where it can)
   for (int it = 0; it < n_iter; ++it) {
     // Jacobi over directions (ISGMR_forward.cu:506-622): every direction reads the old messages,
     // through U; the two buffers alternate instead of being copied.  U normally overwrites the
@@ -1419,17 +1529,12 @@ int mpl_isgmr_forward(const mpl_shape* s, unsigned flags, int enable_sgm, float 
       const bool last = it + 1 == n_iter;
       const bool stored = launch_labels(unary, nxt, s->n_dir, P, s->n_disp, factor, enable_min_a_dir,
                                         label_all + it * P, st, ew_hint(s), last ? kLabelSum : kLabelU,
-                                        last ? cost_final : fuse_u ? nullptr : nxt, rho, p.u_pair_share);
+                                        last ? cost_plane : fuse_u ? nullptr : nxt, rho, p.u_pair_share);
       (last ? have_cost : have_u) = stored;
     }
     have = nxt;
   }
-  if (!have_cost) {
-    Timed timed(MPL_KERNEL_AGGREGATE, st);
-    const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
-    MPL_EW_LAUNCH(aggregate_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, factor,
-                  enable_min_a_dir, cost_final);
-  }
+  if (!have_cost) aggregate(s, flags, unary, msg, factor, enable_min_a_dir, cost_final, st);
   return launch_ok("isgmr_forward");
 }
 
@@ -1594,6 +1699,7 @@ int mpl_trwp_soft_forward(const mpl_shape* s, unsigned flags, float rho, int n_i
   p.msg_out = msg;
   const int rebuild = belief_rebuild_interval(s->n_dir, n_iter);
   bool have_belief = false, have_cost = false;  // the pass that writes the labels has stored it
+  float* const cost_plane = (flags & MPL_F_COST_LABELS_FIRST) ? nullptr : cost_final;  // (where it can)
   for (int it = 0; it < n_iter; ++it) {
     if (rebuild > 0 && it > 0 && it % rebuild == 0 && !have_belief)
       rebuild_belief(s, unary, msg, unary_update, st);
@@ -1618,18 +1724,13 @@ int mpl_trwp_soft_forward(const mpl_shape* s, unsigned flags, float rho, int n_i
       Timed timed(MPL_KERNEL_LABEL, st);
       // the next pass over the same planes, if one is due: cost_final, the re-summed belief plane
       const bool last = it + 1 == n_iter;
-      float* out = last ? cost_final : (rebuild > 0 && (it + 1) % rebuild == 0) ? unary_update : nullptr;
+      float* out = last ? cost_plane : (rebuild > 0 && (it + 1) % rebuild == 0) ? unary_update : nullptr;
       const bool stored = launch_labels(unary, msg, s->n_dir, P, s->n_disp, 1.f, 0,
                                         label_all + it * P, st, ew_hint(s), kLabelSum, out);
       (last ? have_cost : have_belief) = stored;
     }
   }
-  if (!have_cost) {
-    Timed timed(MPL_KERNEL_AGGREGATE, st);
-    const bool v4 = (N % 4 == 0) && aligned16(unary) && aligned16(msg) && aligned16(cost_final);
-    MPL_EW_LAUNCH(aggregate_kernel, v4, ew_hint(s), s->n_dir, N, st, unary, msg, s->n_dir, N, 1.f, 0,
-                  cost_final);
-  }
+  if (!have_cost) aggregate(s, flags, unary, msg, 1.f, 0, cost_final, st);
   return launch_ok("trwp_soft_forward");
 }
 

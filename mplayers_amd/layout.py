@@ -56,6 +56,11 @@ class _LabelsFirst(torch.autograd.Function):
     return _transpose(grad.contiguous(), b * cv, n, h * w, (b, cv, h, w, n))
 
 
+def gradient_labels_last(grad):
+  """The gradient of a (batch, cv, labels, H, W) result as (batch, cv, H, W, labels), contiguous."""
+  return _LabelsFirst.backward(None, grad)
+
+
 def labels_last(x):
   """x.permute(0, 1, 3, 4, 2).contiguous() for a (batch, cv, labels, H, W) tensor."""
   if _usable(x):
