@@ -517,42 +517,42 @@ __device__ __forceinline__ void band_head(const float (&a)[4], float w, float c0
   dn[2] = a[1];
   dn[3] = a[2];
 }
-// One label per lane, the same.  KT == 1 (a Potts table): the centre tap alone.
+// One label per lane, the same.  KT == 1 (a Potts table): the centre tap alone.  The minimum goes round each row of
+// lanes first: a rotation reaches every lane, so it needs no copy of the beliefs to fall back on.
 template <int KT>
 __device__ __forceinline__ void band_head(const float (&a)[1], float w, float c0, float c1, float& red,
                                           float (&v)[1], float (&up)[1], float (&dn)[1]) {
-  red = a[0];  // (the same value as an input: hence the early clobber)
   if constexpr (KT == 1) {
     asm("v_fma_f32 %1, %3, %4, %2\n\ts_nop 0\n\t"
-        MPL_RED("row_shr:1 row_mask:0xf") "s_nop 1\n\t"
-        MPL_RED("row_shr:2 row_mask:0xf") "s_nop 1\n\t"
-        MPL_RED("row_shr:4 row_mask:0xf") "s_nop 1\n\t"
-        MPL_RED("row_shr:8 row_mask:0xf") "s_nop 1\n\t"
+        "v_min_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xf\n\ts_nop 1\n\t"
+        MPL_RED("row_ror:4 row_mask:0xf") "s_nop 1\n\t"
+        MPL_RED("row_ror:2 row_mask:0xf") "s_nop 1\n\t"
+        MPL_RED("row_ror:1 row_mask:0xf") "s_nop 1\n\t"
         MPL_RED("row_bcast:15 row_mask:0xa") "s_nop 1\n\t"
         "v_min_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
-        : "+&v"(red), "=&v"(v[0])
+        : "=&v"(red), "=&v"(v[0])
         : "v"(a[0]), "v"(w), "v"(c0));
     up[0] = dn[0] = a[0];
   } else {
     float tu, td, q, p;
     asm("v_mov_b32 %1, 0x7f800000\n\t"
         "v_mov_b32 %2, 0x7f800000\n\t"
-        MPL_RED("row_shr:1 row_mask:0xf")
+        "v_min_f32_dpp %0, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
         "v_mov_b32_dpp %1, %5 wave_shl:1 row_mask:0xf bank_mask:0xf\n\t"
         "v_mov_b32_dpp %2, %5 wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
-        MPL_RED("row_shr:2 row_mask:0xf")
+        MPL_RED("row_ror:4 row_mask:0xf")
         "v_fma_f32 %4, %6, %7, %5\n\t"
         "v_min_f32 %3, %1, %2\n\t"
-        MPL_RED("row_shr:4 row_mask:0xf")
+        MPL_RED("row_ror:2 row_mask:0xf")
         "v_fmac_f32 %3, %6, %8\n\t"
         "s_nop 0\n\t"
-        MPL_RED("row_shr:8 row_mask:0xf")
+        MPL_RED("row_ror:1 row_mask:0xf")
         "v_min_f32 %4, %4, %3\n\t"
         "s_nop 0\n\t"
         MPL_RED("row_bcast:15 row_mask:0xa")
         "s_nop 1\n\t"
         "v_min_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
-        : "+&v"(red), "=&v"(tu), "=&v"(td), "=&v"(q), "=&v"(p)
+        : "=&v"(red), "=&v"(tu), "=&v"(td), "=&v"(q), "=&v"(p)
         : "v"(a[0]), "v"(w), "v"(c0), "v"(c1));
     v[0] = p;
     up[0] = tu;

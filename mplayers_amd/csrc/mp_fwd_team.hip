@@ -16,7 +16,7 @@
 // iterations on by the helpers that own them, so two sets suffice.
 //
 // Measured, ns per pixel of rows of 256 / 512 chains, one wavefront per chain -> this: 60 labels, Potts, no
-// argmin labels 150 / 158 -> 95 / 103; 96 labels, min(k, 3), kept 418 / 439 -> 204 / 241; 192 labels 469 / 500 ->
+// argmin labels 150 / 158 -> 90 / 101; 96 labels, min(k, 3), kept 418 / 439 -> 204 / 241; 192 labels 469 / 500 ->
 // 241 / 364 (with six helpers 183 / 236 and 228 / 385 on rows of 129), where the planes move at 4.7 TB/s.  The main wavefront of the first issues 29 instructions per
 // pixel, of the last 57.  Which launches take it: team_fwd_chains_per_cu (mp_api.hip).
 //
@@ -247,48 +247,63 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
     float prev[R], uf[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) prev[j] = uf[j] = 0.f;
-    auto pixel = [&](Slot<R>& s, const float (&un)[R], const float w, const bool start, const auto plain)
+    auto pixel = [&](float (&out)[R], const float (&un)[R], const float w, const bool start, const auto plain)
         __attribute__((always_inline)) {
       float a[R], v[R], nmin;
       int fd_idx[R];
 #pragma unroll
       for (int j = 0; j < R; ++j) a[j] = fmaf(rho, prev[j], uf[j]);
-      if (TRAIN) lds_put(s.out[lane], a);
+#pragma unroll
+      for (int j = 0; j < R; ++j) out[j] = a[j];
       team_step<R, KT, C0, false, decltype(plain)::value>(c, a, w, v, fd_idx, nmin);
 #pragma unroll
       for (int j = 0; j < R; ++j) {
         const float m = v[j] - nmin;
         prev[j] = start ? 0.f : m;  // (the chain start has no front pixel and no message)
         uf[j] = un[j];
+        if (!TRAIN) out[j] = prev[j];
       }
-      if (!TRAIN) lds_put(s.out[lane], prev);
     };
     for (int k = 0; k < iters; ++k) {
       if (k >= 1 && k <= blocks) {
         Slot<R>* s = slots + ((k - 1) & 1) * kT;
         const Flags& f = flags[(k - 1) & 1];
+        // Up to two labels per lane a group of two pixels is read and written at once: one LDS instruction takes both
+        // and costs the main wavefront as much as three others.  Two over one, 256 chains of 129 / 450, no argmin labels
+        // kept: 60 labels 0.94 / 0.94, 96 labels 0.93 / 0.90, 128 labels 0.93 / 0.91; kept, where the helpers do most, 0.96 to
+        // 1.01.  Three and four labels fill an access of 16 bytes by themselves.
+        constexpr int kGroup = R <= 2 ? 2 : 1;
+        float un[kGroup][R], w[kGroup], out[kGroup][R];
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) get_in<R>(s[u], f, u, lane, un[u], w[u]);  // (ahead of the question, which takes as long)
         bool neg = false;
         if constexpr (KT >= 0 || KT == -2) neg = ballot(f.neg[lane < kT ? lane : 0] != 0) != 0;
         if (__builtin_expect(!neg, 1)) {
-          float un[R], w;
-          get_in<R>(s[0], f, 0, lane, un, w);
 #pragma unroll
-          for (int i = 0; i < kT; ++i) {
-            float nun[R], nw = 0.f;
-            if (i + 1 < kT) get_in<R>(s[i + 1], f, i + 1, lane, nun, nw);
-            pixel(s[i], un, w, i == 0 && k == 1, std::true_type());
-            if (i + 1 < kT) {
+          for (int i = 0; i < kT; i += kGroup) {
+            float nun[kGroup][R], nw[kGroup];
+            if (i + kGroup < kT) {
 #pragma unroll
-              for (int j = 0; j < R; ++j) un[j] = nun[j];
-              w = nw;
+              for (int u = 0; u < kGroup; ++u) get_in<R>(s[i + kGroup + u], f, i + kGroup + u, lane, nun[u], nw[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < kGroup; ++u) pixel(out[u], un[u], w[u], i + u == 0 && k == 1, std::true_type());
+#pragma unroll
+            for (int u = 0; u < kGroup; ++u) {
+              lds_put(s[i + u].out[lane], out[u]);
+              if (i + kGroup < kT) {
+#pragma unroll
+                for (int j = 0; j < R; ++j) un[u][j] = nun[u][j];
+                w[u] = nw[u];
+              }
             }
           }
         } else {
 #pragma clang loop unroll(disable)
           for (int i = 0; i < kT; ++i) {
-            float un[R], w;
-            get_in<R>(s[i], f, i, lane, un, w);
-            pixel(s[i], un, w, i == 0 && k == 1, std::false_type());
+            get_in<R>(s[i], f, i, lane, un[0], w[0]);
+            pixel(out[0], un[0], w[0], i == 0 && k == 1, std::false_type());
+            lds_put(s[i].out[lane], out[0]);
           }
         }
       }

@@ -297,13 +297,22 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
     for (int k = 0; k < iters; ++k) {
       if (k >= 1 && k <= blocks) {
         FwdSlots& s = sets[(k - 1) & 1];
-        f32x2 cur = *reinterpret_cast<const f32x2*>(s.in[0][sl]);
+        // (two pixels to an LDS instruction, as in mp_fwd_team.hip: 1 to 2 % of a scan of rows of 129; the reverse scan,
+        // whose masks are most of what it reads, has nothing from it)
+        f32x2 two[2], nxt[2], out[2];
+        float as[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) two[u] = *reinterpret_cast<const f32x2*>(s.in[u][sl]);
 #pragma unroll
         for (int i = 0; i < kT; ++i) {
-          f32x2 nxt = cur;
-          if (i + 1 < kT) nxt = *reinterpret_cast<const f32x2*>(s.in[i + 1][sl]);
+          const int u = i & 1;
+          if (u == 0 && i + 2 < kT) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) nxt[j] = *reinterpret_cast<const f32x2*>(s.in[i + 2 + j][sl]);
+          }
+          const f32x2 cur = two[u];
           const float a = fmaf(rho, prev, uf);
-          if (TRAIN) s.a[i][sl] = a;
+          as[u] = a;
           float c[kSrc];
           static_for<kSrc>([&](auto ii) __attribute__((always_inline)) {
             constexpr int q = decltype(ii)::value;
@@ -337,12 +346,19 @@ __global__ void __launch_bounds__(kTeam) fwd_team21_kernel(const SweepParams p) 
             join_min(best, pad, v, vs, nmin);
           }
           prev = (i == 0 && k == 1) ? 0.f : vs - nmin;  // (the chain start has no front pixel and no message)
-          if (TRAIN || SOFT)
-            *reinterpret_cast<f32x2*>(s.out[i][l]) = f32x2{v, nmin};
-          else
-            s.out[i][sl][0] = prev;
+          out[u] = (TRAIN || SOFT) ? f32x2{v, nmin} : f32x2{prev, 0.f};
           uf = cur[0];
-          cur = nxt;
+          if (u == 1) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              if (TRAIN) s.a[i - 1 + j][sl] = as[j];
+              if (TRAIN || SOFT)
+                *reinterpret_cast<f32x2*>(s.out[i - 1 + j][l]) = out[j];
+              else
+                s.out[i - 1 + j][sl][0] = out[j][0];
+              two[j] = nxt[j];
+            }
+          }
         }
       }
       lds_barrier();
