@@ -683,9 +683,9 @@ int elementwise_blocks(int64_t n) {
 // 300x400 1.03 / 1.01 / 1.04; 100 labels 200x300 0.93 / 0.94 / 0.98.  Whole lines: 64 labels 100x150 1.04, 300x400 1.03;
 // 96 labels 384x1248 1.04.
 constexpr int64_t kCachedMessages = (int64_t)208 << 20;
+int64_t message_bytes(const mpl_shape* s) { return (int64_t)s->n_dir * s->batch * s->height * s->width * s->n_disp * 4; }
 bool ew_hint(const mpl_shape* s) {
-  const int64_t messages = (int64_t)s->n_dir * s->batch * s->height * s->width * s->n_disp * 4;
-  return (s->n_disp * 4) % kLineBytes == 0 || messages > kCachedMessages;
+  return (s->n_disp * 4) % kLineBytes == 0 || message_bytes(s) > kCachedMessages;
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1392,6 +1392,7 @@ int mpl_trwp_forward(const mpl_shape* s, unsigned flags, float rho, int n_iter,
       p.dense_team = decide_dense_team(p, opts, train);
       p.team = decide_team_fwd(p, opts, train);
       p.skip_dense = (p.dense_team && s->n_disp <= kWave) ? 1 : 0;
+      p.through = message_bytes(s) <= kCachedMessages ? 1 : 0;
       p.first_iter = (it == 0);
       p.pair_q = 1;
       p.belief = (uninit && it == 0 && d <= 1) ? unary : unary_update;

@@ -563,6 +563,7 @@ struct SweepParams {
                                    // sweep would read (Gauss-Seidel, first pair of directions: the belief
                                    // plane, which then need not exist; Jacobi, first iteration: U), and
                                    // the even sweep of that pair stores no plane
+  int through;                     // Gauss-Seidel, mp_fwd_team.hip: stores go through the L2 (kCachedMessages)
   const float* belief_zero;        // the unary terms
   float* edge_label;               // soft TRWP: (n_dir_total, P, L, L) duals of this iteration, or null
 };

@@ -201,7 +201,7 @@ struct PixT {
   float s[R], md[R], mi[R];
 };
 
-template <int R, bool VEC, bool TRAIN, int KT, bool C0, int kHelpers>
+template <int R, bool VEC, bool TRAIN, int KT, bool C0, int kHelpers, bool THROUGH>
 __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& desc, const ChainCtx& ch0,
                                           Slot<R>* slots, Flags* flags, float* a_s, const float* ctx_s,
                                           const int role) {
@@ -349,8 +349,16 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
           x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, vec_off(on, so, j), 0, load_policy(false)));
       }
     };
+    // THROUGH: where the messages fit the last-level cache (p.through, kCachedMessages) what is stored had better stay there.
+    // Stores that go through the L2 at once (sc1) without the hint, over the hint, 5 iterations, 4 directions: 240x320, 60
+    // labels 0.95 (8 directions 0.95), 96 labels 0.95, 128 labels 0.89; 375x450, 64 labels 0.93; argmin labels kept, the layer's
+    // whole pass, 0.97 to 0.99.  Larger ones 300x400, 64 labels, 8 directions (246 MB) 1.01, 375x450, 60 labels, 8 directions
+    // 1.19; three labels per lane 1.00 to 1.07.  (Neither hint nor sc1: 0.98, 0.97, 0.90, 0.96.  A branch
+    // at every store in place of a kernel of its own costs more than it gives: training 96 labels 2.17 -> 3.38 ms.)
     auto store_plane = [&](rsrc_t r, bool on, unsigned so, const float (&x)[R]) __attribute__((always_inline)) {
-      if constexpr (VEC) {
+      if constexpr (THROUGH) {
+        buf_store<R, true, kStoreThrough>(r, vec_off(on, so, 0), 0u, x);
+      } else if constexpr (VEC) {
         buf_store<R, true>(r, vec_off(on, so, 0), 0u, x);
       } else {
 #pragma unroll
@@ -511,7 +519,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
   }
 }
 
-template <int R, bool VEC, bool TRAIN, int kHelpers>
+template <int R, bool VEC, bool TRAIN, int kHelpers, bool THROUGH>
 __global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_fwd_team_kernel(const SweepParams p) {
   constexpr int kTeam = (kHelpers + 1) * kWave;
   extern __shared__ __align__(16) char smem_raw[];
@@ -560,7 +568,7 @@ __global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_fwd_team_kernel(
   __syncthreads();
   if (role == kHelpers) __builtin_amdgcn_s_setprio(3);
 
-#define MPL_WALK(KT, C0) team_walk<R, VEC, TRAIN, KT, C0, kHelpers>(p, desc, ch, slots, flags, a_s, ctx_s, role)
+#define MPL_WALK(KT, C0) team_walk<R, VEC, TRAIN, KT, C0, kHelpers, THROUGH>(p, desc, ch, slots, flags, a_s, ctx_s, role)
   // (the choice of the step: sweep_fwd_kernel)
   if (desc.linear && !p.ctx2d && (desc.band_k == 0 || desc.band_k > 4)) {
     MPL_WALK(-2, false);
@@ -601,7 +609,14 @@ inline size_t team_lds_bytes(int L, int R, bool ctx2d, size_t slot, int helpers)
 template <int R, bool VEC, bool TRAIN, int kHelpers>
 void launch_h(const SweepParams& p, hipStream_t st) {
   const size_t lds = team_lds_bytes(p.L, R, p.ctx2d != 0, sizeof(Slot<R>), kHelpers);
-  sweep_fwd_team_kernel<R, VEC, TRAIN, kHelpers><<<p.block_prefix[p.n_dirs], (kHelpers + 1) * kWave, lds, st>>>(p);
+  const auto launch = [&](auto kernel) { kernel<<<p.block_prefix[p.n_dirs], (kHelpers + 1) * kWave, lds, st>>>(p); };
+  if constexpr (VEC && R <= 2) {
+    if (p.through) {
+      launch(sweep_fwd_team_kernel<R, VEC, TRAIN, kHelpers, true>);
+      return;
+    }
+  }
+  launch(sweep_fwd_team_kernel<R, VEC, TRAIN, kHelpers, false>);
 }
 
 template <int R, bool VEC, bool TRAIN>
