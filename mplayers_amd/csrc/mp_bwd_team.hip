@@ -20,14 +20,15 @@
 // which of its neighbours up to kWin labels away point at it (five bits) and whether it belongs to
 // the ones that share a target (one bit); the main wavefront adds up masked neighbours from registers
 // and sums the others with the wave reduction that the normalisation needs anyway (two interleaved
-// chains of lane shifts).  Where labels are left that share a second target (either side of a slope
+// chains of lane shifts).  In launches of few chains (launch_vj) the bits come as masks as well, 1 or 0 in half precision,
+// so that a masked add is one instruction (v_fma_mix) in place of three.  Where labels are left that share a second target (either side of a slope
 // under a linear table) another wave reduction sums them; a pixel with any further argmin label scatters
 // through LDS float adds.  The normalisation (g[norm_index] -= sum g) reaches dU through its argmin label
 // only, and is subtracted there.
 //
 // Measured, TRWP backward on 4 directions, 5 iterations, min(k, 3) table, one wavefront per chain ->
 // this: 256x512x192 5.16 -> 2.12 ms (rows of 256 chains: 645 -> 246 ns per pixel and walk; the main
-// wavefront issues 112 instructions per pixel, some five clocks each), with dedge_weights and dcontext
+// wavefront issues 112 instructions per pixel, some five clocks each; masks take another 0.2 ms off), with dedge_weights and dcontext
 // 7.18 -> 3.8, 500x800x192 8.91 -> 5.87; bent table 240x320x96 with dcontext 5.95 -> 3.18.  Argmin labels
 // anywhere, so that every pixel scatters through LDS adds, 459 instead of 243 ns with 192 labels.  Three helpers with
 // two pixels each of a block; with one pixel 2.14, with four 2.36; six helpers of one pixel: launch_vj.  Which launches take it: team_chains_per_cu (mp_api.hip).
@@ -96,6 +97,15 @@ struct PixT {
   float w, de;
 };
 
+// LDS of a workgroup, but for the masks of a code byte per label that may follow
+template <int R>
+__host__ __device__ inline size_t team_lds_bytes(int L, bool gr, int helpers) {
+  const size_t bytes = 2 * kT * (sizeof(Slot<R>) + sizeof(Scalars)) +
+                       sizeof(float) * (kAccFloats + (gr ? L + helpers * hist_floats(R, L) : 0));
+  return (bytes + 15) & ~(size_t)15;
+}
+constexpr size_t mask_lds_bytes(int R) { return 2 * kT * R * kWave * 16; }
+
 // sums of x and y over the 64 lanes, the two chains of lane-shifted adds interleaved (a lane shift
 // may read a register two slots after it was written); the same association as wave_sum_fast
 __device__ __forceinline__ void wave_sum2(float& x, float& y) {
@@ -110,6 +120,28 @@ __device__ __forceinline__ void wave_sum2(float& x, float& y) {
   x = readlane_f(x, 63);
   y = readlane_f(y, 63);
 }
+
+// A code byte as eight numbers, 1 where the bit is set, in one 16-byte read: a multiply-add with such a mask (v_fma_mix)
+// takes the place of an extraction, an AND and an add.
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f16x8 masks_of(int byte) {
+  i32x4 m;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int two = (byte >> (2 * k)) & 3;
+    m[k] = (int)__umul24((unsigned)((two | (two << 15)) & 0x10001), 0x3c00u);  // (1 in half precision, in either half)
+  }
+  return __builtin_bit_cast(f16x8, m);
+}
+// the same masks (left to itself the compiler shifts upper halves down ahead of the branch that uses them)
+__device__ __forceinline__ f16x8 opaque(f16x8 m) {
+  i32x4 x = __builtin_bit_cast(i32x4, m);
+  int x0 = x[0], x1 = x[1], x2 = x[2];
+  asm("" : "+v"(x0), "+v"(x1), "+v"(x2));
+  return __builtin_bit_cast(f16x8, i32x4{x0, x1, x2, x[3]});
+}
+__device__ __forceinline__ float mask_add(_Float16 mask, float x, float sum) { return fmaf((float)mask, x, sum); }
 
 // x where bit BIT of the code is set, else 0 (the compiler makes a comparison, a wait state and a
 // select of an arithmetic form)
@@ -271,8 +303,8 @@ __device__ __forceinline__ void lds_order() {  // of this wavefront's own LDS in
   __builtin_amdgcn_wave_barrier();
 }
 
-// GR: dedge_weights and / or dcontext are wanted
-template <int R, bool VEC, bool JACOBI, bool GR, int kHelpers>
+// GR: dedge_weights and / or dcontext are wanted.  MASKS: the helpers put the codes into LDS as masks too (masks_of).
+template <int R, bool VEC, bool JACOBI, bool GR, int kHelpers, bool MASKS>
 __global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_bwd_team_kernel(const BackParams p, const int turn_every) {
   constexpr int kPer = kT / kHelpers;  // pixels of a block per helper
   constexpr int kTeam = (kHelpers + 1) * kWave;
@@ -284,6 +316,7 @@ __global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_bwd_team_kernel(
   const int L = p.L;
   const int n_ctx = L;  // (1-D tables only)
   float* hist_s = ctx_s + n_ctx;  // dcontext, one histogram per helper
+  f16x8* masks = reinterpret_cast<f16x8*>(smem_raw + team_lds_bytes<R>(L, GR, kHelpers));  // [2 kT][R][kWave]
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   // The last wavefront is the main one in every workgroup: the wavefronts of the workgroups that a compute
@@ -321,85 +354,155 @@ __global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_bwd_team_kernel(
 #pragma unroll
     for (int j = 0; j < R; ++j) sc[j] = 0.f;
     float* const mine = acc + lab0;
+    // one pixel: sc is dU of the one before, then of this one
+    auto pixel = [&](Slot<R>& s, Scalars& sv, const float (&base)[R], const int code, const int rest, const f16x8 (&m)[R],
+                     const auto read_next, const auto masked) __attribute__((always_inline)) {
+      constexpr bool M = decltype(masked)::value;
+      float g[R], part, pop;
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+        // gradient w.r.t. the normalised message of this pixel, including what the previous
+        // step added through the recurrence (dmsg[front] += rho * value, TRWP_backward.cu:108)
+        g[j] = fmaf(rho, sc[j], base[j]);
+      lds_put(s.sc[lane], sc);
+      read_next();
+      part = g[0];
+      pop = M ? mask_add(m[0][kPop], g[0], 0.f) : if_bit<kPop>(code, g[0]);
+      static_for<R - 1>([&](auto jj) __attribute__((always_inline)) {
+        constexpr int j = decltype(jj)::value + 1;
+        part += g[j];
+        if constexpr (M)
+          pop = mask_add(m[j][kPop], g[j], pop);
+        else
+          add_popular<8 * j>(code, g[j], pop);
+      });
+      wave_sum2(part, pop);
+      float near[R];
+      auto near_sums = [&]() __attribute__((always_inline)) {
+        float nb[R + 2 * kWin];
+        neighbours<R>(g, nb);
+        if constexpr (M) {
+          f16x8 mj[R];
+#pragma unroll
+          for (int j = 0; j < R; ++j) mj[j] = opaque(m[j]);
+          // (the labels' sums side by side: one that follows another of its label waits a slot)
+#pragma unroll
+          for (int b = 0; b <= 2 * kWin; ++b)
+#pragma unroll
+            for (int j = 0; j < R; ++j) near[j] = mask_add(mj[j][b], nb[j + b], b == 0 ? 0.f : near[j]);
+        } else {
+          static_for<R>([&](auto jj) __attribute__((always_inline)) {
+            constexpr int j = decltype(jj)::value;
+            near[j] = window_sum<8 * j>(code, nb[j], nb[j + 1], nb[j + 2], nb[j + 3], nb[j + 4]);
+          });
+        }
+      };
+      const int kind = __builtin_amdgcn_readfirstlane(rest);
+      if (__builtin_expect((kind & (1 << kRest)) == 0, 1)) {
+        near_sums();
+      } else if (kind >= 0) {  // (bit kMore) two shared targets
+        near_sums();
+        float pop2 = 0.f;
+        static_for<R>([&](auto jj) __attribute__((always_inline)) {
+          constexpr int j = decltype(jj)::value;
+          pop2 += if_bit<pop2_bit(R) + j>(rest, g[j]);
+        });
+        pop2 = wave_sum_fast(pop2);
+        static_for<R>([&](auto jj) __attribute__((always_inline)) {
+          constexpr int j = decltype(jj)::value;
+          near[j] += if_bit<is_pop2_bit(R) + j>(rest, pop2);
+        });
+      } else {
+        const int fds = s.fds[lane];
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          const bool skip = ((code >> (8 * j + kPop)) & 1) != 0 || lab0 + j >= L;
+          atomicAdd(&acc[skip ? kMaxL + lane : ((fds >> (8 * j)) & 0xff)], g[j]);
+        }
+        lds_order();
+#pragma unroll
+        for (int j = 0; j < R; ++j) near[j] = mine[j];
+        lds_order();
+#pragma unroll
+        for (int j = 0; j < R; ++j) mine[j] = 0.f;
+        lds_order();
+      }
+      if (GR) sv.tot = part;  // (every lane stores the same value to the same address)
+      static_for<R>([&](auto jj) __attribute__((always_inline)) {
+        constexpr int j = decltype(jj)::value;
+        if constexpr (M)
+          sc[j] = near[j] + mask_add(-m[j][kIsNrm], part, mask_add(m[j][kIsPop], pop, 0.f));
+        else
+          sc[j] = window_finish<8 * j>(code, near[j], pop, part);
+      });
+    };
     for (int k = 0; k < iters; ++k) {
       if (k >= 1 && k <= blocks) {
         Slot<R>* s = slots + ((k - 1) & 1) * kT;
         Scalars* sv = scal + ((k - 1) & 1) * kT;
-        float base[R];
-        int code, rest;
-        get_in<R>(s[0].in[lane], base, code, rest);
+        const f16x8* const mk = masks + (((k - 1) & 1) * kT * R) * kWave + lane;
+        auto block = [&](const auto masked) __attribute__((always_inline)) {
+          constexpr bool M = decltype(masked)::value;
+          float base[R];
+          int code, rest;
+          f16x8 m[R] = {};
+          get_in<R>(s[0].in[lane], base, code, rest);
+          if constexpr (M) {
 #pragma unroll
-        for (int i = 0; i < kT; ++i) {
-          float g[R], part, pop;
-#pragma unroll
-          for (int j = 0; j < R; ++j)
-            // gradient w.r.t. the normalised message of this pixel, including what the previous
-            // step added through the recurrence (dmsg[front] += rho * value, TRWP_backward.cu:108)
-            g[j] = fmaf(rho, sc[j], base[j]);
-          lds_put(s[i].sc[lane], sc);
-          float nbase[R];
-          int ncode = 0, nrest = 0;
-          if (i + 1 < kT) {
-            get_in<R>(s[i + 1].in[lane], nbase, ncode, nrest);
+            for (int j = 0; j < R; ++j) m[j] = mk[j * kWave];
           }
-          part = g[0];
-          pop = if_bit<kPop>(code, g[0]);
-          static_for<R - 1>([&](auto jj) __attribute__((always_inline)) {
-            constexpr int j = decltype(jj)::value + 1;
-            part += g[j];
-            add_popular<8 * j>(code, g[j], pop);
-          });
-          wave_sum2(part, pop);
-          float near[R];
-          auto near_sums = [&]() __attribute__((always_inline)) {
-            float nb[R + 2 * kWin];
-            neighbours<R>(g, nb);
-            static_for<R>([&](auto jj) __attribute__((always_inline)) {
-              constexpr int j = decltype(jj)::value;
-              near[j] = window_sum<8 * j>(code, nb[j], nb[j + 1], nb[j + 2], nb[j + 3], nb[j + 4]);
-            });
-          };
-          const int kind = __builtin_amdgcn_readfirstlane(rest);
-          if (__builtin_expect((kind & (1 << kRest)) == 0, 1)) {
-            near_sums();
-          } else if (kind >= 0) {  // (bit kMore) two shared targets
-            near_sums();
-            float pop2 = 0.f;
-            static_for<R>([&](auto jj) __attribute__((always_inline)) {
-              constexpr int j = decltype(jj)::value;
-              pop2 += if_bit<pop2_bit(R) + j>(rest, g[j]);
-            });
-            pop2 = wave_sum_fast(pop2);
-            static_for<R>([&](auto jj) __attribute__((always_inline)) {
-              constexpr int j = decltype(jj)::value;
-              near[j] += if_bit<is_pop2_bit(R) + j>(rest, pop2);
-            });
-          } else {
-            const int fds = s[i].fds[lane];
 #pragma unroll
-            for (int j = 0; j < R; ++j) {
-              const bool skip = ((code >> (8 * j + kPop)) & 1) != 0 || lab0 + j >= L;
-              atomicAdd(&acc[skip ? kMaxL + lane : ((fds >> (8 * j)) & 0xff)], g[j]);
+          for (int i = 0; i < kT; ++i) {
+            float nbase[R];
+            int ncode = 0, nrest = 0;
+            f16x8 nm[R] = {};
+            pixel(
+                s[i], sv[i], base, code, rest, m,
+                [&]() __attribute__((always_inline)) {  // (the next pixel's reads, once this one's dU is on its way)
+                  if (i + 1 < kT) {
+                    get_in<R>(s[i + 1].in[lane], nbase, ncode, nrest);
+                    if constexpr (M) {
+#pragma unroll
+                      for (int j = 0; j < R; ++j) nm[j] = mk[((i + 1) * R + j) * kWave];
+                    }
+                  }
+                },
+                masked);
+            if (i + 1 < kT) {
+#pragma unroll
+              for (int j = 0; j < R; ++j) {
+                base[j] = nbase[j];
+                m[j] = nm[j];
+              }
+              code = ncode;
+              rest = nrest;
             }
-            lds_order();
-#pragma unroll
-            for (int j = 0; j < R; ++j) near[j] = mine[j];
-            lds_order();
-#pragma unroll
-            for (int j = 0; j < R; ++j) mine[j] = 0.f;
-            lds_order();
           }
-          if (GR) sv[i].tot = part;  // (every lane stores the same value to the same address)
-          static_for<R>([&](auto jj) __attribute__((always_inline)) {
-            constexpr int j = decltype(jj)::value;
-            sc[j] = window_finish<8 * j>(code, near[j], pop, part);
-          });
-          if (i + 1 < kT) {
+        };
+        if constexpr (MASKS) {
+          float sc_was[R];
 #pragma unroll
-            for (int j = 0; j < R; ++j) base[j] = nbase[j];
-            code = ncode;
-            rest = nrest;
+          for (int j = 0; j < R; ++j) sc_was[j] = sc[j];
+          block(std::true_type());
+          // A zero mask does not switch off what is not finite: an infinity or a NaN in a gradient, or in a sum, makes
+          // NaN of every label's dU, there and from there on (tested as an integer: the compiler may take NaN for
+          // anything).  The pixels of such a block go by the codes, one after another.
+          int probe = uniform_i(__builtin_bit_cast(int, sc[0]));
+          asm("" : "+s"(probe));
+          if (__builtin_expect((probe & 0x7f800000) == 0x7f800000, 0)) {
+#pragma unroll
+            for (int j = 0; j < R; ++j) sc[j] = sc_was[j];
+            const f16x8 none[R] = {};
+#pragma clang loop unroll(disable)
+            for (int i = 0; i < kT; ++i) {
+              float base[R];
+              int code, rest;
+              get_in<R>(s[i].in[lane], base, code, rest);
+              pixel(s[i], sv[i], base, code, rest, none, []() {}, std::false_type());
+            }
           }
+        } else {
+          block(std::false_type());
         }
       }
       lds_barrier();
@@ -486,7 +589,7 @@ __global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_bwd_team_kernel(
     };
 
     // what the recurrence needs of a pixel, into its slot
-    auto prepare = [&](const PixT<R>& px, Slot<R>& s, Scalars& sv) __attribute__((always_inline)) {
+    auto prepare = [&](const PixT<R>& px, Slot<R>& s, Scalars& sv, f16x8* const mk) __attribute__((always_inline)) {
       const int nidx = __builtin_amdgcn_readfirstlane(px.nidx);
       int fn = 0;  // argmin label of the normalisation label
 #pragma unroll
@@ -526,6 +629,7 @@ __global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_bwd_team_kernel(
         c |= l == pop ? 1 << kIsPop : 0;
         c |= l == fn ? 1 << kIsNrm : 0;
         code |= c << (8 * j);
+        if constexpr (MASKS) mk[j * kWave + lane] = masks_of(c);
         ap[j] = EVEN ? fmaf(rho, px.hi[j], px.a[j]) : px.a[j];
         base[j] = JACOBI ? px.a[j] : ap[j] + (EVEN ? -px.hd[j] - px.hi[j] : px.hd[j]);
         if (l >= L) base[j] = 0.f;
@@ -632,7 +736,7 @@ __global__ void __launch_bounds__((kHelpers + 1) * kWave) sweep_bwd_team_kernel(
         Scalars& sv = scal[set * kT + i];
         finish(n - 1 - ((k - 2) * kT + i), s, sv);
         lds_order();
-        prepare(ring[u], s, sv);
+        prepare(ring[u], s, sv, masks + (set * kT + i) * R * kWave);
         ring[u] = load_pix((k + 2) * kT + i);
       }
       lds_barrier();
@@ -704,9 +808,10 @@ template <int R, bool VEC, bool JACOBI>
 void launch_vj(const BackParams& p, hipStream_t st) {
   const int blocks = p.block_prefix[p.n_dirs];
   const bool gr = p.dedge != nullptr || p.dctx != nullptr;
-  const auto launch = [&](auto kernel, int helpers, int turn_every) {
-    const size_t lds = 2 * kT * (sizeof(Slot<R>) + sizeof(Scalars)) +
-                       sizeof(float) * (kAccFloats + (gr ? p.L + helpers * hist_floats(R, p.L) : 0));
+  const auto launch = [&](auto kernel, int helpers, int turn_every, size_t extra = 0) {
+    const size_t lds = team_lds_bytes<R>(p.L, gr, helpers) + extra;
+    if (lds > (64 << 10))
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     kernel<<<blocks, (helpers + 1) * kWave, lds, st>>>(p, turn_every);
   };
   // With four labels per lane the LDS holds two workgroups of a unit, and a launch of more runs in rounds.  When
@@ -725,11 +830,22 @@ void launch_vj(const BackParams& p, hipStream_t st) {
   // 500x700, 192 labels, 1199 diagonals 1.04 / 0.94 / 1.04.
   if constexpr (R < 4) {
     if (blocks <= 3 * n_cu) {
-      launch(gr ? sweep_bwd_team_kernel<R, VEC, JACOBI, true, 6> : sweep_bwd_team_kernel<R, VEC, JACOBI, false, 6>, 6, 0);
+      // Masks where the LDS holds those of all the launch's chains (160 KB a unit, given out in 1280 bytes): a chain per
+      // unit more would wait for another to end.  Over the codes, the layer's whole pass, 4 directions, 5 iterations, dunary
+      // alone: 192 labels 256x512 0.946, 130x160 0.92, 96 and 128 labels 240x320 0.91, 191 labels 0.98; with 8 directions, whose
+      // diagonals are more chains than that, 200x260 0.93, 375x450 0.99; a learned table 96 labels 240x320 0.975; ISGMR
+      // 128 labels 130x160 0.96.
+      const size_t with_masks = (team_lds_bytes<R>(p.L, gr, 6) + mask_lds_bytes(R) + 1279) / 1280 * 1280;
+      if ((size_t)blocks <= n_cu * ((160 << 10) / with_masks)) {
+        launch(gr ? sweep_bwd_team_kernel<R, VEC, JACOBI, true, 6, true> : sweep_bwd_team_kernel<R, VEC, JACOBI, false, 6, true>, 6, 0,
+               mask_lds_bytes(R));
+        return;
+      }
+      launch(gr ? sweep_bwd_team_kernel<R, VEC, JACOBI, true, 6, false> : sweep_bwd_team_kernel<R, VEC, JACOBI, false, 6, false>, 6, 0);
       return;
     }
   }
-  launch(gr ? sweep_bwd_team_kernel<R, VEC, JACOBI, true, 3> : sweep_bwd_team_kernel<R, VEC, JACOBI, false, 3>, 3, turn_every);
+  launch(gr ? sweep_bwd_team_kernel<R, VEC, JACOBI, true, 3, false> : sweep_bwd_team_kernel<R, VEC, JACOBI, false, 3, false>, 3, turn_every);
 }
 
 }  // namespace
