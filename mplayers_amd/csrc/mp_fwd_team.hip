@@ -386,11 +386,19 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
       return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
                                            dW, (lane < kWs && tl < n) ? (int)(pp * 4u) : kDeadOffset, 0, 0));
     };
+    const int first_stored = p.zero_start ? 0 : 1;
     float md0[R];  // second sweep: the old message of the chain start (helper 0)
     if (!EVEN) load_plane(rMd, role == 0, (unsigned)ch.pix0 * (unsigned)L * 4u, md0);
 
     float tt[2][kPer][R], ww[2][kPer];  // of the blocks in the slots
 
+    // Whether chain position t is one of first .. n - 1, in one comparison: half of the helpers' instructions were scalar
+    // ones that asked about either end.  60 and 64 labels, argmin labels kept, rows of 200 to 450, two comparisons -> one:
+    // 128 and 256 chains 0.97, 320 to 512 chains 0.91 to 0.94, 700 chains 0.94; 96 and 128 labels 0.98 to 1.00; 191
+    // labels 512 chains 0.95.  Without argmin labels 0.97 to 1.01.
+    auto within = [&](const int t, const int first) __attribute__((always_inline)) {
+      return (unsigned)(t - first) < (unsigned)(n - first);
+    };
     auto prepare = [&](const PixT<R>& px, const float w, const int t, const int i, Slot<R>& s, Flags& f,
                        float (&tk)[R], float& wk)
         __attribute__((always_inline)) {
@@ -403,7 +411,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
       }
       wk = w;
       put_in<R>(s, f, i, lane, un, w);
-      if (KT >= 0 || KT == -2) f.neg[i] = (t >= 1 && t < n && !(w >= 0.f)) ? 1 : 0;
+      if (KT >= 0 || KT == -2) f.neg[i] = (within(t, 1) && !(w >= 0.f)) ? 1 : 0;
       // Q of the pixel is known already, whatever its message
       if (EVEN) store_plane(rSo, t < n, (unsigned)(ch.pix0 + t * ch.pstep) * (unsigned)L * 4u, q);
     };
@@ -411,7 +419,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
     // what is left of a pixel once its message is known (nothing outside the chain)
     auto finish = [&](const int t, const Slot<R>& s, const float (&tk)[R], const float wk)
         __attribute__((always_inline)) {
-      const bool on = t >= 0 && t < n;
+      const bool on = within(t, 0);
       const unsigned pp = (unsigned)(ch.pix0 + t * ch.pstep);
       const unsigned so = pp * (unsigned)L * 4u;
       float m[R];
@@ -429,7 +437,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
           pr[j] = lab0 + j < L && v[j] == nmin;
         }
         const int nidx = last_label<R>(pr, L - 1);
-        const bool idx_on = on && t > 0;
+        const bool idx_on = within(t, 1);
         if constexpr (VEC) {
           buf_store_u8<R, true>(rImin, (int)((idx_on && lane_ok) ? pp * (unsigned)L + (unsigned)lab0 : kDeadWide), 0u, fd_idx);
         } else {
@@ -443,7 +451,7 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
         __builtin_amdgcn_raw_buffer_store_b8((unsigned char)nidx, dInorm, idx_on ? (int)pp : kDeadOffset, 0, 0);
       }
       // (the reference never writes the chain start)
-      store_plane(rMo, on && (t > 0 || p.zero_start), so, m);
+      store_plane(rMo, within(t, first_stored), so, m);
       if constexpr (!EVEN) {
         float sn[R];
 #pragma unroll
