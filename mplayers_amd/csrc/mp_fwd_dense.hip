@@ -99,6 +99,69 @@ __device__ __forceinline__ void get_words(const float* src, float (&x)[R]) {
   }
 }
 
+// +inf that the compiler cannot see through: what starts from it is +inf where no candidate is a number (a candidate
+// that is none drops out of a minimum; left to itself the compiler leaves out a minimum with +inf), so a share without
+// a number says nothing about the labels or their least one.  Argmin labels kept, rows of 257 on 256 chains, with what
+// finds the labels of such pixels, over neither: 17 to 64 labels 1.01 to 1.02, 96 and 128 labels 1.00 to 1.01, 192 labels 1.00.
+__device__ __forceinline__ float opaque_inf() {
+  float x = INFINITY;
+  asm volatile("" : "+s"(x));
+  return x;
+}
+
+// Comparisons that are false of what is no number, whichever way round the compiler puts the select behind them (of a
+// plain one it takes the opposite, which is false of it too).
+__device__ __forceinline__ bool equal(const float a, const float b) {
+  return __builtin_amdgcn_inverse_ballot_w64(__builtin_amdgcn_fcmpf(a, b, 1));  // (ordered, equal)
+}
+__device__ __forceinline__ bool at_most(const float a, const float b) {
+  return __builtin_amdgcn_inverse_ballot_w64(__builtin_amdgcn_fcmpf(a, b, 5));  // (ordered, less or equal)
+}
+
+constexpr int kNoLabel = kMaxL;
+// the candidates of label l in the trip from front label f0 on (the same multiply-adds on the same operands as in the
+// scan: the same bits)
+template <int R>
+__device__ __forceinline__ void trip_candidates(const float* a, const float* csym_s, const float w, const int f0, const int l,
+                                                float (&val)[kTrip]) {
+  const f32x4 a0 = *reinterpret_cast<const f32x4*>(a + f0);
+  const f32x4 a1 = *reinterpret_cast<const f32x4*>(a + f0 + 4);
+  const float* cp = csym_s + (dense_sym_centre<R>() + l - f0 - (kTrip - 1));  // entry of front label f0 + kTrip - 1
+#pragma unroll
+  for (int u = 0; u < kTrip; ++u) val[u] = fmaf(w, cp[kTrip - 1 - u], u < 4 ? a0[u & 3] : a1[u & 3]);
+}
+// the largest front label of them whose candidate is the minimum v; kNoLabel or more: none
+__device__ __forceinline__ int trip_label(const float (&val)[kTrip], const float v, const int f0) {
+  int arg = kNoLabel;
+#pragma unroll
+  for (int u = 0; u < kTrip; ++u) arg = equal(val[u], v) ? u : arg;
+  return f0 + arg;
+}
+// The labels that trip_label has not found: of a minimum of +inf, which a share without a number reaches too and whose
+// trip it then is.  All front labels are looked at, and the last one is taken where no candidate is a number, as in
+// the other scans.
+template <int R>
+__device__ __forceinline__ void labels_without_trip(const float* a, const float* csym_s, const float w, const float (&v)[R],
+                                                    const int lab0, const int L, int (&fd_idx)[R]) {
+  bool none[R], any = false;
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    none[j] = fd_idx[j] >= L;
+    any |= none[j];
+    fd_idx[j] = min(fd_idx[j], L - 1);
+  }
+  if (__builtin_expect(ballot(any) == 0, 1)) return;
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const float* cp = csym_s + (dense_sym_centre<R>() + lab0 + j);
+#pragma clang loop unroll(disable)
+    for (int fd = 0; fd < L; ++fd) {
+      const bool is_min = equal(fmaf(w, cp[-fd], a[fd]), v[j]);
+      fd_idx[j] = none[j] && is_min ? fd : fd_idx[j];
+    }
+  }
+}
+
 // NT: trips per wavefront
 template <int R, bool TRAIN, int NT>
 __device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx& ch0, const bool msg_zero,
@@ -119,6 +182,7 @@ __device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx&
   const int64_t N = P * L;
   const int blocks = (n + kBlock - 1) / kBlock;
   const int fd_lo = wave * kShare;
+  const float inf = opaque_inf();
 
   float floor_l[R];
 #pragma unroll
@@ -163,7 +227,7 @@ __device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx&
       int trip[R];
 #pragma unroll
       for (int j = 0; j < R; ++j) {
-        v[j] = INFINITY;
+        v[j] = inf;
         trip[j] = wave * NT;
       }
       f32x4 x[2 * NT];
@@ -180,13 +244,8 @@ __device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx&
           for (int u = 0; u < kTrip; ++u) c[u] = fmaf(w, tab[k * kTrip + u][j], u < 4 ? x0[u & 3] : x1[u & 3]);
           if constexpr (TRAIN) {
             const float lm = fminf(fminf(fminf(fminf(fminf(c[0], c[1]), c[2]), fminf(fminf(c[3], c[4]), c[5])), c[6]), c[7]);
-            if (k > 0) {
-              const bool take = lm <= v[j];
-              v[j] = fminf(v[j], lm);
-              trip[j] = take ? wave * NT + k : trip[j];
-            } else {
-              v[j] = lm;
-            }
+            if (k > 0) trip[j] = at_most(lm, v[j]) ? wave * NT + k : trip[j];
+            v[j] = fminf(lm, v[j]);
           } else {
 #pragma unroll
             for (int u = 0; u < kTrip; u += 2) v[j] = fminf(fminf(v[j], c[u]), c[u + 1]);
@@ -316,29 +375,21 @@ __device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx&
       if constexpr (TRAIN) {
         float un[R], w;
         get_slot<R>(st.in[i][lane], un, w);
-        int fd_idx[R];
+        int fd_idx[R], f0[R];
         bool pr[R];
+        float val[R][kTrip];
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-          const int f0 = ((trips >> (8 * j)) & 0xff) * kTrip;
-          const int l = lab0 + j < L ? lab0 + j : L - 1;
-          const f32x4 a0 = *reinterpret_cast<const f32x4*>(&st.a[i][f0]);
-          const f32x4 a1 = *reinterpret_cast<const f32x4*>(&st.a[i][f0 + 4]);
-          const float* cp = csym_s + (dense_sym_centre<R>() + l - f0 - (kTrip - 1));  // entry of front label f0 + kTrip - 1
-          int arg = 0;
-#pragma unroll
-          for (int u = 0; u < kTrip; ++u) {
-            const float val = fmaf(w, cp[kTrip - 1 - u], u < 4 ? a0[u & 3] : a1[u & 3]);
-            arg = val == v[j] ? u : arg;
-          }
-          const int fd = f0 + arg;
-          // (the last label where no candidate is a number, as in the other scans: a test of the bits, which the
-          // compiler may not take for false)
-          const bool none = (__builtin_bit_cast(unsigned, v[j]) & 0x7fffffffu) > 0x7f800000u;
-          fd_idx[j] = fd < L && !none ? fd : L - 1;
-          pr[j] = lab0 + j < L && v[j] == nmin;
+          f0[j] = ((trips >> (8 * j)) & 0xff) * kTrip;
+          trip_candidates<R>(st.a[i], csym_s, w, f0[j], lab0 + j, val[j]);
         }
         pause();
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          fd_idx[j] = trip_label(val[j], v[j], f0[j]);
+          pr[j] = lab0 + j < L && v[j] == nmin;
+        }
+        labels_without_trip<R>(st.a[i], csym_s, w, v, lab0, L, fd_idx);
         const int nidx = last_label<R>(pr, L - 1);
         const bool idx_on = on && t > 0;
         const unsigned sob = pp * (unsigned)L;
@@ -467,6 +518,7 @@ __device__ __forceinline__ void walk_chain_alone(const SweepParams& p, const Cha
   const int64_t N = P * L;
   const int blocks = (n + kBlockAlone - 1) / kBlockAlone;
   const int fd_lo = wave * kShare;
+  const float inf = opaque_inf();
 
   float floor_l[R];
 #pragma unroll
@@ -587,23 +639,12 @@ __device__ __forceinline__ void walk_chain_alone(const SweepParams& p, const Cha
 #pragma unroll
         for (int j = 0; j < R; ++j) {
           const int f0 = ((trips >> (8 * j)) & 0xff) * kTrip;
-          const int l = lab0 + j < L ? lab0 + j : L - 1;
-          const f32x4 a0 = *reinterpret_cast<const f32x4*>(&s.a[i][f0]);
-          const f32x4 a1 = *reinterpret_cast<const f32x4*>(&s.a[i][f0 + 4]);
-          const float* cp = csym_s + (dense_sym_centre<R>() + l - f0 - (kTrip - 1));  // entry of front label f0 + kTrip - 1
-          int arg = 0;
-#pragma unroll
-          for (int u = 0; u < kTrip; ++u) {
-            const float val = fmaf(w, cp[kTrip - 1 - u], u < 4 ? a0[u & 3] : a1[u & 3]);
-            arg = val == v[j] ? u : arg;
-          }
-          const int fd = f0 + arg;
-          // (the last label where no candidate is a number, as in the other scans: a test of the bits, which the
-          // compiler may not take for false)
-          const bool none = (__builtin_bit_cast(unsigned, v[j]) & 0x7fffffffu) > 0x7f800000u;
-          fd_idx[j] = fd < L && !none ? fd : L - 1;
+          float val[kTrip];
+          trip_candidates<R>(s.a[i], csym_s, w, f0, lab0 + j, val);
+          fd_idx[j] = trip_label(val, v[j], f0);
           pr[j] = lab0 + j < L && v[j] == nmin;
         }
+        labels_without_trip<R>(s.a[i], csym_s, w, v, lab0, L, fd_idx);
         const int nidx = last_label<R>(pr, L - 1);
         const bool idx_on = on && t > 0;
         const unsigned sob = pp * (unsigned)L;
@@ -641,7 +682,7 @@ __device__ __forceinline__ void walk_chain_alone(const SweepParams& p, const Cha
       int trip[R];
 #pragma unroll
       for (int j = 0; j < R; ++j) {
-        v[j] = INFINITY;
+        v[j] = inf;
         trip[j] = wave * NT;
       }
 #pragma unroll
@@ -655,13 +696,8 @@ __device__ __forceinline__ void walk_chain_alone(const SweepParams& p, const Cha
           for (int u = 0; u < kTrip; ++u) c[u] = fmaf(w, tab[k * kTrip + u][j], u < 4 ? x0[u & 3] : x1[u & 3]);
           if constexpr (TRAIN) {
             const float lm = fminf(fminf(fminf(fminf(fminf(c[0], c[1]), c[2]), fminf(fminf(c[3], c[4]), c[5])), c[6]), c[7]);
-            if (k > 0) {
-              const bool take = lm <= v[j];
-              v[j] = fminf(v[j], lm);
-              trip[j] = take ? wave * NT + k : trip[j];
-            } else {
-              v[j] = lm;
-            }
+            if (k > 0) trip[j] = at_most(lm, v[j]) ? wave * NT + k : trip[j];
+            v[j] = fminf(lm, v[j]);
           } else {
 #pragma unroll
             for (int u = 0; u < kTrip; u += 2) v[j] = fminf(fminf(v[j], c[u]), c[u + 1]);
