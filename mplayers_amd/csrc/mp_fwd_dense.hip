@@ -109,15 +109,6 @@ __device__ __forceinline__ float opaque_inf() {
   return x;
 }
 
-// Comparisons that are false of what is no number, whichever way round the compiler puts the select behind them (of a
-// plain one it takes the opposite, which is false of it too).
-__device__ __forceinline__ bool equal(const float a, const float b) {
-  return __builtin_amdgcn_inverse_ballot_w64(__builtin_amdgcn_fcmpf(a, b, 1));  // (ordered, equal)
-}
-__device__ __forceinline__ bool at_most(const float a, const float b) {
-  return __builtin_amdgcn_inverse_ballot_w64(__builtin_amdgcn_fcmpf(a, b, 5));  // (ordered, less or equal)
-}
-
 constexpr int kNoLabel = kMaxL;
 // the candidates of label l in the trip from front label f0 on (the same multiply-adds on the same operands as in the
 // scan: the same bits)

@@ -16,6 +16,15 @@ __device__ __forceinline__ void lds_order() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Comparisons that are false of what is no number, whichever way round the compiler puts the select behind them (of a
+// plain one it takes the opposite, which is false of it too).
+__device__ __forceinline__ bool equal(const float a, const float b) {
+  return __builtin_amdgcn_inverse_ballot_w64(__builtin_amdgcn_fcmpf(a, b, 1));  // (ordered, equal)
+}
+__device__ __forceinline__ bool at_most(const float a, const float b) {
+  return __builtin_amdgcn_inverse_ballot_w64(__builtin_amdgcn_fcmpf(a, b, 5));  // (ordered, less or equal)
+}
+
 // Dense O(L^2) step: v[cd] = min_fd( a[fd] + w * ctx(cd, fd) ), largest fd on ties.
 // HorizontalKernel inner loop, TRWP_forward.cu:127-153.  a_s / ctx_s live in LDS.
 template <int R, bool TRAIN>
@@ -103,7 +112,7 @@ __device__ __forceinline__ void dense1d_step(const float (&a)[R], const float w,
   auto close_trip = [&](const float (&lm)[R]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-      const bool take = lm[j] <= v[j];
+      const bool take = at_most(lm[j], v[j]);
       v[j] = fminf(v[j], lm[j]);
       rel[j] = take ? 0 : rel[j] - 1;
     }
@@ -224,7 +233,7 @@ __device__ __forceinline__ void dense1d_argmin(const float (&v)[R], const int (&
 #pragma unroll
     for (int u = 0; u < T; ++u) {
       const float val = fmaf(w, cp[T - 1 - u], af[u]);
-      arg = val == v[j] ? u : arg;
+      arg = equal(val, v[j]) ? u : arg;
     }
     const int fd = t0 + arg;
     fd_idx[j] = fd < L ? fd : L - 1;
@@ -266,7 +275,7 @@ __device__ __forceinline__ void dense1d_step_lanes(const float (&a)[R], float w,
       if (TRAIN) {
         // (the minimum and the comparison are independent instructions; a select of the value
         // would wait for the comparison's lane mask like the select of the label does)
-        const bool take = val <= v[j];
+        const bool take = at_most(val, v[j]);
         v[j] = fminf(v[j], val);
         fd_idx[j] = take ? fd : fd_idx[j];
       } else {

@@ -22,7 +22,7 @@ def _table_with_forbidden_jumps(L, lo, hi, W, iterations, training, B=1):
 
 
 def _same(four, one, training):
-  for k in ("msg", "cost_final", "label_all") + (("msg_norm_index",) if training else ()):
+  for k in ("msg", "cost_final", "label_all") + (("msg_min_index", "msg_norm_index") if training else ()):
     assert np.array_equal(four[k], one[k], equal_nan=True), k
 
 
@@ -78,8 +78,10 @@ def test_argmin_labels_against_the_definition(gpu, L, many):
     least = np.where(np.isnan(cand), np.inf, cand).min(1)
     want = np.where((cand == least[:, None]).any(1), L - 1 - np.argmax((cand == least[:, None])[:, ::-1], 1), L - 1)
     print("case", L, B, kind, flush=True)
-    got = _run(gpu, 2, np.repeat(u, B, 0), ctx, np.repeat(ew, B, 1), 2, 1, True, _lib.F_PACKED_OFF | _lib.F_DENSE_TABLE)
-    for b in (0, B - 1):
-      assert np.array_equal(got["msg_min_index"][0, 0, b, 0, 0, 1], want), kind
-      with np.errstate(invalid="ignore"):
-        assert np.array_equal(got["msg"][0, b, 0, 0, 1], (least - least.min()).astype(np.float32), equal_nan=True), kind
+    # one wavefront per chain, four with the same step, four that share the front labels
+    for option, flags in ((0, 0), (2, 0), (2, _lib.F_DENSE_TABLE)):
+      got = _run(gpu, option, np.repeat(u, B, 0), ctx, np.repeat(ew, B, 1), 2, 1, True, _lib.F_PACKED_OFF | flags)
+      for b in (0, B - 1):
+        assert np.array_equal(got["msg_min_index"][0, 0, b, 0, 0, 1], want), (kind, option, flags)
+        with np.errstate(invalid="ignore"):
+          assert np.array_equal(got["msg"][0, b, 0, 0, 1], (least - least.min()).astype(np.float32), equal_nan=True), kind
