@@ -313,6 +313,9 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
     MPL_ORDER_LOADS();
   }
 
+  // The dense 1-D steps leave out candidates that are no number, so a term that is none must not become the -inf
+  // that a maximum with the floor makes of it.
+  const bool keep_nan = kDenseMain && !(R == 1 && (p.ctx2d || (KT == -1 && L < kSlidingMinL)));
   int st_p = ch.pix0 + ch.pstep;
   // in_chain: a constant `true` where the caller knows that step t lies inside the chain and that
   // no edge weight of the chain is negative
@@ -331,7 +334,7 @@ __device__ __forceinline__ void run_chain_fwd(const SweepParams& p, const CtxDes
         } else {
           tt[j] = 0.f;
         }
-        un[j] = MASK ? fmaxf(x, floor_l[j]) : x;
+        un[j] = !MASK ? x : keep_nan ? (valid[j] ? x : inf) : fmaxf(x, floor_l[j]);
       }
       const float w = uniform_f(px.w);
       float a[R], v[R];

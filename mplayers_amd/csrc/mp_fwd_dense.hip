@@ -330,7 +330,8 @@ __device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx&
 #pragma unroll
       for (int j = 0; j < R; ++j) {
         tk[j] = EVEN ? px.s[j] - px.md[j] : px.s[j] + px.mi[j];
-        un[j] = fmaxf(fmaf(tk[j], rho, -px.mi[j]), floor_l[j]);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
+        // UpdateUnaryKernel, TRWP_forward.cu:70-78 (no maximum with the floor, which is -inf where a term is no number)
+        un[j] = lab0 + j < L ? fmaf(tk[j], rho, -px.mi[j]) : INFINITY;
         q[j] = tk[j] - px.mi[j];
       }
       put_slot<R>(st.in[i][lane], un, px.w);
@@ -589,7 +590,8 @@ __device__ __forceinline__ void walk_chain_alone(const SweepParams& p, const Cha
 #pragma unroll
       for (int j = 0; j < R; ++j) {
         tk[j] = EVEN ? px.s[j] - px.md[j] : px.s[j] + px.mi[j];
-        un[j] = fmaxf(fmaf(tk[j], rho, -px.mi[j]), floor_l[j]);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
+        // UpdateUnaryKernel, TRWP_forward.cu:70-78 (no maximum with the floor, which is -inf where a term is no number)
+        un[j] = lab0 + j < L ? fmaf(tk[j], rho, -px.mi[j]) : INFINITY;
         q[j] = tk[j] - px.mi[j];
       }
       put_slot<R>(s.in[i][lane], un, px.w);

@@ -406,7 +406,8 @@ __device__ __forceinline__ void team_walk(const SweepParams& p, const CtxDesc& d
 #pragma unroll
       for (int j = 0; j < R; ++j) {
         tk[j] = EVEN ? px.s[j] - px.md[j] : px.s[j] + px.mi[j];
-        un[j] = fmaxf(fmaf(tk[j], rho, -px.mi[j]), c.floor_l[j]);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
+        un[j] = fmaf(tk[j], rho, -px.mi[j]);  // UpdateUnaryKernel, TRWP_forward.cu:70-78
+        un[j] = KT == -1 && !c.full_table ? (lab0 + j < L ? un[j] : INFINITY) : fmaxf(un[j], c.floor_l[j]);  // (keep_nan, mp_fwd.hip)
         q[j] = tk[j] - px.mi[j];
       }
       wk = w;

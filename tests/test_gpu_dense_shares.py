@@ -85,3 +85,31 @@ def test_argmin_labels_against_the_definition(gpu, L, many):
         assert np.array_equal(got["msg_min_index"][0, 0, b, 0, 0, 1], want), (kind, option, flags)
         with np.errstate(invalid="ignore"):
           assert np.array_equal(got["msg"][0, b, 0, 0, 1], (least - least.min()).astype(np.float32), equal_nan=True), kind
+
+
+@pytest.mark.parametrize("L", [8, 17, 32, 64, 96, 128, 160, 192, 256])
+@pytest.mark.parametrize("share", [0, 1, 2, 3])
+@pytest.mark.parametrize("training", [True, False])
+def test_unary_terms_without_a_number(gpu, L, share, training):
+  """Unary terms of a quarter of the labels that are NaN, at a chain's start and inside it: the messages stay numbers, in
+  every scan the same ones."""
+  import torch
+  from mplayers_amd import _lib
+  n = SHARE.get(L, -(-L // 4))
+  rng = np.random.default_rng(L + share)
+  ctx = rng.random(L).astype(np.float32)
+  ctx[[0, L - 1]] = 0  # (no band: entries above the last one)
+  many = 3 + torch.cuda.get_device_properties(0).multi_processor_count // 2
+  for B in (1,) if L <= 128 else (1, many):
+    for x in (0, 4, 8):
+      unary = (3 * rng.random((1, 1, 2, 9, L))).astype(np.float32)
+      unary[0, 0, 1, x, share * n:(share + 1) * n] = np.nan
+      ew = (0.1 + 0.9 * rng.random((4, 1, 1, 2, 9))).astype(np.float32)
+      problem = np.repeat(unary, B, 0), ctx, np.repeat(ew, B, 1), 4, 2, training
+      print("case", L, share, training, B, x, flush=True)
+      one = _run(gpu, 0, *problem, _lib.F_PACKED_OFF)
+      assert np.isfinite(one["msg"]).all()
+      for option, flags in ((2, 0), (2, _lib.F_DENSE_TABLE), (0, _lib.F_DENSE_TABLE)):
+        if L < 17 and flags:
+          continue
+        _same(_run(gpu, option, *problem, _lib.F_PACKED_OFF | flags), one, training)
