@@ -314,7 +314,17 @@ __global__ void __launch_bounds__(256) aggregate_first_kernel(const float* __res
 #pragma unroll
         for (int k = 0; k < ND; ++k) fold(k, m[k]);
       } else {
-        for (int k = 0; k < n_dir; ++k) fold(k, ld_pack<V, NT>(msg + (int64_t)k * N + i));
+        int k = 0;
+        if constexpr (V == 1) {  // (four planes' loads at a time: 97 labels 241x321, 12 directions 164 -> 85 us, 6 directions 90 -> 64)
+          for (; k + 4 <= n_dir; k += 4) {
+            Pack<V> m[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) m[q] = ld_pack<V, NT>(msg + (int64_t)(k + q) * N + i);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) fold(k + q, m[q]);
+          }
+        }
+        for (; k < n_dir; ++k) fold(k, ld_pack<V, NT>(msg + (int64_t)k * N + i));
       }
       if (min_a_dir) {
 #pragma unroll

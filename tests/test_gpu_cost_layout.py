@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("L", [1, 3, 16, 21, 32, 33, 64, 96, 128, 129, 192, 255, 256])
-@pytest.mark.parametrize("B,H,W,n_dir", [(1, 1, 1, 4), (2, 5, 7, 8), (3, 8, 16, 4), (1, 32, 33, 16), (2, 3, 43, 2), (2, 3, 43, 16)])
+@pytest.mark.parametrize("B,H,W,n_dir", [(1, 1, 1, 4), (2, 5, 7, 8), (3, 8, 16, 4), (1, 32, 33, 16), (2, 3, 43, 2), (2, 3, 43, 16), (2, 5, 7, 6), (1, 3, 43, 12)])
 def test_costs_turned_over(gpu, L, B, H, W, n_dir):
   from mplayers_amd import _lib, ops
   gen = torch.Generator(device=gpu.DEV).manual_seed(L + H)
