@@ -32,3 +32,30 @@ def test_costs_turned_over(gpu, L, B, H, W, n_dir):
       out.append((cost, msg, label))
     assert torch.equal(out[0][0].permute(0, 1, 4, 2, 3), out[1][0]), what
     assert torch.equal(out[0][1], out[1][1]) and torch.equal(out[0][2], out[1][2]), what
+
+
+@pytest.mark.parametrize("L,tile,H,W", [(3, 128, 512, 513), (21, 128, 513, 513), (32, 128, 512, 513), (32, 128, 513, 513),
+                                        (33, 64, 384, 342), (96, 64, 384, 342), (96, 64, 363, 363), (128, 64, 363, 363),
+                                        (129, 32, 211, 317), (256, 32, 192, 346)])
+@pytest.mark.parametrize("n_dir", [2, 4])
+def test_every_tile(gpu, L, tile, H, W, n_dir):
+  """Images large enough for each tile of pixels, of whole lines and of odd sizes, whose last tile is partial, and for the
+  regrouping of workgroups, with the last round of groups incomplete."""
+  from mplayers_amd import _lib, ops
+  cus = torch.cuda.get_device_properties(0).multi_processor_count
+  tiles = -(-H * W // tile)
+  assert tiles >= 2 * 4 * cus and tiles % 64 != 0 and tiles > 64
+  gen = torch.Generator(device=gpu.DEV).manual_seed(L + H)
+  unary = torch.rand(1, 1, H, W, L, generator=gen, device=gpu.DEV)
+  ew = torch.rand(n_dir, 1, 1, H, W, generator=gen, device=gpu.DEV)
+  ctx = torch.triu(torch.rand(L, L, generator=gen, device=gpu.DEV), 1) if L == 21 else \
+      0.1 * torch.arange(L, device=gpu.DEV).clamp(max=3)
+  none = torch.empty(0, dtype=torch.uint8)
+  out = []
+  for flags in (0, _lib.F_COST_LABELS_FIRST):
+    msg, scratch = torch.zeros(n_dir, 1, 1, H, W, L, device=gpu.DEV), torch.empty_like(unary)
+    cost = torch.full((1, 1, L, H, W) if flags else (1, 1, H, W, L), float("nan"), device=gpu.DEV)
+    print("case", L, H, W, n_dir, flags, flush=True)
+    ops.TRWP.forward(0.5, 1, 0, unary, ctx, ew, msg, cost, none, none, scratch, none, flags=flags)
+    out.append(cost)
+  assert torch.equal(out[0].permute(0, 1, 4, 2, 3), out[1])

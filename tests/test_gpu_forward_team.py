@@ -95,7 +95,8 @@ def test_chain_lengths_and_launches(gpu, L, table, training):
 @pytest.mark.parametrize("training", [True, False])
 def test_tables_declared_dense(gpu, L, training):
   """Four wavefronts that share the front labels: label counts at the edges of a wavefront's trips, of a lane's
-  labels and of the front labels per wavefront; chains around a block of eight pixels."""
+  labels and of the front labels per wavefront; short and long chains (around a block of pixels:
+  tests/test_gpu_dense_chains.py)."""
   from mplayers_amd import _lib
   flags = _lib.F_PACKED_OFF | _lib.F_DENSE_TABLE
   for H, W, table, negative in ((3, 1, "random", False), (8, 9, "random", True), (7, 16, "random", False),
