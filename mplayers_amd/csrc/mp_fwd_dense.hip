@@ -130,10 +130,11 @@ __device__ __forceinline__ int trip_label(const float (&val)[kTrip], const float
 }
 // The labels that trip_label has not found: of a minimum of +inf, which a share without a number reaches too and whose
 // trip it then is.  All front labels are looked at, and the last one is taken where no candidate is a number, as in
-// the other scans.
+// the other scans.  stored: uniform; the labels are kept (a chain start's beliefs are zero, also past the last label, and
+// its trips end there).
 template <int R>
 __device__ __forceinline__ void labels_without_trip(const float* a, const float* csym_s, const float w, const float (&v)[R],
-                                                    const int lab0, const int L, int (&fd_idx)[R]) {
+                                                    const bool stored, const int lab0, const int L, int (&fd_idx)[R]) {
   bool none[R], any = false;
 #pragma unroll
   for (int j = 0; j < R; ++j) {
@@ -141,7 +142,7 @@ __device__ __forceinline__ void labels_without_trip(const float* a, const float*
     any |= none[j];
     fd_idx[j] = min(fd_idx[j], L - 1);
   }
-  if (__builtin_expect(ballot(any) == 0, 1)) return;
+  if (__builtin_expect(!stored || ballot(any) == 0, 1)) return;
 #pragma unroll
   for (int j = 0; j < R; ++j) {
     const float* cp = csym_s + (dense_sym_centre<R>() + lab0 + j);
@@ -381,9 +382,9 @@ __device__ __forceinline__ void walk_chain(const SweepParams& p, const ChainCtx&
           fd_idx[j] = trip_label(val[j], v[j], f0[j]);
           pr[j] = lab0 + j < L && v[j] == nmin;
         }
-        labels_without_trip<R>(st.a[i], csym_s, w, v, lab0, L, fd_idx);
-        const int nidx = last_label<R>(pr, L - 1);
         const bool idx_on = on && t > 0;
+        labels_without_trip<R>(st.a[i], csym_s, w, v, idx_on, lab0, L, fd_idx);
+        const int nidx = last_label<R>(pr, L - 1);
         const unsigned sob = pp * (unsigned)L;
         if (R == 1 || whole) {
           buf_store_u8<R, true>(rImin, (int)((idx_on && lab0 < L) ? sob + (unsigned)lab0 : kDeadWide), 0u, fd_idx);
@@ -637,9 +638,9 @@ __device__ __forceinline__ void walk_chain_alone(const SweepParams& p, const Cha
           fd_idx[j] = trip_label(val, v[j], f0);
           pr[j] = lab0 + j < L && v[j] == nmin;
         }
-        labels_without_trip<R>(s.a[i], csym_s, w, v, lab0, L, fd_idx);
-        const int nidx = last_label<R>(pr, L - 1);
         const bool idx_on = on && t > 0;
+        labels_without_trip<R>(s.a[i], csym_s, w, v, idx_on, lab0, L, fd_idx);
+        const int nidx = last_label<R>(pr, L - 1);
         const unsigned sob = pp * (unsigned)L;
         if (R == 1 || whole) {
           buf_store_u8<R, true>(rImin, (int)((idx_on && lab0 < L) ? sob + (unsigned)lab0 : kDeadWide), 0u, fd_idx);
