@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "mp_common.h"
@@ -290,7 +291,9 @@ __global__ void __launch_bounds__(256) aggregate_first_kernel(const float* __res
   const int pixels = HW - p0 < tile ? HW - p0 : tile;
   for (int64_t b = blockIdx.y; b * HW * L < N; b += gridDim.y) {
     const int64_t first = (b * HW + p0) * L;
-    for (int e = (int)threadIdx.x * V; e < pixels * L; e += 256 * V) {
+    const int lead = V == 4 ? (int)first & 3 : 0;  // (fours of the planes, not of the tile)
+    const bool whole = V == 1 || (lead == 0 && ((pixels * L) & 3) == 0);
+    for (int e = (int)threadIdx.x * V - lead; e < pixels * L; e += 256 * V) {
       const int64_t i = first + e;
       Pack<V> v = ld_pack<V, NT>(unary + i);
 #pragma unroll
@@ -331,14 +334,20 @@ __global__ void __launch_bounds__(256) aggregate_first_kernel(const float* __res
         for (int j = 0; j < V; ++j) v.v[j] += mn.v[j];
       }
       int p = e / L, l = e - p * L;
+      const auto put = [&](const auto checked) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < V; ++j) {
-        turn[p * stride + l] = v.v[j];
-        if (++l == L) {
-          l = 0;
-          ++p;
+        for (int j = 0; j < V; ++j) {
+          if (!decltype(checked)::value || (unsigned)(e + j) < (unsigned)(pixels * L)) turn[p * stride + l] = v.v[j];
+          if (++l == L) {
+            l = 0;
+            ++p;
+          }
         }
-      }
+      };
+      if (whole)
+        put(std::false_type());
+      else
+        put(std::true_type());
     }
     __syncthreads();
     float* const out = cost + b * HW * L + p0;
@@ -1153,10 +1162,19 @@ void aggregate(const mpl_shape* s, unsigned flags, const float* unary, const flo
     MPL_EW_LAUNCH(aggregate_kernel, v4, nt, n_dir, N, st, unary, msg, n_dir, N, factor, min_a_dir, cost_final);
     return;
   }
-  // some 32 KB of LDS at most, a run of a few KB per plane; one line of the result, where that is not enough to go round
+  // Some 32 KB of LDS at most, a run of a few KB per plane; one line of the result, where that is not enough to go
+  // round, and less of it for the few tiles of a small image with many labels, whose workgroups pass over theirs again
+  // and again.  Tiles of 32 pixels -> this, us: 255 labels 23x29, 8 directions 26 -> 10, batch 4 16 -> 10; 191 labels 4x46x65,
+  // 12 directions 51 -> 30; 256 labels 60x80, 4 directions 14 -> 10; 97 labels 4x63x77, 6 directions 22 -> 16; 192 labels
+  // 100x150 15.9 -> 16.2.
+  const auto tiles = [&](int log) { return (((HW - 1) >> log) + 1) * s->batch; };
+  const int n_simd = launch_policy().n_simd;
   int tile_log = L <= 32 ? 7 : L <= 128 ? 6 : 5;
-  while (tile_log > 5 && (((HW - 1) >> tile_log) + 1) * s->batch < 2 * launch_policy().n_simd) --tile_log;
-  const bool v4 = (HW * L) % 4 == 0 && aligned16(unary) && aligned16(msg);
+  while (tile_log > 5 && tiles(tile_log) < 2 * n_simd) --tile_log;
+  while (L > 32 && tile_log > 3 && tiles(tile_log) < n_simd) --tile_log;
+  // (fours that lie across two tiles are loaded for both: 191 labels 4x46x65, 12 directions 60 -> 51 us, 21 labels
+  // 4x129x129 9.5 -> 8.8)
+  const bool v4 = N % 4 == 0 && aligned16(unary) && aligned16(msg);
   const bool lines = (HW * (int64_t)sizeof(float)) % kLineBytes == 0 && ((uintptr_t)cost_final & (kLineBytes - 1)) == 0;
   const dim3 grid((unsigned)(((HW - 1) >> tile_log) + 1), (unsigned)std::min(s->batch, 65535));
   const size_t lds = sizeof(float) * ((size_t)(L | 1) << tile_log);

@@ -59,3 +59,27 @@ def test_every_tile(gpu, L, tile, H, W, n_dir):
     ops.TRWP.forward(0.5, 1, 0, unary, ctx, ew, msg, cost, none, none, scratch, none, flags=flags)
     out.append(cost)
   assert torch.equal(out[0].permute(0, 1, 4, 2, 3), out[1])
+
+
+@pytest.mark.parametrize("L,H,W", [(1, 33, 35), (2, 33, 35), (3, 21, 23), (5, 9, 7), (21, 65, 65), (33, 9, 11), (97, 63, 77),
+                                   (191, 46, 65), (255, 23, 29)])
+@pytest.mark.parametrize("B,n_dir", [(4, 4), (4, 6), (2, 8), (1, 4)])
+def test_fours_across_tiles_and_images(gpu, L, H, W, B, n_dir):
+  """Images of a number of elements that four does not divide, in batches that make the planes whole fours, with tiles of
+  32, 16 and 8 pixels: fours that begin before the tile, or end after it."""
+  from mplayers_amd import _lib, ops
+  gen = torch.Generator(device=gpu.DEV).manual_seed(L + B)
+  unary = torch.rand(B, 1, H, W, L, generator=gen, device=gpu.DEV)
+  ew = torch.rand(n_dir, B, 1, H, W, generator=gen, device=gpu.DEV)
+  ctx = torch.triu(torch.rand(L, L, generator=gen, device=gpu.DEV), 1) if L == 21 else \
+      0.1 * torch.arange(L, device=gpu.DEV).clamp(max=3)
+  none = torch.empty(0, dtype=torch.uint8)
+  for min_a_dir in (0, 1):
+    out = []
+    for flags in (0, _lib.F_COST_LABELS_FIRST):
+      msg, scratch = torch.zeros(n_dir, B, 1, H, W, L, device=gpu.DEV), torch.empty_like(unary)
+      cost = torch.full((B, 1, L, H, W) if flags else (B, 1, H, W, L), float("nan"), device=gpu.DEV)
+      print("case", L, H, W, B, n_dir, min_a_dir, flags, flush=True)
+      ops.TRWP.forward(0.5, 1, min_a_dir, unary, ctx, ew, msg, cost, none, none, scratch, none, flags=flags)
+      out.append(cost)
+    assert torch.equal(out[0].permute(0, 1, 4, 2, 3), out[1])
