@@ -1075,7 +1075,11 @@ void launch_team21_bwd(const BackParams& p, hipStream_t st) {
                            : bwd_team21_kernel<false, false, SOFT, N>,                                           \
          N, sizeof(BwdSlots<2 * N>))
   const int cus = launch_policy().n_simd / 4;
-  if (p.edge_label == nullptr && p.dctx != nullptr && blocks <= 2 * cus)
+  // (dynamic LDS beyond 64 KB would have to be asked for)
+  constexpr size_t kManyLds = 2 * sizeof(BwdSlots<2 * kManyHelpers>) + sizeof(float) * (kMaxL + 2 * kPairs);
+  static_assert(kManyLds <= (64 << 10), "LDS of the reverse scans with many helpers");
+  constexpr int kManyPerCu = (160 << 10) / ((kManyLds + 1279) / 1280 * 1280);  // (given out in 1280 bytes)
+  if (p.edge_label == nullptr && p.dctx != nullptr && blocks <= kManyPerCu * cus)
     launch(bwd_team21_kernel<true, true, false, kManyHelpers>, kManyHelpers, sizeof(BwdSlots<2 * kManyHelpers>));
   else if (p.edge_label == nullptr)
     MPL_BWD21(false, kHelpers);
