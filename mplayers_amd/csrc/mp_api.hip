@@ -1146,8 +1146,8 @@ void fold_dcontext(const BackParams& p, float* dcontext, hipStream_t st) {
 // 16 directions, labels first: the loads of all planes go out together, but of four floats each only up to this much of
 // messages.  Measured, us, one plane after another / together: 96 labels 150x200 30.8 / 30.5, 240x320 92 / 77, 300x400
 // 123 / 122, 64 labels 480x640 (1.2 GiB) 241 / 237, 96 labels 384x800 (1.8 GiB) 348 / 385, 384x1248 516 / 596, 190 labels
-// 375x450 (1.9 GiB) 420 / 432.  Single floats: 21 labels 65x65 14.9 / 4.0, 4x129x129 33 / 16, 97 labels 241x321
-// 213 / 99, 383x1247 1167 / 752.
+// 375x450 (1.9 GiB) 420 / 432.  Single floats: 21 labels 65x65 14.9 / 4.0, 97 labels 241x321 213 / 99, 383x1247
+// 1167 / 752.
 constexpr int64_t kFirst16Bytes = (int64_t)5 << 28;
 
 // cost_final from the unary terms and the messages, in either layout.

@@ -15,8 +15,8 @@
 //     while a block is scanned they finish the one before and prepare the one after it.  They issue where the
 //     scanners wait for LDS and for each other, some half of the time.
 // Measured, argmin labels kept / not, rows of 257 on 256 chains, ns per pixel, every wavefront serving two pixels of a
-// block it has scanned -> this: 64 labels 443 / 385 -> 320 / 308, 96 labels 697 / 608 -> 452 / 441, 128 labels 811 / 652 ->
-// 519 / 506; 192 labels, rows of 129, 1290 / 973 -> 891 / 845.  A third of that is that what follows the barrier reads
+// block it has scanned -> this: 64 labels 443 / 385 -> 323 / 312, 96 labels 697 / 608 -> 453 / 445, 128 labels 811 / 652 ->
+// 522 / 509; 192 labels, rows of 129, 1290 / 973 -> 891 / 845.  A third of that is that what follows the barrier reads
 // everything it needs before it waits for any of it.
 // The argmin labels take two steps, as in dense1d_step: the scan notes the trip (eight front labels) whose
 // candidates last reached the running minimum; the servers evaluate that one trip again.
@@ -102,7 +102,7 @@ __device__ __forceinline__ void get_words(const float* src, float (&x)[R]) {
 // +inf that the compiler cannot see through: what starts from it is +inf where no candidate is a number (a candidate
 // that is none drops out of a minimum; left to itself the compiler leaves out a minimum with +inf), so a share without
 // a number says nothing about the labels or their least one.  Argmin labels kept, rows of 257 on 256 chains, with what
-// finds the labels of such pixels, over neither: 17 to 64 labels 1.01 to 1.02, 96 and 128 labels 1.00 to 1.01, 192 labels 1.00.
+// finds the labels of such pixels, over neither: 17 to 64 labels 1.01 to 1.025, 96 and 128 labels 1.00 to 1.01, 192 labels 1.00.
 __device__ __forceinline__ float opaque_inf() {
   float x = INFINITY;
   asm volatile("" : "+s"(x));
