@@ -810,7 +810,7 @@ void launch_vj(const BackParams& p, hipStream_t st) {
   const bool gr = p.dedge != nullptr || p.dctx != nullptr;
   const auto launch = [&](auto kernel, int helpers, int turn_every, size_t extra = 0) {
     const size_t lds = team_lds_bytes<R>(p.L, gr, helpers) + extra;
-    if (lds > (64 << 10))
+    if (lds > (64 << 10))  // (a refusal shows as the launch's, and is reported with it)
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     kernel<<<blocks, (helpers + 1) * kWave, lds, st>>>(p, turn_every);
   };
